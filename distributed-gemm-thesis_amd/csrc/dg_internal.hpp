@@ -88,13 +88,14 @@ struct Prob {
     int64_t ldc;
     double alpha, beta;
     int32_t seg0, nseg;    // segment range in the segment table
-    int32_t tile0[2];      // first global tile id of this problem, per tile shape
-    int32_t tiles_m[2], tiles_n[2];
+    int32_t tile0;         // first tile id of this problem in its list
     // direct-to-LDS kernel: bit 0 (bit 1) set when the row-contiguous A (B)
     // starts 8 bytes past a 16-byte boundary; its loads then start one row
-    // earlier and the tile grid runs over rows + 1
+    // earlier and the tile grid runs over rows + 1; register-staged kernel:
+    // kByElements or 0
     int32_t shift;
 };
+constexpr int32_t kByElements = 4;  // load single elements instead of pairs
 
 // Division of 32-bit unsigned integers by a launch constant d >= 1 with
 // one high multiply, a subtract, an add and two shifts (Granlund and
@@ -128,12 +129,13 @@ enum {
     DG_GEMM_MODE_PERSISTENT = 2,   // CU-count workgroups pull tiles from an atomic counter
 };
 
-// Output tile shapes of the FP64 GEMM.
+// Output tiles of an FP64 GEMM batch.
 enum {
-    DG_GEMM_TILE_128x128 = 0,  // 4 waves, two workgroups per CU
-    DG_GEMM_TILE_256x128 = 1,  // 8 waves, one workgroup per CU
-    DG_GEMM_TILE_128x128W8 = 2,  // 8 waves of 64x32, two workgroups per CU
-    DG_GEMM_TILE_DEFAULT = DG_GEMM_TILE_128x128,
+    DG_GEMM_TILE_AUTO = -1,    // the one whose estimated time is least
+    DG_GEMM_TILE_128x128 = 0,  // direct-to-LDS kernels where they apply, 64x64 register-staged elsewhere
+    DG_GEMM_TILE_64x64 = 1,    // register-staged kernel
+    DG_GEMM_TILE_32x32 = 2,    // register-staged kernel
+    DG_GEMM_TILES = 3,
 };
 
 // Launches the FP64 MFMA GEMM over `probs` (host vector; uploaded through
@@ -141,64 +143,62 @@ enum {
 int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs,
                     const std::vector<Seg>& segs, hipStream_t stream, int mode);
 
-// A batch split by kernel.  Each problem is routed on its own properties,
-// so it sums in the same order alone or inside any batch: the direct-to-LDS
-// kernel takes it when every segment has K > 0 and even leading dimensions,
-// its k-contiguous operand (A with opA = T, B with opB = N) has 16-byte
-// aligned bases and even K, and its row-contiguous operand (A with opA = N,
-// B with opB = T) has 8-byte aligned bases with the same offset within 16
-// bytes in every segment; the register-staged kernel takes the others.
-// DG_GEMM_NO_DMA routes everything to the register-staged kernel.
+// A batch split by kernel.  With DG_GEMM_TILE_128x128, the direct-to-LDS
+// kernels take a problem when every segment has K > 0 and even leading
+// dimensions, its k-contiguous operand (A with opA = T, B with opB = N) has
+// 16-byte aligned bases and even K, and its row-contiguous operand (A with
+// opA = N, B with opB = T) has 8-byte aligned bases with the same offset
+// within 16 bytes in every segment; the register-staged kernel takes the
+// others, and all of them with the other tiles.  DG_GEMM_TILE_AUTO estimates
+// each choice's time from its tiles and takes the least: 128x128 tiles keep
+// the matrix cores busiest but leave CUs idle until there are a few hundred
+// of them (DG_GEMM_TILE forces a choice, DG_GEMM_NO_DMA routes everything to
+// the register-staged kernel).  Every kernel and tile sums an element in the
+// same order, so a problem gives the same bits alone, in any batch and on any
+// tile.
 // Direct-to-LDS problems whose tiles are all interior (no row shift, m and n
 // multiples of 128, whole k-steps, an even step count) go to `dma`, which
 // the A-in-registers kernel runs; the others go to `dmae` (the edge-handling
 // kernel).  With split_edges, a direct-to-LDS problem with edges and at
 // least 8 interior tiles is cut into sub-problems: an interior block on
-// `dma`, and strips on `dmae` around it, placed so that the tile count does
-// not grow (a row-shifted problem's interior starts at its row 127).  The
-// sub-problems' segments are appended to `segs` (which starts as a copy of
-// the input segments); every element still sums in the same order.  The
-// strips past the interior that are narrower than a tile go instead to
-// `nar[0]` (columns past it, 128x32 tiles) and `nar[1]` (rows past it, 64x128
-// tiles), which the register-staged kernel runs in the same k order
-// (DG_GEMM_NO_NARROW keeps them on `dmae`).
+// `dma` (a row-shifted problem's interior starts at its row 127), and strips
+// around it on the register-staged kernel (on `dmae` under
+// DG_GEMM_NO_NARROW).  The sub-problems' segments are appended to `segs`
+// (which starts as a copy of the input segments).
+// Register-staged problems and strips go to gen[0] (64x64 tiles), or gen[1]
+// (32x32) when 32x32 is the choice or they are at most 32 rows or columns.
 struct GemmBatch {
-    std::vector<Prob> dma, dmae, gen;  // tile ranges assigned per list
-    int tiles_dma = 0;                 // 128x128 tiles of `dma`
-    int tiles_dmae = 0;                // 128x128 tiles of `dmae`
-    int tiles_gen[2] = {0, 0};         // tiles of `gen` per tile shape
-    bool vec = true;                   // every `gen` segment allows 128-bit loads
-    std::vector<Prob> nar[2];          // narrow strips: 128x32 tiles, 64x128 tiles
-    int tiles_nar[2] = {0, 0};
-    bool vec_nar[2] = {true, true};
-    std::vector<Seg> segs;             // the segment table all lists index
+    std::vector<Prob> dma, dmae, gen[2];  // tile ranges assigned per list
+    int tiles_dma = 0, tiles_dmae = 0, tiles_gen[2] = {0, 0};
+    std::vector<Seg> segs;                // the segment table all lists index
+    bool empty() const { return dma.empty() && dmae.empty() && gen[0].empty() && gen[1].empty(); }
 };
-int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs_in, const std::vector<Seg>& segs,
-                 GemmBatch& out, bool split_edges = true);
+int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, const std::vector<Seg>& segs, GemmBatch& out,
+                 bool split_edges = true, int tile = DG_GEMM_TILE_AUTO);
 
 // The same batch with its tables resident on the device.
 struct GemmBatchDev {
-    const Prob* dma = nullptr;
-    int ndma = 0, tiles_dma = 0;
-    const Prob* dmae = nullptr;
-    int ndmae = 0, tiles_dmae = 0;
-    const Prob* gen = nullptr;
-    int ngen = 0, tiles_gen[2] = {0, 0};
-    bool vec = true;
-    const Prob* nar[2] = {nullptr, nullptr};
-    int nnar[2] = {0, 0}, tiles_nar[2] = {0, 0};
-    bool vec_nar[2] = {true, true};
+    const Prob *dma = nullptr, *dmae = nullptr, *gen[2] = {nullptr, nullptr};
+    int ndma = 0, ndmae = 0, ngen[2] = {0, 0};
+    int tiles_dma = 0, tiles_dmae = 0, tiles_gen[2] = {0, 0};
     const Seg* segs = nullptr;
+    void set_counts(const GemmBatch& h) {
+        ndma = (int)h.dma.size();
+        ndmae = (int)h.dmae.size();
+        tiles_dma = h.tiles_dma;
+        tiles_dmae = h.tiles_dmae;
+        for (int w = 0; w < 2; ++w) {
+            ngen[w] = (int)h.gen[w].size();
+            tiles_gen[w] = h.tiles_gen[w];
+        }
+    }
 };
 // Device half.  The persistent mode needs a device int `counter`, which it
 // zeroes with a kernel before each launch (graph safe).  `dma` runs the
 // A-in-registers kernel (the lean direct-to-LDS kernel under
 // DG_GEMM_NO_AREG), `dmae` the edge-handling direct-to-LDS kernel, `gen` the
-// register-staged kernel of tile shape cfg; one launch per non-empty list.
-int launch_gemm_f64_dev(char opA, char opB, int mode, int cfg, const GemmBatchDev& b, int* counter,
-                        hipStream_t stream);
-// Tile shape used by the one-shot entry points (DG_GEMM_TILE env override).
-int default_tile_cfg();
+// register-staged kernel; one launch per non-empty list.
+int launch_gemm_f64_dev(char opA, char opB, int mode, const GemmBatchDev& b, int* counter, hipStream_t stream);
 
 // C[x] = beta*C[x] over an m x n column-major matrix (beta == 0 writes 0).
 int launch_scale(int64_t m, int64_t n, double beta, double* C, int64_t ldc, hipStream_t stream);

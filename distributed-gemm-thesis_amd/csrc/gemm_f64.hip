@@ -9,23 +9,28 @@
 // would have brought in; a SUMMA rank is one problem whose segments are the
 // owners' panels.
 //
-// Three kernels share the problem/segment tables and the tile order.  Batches
-// whose tiles are all interior run gemm_f64_dma_ar_kernel (A straight into
-// registers, B direct to LDS); the others that take direct loads run
-// gemm_f64_dma_kernel (both operands direct to LDS); both are described below.  The rest run gemm_f64_kernel:
-// Tiling (256 threads = 4 waves of 64 lanes):
-//   block tile 128 x 128, k-step 16, LDS double buffered (2 blocks per CU);
-//   each wave owns a 64 x 64 sub-tile = 4 x 4 MFMA tiles of 16 x 16.
-// LDS holds both operands k-contiguous, [row][k] with a padded stride of 18
-// doubles (144 B), so a lane reads its 4 consecutive k values with two
-// 128-bit LDS reads and 16 lanes of one read touch 64 distinct banks.
-// Lane l of an MFMA supplies k = 4*(l/16) + kk for sub-step kk; A and B use
-// the same k assignment, so the product is exact whatever k order the
-// matrix core sums in.
+// Three kernels share the problem/segment tables and the tile order: problems
+// whose 128x128 tiles are all interior run gemm_f64_dma_ar_kernel (A straight
+// into registers, B direct to LDS); the others that take direct loads run
+// gemm_f64_dma_kernel (both operands direct to LDS); both are described below.
+// gemm_f64_kernel takes everything else on 64x64 or 32x32 tiles: operands that
+// direct loads do not take (odd leading dimensions, odd K), strips cut off
+// uneven problems, and batches too small to fill the chip with 128x128 tiles
+// (prepare_gemm chooses).  It stages both operands through registers into a
+// double-buffered LDS; four waves a workgroup, each owning a quarter of the
+// tile.
+// What bounds it: the FP64 MFMA (64 cycles each, on the vector ALU's pipes).
+// Measured (TFLOP/s, against the 128x128 tiles and guarded loads before):
+// 512^3 3.8 -> 28.9 (32x32 tiles; 70 -> 9.3 us), 1024^3 16.6 -> 50.4, 2000^3
+// 32.8 -> 65.9, 3072^3 55.3 -> 70.9, 4097^3 (odd leading dimensions) 48.6 ->
+// 64.4, TN 1500 x 1333 x 2001 22.7 -> 61.8.
+// Lane l of an MFMA supplies k = 2*(l/16) + q to sub-step q for both operands,
+// so the product is exact whatever k order the matrix core sums in.
 // The MFMA is issued as D = B^T A^T, so each output register holds 16
 // consecutive rows of one C column: the epilogue stores are 128-byte runs.
 // Result layout of v_mfma_f64_16x16x4_f64: lane l, register v holds
 // D(l/16 + 4v, l%16) (checked on the device by the exact-integer tests).
+#include <algorithm>
 #include <string>
 
 #include "dg_internal.hpp"
@@ -44,32 +49,29 @@ typedef __attribute__((address_space(1))) const double gdouble;
 typedef __attribute__((address_space(1))) const dv2 gdv2;
 __device__ __forceinline__ double gld(const double* p) { return *(gdouble*)p; }
 __device__ __forceinline__ dv2 gld2(const double* p) { return *(gdv2*)p; }
+// a pair at any element alignment: one 16-byte load all the same
+typedef dv2 dv2u __attribute__((aligned(8)));
+typedef __attribute__((address_space(1))) const dv2u gdv2u;
+__device__ __forceinline__ dv2 gld2u(const double* p) { return *(gdv2u*)p; }
 
-constexpr int BK = 16;
-constexpr int LDK = BK + 2;  // padded LDS row stride (doubles)
 constexpr int GROUP_M = 8;   // tile rows per raster group
 
-// Tile shapes: BM x BN output tiles computed by NTH threads, each wave owning
-// a WM x WN sub-tile (WM/16 x WN/16 MFMA tiles of 16 x 16); OCC workgroups
-// per CU.
-template <int BM_, int BN_, int NTH_, int OCC_, int WM_ = 64, int WN_ = 64>
+// Shapes of the register-staged kernel: BM x BN output tiles of four waves,
+// each owning a WM x WN sub-tile (WM/16 x WN/16 MFMA tiles of 16 x 16);
+// BK-deep k-stages (a multiple of 8), D of them in flight in registers; OCC
+// workgroups per CU.
+template <int BM_, int BN_, int WM_, int WN_, int BK_, int D_, int OCC_>
 struct TileCfg {
-    static constexpr int BM = BM_, BN = BN_, NTH = NTH_, OCC = OCC_, WM = WM_, WN = WN_;
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, BK = BK_, D = D_, OCC = OCC_;
+    static constexpr int NTH = 256;
     static constexpr int WAVES_N = BN / WN;
     static constexpr int FM = WM / 16, FN = WN / 16;
-    static constexpr int PA = BM * BK / (2 * NTH);  // 128-bit loads per thread per k-step (A)
-    static constexpr int PB = BN * BK / (2 * NTH);  // (B)
     static_assert((BM / WM) * (BN / WN) * 64 == NTH, "one wave per WM x WN sub-tile");
 };
-using Cfg128 = TileCfg<128, 128, 256, 2>;  // 73.7 KB LDS, two workgroups per CU
-using Cfg256 = TileCfg<256, 128, 512, 1>;  // 110.6 KB LDS, 8 waves, half the B traffic per flop
-using Cfg128w8 = TileCfg<128, 128, 512, 2, 64, 32>;  // 8 waves of 64 x 32: four waves per SIMD
-// Strips narrower than a 128x128 tile, cut off uneven direct-to-LDS problems:
-// columns past the interior (fewer than 128) and rows past it.
-using CfgN32 = TileCfg<128, 32, 256, 2, 32, 32>;  // 4 waves of 32 x 32 stacked in M
-using CfgM64 = TileCfg<64, 128, 256, 2, 32, 64>;  // 2 x 2 waves of 32 x 64 (2 ms per step faster than
-                                                  // 32 x 128 tiles on the 20000 batch's 41-row strips)
-constexpr int64_t kNarrowMax = 64;  // widest strip (rows or columns) put on narrow tiles
+using Cfg64 = TileCfg<64, 64, 32, 32, 16, 2, 4>;
+using Cfg32 = TileCfg<32, 32, 16, 16, 32, 2, 3>;
+constexpr int64_t kMaxPairLd = (1 << 22) - 64;  // 8 * (127 ld + BK) stays below 2^32
+constexpr int64_t kNarrowMax = 32;  // problems and strips up to this many rows or columns wide take the 32 x 32 tiles
 
 // Block id -> tile id so that each XCD (blocks are dealt round-robin to the
 // 8 XCDs) receives one contiguous range of tiles, which the grouped raster
@@ -81,143 +83,137 @@ __device__ __forceinline__ int xcd_remap(int bid, int total) {
     return x * q + min(x, r) + slot;
 }
 
-// Loads one k-step of an operand stored "k-contiguous" (element (row, k) at
-// base[k + row*ld]) into registers: ROWS rows x 16 k; thread t takes k pair
-// 2*(t%8) of rows t/8 + (NTH/8)*q.
-template <int ROWS, int NTH, bool EDGE, bool VEC>
-__device__ __forceinline__ void load_kc(dv2 (&r)[ROWS * BK / (2 * NTH)], const double* __restrict__ base, int64_t ld,
-                                        int64_t row0, int64_t rows, int64_t k0, int64_t klen) {
-    const int t = threadIdx.x;
-    const int kp = (t & 7) * 2;
-    const int rr = t >> 3;
+// One operand of the register-staged kernel: BK-deep stages of ROWS rows,
+// loaded in 16-byte pairs at whatever alignment the matrix has (the hardware
+// takes unaligned global loads; a pair per load instead of two elements is
+// what lets odd leading dimensions run like even ones), stored to LDS in the
+// direction memory has so that both the store and the fragment reads are
+// conflict-free runs.
+//  * KC, element (row, k) at base[k + row*ld]: a thread takes the k pair
+//    kt = 2*(t % CH) of rows t/CH + RPP*q; LDS [row][k], rows padded by one
+//    pair.
+//  * else, element (row, k) at base[row + k*ld]: a thread takes the row pair
+//    2*(t % HP) of k kt + KPP*q, kt = t/HP; LDS [k][row], k-rows padded by 64
+//    bytes.
+// Rows past the end are read from the last row; they feed only outputs that
+// are never stored.  A segment's last stage is read by elements (read_last),
+// with k past the end turned into zeros; in the stages before it every pair
+// is inside the matrix: a pair that starts at the last row ends at the next
+// k's first row or in the columns' padding.
+// An FP64 MFMA runs on the vector ALU's own pipes, so every vector
+// instruction of the loop is time taken from the product (1.4 to 3.7 of them
+// per MFMA cost a fifth of the rate): a whole stage uses none but the memory
+// instructions, with a scalar base that moves and 32-bit lane offsets that
+// stay.  The compiler counts loads in flight only along straight code, so
+// whole stages also have no branch around their loads (with one it waited
+// for all of them every stage).
+template <bool KC, int ROWS, int BK>
+struct Staged {
+    static constexpr int CH = BK / 2, RPP = 256 / CH;          // KC
+    static constexpr int HP = ROWS / 2, KPP = 256 / HP;        // else
+    static constexpr int NL = ROWS * BK / 512;                 // loads per thread and stage
+    static constexpr int LROW = KC ? (BK + 2) * 8 : ROWS * 8 + 64;  // bytes
+    static constexpr int BYTES = KC ? ROWS * LROW : BK * LROW;
+
+    const double* base;   // the tile's first row at the next stage's first k (uniform)
+    int64_t ld;
+    uint32_t off[NL];     // bytes from it to this thread's pairs
+
+    // row of this thread's pair q within the tile, k of it within the stage
+    static __device__ __forceinline__ int row(int q) { return KC ? (int)threadIdx.x / CH + RPP * q : 2 * ((int)threadIdx.x % HP); }
+    static __device__ __forceinline__ int kk(int q) { return KC ? 2 * ((int)threadIdx.x % CH) : (int)threadIdx.x / HP + KPP * q; }
+
+    // At a segment's first k; the tile has `rows` rows from row0 on.
+    __device__ __forceinline__ void start(const double* x, int64_t ld_, int64_t row0, int rows) {
+        ld = ld_;
+        base = x + row0 * (KC ? ld : 1);
 #pragma unroll
-    for (int q = 0; q < ROWS * BK / (2 * NTH); ++q) {
-        int64_t row = row0 + rr + (NTH / 8) * q;
-        int64_t k = k0 + kp;
-        if (!EDGE) {
-            const double* p = base + k + row * ld;
-            if (VEC) {
-                r[q] = gld2(p);
-            } else {
-                r[q].x = gld(p);
-                r[q].y = gld(p + 1);
-            }
-        } else {
-            row = row < rows ? row : rows - 1;  // clamped rows feed outputs that are never stored
-            const double* p = base + row * ld;
-            r[q].x = (k < klen) ? gld(p + k) : 0.0;
-            r[q].y = (k + 1 < klen) ? gld(p + k + 1) : 0.0;
+        for (int q = 0; q < NL; ++q) {
+            const uint32_t r = min(row(q), rows - 1), k = kk(q);
+            off[q] = 8u * (KC ? r * (uint32_t)ld + k : k * (uint32_t)ld + r);
         }
     }
-}
-
-// Loads one k-step of an operand stored "row-contiguous" (element (row, k)
-// at base[row + k*ld]): thread t takes rows 2*(t%(ROWS/2)), +1 of k column
-// t/(ROWS/2) + (NTH/(ROWS/2))*q.
-template <int ROWS, int NTH, bool EDGE, bool VEC>
-__device__ __forceinline__ void load_rc(dv2 (&r)[ROWS * BK / (2 * NTH)], const double* __restrict__ base, int64_t ld,
-                                        int64_t row0, int64_t rows, int64_t k0, int64_t klen) {
-    constexpr int HP = ROWS / 2;
-    const int t = threadIdx.x;
-    const int rp = (t % HP) * 2;
-    const int kc = t / HP;
+    __device__ __forceinline__ void advance() {
+        base += KC ? BK : BK * ld;
+        asm volatile("" : "+s"(base));  // stays a scalar: not folded into vector address increments
+    }
+    __device__ __forceinline__ void read(dv2 (&v)[NL]) {
 #pragma unroll
-    for (int q = 0; q < ROWS * BK / (2 * NTH); ++q) {
-        int64_t row = row0 + rp;
-        int64_t k = k0 + kc + (NTH / HP) * q;
-        if (!EDGE) {
-            const double* p = base + row + k * ld;
-            if (VEC) {
-                r[q] = gld2(p);
+        for (int q = 0; q < NL; ++q) {
+            asm volatile("" : "+v"(off[q]));  // stays 32 bits: the load adds it to the scalar base itself
+            v[q] = gld2u((const double*)((const char*)base + off[q]));
+        }
+        advance();
+    }
+    // The segment's last stage, `left` <= BK of its k real (or any stage of a
+    // matrix that read() does not take).
+    __device__ __forceinline__ void read_last(dv2 (&v)[NL], int left, int rows) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const int r = min(row(q), rows - 1), k = min(kk(q), left - 1);
+            const double* x = base + (KC ? r * ld + k : k * ld + r);
+            v[q] = dv2{gld(x), gld(x + (KC ? k + 1 < left : r + 1 < rows))};
+        }
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const int k = kk(q);
+            v[q] = dv2{k < left ? v[q].x : 0.0, (KC ? k + 1 : k) < left ? v[q].y : 0.0};
+        }
+        advance();
+    }
+    static __device__ __forceinline__ void store(char* s, const dv2 (&v)[NL]) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+            *reinterpret_cast<dv2*>(s + (KC ? row(q) * LROW + kk(q) * 8 : kk(q) * LROW + row(q) * 8)) = v[q];
+    }
+    // f[i][q] = X(row w0 + 16i + lr, k = 8h + 2lg + q)
+    template <int F>
+    static __device__ __forceinline__ void fragments(double (&f)[F][2], const char* s, int w0, int lr, int lg, int h) {
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+            if constexpr (KC) {
+                const dv2 v = *reinterpret_cast<const dv2*>(s + (w0 + 16 * i + lr) * LROW + (8 * h + 2 * lg) * 8);
+                f[i][0] = v.x;
+                f[i][1] = v.y;
             } else {
-                r[q].x = gld(p);
-                r[q].y = gld(p + 1);
-            }
-        } else {
-            if (k < klen) {
-                const double* p = base + k * ld;
-                int64_t ra = row < rows ? row : rows - 1;
-                int64_t rb = row + 1 < rows ? row + 1 : rows - 1;
-                r[q].x = gld(p + ra);
-                r[q].y = gld(p + rb);
-            } else {
-                r[q].x = 0.0;
-                r[q].y = 0.0;
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+                    f[i][q] = *reinterpret_cast<const double*>(s + (8 * h + 2 * lg + q) * LROW + (w0 + 16 * i + lr) * 8);
             }
         }
     }
-}
+};
 
-template <int ROWS, int NTH>
-__device__ __forceinline__ void store_kc(double* __restrict__ s, const dv2 (&r)[ROWS * BK / (2 * NTH)]) {
-    const int t = threadIdx.x;
-    const int kp = (t & 7) * 2;
-    const int rr = t >> 3;
-#pragma unroll
-    for (int q = 0; q < ROWS * BK / (2 * NTH); ++q) *reinterpret_cast<dv2*>(&s[(rr + (NTH / 8) * q) * LDK + kp]) = r[q];
-}
+template <class C, bool TA, bool TB>
+struct TileLds {
+    using OA = Staged<TA, C::BM, C::BK>;    // op(A) is k-contiguous when A is transposed
+    using OB = Staged<!TB, C::BN, C::BK>;   // op(B) when B is not
+    static constexpr int STAGE = OA::BYTES + OB::BYTES;
+};
 
-template <int ROWS, int NTH>
-__device__ __forceinline__ void store_rc(double* __restrict__ s, const dv2 (&r)[ROWS * BK / (2 * NTH)]) {
-    constexpr int HP = ROWS / 2;
-    const int t = threadIdx.x;
-    const int rp = (t % HP) * 2;
-    const int kc = t / HP;
-#pragma unroll
-    for (int q = 0; q < ROWS * BK / (2 * NTH); ++q) {
-        s[rp * LDK + kc + (NTH / HP) * q] = r[q].x;
-        s[(rp + 1) * LDK + kc + (NTH / HP) * q] = r[q].y;
-    }
-}
+// Computes one output tile of problem P.  Two LDS buffers, one barrier per
+// stage: while stage s is multiplied, stages s+1 .. s+D are in flight to
+// registers; s+1 is stored to the other buffer and s+1+D requested before the
+// stage's last MFMAs.
+template <class C, bool TA, bool TB>
+__device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__ segs, int local, char* lds) {
+    constexpr int BM = C::BM, BN = C::BN, BK = C::BK, D = C::D;
+    using L = TileLds<C, TA, TB>;
+    using OA = typename L::OA;
+    using OB = typename L::OB;
 
-// op(A) is k-contiguous in memory when A is transposed; op(B) when B is not.
-template <class C, bool TA, bool EDGE, bool VEC>
-__device__ __forceinline__ void load_a(dv2 (&r)[C::PA], const Seg& s, int64_t m0, int64_t M, int64_t k0) {
-    if (TA) load_kc<C::BM, C::NTH, EDGE, VEC>(r, s.a, s.lda, m0, M, k0, s.klen);
-    else    load_rc<C::BM, C::NTH, EDGE, VEC>(r, s.a, s.lda, m0, M, k0, s.klen);
-}
-template <class C, bool TB, bool EDGE, bool VEC>
-__device__ __forceinline__ void load_b(dv2 (&r)[C::PB], const Seg& s, int64_t n0, int64_t N, int64_t k0) {
-    if (TB) load_rc<C::BN, C::NTH, EDGE, VEC>(r, s.b, s.ldb, n0, N, k0, s.klen);
-    else    load_kc<C::BN, C::NTH, EDGE, VEC>(r, s.b, s.ldb, n0, N, k0, s.klen);
-}
-template <class C, bool TA>
-__device__ __forceinline__ void store_a(double* s, const dv2 (&r)[C::PA]) {
-    if (TA) store_kc<C::BM, C::NTH>(s, r); else store_rc<C::BM, C::NTH>(s, r);
-}
-template <class C, bool TB>
-__device__ __forceinline__ void store_b(double* s, const dv2 (&r)[C::PB]) {
-    if (TB) store_rc<C::BN, C::NTH>(s, r); else store_kc<C::BN, C::NTH>(s, r);
-}
-
-// Computes one output tile of the grouped problem set.
-template <class C, bool TA, bool TB, bool VEC>
-__device__ __forceinline__ void gemm_tile(const Prob* __restrict__ probs, int nprob, const Seg* __restrict__ segs,
-                                          int tile, double (&As)[2][C::BM * LDK], double (&Bs)[2][C::BN * LDK]) {
-    constexpr int BM = C::BM, BN = C::BN;
-    constexpr int ci = BM == 256 ? 1 : 0;  // which tile range of the problem table
-
-    // Problem owning this tile: last problem with tile0 <= tile.
-    int lo = 0, hi = nprob - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (probs[mid].tile0[ci] <= tile) lo = mid; else hi = mid - 1;
-    }
-    const Prob P = probs[lo];
-    const int local = tile - P.tile0[ci];
-
+    const int tiles_m = (int)((P.m + BM - 1) / BM), tiles_n = (int)((P.n + BN - 1) / BN);
     // Grouped raster: GROUP_M tile rows sweep the tile columns together.
-    const int per_group = GROUP_M * P.tiles_n[ci];
+    const int per_group = GROUP_M * tiles_n;
     const int group = local / per_group;
     const int first_m = group * GROUP_M;
-    const int gsize = min(P.tiles_m[ci] - first_m, GROUP_M);
+    const int gsize = min(tiles_m - first_m, GROUP_M);
     const int in_group = local - group * per_group;
     const int tm = first_m + in_group % gsize;
     const int tn = in_group / gsize;
 
     const int64_t m0 = (int64_t)tm * BM;
     const int64_t n0 = (int64_t)tn * BN;
-    const bool interior = (m0 + BM <= P.m) && (n0 + BN <= P.n);
 
     const int lane = threadIdx.x & 63;
     const int wave = threadIdx.x >> 6;
@@ -233,102 +229,158 @@ __device__ __forceinline__ void gemm_tile(const Prob* __restrict__ probs, int np
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = dv4{0.0, 0.0, 0.0, 0.0};
 
-    int s = P.seg0;
-    const int s_end = P.seg0 + P.nseg;
-    Seg cur = segs[s];
-    int64_t kk = 0;
+    // load cursor over the problem's segments, one stage at a time
+    const int rows = (int)min(P.m - m0, (int64_t)BM), cols = (int)min(P.n - n0, (int64_t)BN);
+    const bool pairs = !(P.shift & kByElements);
+    int sg = P.seg0;
+    const int sg_last = P.seg0 + P.nseg - 1;
+    int64_t left;  // k of the segment from the next stage on (0 or less: past the last segment)
+    OA oa;
+    OB ob;
+    auto enter = [&]() {
+        const Seg cur = segs[sg];
+        left = cur.klen;
+        oa.start(cur.a, cur.lda, m0, rows);
+        ob.start(cur.b, cur.ldb, n0, cols);
+    };
+    dv2 va[D][OA::NL], vb[D][OB::NL];
+    auto read = [&](int d) {
+        if (left <= 0) return;
+        if (pairs && left > BK) {
+            oa.read(va[d]);
+            ob.read(vb[d]);
+        } else {
+            const int real = (int)min(left, (int64_t)BK);
+            oa.read_last(va[d], real, rows);
+            ob.read_last(vb[d], real, cols);
+        }
+        left -= BK;
+        if (left <= 0 && sg < sg_last) {
+            ++sg;
+            enter();
+        }
+    };
+    auto store = [&](char* buf, int d) {
+        OA::store(buf, va[d]);
+        OB::store(buf + OA::BYTES, vb[d]);
+    };
+    int64_t ns = 0;
+    for (int x = P.seg0; x <= sg_last; ++x) ns += (segs[x].klen + BK - 1) / BK;
 
-    dv2 ra[C::PA], rb[C::PB];
-    if (interior && BK <= cur.klen) {
-        load_a<C, TA, false, VEC>(ra, cur, m0, P.m, 0);
-        load_b<C, TB, false, VEC>(rb, cur, n0, P.n, 0);
-    } else {
-        load_a<C, TA, true, false>(ra, cur, m0, P.m, 0);
-        load_b<C, TB, true, false>(rb, cur, n0, P.n, 0);
-    }
-    int buf = 0;
-    store_a<C, TA>(As[0], ra);
-    store_b<C, TB>(Bs[0], rb);
+    enter();
+#pragma unroll
+    for (int d = 0; d < D; ++d) read(d);
+    store(lds, 0);
+    read(0);
     __syncthreads();
 
-    while (true) {
-        // Next k-step position (possibly in the next segment).
-        int64_t nk = kk + BK;
-        int ns = s;
-        Seg nxt = cur;
-        if (nk >= cur.klen) {
-            ++ns;
-            nk = 0;
-            if (ns < s_end) nxt = segs[ns];
-        }
-        const bool has_next = ns < s_end;
-        if (has_next) {
-            if (interior && nk + BK <= nxt.klen) {
-                load_a<C, TA, false, VEC>(ra, nxt, m0, P.m, nk);
-                load_b<C, TB, false, VEC>(rb, nxt, n0, P.n, nk);
-            } else {
-                load_a<C, TA, true, false>(ra, nxt, m0, P.m, nk);
-                load_b<C, TB, true, false>(rb, nxt, n0, P.n, nk);
-            }
-        }
-
-        const double* as = As[buf];
-        const double* bs = Bs[buf];
-        // Each half h of the k-step is one 8-deep step of the direct-to-LDS
-        // kernels, summed in their order: lane group lg supplies k = 8h + 2lg
-        // + q to MFMA q (one 128-bit LDS read per half), so every element
-        // takes the same sequence of MFMAs in all three kernels and a
-        // problem cut between them gives the same bits (but for the sign of
-        // an exactly zero sum when K leaves this kernel a zero-padded half).
+    // Each 8-deep part h of a stage is one step of the direct-to-LDS kernels,
+    // summed in their order: lane group lg supplies k = 8h + 2lg + q to MFMA q,
+    // so every element takes the same sequence of MFMAs in all FP64 kernels
+    // and a problem cut between them, or run on other tiles, gives the same
+    // bits (but for the sign of an exactly zero sum when K leaves this kernel
+    // zero-padded parts).
+    // A part's fragments are read while the part before it is multiplied, the
+    // first part's of stage s + 1 during the last part of stage s: the stage's
+    // barrier sits before that part, when the fragments of stage s are all in
+    // registers and stage s + 1 is stored.
+    constexpr int H = BK / 8;
+    static_assert(H % 2 == 0, "fragment set of part h: h & 1");
+    double fa[2][FM][2], fb[2][FN][2];
+    auto fragments = [&](const char* buf, int h) {
+        OA::template fragments<FM>(fa[h & 1], buf, wm, lr, lg, h);
+        OB::template fragments<FN>(fb[h & 1], buf + OA::BYTES, wn, lr, lg, h);
+    };
+    auto multiply = [&](int h, int q) {
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            dv2 af[FM], bf[FN];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-                af[i] = *reinterpret_cast<const dv2*>(&as[(wm + 16 * i + lr) * LDK + 8 * h + 2 * lg]);
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j)
-                bf[j] = *reinterpret_cast<const dv2*>(&bs[(wn + 16 * j + lr) * LDK + 8 * h + 2 * lg]);
+                acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[h & 1][j][q], fa[h & 1][i][q], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Two stages a turn: s, even, in buffer 0, and s + 1; stage s + 1 waits in
+    // register set (s + 1) % D.  Turns that read only whole stages of one
+    // segment run without conditions.
+    static_assert(D == 1 || D == 2, "the register set of an odd stage is D - 1, of an even one 0");
+    char* const bufs[2] = {lds, lds + L::STAGE};
+    fragments(lds, 0);
+    for (int64_t s = 0; s < ns;) {
+        const int64_t turns = pairs && left > 0 ? (left - 1) / (2 * BK) : 0;
+        for (int64_t i = 0; i < turns; ++i) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q)
+            for (int u = 0; u < 2; ++u) {
+                const int nx = (u + 1) % D;
 #pragma unroll
-                for (int i = 0; i < FM; ++i)
-#pragma unroll
-                    for (int j = 0; j < FN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j][q], af[i][q], acc[i][j], 0, 0, 0);
+                for (int h = 0; h < H; ++h) {
+                    if (h < H - 1) {
+                        fragments(bufs[u], h + 1);
+                    } else {
+                        __syncthreads();
+                        fragments(bufs[u ^ 1], 0);
+                    }
+                    multiply(h, 0);
+                    if (h == H - 2) {
+                        store(bufs[u ^ 1], nx);
+                        oa.read(va[nx]);
+                        ob.read(vb[nx]);
+                    }
+                    multiply(h, 1);
+                }
+            }
         }
-
-        if (!has_next) break;
-        buf ^= 1;
-        store_a<C, TA>(As[buf], ra);
-        store_b<C, TB>(Bs[buf], rb);
-        __syncthreads();
-        s = ns;
-        kk = nk;
-        cur = nxt;
+        s += 2 * turns;
+        left -= 2 * BK * turns;
+#pragma unroll
+        for (int u = 0; u < 2; ++u, ++s) {
+            if (s >= ns) break;
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                if (h < H - 1) {
+                    fragments(bufs[u], h + 1);
+                } else if (s + 1 < ns) {
+                    __syncthreads();
+                    fragments(bufs[u ^ 1], 0);
+                }
+                multiply(h, 0);
+                if (h == H - 2 && s + 1 < ns) {
+                    store(bufs[u ^ 1], (u + 1) % D);
+                    read((u + 1) % D);
+                }
+                multiply(h, 1);
+            }
+        }
     }
 
     // Epilogue.  Register v of lane group lg holds MFMA result row lg + 4v
     // (the f64 16x16x4 result layout), i.e.
     // acc[i][j][v] = sum for C(m0 + wm + 16i + lr, n0 + wn + 16j + lg + 4v).
+    // The old values of a column block are all requested, at clamped
+    // addresses, before the first is used.
     const double alpha = P.alpha, beta = P.beta;
+    typedef __attribute__((address_space(1))) double gd;
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const int64_t m = m0 + wm + 16 * i + lr;
+    for (int j = 0; j < FN; ++j) {
+        double old[FM][4];
+        if (beta != 0.0) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) {
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int64_t m = m0 + wm + 16 * i + lr, n = n0 + wn + 16 * j + lg + 4 * v;
+                    old[i][v] = *(gd*)(P.c + (m < P.m ? m : P.m - 1) + (n < P.n ? n : P.n - 1) * P.ldc);
+                }
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int64_t n = n0 + wn + 16 * j + lg + 4 * v;
-                if (interior || (m < P.m && n < P.n)) {
-                    __attribute__((address_space(1))) double* cp =
-                        (__attribute__((address_space(1))) double*)(P.c + m + n * P.ldc);
-                    double val = alpha * acc[i][j][v];
-                    if (beta != 0.0) val = fma(beta, *cp, val);
-                    *cp = val;
-                }
+                const int64_t m = m0 + wm + 16 * i + lr, n = n0 + wn + 16 * j + lg + 4 * v;
+                double val = alpha * acc[i][j][v];
+                if (beta != 0.0) val = fma(beta, old[i][v], val);
+                if (m < P.m && n < P.n) *(gd*)(P.c + m + n * P.ldc) = val;
             }
-        }
     }
 }
 
@@ -336,16 +388,25 @@ __device__ __forceinline__ void gemm_tile(const Prob* __restrict__ probs, int np
 // MODE 1: one workgroup per tile, XCD-contiguous tile ranges (xcd_remap);
 // MODE 2: persistent: every workgroup takes tiles from `counter` (zeroed
 //         before the launch) until the tile space is exhausted.
-template <class C, bool TA, bool TB, bool VEC, int MODE>
+template <class C, bool TA, bool TB, int MODE>
 __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_kernel(const Prob* __restrict__ probs, int nprob,
                                                                   const Seg* __restrict__ segs, int total_tiles,
                                                                   int* __restrict__ counter) {
-    __shared__ double As[2][C::BM * LDK];
-    __shared__ double Bs[2][C::BN * LDK];
+    __shared__ __attribute__((aligned(16))) char lds[2 * TileLds<C, TA, TB>::STAGE];
+    auto run = [&](int tile) {
+        // Problem owning this tile: last problem with tile0 <= tile.
+        int lo = 0, hi = nprob - 1;
+        while (lo < hi) {
+            int mid = (lo + hi + 1) >> 1;
+            if (probs[mid].tile0 <= tile) lo = mid; else hi = mid - 1;
+        }
+        const Prob P = probs[lo];
+        gemm_tile<C, TA, TB>(P, segs, tile - P.tile0, lds);
+    };
     if (MODE == 0) {
-        gemm_tile<C, TA, TB, VEC>(probs, nprob, segs, blockIdx.x, As, Bs);
+        run(blockIdx.x);
     } else if (MODE == 1) {
-        gemm_tile<C, TA, TB, VEC>(probs, nprob, segs, xcd_remap(blockIdx.x, total_tiles), As, Bs);
+        run(xcd_remap(blockIdx.x, total_tiles));
     } else {
         __shared__ int next;
         while (true) {
@@ -354,7 +415,7 @@ __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_kernel(const Prob* __
             __syncthreads();
             const int tile = next;
             if (tile >= total_tiles) break;
-            gemm_tile<C, TA, TB, VEC>(probs, nprob, segs, tile, As, Bs);
+            run(tile);
         }
     }
 }
@@ -507,14 +568,16 @@ __device__ __forceinline__ void dma_tile(const Prob* __restrict__ probs, int npr
     int lo = 0, hi = nprob - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
-        if (probs[mid].tile0[0] <= tile) lo = mid; else hi = mid - 1;
+        if (probs[mid].tile0 <= tile) lo = mid; else hi = mid - 1;
     }
     const Prob P = probs[lo];
-    const int local = tile - P.tile0[0];
-    const int per_group = GROUP_M * P.tiles_n[0];
+    const int local = tile - P.tile0;
+    const int tiles_m = (int)((P.m + (P.shift & 1) + DBM - 1) / DBM);
+    const int tiles_n = (int)((P.n + ((P.shift >> 1) & 1) + DBN - 1) / DBN);
+    const int per_group = GROUP_M * tiles_n;
     const int group = local / per_group;
     const int first_m = group * GROUP_M;
-    const int gsize = min(P.tiles_m[0] - first_m, GROUP_M);
+    const int gsize = min(tiles_m - first_m, GROUP_M);
     const int in_group = local - group * per_group;
     const int64_t m0 = (int64_t)(first_m + in_group % gsize) * DBM;
     const int64_t n0 = (int64_t)(in_group / gsize) * DBN;
@@ -710,14 +773,16 @@ __device__ __forceinline__ void dma_tile_ar(const Prob* __restrict__ probs, int 
     int lo = 0, hi = nprob - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
-        if (probs[mid].tile0[0] <= tile) lo = mid; else hi = mid - 1;
+        if (probs[mid].tile0 <= tile) lo = mid; else hi = mid - 1;
     }
     const Prob P = probs[lo];
-    const int local = tile - P.tile0[0];
-    const int per_group = GROUP_M * P.tiles_n[0];
+    const int local = tile - P.tile0;
+    const int tiles_m = (int)((P.m + (P.shift & 1) + DBM - 1) / DBM);
+    const int tiles_n = (int)((P.n + ((P.shift >> 1) & 1) + DBN - 1) / DBN);
+    const int per_group = GROUP_M * tiles_n;
     const int group = local / per_group;
     const int first_m = group * GROUP_M;
-    const int gsize = min(P.tiles_m[0] - first_m, GROUP_M);
+    const int gsize = min(tiles_m - first_m, GROUP_M);
     const int in_group = local - group * per_group;
     const int64_t m0 = (int64_t)(first_m + in_group % gsize) * DBM;
     const int64_t n0 = (int64_t)(in_group / gsize) * DBN;
@@ -962,35 +1027,25 @@ __global__ void scale_kernel(int64_t m, int64_t n, double beta, double* __restri
     }
 }
 
-template <class C, bool TA, bool TB, bool VEC>
+template <class C, bool TA, bool TB>
 void launch_mode(int mode, const Prob* dp, int np, const Seg* ds, int tiles, int grid, int* counter,
                  hipStream_t st) {
     if (mode == DG_GEMM_MODE_ROUND_ROBIN)
-        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, VEC, 0>), dim3(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles,
-                           counter);
+        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 0>), dim3(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
     else if (mode == DG_GEMM_MODE_XCD)
-        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, VEC, 1>), dim3(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles,
-                           counter);
+        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 1>), dim3(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
     else
-        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, VEC, 2>), dim3(grid), dim3(C::NTH), 0, st, dp, np, ds, tiles,
-                           counter);
-}
-
-template <class C, bool TA, bool TB>
-void launch_kind(bool vec, int mode, const Prob* dp, int np, const Seg* ds, int tiles, int grid, int* counter,
-                 hipStream_t st) {
-    if (vec) launch_mode<C, TA, TB, true>(mode, dp, np, ds, tiles, grid, counter, st);
-    else     launch_mode<C, TA, TB, false>(mode, dp, np, ds, tiles, grid, counter, st);
+        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 2>), dim3(grid), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
 }
 
 template <class C>
-void launch_cfg(char opA, char opB, bool vec, int mode, const Prob* dp, int np, const Seg* ds, int tiles, int grid,
-                int* counter, hipStream_t st) {
+void launch_cfg(char opA, char opB, int mode, const Prob* dp, int np, const Seg* ds, int tiles, int grid, int* counter,
+                hipStream_t st) {
     const bool ta = opA == 'T', tb = opB == 'T';
-    if (!ta && !tb) launch_kind<C, false, false>(vec, mode, dp, np, ds, tiles, grid, counter, st);
-    else if (!ta && tb) launch_kind<C, false, true>(vec, mode, dp, np, ds, tiles, grid, counter, st);
-    else if (ta && !tb) launch_kind<C, true, false>(vec, mode, dp, np, ds, tiles, grid, counter, st);
-    else launch_kind<C, true, true>(vec, mode, dp, np, ds, tiles, grid, counter, st);
+    if (!ta && !tb) launch_mode<C, false, false>(mode, dp, np, ds, tiles, grid, counter, st);
+    else if (!ta && tb) launch_mode<C, false, true>(mode, dp, np, ds, tiles, grid, counter, st);
+    else if (ta && !tb) launch_mode<C, true, false>(mode, dp, np, ds, tiles, grid, counter, st);
+    else launch_mode<C, true, true>(mode, dp, np, ds, tiles, grid, counter, st);
 }
 
 }  // namespace
@@ -1005,24 +1060,78 @@ int launch_scale(int64_t m, int64_t n, double beta, double* C, int64_t ldc, hipS
     return DG_OK;
 }
 
-int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs_in, const std::vector<Seg>& segs,
-                 GemmBatch& out, bool split_edges) {
+// Whether the register-staged kernel must load a problem by single elements:
+// bases off 8-byte alignment, or rows so far apart that a tile's offsets
+// leave 32 bits.
+static bool by_elements(const Prob& p, const std::vector<Seg>& segs) {
+    for (int s = p.seg0; s < p.seg0 + p.nseg; ++s) {
+        const Seg& g = segs[s];
+        if (((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 7) || g.lda > kMaxPairLd || g.ldb > kMaxPairLd)
+            return true;
+    }
+    return false;
+}
+
+// Time (us) of one list's launch, to choose between the tile shapes: the
+// fullest CU's tiles at the rate that `conc` resident workgroups reach (eff,
+// by how many there are), plus 4 us of prologue and epilogue per round of
+// resident tiles.  Measured rates, share of 78.6 TFLOP/s: 128x128 direct to
+// LDS 0.91 (256 tiles, one workgroup per CU) and 0.95 (two); 64x64 0.74, 0.83,
+// 0.865, 0.895 with one to four; 32x32 0.58, 0.68, 0.72, 0.76.
+struct ListCost {
+    int64_t tiles = 0;
+    double sum = 0, most = 0, least = 1e300;  // us of CU time: all tiles, the longest, the shortest
+    void add(int64_t n, int64_t area, int64_t k) {
+        const double u = 2.0 * (double)area * (double)k / (78.6e6 / 256);
+        tiles += n;
+        sum += (double)n * u;
+        most = std::max(most, u);
+        least = std::min(least, u);
+    }
+    double time(int conc, const double* eff) const {
+        if (!tiles) return 0;
+        const int64_t c = (tiles + 255) / 256;
+        const double load = most == least ? (double)c * most : std::max(sum / 256 + most / 2, most);
+        return load / eff[std::min<int64_t>(c, conc) - 1] + 4.0 * std::max(1.0, (double)c / conc);
+    }
+};
+constexpr double kEffInterior[2] = {0.91, 0.95}, kEffEdge[2] = {0.85, 0.93};
+constexpr double kEff64[4] = {0.74, 0.83, 0.865, 0.895}, kEff32[4] = {0.58, 0.68, 0.72, 0.76};
+
+// prepare_gemm for one tile choice; *time receives the estimate (us).
+static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, const std::vector<Seg>& segs,
+                        GemmBatch& out, bool split_edges, int tile, double* time) {
     out = GemmBatch{};
     out.segs = segs;
     const bool ak = opA == 'T', bkc = opB != 'T';  // k-contiguous operands
-    static const bool no_dma = getenv("DG_GEMM_NO_DMA") != nullptr;
     int64_t tdma = 0, tdmae = 0, tgen[2] = {0, 0};
-    const int bm[2] = {Cfg128::BM, Cfg256::BM}, bn[2] = {Cfg128::BN, Cfg256::BN};
+    ListCost cdma, cdmae, cgen[2];
     constexpr int64_t TM = dmak::DBM, TN = dmak::DBN;
+    auto depth = [&](const Prob& p) {
+        int64_t k = 0;
+        for (int s = p.seg0; s < p.seg0 + p.nseg; ++s) k += out.segs[s].klen;
+        return k;
+    };
     // a direct-to-LDS problem (or sub-problem) onto its list
     auto add_dma = [&](Prob p, bool interior) {
         const int sa = p.shift & 1, sb = (p.shift >> 1) & 1;
-        p.tiles_m[0] = p.tiles_m[1] = (int32_t)((p.m + sa + TM - 1) / TM);
-        p.tiles_n[0] = p.tiles_n[1] = (int32_t)((p.n + sb + TN - 1) / TN);
         int64_t& t = interior ? tdma : tdmae;
-        p.tile0[0] = p.tile0[1] = (int32_t)t;
-        t += (int64_t)p.tiles_m[0] * p.tiles_n[0];
+        p.tile0 = (int32_t)t;
+        const int64_t n = ((p.m + sa + TM - 1) / TM) * ((p.n + sb + TN - 1) / TN);
+        t += n;
+        (interior ? cdma : cdmae).add(n, TM * TN, depth(p));
         (interior ? out.dma : out.dmae).push_back(p);
+    };
+    // a problem, or a strip of one, onto the register-staged kernel's list
+    auto add_gen = [&](Prob q) {
+        const int w = tile == DG_GEMM_TILE_32x32 || q.m <= kNarrowMax || q.n <= kNarrowMax ? 1 : 0;
+        const int64_t e = w ? 32 : 64;
+        q.shift = by_elements(q, out.segs) ? kByElements : 0;
+        q.tile0 = (int32_t)tgen[w];
+        const int64_t n = ((q.m + e - 1) / e) * ((q.n + e - 1) / e);
+        tgen[w] += n;
+        cgen[w].add(n, e * e, depth(q));
+        out.gen[w].push_back(q);
     };
     // rows [r0, r0 + nr) x columns [c0, c0 + nc) of p as a problem of its own,
     // its segments re-based and appended; its shifts follow from the new bases
@@ -1044,35 +1153,14 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs_in, const st
         q.shift = sa | (sb << 1);
         return q;
     };
-    // a strip narrower than a tile onto narrow list w (0: 128x32 tiles, 1: 64x128)
     static const bool no_narrow = getenv("DG_GEMM_NO_NARROW") != nullptr;
-    const int nbm[2] = {CfgN32::BM, CfgM64::BM}, nbn[2] = {CfgN32::BN, CfgM64::BN};
-    int64_t tnar[2] = {0, 0};
-    auto add_nar = [&](Prob q, int w) {
-        for (int s = q.seg0; s < q.seg0 + q.nseg; ++s) {
-            const Seg& g = out.segs[s];
-            if ((reinterpret_cast<uintptr_t>(g.a) & 15) || (reinterpret_cast<uintptr_t>(g.b) & 15) || (g.lda & 1) ||
-                (g.ldb & 1))
-                out.vec_nar[w] = false;
-        }
-        q.tiles_m[0] = q.tiles_m[1] = (int32_t)((q.m + nbm[w] - 1) / nbm[w]);
-        q.tiles_n[0] = q.tiles_n[1] = (int32_t)((q.n + nbn[w] - 1) / nbn[w]);
-        q.tile0[0] = q.tile0[1] = (int32_t)tnar[w];
-        tnar[w] += (int64_t)q.tiles_m[0] * q.tiles_n[0];
-        out.nar[w].push_back(q);
-    };
-    // a strip of `width` rows (columns) fills 128-wide tiles to width / 128,
-    // a 64-row (32-column) tile to width / 64 (width / (32 ceil(width / 32))),
-    // and the narrow tiles pay up to this width
-    auto narrow = [&](int64_t width) { return !no_narrow && width <= kNarrowMax; };
     for (const Prob& p0 : probs_in) {
         if (p0.m <= 0 || p0.n <= 0 || p0.nseg <= 0) continue;
-        bool v = true, d = !no_dma;
+        bool d = tile == DG_GEMM_TILE_128x128;
         int off_a = -1, off_b = -1;  // byte offset within 16 of a row-contiguous A / B
-        for (int s = p0.seg0; s < p0.seg0 + p0.nseg; ++s) {
+        for (int s = p0.seg0; d && s < p0.seg0 + p0.nseg; ++s) {
             const Seg& g = segs[s];
             const int oa = (int)(reinterpret_cast<uintptr_t>(g.a) & 15), ob = (int)(reinterpret_cast<uintptr_t>(g.b) & 15);
-            if (oa || ob || (g.lda & 1) || (g.ldb & 1)) v = false;
             if ((g.lda & 1) || (g.ldb & 1) || g.klen <= 0) d = false;
             if (ak) { if (oa || (g.klen & 1)) d = false; }   // k pairs, 16-byte aligned
             else { if ((oa & 7) || (off_a >= 0 && oa != off_a)) d = false; off_a = oa; }
@@ -1081,14 +1169,7 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs_in, const st
         }
         Prob p = p0;
         if (!d) {
-            out.vec = out.vec && v;
-            for (int c = 0; c < 2; ++c) {
-                p.tiles_m[c] = (int32_t)((p.m + bm[c] - 1) / bm[c]);
-                p.tiles_n[c] = (int32_t)((p.n + bn[c] - 1) / bn[c]);
-                p.tile0[c] = (int32_t)tgen[c];
-                tgen[c] += (int64_t)p.tiles_m[c] * p.tiles_n[c];
-            }
-            out.gen.push_back(p);
+            add_gen(p);
             continue;
         }
         const int sa = off_a == 8, sb = off_b == 8;
@@ -1113,54 +1194,77 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs_in, const st
             add_dma(p, false);
             continue;
         }
+        auto strip = [&](const Prob& q) { if (no_narrow) add_dma(q, false); else add_gen(q); };
         add_dma(sub(p, r0, mi, c0, ni), true);                                       // interior
-        if (r0 > 0) add_dma(sub(p, 0, r0, 0, p.n), false);                           // rows before it
-        if (r0 + mi < p.m) {                                                         // rows after it
-            const Prob q = sub(p, r0 + mi, p.m - r0 - mi, 0, p.n);
-            if (narrow(q.m)) add_nar(q, 1); else add_dma(q, false);
-        }
-        if (c0 > 0) add_dma(sub(p, r0, mi, 0, c0), false);                           // columns before it
-        if (c0 + ni < p.n) {                                                         // columns after it
-            const Prob q = sub(p, r0, mi, c0 + ni, p.n - c0 - ni);
-            if (narrow(q.n)) add_nar(q, 0); else add_dma(q, false);
-        }
+        if (r0 > 0) strip(sub(p, 0, r0, 0, p.n));                                    // rows before it
+        if (r0 + mi < p.m) strip(sub(p, r0 + mi, p.m - r0 - mi, 0, p.n));            // rows after it
+        if (c0 > 0) strip(sub(p, r0, mi, 0, c0));                                    // columns before it
+        if (c0 + ni < p.n) strip(sub(p, r0, mi, c0 + ni, p.n - c0 - ni));            // columns after it
     }
     if (tdma > INT32_MAX || tdmae > INT32_MAX || tgen[0] > INT32_MAX || tgen[1] > INT32_MAX ||
-        tnar[0] > INT32_MAX || tnar[1] > INT32_MAX || out.segs.size() > (size_t)INT32_MAX)
+        out.segs.size() > (size_t)INT32_MAX)
         return fail(DG_ERR_INVALID, "gemm: output tiles exceed one launch");
-    out.tiles_nar[0] = (int)tnar[0];
-    out.tiles_nar[1] = (int)tnar[1];
     out.tiles_dma = (int)tdma;
     out.tiles_dmae = (int)tdmae;
-    out.tiles_gen[0] = (int)tgen[0];
-    out.tiles_gen[1] = (int)tgen[1];
+    for (int w = 0; w < 2; ++w) out.tiles_gen[w] = (int)tgen[w];
+    *time = cdma.time(2, kEffInterior) + cdmae.time(2, kEffEdge) + cgen[0].time(4, kEff64) + cgen[1].time(4, kEff32);
     return DG_OK;
 }
 
-int persistent_grid(int cfg) {
+int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, const std::vector<Seg>& segs, GemmBatch& out,
+                 bool split_edges, int tile) {
+    // DG_GEMM_TILE forces a shape; DG_GEMM_NO_DMA keeps everything on the register-staged kernel
+    static const int forced = [] {
+        const char* e = getenv("DG_GEMM_TILE");
+        const std::string v = e ? e : "";
+        if (v == "128x128") return (int)DG_GEMM_TILE_128x128;
+        if (v == "64x64") return (int)DG_GEMM_TILE_64x64;
+        if (v == "32x32") return (int)DG_GEMM_TILE_32x32;
+        return (int)DG_GEMM_TILE_AUTO;
+    }();
+    static const bool no_dma = getenv("DG_GEMM_NO_DMA") != nullptr;
+    if (forced != DG_GEMM_TILE_AUTO) tile = forced;
+    if (no_dma && tile == DG_GEMM_TILE_128x128) tile = DG_GEMM_TILE_64x64;
+    double t = 0;
+    if (tile != DG_GEMM_TILE_AUTO) return prepare_tile(opA, opB, probs, segs, out, split_edges, tile, &t);
+    double best = 0;
+    int rc_best = DG_ERR_INVALID;
+    for (int c = no_dma ? DG_GEMM_TILE_64x64 : DG_GEMM_TILE_128x128; c < DG_GEMM_TILES; ++c) {
+        GemmBatch b;
+        const int rc = prepare_tile(opA, opB, probs, segs, b, split_edges, c, &t);
+        if (rc == DG_OK && (rc_best != DG_OK || t < best)) {
+            out = std::move(b);
+            best = t;
+            rc_best = DG_OK;
+        }
+    }
+    return rc_best;
+}
+
+int persistent_grid(int occ) {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
         cus = 256;
-    return cus * (cfg == DG_GEMM_TILE_256x128 ? Cfg256::OCC : cfg == DG_GEMM_TILE_128x128W8 ? Cfg128w8::OCC : Cfg128::OCC);
+    return cus * occ;
 }
 
-int launch_gemm_f64_dev(char opA, char opB, int mode, int cfg, const GemmBatchDev& b, int* counter,
-                        hipStream_t stream) {
+int launch_gemm_f64_dev(char opA, char opB, int mode, const GemmBatchDev& b, int* counter, hipStream_t stream) {
     if (mode == DG_GEMM_MODE_PERSISTENT && !counter)
         return fail(DG_ERR_INVALID, "gemm: persistent launch without a work counter");
+    // grid of a list's launch: its tiles, or as many workgroups as are resident
+    auto grid_of = [&](int tiles, int occ) {
+        if (mode != DG_GEMM_MODE_PERSISTENT) return tiles;
+        hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(1), 0, stream, counter);
+        return std::min(tiles, persistent_grid(occ));
+    };
     for (int e = 0; e < 2; ++e) {  // interior list, then edge list
         const bool edge = e == 1;
         const int t0 = edge ? b.tiles_dmae : b.tiles_dma;
         if (t0 <= 0) continue;
         const Prob* dp = edge ? b.dmae : b.dma;
         const int np = edge ? b.ndmae : b.ndma;
-        int grid = 0;
-        if (mode == DG_GEMM_MODE_PERSISTENT) {
-            grid = persistent_grid(DG_GEMM_TILE_128x128);
-            if (grid > t0) grid = t0;
-            hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(1), 0, stream, counter);
-        }
+        const int grid = grid_of(t0, 2);
         const bool ak = opA == 'T', bkc = opB != 'T';
         if (ak && bkc) launch_dma<true, true>(edge, mode, dp, np, b.segs, t0, grid, counter, stream);
         else if (ak) launch_dma<true, false>(edge, mode, dp, np, b.segs, t0, grid, counter, stream);
@@ -1168,43 +1272,15 @@ int launch_gemm_f64_dev(char opA, char opB, int mode, int cfg, const GemmBatchDe
         else launch_dma<false, false>(edge, mode, dp, np, b.segs, t0, grid, counter, stream);
         DG_LAUNCH_CHECK();
     }
-    for (int w = 0; w < 2; ++w) {  // narrow strips: 128x32 tiles, then 64x128 tiles
-        const int tw = b.tiles_nar[w];
-        if (tw <= 0) continue;
-        int grid = 0;
-        if (mode == DG_GEMM_MODE_PERSISTENT) {
-            grid = persistent_grid(DG_GEMM_TILE_128x128);  // two workgroups per CU, as CfgN32 / CfgM64
-            if (grid > tw) grid = tw;
-            hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(1), 0, stream, counter);
-        }
-        if (w == 0) launch_cfg<CfgN32>(opA, opB, b.vec_nar[0], mode, b.nar[0], b.nnar[0], b.segs, tw, grid, counter, stream);
-        else launch_cfg<CfgM64>(opA, opB, b.vec_nar[1], mode, b.nar[1], b.nnar[1], b.segs, tw, grid, counter, stream);
+    for (int w = 0; w < 2; ++w) {  // 64x64 tiles, then 32x32
+        const int t = b.tiles_gen[w];
+        if (t <= 0) continue;
+        const int grid = grid_of(t, w ? Cfg32::OCC : Cfg64::OCC);
+        if (w == 0) launch_cfg<Cfg64>(opA, opB, mode, b.gen[0], b.ngen[0], b.segs, t, grid, counter, stream);
+        else launch_cfg<Cfg32>(opA, opB, mode, b.gen[1], b.ngen[1], b.segs, t, grid, counter, stream);
         DG_LAUNCH_CHECK();
     }
-    const int t = b.tiles_gen[cfg == DG_GEMM_TILE_256x128 ? 1 : 0];
-    if (t <= 0) return DG_OK;
-    int grid = 0;
-    if (mode == DG_GEMM_MODE_PERSISTENT) {
-        grid = persistent_grid(cfg);
-        if (grid > t) grid = t;
-        hipLaunchKernelGGL(zero_counter_kernel, dim3(1), dim3(1), 0, stream, counter);
-    }
-    if (cfg == DG_GEMM_TILE_256x128) launch_cfg<Cfg256>(opA, opB, b.vec, mode, b.gen, b.ngen, b.segs, t, grid, counter, stream);
-    else if (cfg == DG_GEMM_TILE_128x128W8) launch_cfg<Cfg128w8>(opA, opB, b.vec, mode, b.gen, b.ngen, b.segs, t, grid, counter, stream);
-    else launch_cfg<Cfg128>(opA, opB, b.vec, mode, b.gen, b.ngen, b.segs, t, grid, counter, stream);
-    DG_LAUNCH_CHECK();
     return DG_OK;
-}
-
-int default_tile_cfg() {
-    static const int cfg = [] {
-        const char* e = getenv("DG_GEMM_TILE");
-        if (e && std::string(e) == "256x128") return (int)DG_GEMM_TILE_256x128;
-        if (e && std::string(e) == "128x128") return (int)DG_GEMM_TILE_128x128;
-        if (e && std::string(e) == "128x128w8") return (int)DG_GEMM_TILE_128x128W8;
-        return (int)DG_GEMM_TILE_DEFAULT;
-    }();
-    return cfg;
 }
 
 int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs_in, const std::vector<Seg>& segs,
@@ -1212,7 +1288,7 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs_in, const
     GemmBatch hb;
     int rc = prepare_gemm(opA, opB, probs_in, segs, hb);
     if (rc) return rc;
-    if (hb.dma.empty() && hb.dmae.empty() && hb.gen.empty() && hb.nar[0].empty() && hb.nar[1].empty()) return DG_OK;
+    if (hb.empty()) return DG_OK;
     GemmBatchDev b;
     TableUseScope uses{stream};  // after the launch below returns
     auto table = [&](const auto& v, auto** dst) -> bool {
@@ -1222,24 +1298,12 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs_in, const
         *dst = static_cast<const T*>(cached_table(v.data(), v.size() * sizeof(T), stream));
         return *dst != nullptr;
     };
-    if (!table(hb.dma, &b.dma) || !table(hb.dmae, &b.dmae) || !table(hb.gen, &b.gen) || !table(hb.segs, &b.segs) ||
-        !table(hb.nar[0], &b.nar[0]) || !table(hb.nar[1], &b.nar[1]))
+    if (!table(hb.dma, &b.dma) || !table(hb.dmae, &b.dmae) || !table(hb.gen[0], &b.gen[0]) ||
+        !table(hb.gen[1], &b.gen[1]) || !table(hb.segs, &b.segs))
         return DG_ERR_ALLOC;
-    for (int w = 0; w < 2; ++w) {
-        b.nnar[w] = (int)hb.nar[w].size();
-        b.tiles_nar[w] = hb.tiles_nar[w];
-        b.vec_nar[w] = hb.vec_nar[w];
-    }
-    b.ndma = (int)hb.dma.size();
-    b.tiles_dma = hb.tiles_dma;
-    b.ndmae = (int)hb.dmae.size();
-    b.tiles_dmae = hb.tiles_dmae;
-    b.ngen = (int)hb.gen.size();
-    b.tiles_gen[0] = hb.tiles_gen[0];
-    b.tiles_gen[1] = hb.tiles_gen[1];
-    b.vec = hb.vec;
+    b.set_counts(hb);
     if (mode == DG_GEMM_MODE_PERSISTENT) mode = DG_GEMM_MODE_XCD;  // needs a counter: plans only
-    return launch_gemm_f64_dev(opA, opB, mode, default_tile_cfg(), b, nullptr, stream);
+    return launch_gemm_f64_dev(opA, opB, mode, b, nullptr, stream);
 }
 
 }  // namespace dg

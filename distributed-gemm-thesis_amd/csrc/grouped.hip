@@ -15,12 +15,13 @@
 struct dg_grouped_plan {
     struct Group {
         char opA, opB;
-        dg::GemmBatchDev b;         // device tables owned by the plan
+        dg::GemmBatchDev b;
     };
-    std::vector<Group> groups;
+    std::vector<Group> groups[dg::DG_GEMM_TILES];  // per tile choice; [0] alone unless autotuned
+    void* tables = nullptr;                        // the tables of all of them
     int mode = DG_PLAN_AUTOTUNE;   // requested
     int variant = -1;              // DG_GEMM_MODE_* in use (-1: not tuned yet)
-    int cfg = 0;                   // DG_GEMM_TILE_* in use
+    int cfg = 0;                   // which of `groups` is in use
     std::string shape_key;
     int* counter = nullptr;        // device work counter (persistent mode)
     hipGraphExec_t graph = nullptr;
@@ -166,8 +167,8 @@ int launch_ozaki_problem(const dg_grouped_plan* p, int i, hipStream_t st) {
 }
 
 int plan_launch(dg_grouped_plan* p, int variant, int cfg, hipStream_t st, bool with_ozaki = true) {
-    for (auto& g : p->groups) {
-        int rc = launch_gemm_f64_dev(g.opA, g.opB, variant, cfg, g.b, p->counter, st);
+    for (auto& g : p->groups[cfg]) {
+        int rc = launch_gemm_f64_dev(g.opA, g.opB, variant, g.b, p->counter, st);
         if (rc) return rc;
     }
     if (!with_ozaki) return DG_OK;
@@ -261,51 +262,57 @@ int share_operands(dg_grouped_plan* p) {
     return DG_OK;
 }
 
-// Device tables of the FP64 problems listed in `use` (all when empty).
+// Device tables of the FP64 problems listed in `use` (all when null), one
+// allocation and one copy for all: with the autotuner a set per tile choice
+// for it to time, else the estimated best.
 int build_groups(dg_grouped_plan* p, const dg_gemm_desc* descs, int count, const std::vector<char>* use) {
     std::vector<dg_gemm_desc> sel;
     sel.reserve(count);
     for (int i = 0; i < count; ++i)
         if (!use || (*use)[i]) sel.push_back(descs[i]);
-    for (auto& kv : by_ops(sel.data(), (int)sel.size())) {
-        std::vector<Prob> probs0;
-        std::vector<Seg> segs;
-        build_group(sel.data(), kv.second, probs0, segs);
-        GemmBatch hb;
-        int rc = prepare_gemm(kv.first.first, kv.first.second, probs0, segs, hb);
-        if (rc) return rc;
-        if (hb.dma.empty() && hb.dmae.empty() && hb.gen.empty() && hb.nar[0].empty() && hb.nar[1].empty()) continue;
-        dg_grouped_plan::Group g;
-        g.opA = kv.first.first;
-        g.opB = kv.first.second;
-        p->groups.push_back(g);
-        GemmBatchDev& b = p->groups.back().b;  // owned by the plan from here on (freed on failure too)
-        auto upload = [&](const auto& v, auto** dst) -> bool {
-            using T = typename std::decay_t<decltype(v)>::value_type;
-            *dst = nullptr;
-            if (v.empty()) return true;
-            void* d = nullptr;
-            if (hipMalloc(&d, v.size() * sizeof(T)) != hipSuccess) return false;
-            *dst = static_cast<const T*>(d);
-            return hipMemcpy(d, v.data(), v.size() * sizeof(T), hipMemcpyHostToDevice) == hipSuccess;
-        };
-        if (!upload(hb.dma, &b.dma) || !upload(hb.dmae, &b.dmae) || !upload(hb.gen, &b.gen) ||
-            !upload(hb.nar[0], &b.nar[0]) || !upload(hb.nar[1], &b.nar[1]) || !upload(hb.segs, &b.segs))
-            return fail(DG_ERR_ALLOC, "plan: table upload");
-        for (int w = 0; w < 2; ++w) {
-            b.nnar[w] = (int)hb.nar[w].size();
-            b.tiles_nar[w] = hb.tiles_nar[w];
-            b.vec_nar[w] = hb.vec_nar[w];
+    std::vector<unsigned char> image;
+    struct Put { const void** dst; size_t off; };
+    std::vector<Put> puts;
+    auto put = [&](const auto& v, auto** dst) {
+        *dst = nullptr;
+        if (v.empty()) return;
+        const size_t off = (image.size() + 255) / 256 * 256, bytes = v.size() * sizeof(v[0]);
+        image.resize(off + bytes);
+        memcpy(image.data() + off, v.data(), bytes);
+        puts.push_back({reinterpret_cast<const void**>(dst), off});
+    };
+    for (auto& g : p->groups) g.clear();  // a build that failed before
+    if (p->tables) (void)hipFree(p->tables);
+    p->tables = nullptr;
+    const bool tune = p->mode == DG_PLAN_AUTOTUNE;
+    const auto kinds = by_ops(sel.data(), (int)sel.size());
+    for (int t = 0; t < (tune ? (int)DG_GEMM_TILES : 1); ++t) {
+        p->groups[t].reserve(kinds.size());  // `puts` points into it
+        for (auto& kv : kinds) {
+            std::vector<Prob> probs0;
+            std::vector<Seg> segs;
+            build_group(sel.data(), kv.second, probs0, segs);
+            GemmBatch hb;
+            int rc = prepare_gemm(kv.first.first, kv.first.second, probs0, segs, hb, true, tune ? t : (int)DG_GEMM_TILE_AUTO);
+            if (rc) return rc;
+            if (hb.empty()) continue;
+            p->groups[t].push_back({kv.first.first, kv.first.second, GemmBatchDev{}});
+            GemmBatchDev& b = p->groups[t].back().b;
+            put(hb.dma, &b.dma);
+            put(hb.dmae, &b.dmae);
+            for (int w = 0; w < 2; ++w) put(hb.gen[w], &b.gen[w]);
+            put(hb.segs, &b.segs);
+            b.set_counts(hb);
         }
-        b.ndma = (int)hb.dma.size();
-        b.tiles_dma = hb.tiles_dma;
-        b.ndmae = (int)hb.dmae.size();
-        b.tiles_dmae = hb.tiles_dmae;
-        b.ngen = (int)hb.gen.size();
-        b.tiles_gen[0] = hb.tiles_gen[0];
-        b.tiles_gen[1] = hb.tiles_gen[1];
-        b.vec = hb.vec;
     }
+    if (image.empty()) return DG_OK;
+    if (hipMalloc(&p->tables, image.size()) != hipSuccess) {
+        p->tables = nullptr;
+        return fail(DG_ERR_ALLOC, "plan: tables of %zu bytes", image.size());
+    }
+    if (hipMemcpy(p->tables, image.data(), image.size(), hipMemcpyHostToDevice) != hipSuccess)
+        return fail(DG_ERR_ALLOC, "plan: table upload");
+    for (const Put& x : puts) *x.dst = static_cast<char*>(p->tables) + x.off;
     return DG_OK;
 }
 
@@ -458,7 +465,7 @@ int choose_forms(dg_grouped_plan* p, hipStream_t st) {
     return DG_OK;
 }
 
-// Times each scheduling variant (best of three) on the plan's own operands
+// Times each tile choice and scheduling variant (best of three) on the plan's own operands
 // and keeps the fastest.  The outputs are saved before the trials and
 // restored after them, also when a trial fails, so tuning leaves C as it
 // found it.
@@ -468,18 +475,21 @@ int autotune(dg_grouped_plan* p, hipStream_t st) {
         std::lock_guard<std::mutex> lock(c.mu);
         tune_load_locked(c);
         auto it = c.best.find(p->shape_key);
-        if (it != c.best.end()) { p->variant = it->second % 4; p->cfg = it->second / 4; return DG_OK; }
+        if (it != c.best.end() && it->second >= 0 && it->second / 4 < DG_GEMM_TILES && it->second % 4 < 3) {
+            p->variant = it->second % 4;
+            p->cfg = it->second / 4;
+            return DG_OK;
+        }
     }
     const int variants[3] = {DG_GEMM_MODE_XCD, DG_GEMM_MODE_ROUND_ROBIN, DG_GEMM_MODE_PERSISTENT};
-    const int cfgs[2] = {DG_GEMM_TILE_128x128, DG_GEMM_TILE_256x128};
     float best_ms = 1e30f;
-    int best = DG_GEMM_MODE_XCD;  // encoded cfg * 4 + scheduling mode
+    int best = DG_GEMM_MODE_XCD;  // encoded tile choice * 4 + scheduling mode
     {
         // the outputs are restored when `trial` ends, whether or not the trials succeed
         TrialScope trial;
         int rc = trial.save(st, p->c_spans);
         if (rc) return rc;
-        for (int cfg : cfgs)
+        for (int cfg = 0; cfg < DG_GEMM_TILES; ++cfg)
             for (int v : variants) {
                 float vbest = 1e30f;
                 for (int rep = 0; rep < 3; ++rep) {
@@ -579,7 +589,7 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
     // Lay out every op group's tables (problems routed to each kernel, then
     // segments) in one host image, 256-byte aligned pieces, and check the size
     // before anything is launched.
-    struct Piece { char opA, opB; GemmBatch hb; std::vector<Seg> segs; size_t off_dma, off_dmae, off_gen, off_seg; };
+    struct Piece { char opA, opB; GemmBatch hb; size_t off_dma, off_dmae, off_gen[2], off_seg; };
     std::vector<Piece> pieces;
     size_t total = 0;
     auto take = [&](size_t bytes) { const size_t o = total; total = (total + bytes + 255) / 256 * 256; return o; };
@@ -588,14 +598,13 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
         std::vector<Seg> segs;
         build_group(descs, kv.second, probs, segs);
         if (probs.empty()) continue;
-        Piece pc{kv.first.first, kv.first.second, GemmBatch{}, std::move(segs), 0, 0, 0, 0};
-        // no sub-problems here (so no narrow strips either): the tables stay
-        // within the documented capacity
-        rc = prepare_gemm(pc.opA, pc.opB, probs, pc.segs, pc.hb, false);
+        Piece pc{kv.first.first, kv.first.second, GemmBatch{}, 0, 0, {0, 0}, 0};
+        // no sub-problems here: the tables stay within the documented capacity
+        rc = prepare_gemm(pc.opA, pc.opB, probs, segs, pc.hb, false);
         if (rc) return rc;
         pc.off_dma = take(pc.hb.dma.size() * sizeof(Prob));
         pc.off_dmae = take(pc.hb.dmae.size() * sizeof(Prob));
-        pc.off_gen = take(pc.hb.gen.size() * sizeof(Prob));
+        for (int w = 0; w < 2; ++w) pc.off_gen[w] = take(pc.hb.gen[w].size() * sizeof(Prob));
         pc.off_seg = take(pc.hb.segs.size() * sizeof(Seg));
         pieces.push_back(std::move(pc));
     }
@@ -609,30 +618,23 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
     if (pieces.empty()) return DG_OK;
     std::vector<unsigned char> image(total, 0);
     for (const Piece& pc : pieces) {
-        if (!pc.hb.dma.empty()) memcpy(image.data() + pc.off_dma, pc.hb.dma.data(), pc.hb.dma.size() * sizeof(Prob));
-        if (!pc.hb.dmae.empty())
-            memcpy(image.data() + pc.off_dmae, pc.hb.dmae.data(), pc.hb.dmae.size() * sizeof(Prob));
-        if (!pc.hb.gen.empty()) memcpy(image.data() + pc.off_gen, pc.hb.gen.data(), pc.hb.gen.size() * sizeof(Prob));
-        memcpy(image.data() + pc.off_seg, pc.hb.segs.data(), pc.hb.segs.size() * sizeof(Seg));
+        auto copy = [&](const auto& v, size_t off) { if (!v.empty()) memcpy(image.data() + off, v.data(), v.size() * sizeof(v[0])); };
+        copy(pc.hb.dma, pc.off_dma);
+        copy(pc.hb.dmae, pc.off_dmae);
+        for (int w = 0; w < 2; ++w) copy(pc.hb.gen[w], pc.off_gen[w]);
+        copy(pc.hb.segs, pc.off_seg);
     }
     rc = store_bytes(base, image, st);
     if (rc) return rc;
     unsigned char* b = static_cast<unsigned char*>(base);
     for (const Piece& pc : pieces) {
         GemmBatchDev d;
-        d.dma = pc.hb.dma.empty() ? nullptr : reinterpret_cast<const Prob*>(b + pc.off_dma);
-        d.ndma = (int)pc.hb.dma.size();
-        d.tiles_dma = pc.hb.tiles_dma;
-        d.dmae = pc.hb.dmae.empty() ? nullptr : reinterpret_cast<const Prob*>(b + pc.off_dmae);
-        d.ndmae = (int)pc.hb.dmae.size();
-        d.tiles_dmae = pc.hb.tiles_dmae;
-        d.gen = pc.hb.gen.empty() ? nullptr : reinterpret_cast<const Prob*>(b + pc.off_gen);
-        d.ngen = (int)pc.hb.gen.size();
-        d.tiles_gen[0] = pc.hb.tiles_gen[0];
-        d.tiles_gen[1] = pc.hb.tiles_gen[1];
-        d.vec = pc.hb.vec;
+        d.dma = reinterpret_cast<const Prob*>(b + pc.off_dma);
+        d.dmae = reinterpret_cast<const Prob*>(b + pc.off_dmae);
+        for (int w = 0; w < 2; ++w) d.gen[w] = reinterpret_cast<const Prob*>(b + pc.off_gen[w]);
         d.segs = reinterpret_cast<const Seg*>(b + pc.off_seg);
-        rc = launch_gemm_f64_dev(pc.opA, pc.opB, DG_GEMM_MODE_ROUND_ROBIN, default_tile_cfg(), d, nullptr, st);
+        d.set_counts(pc.hb);
+        rc = launch_gemm_f64_dev(pc.opA, pc.opB, DG_GEMM_MODE_ROUND_ROBIN, d, nullptr, st);
         if (rc) return rc;
     }
     return DG_OK;
@@ -686,11 +688,10 @@ int dg_grouped_plan_create_form(const dg_gemm_desc* descs, int count, int mode, 
     p->form = form;
     p->moduli_req = moduli;
     (void)hipGetDevice(&p->device);
-    p->shape_key = shape_class(descs, count);
+    p->shape_key = "t3:" + shape_class(descs, count);  // three tile choices: entries of other choices stay unread
     if (form == DG_FORM_OZAKI_INT8) p->shape_key = "oz" + std::to_string(moduli) + ":" + p->shape_key;
     if (mode == DG_PLAN_NONPERSISTENT) p->variant = DG_GEMM_MODE_ROUND_ROBIN;
     if (mode == DG_PLAN_PERSISTENT) p->variant = DG_GEMM_MODE_PERSISTENT;
-    p->cfg = default_tile_cfg();
     auto cleanup = [&](int code) { dg_grouped_plan_destroy(p); return code; };
     if (hipMalloc(&p->counter, sizeof(int)) != hipSuccess) return cleanup(fail(DG_ERR_ALLOC, "plan: counter alloc"));
     for (int i = 0; i < count; ++i)
@@ -776,14 +777,7 @@ int dg_grouped_plan_destroy(dg_grouped_plan* p) {
     if (p->oz_shared) (void)hipFree(p->oz_shared);
     if (p->graph) (void)hipGraphExecDestroy(p->graph);
     if (p->capture_stream) (void)hipStreamDestroy(p->capture_stream);
-    for (auto& g : p->groups) {
-        if (g.b.dma) (void)hipFree(const_cast<dg::Prob*>(g.b.dma));
-        if (g.b.dmae) (void)hipFree(const_cast<dg::Prob*>(g.b.dmae));
-        if (g.b.gen) (void)hipFree(const_cast<dg::Prob*>(g.b.gen));
-        for (const dg::Prob* t : g.b.nar)
-            if (t) (void)hipFree(const_cast<dg::Prob*>(t));
-        if (g.b.segs) (void)hipFree(const_cast<dg::Seg*>(g.b.segs));
-    }
+    if (p->tables) (void)hipFree(p->tables);
     if (p->counter) (void)hipFree(p->counter);
     delete p;
     return DG_OK;
