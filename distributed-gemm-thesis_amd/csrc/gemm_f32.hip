@@ -30,8 +30,16 @@
 // Interior problems with a k-contiguous operand (opA = T, or opA = opB = N)
 // run sgemm_dma_xr_kernel instead, which keeps that operand in registers and
 // only the other in LDS (+2.3 % at NN 16384^3; described at the kernel), and
-// uneven ones are cut into such an interior block and edge strips
-// (run_sgemm_dma), with the same bits as the whole problem on this kernel.
+// uneven ones are cut into such an interior block and strips (run_sgemm).
+//
+// sgemm_kernel stages both operands through registers on 64x64 or 32x32
+// tiles: operands the direct loads do not take (bases off 16-byte alignment,
+// leading dimensions not multiples of 4, K % 4 != 0 with a k-contiguous
+// operand), strips, products too small to fill the chip with 128x128 tiles,
+// and long-K products of any size (run_sgemm chooses; all kernels give the
+// same bits).  TFLOP/s before (FMA kernel without matrix cores, or 128x128
+// tiles) and after: 4001^3 38.8 -> 136.5, 1537 x 2051 x 1023 28.5 -> 93.8, 512^3
+// 7.7 -> 36.7, 1024^3 31.5 -> 90, 3072^3 105.9 -> 142.8, 4096^3 142.2 -> 146.1.
 //
 // Edges: rows past the end of a k-contiguous operand read its last row;
 // row chunks past the end of a row-contiguous operand read the last 16-byte
@@ -39,16 +47,18 @@
 // the products of those rows land only in unstored rows / columns of C.
 // k past K reads a zero page (K must be a multiple of 4 when an operand is
 // k-contiguous, so a 16-byte chunk never straddles K), and an odd step count
-// gets one zero step.  Operands that are not 16-byte aligned, leading
-// dimensions that are not multiples of 4, or K % 4 != 0 with a k-contiguous
-// operand run sgemm_generic_kernel (LDS-tiled FMA) instead.
+// gets one zero step.
+#include <algorithm>
+#include <cstdlib>
+#include <string>
+
 #include "dg_internal.hpp"
+#include "staged.hpp"
 
 namespace dg {
 
 namespace {
 
-typedef float fv4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void gvoid_t;
 
@@ -161,6 +171,7 @@ struct SgemmArgs {
     float alpha, beta;
     int tiles_m, tiles_n;
     int cvec;  // C 16-byte aligned with ldc % 4 == 0: vector stores
+    int by_elements;  // sgemm_kernel: operands that Staged::read does not take
 };
 
 __device__ __forceinline__ int xcd_remap(int bid, int total) {
@@ -504,57 +515,220 @@ __global__ __launch_bounds__(256, 2) void sgemm_dma_xr_kernel(SgemmArgs P) {
     }
 }
 
-// Any layout: 64x64 tiles, k-steps of 16 staged through LDS with guarded
-// loads (zeros past the edges), each thread a 4x4 block of C in FP32 FMAs.
-__global__ __launch_bounds__(256) void sgemm_generic_kernel(int ta, int tb, SgemmArgs P) {
-    __shared__ float As[16][64 + 1];
-    __shared__ float Bs[16][64 + 1];
-    const int t = threadIdx.x;
-    const int tx = t & 15, ty = t >> 4;
-    const int64_t m0 = (int64_t)blockIdx.x * 64, n0 = (int64_t)blockIdx.y * 64;
-    float acc[4][4] = {};
-    for (int64_t k0 = 0; k0 < P.k; k0 += 16) {
+// Register-staged form for any layout (Staged) and for problems too small
+// to fill the chip with 128x128 tiles: T x T tiles of four waves of T/2 x T/2,
+// BK-deep stages, two in flight in registers, two LDS buffers and one barrier
+// per stage, placed as in gemm_f64_kernel (a 16-deep part's fragments are
+// read while the part before it is multiplied).  The k order of an element
+// is sgemm_dma_kernel's: lane group lg supplies k = 4lg + s of a 16-deep step
+// to MFMA s, A the first operand, so the tile choice changes no bit (but the
+// sign of an exactly zero sum).
+// A row-contiguous operand's block row r stands for row F*r + i of block i, so
+// that a lane's rows of all F blocks are one LDS read.
+template <int T_, int BK_, int OCC_>
+struct SgemmTile {
+    static constexpr int T = T_, BK = BK_, OCC = OCC_, W = T / 2, F = W / 16, H = BK / 16;
+    static_assert(H % 2 == 0, "fragment set of part h: h & 1");
+};
+using Sgemm64 = SgemmTile<64, 32, 4>;
+using Sgemm32 = SgemmTile<32, 64, 3>;
+
+// f[i][s] = X(row(i), k = 16h + 4lg + s), row(i) = w0 + 16i + lr for a
+// k-contiguous operand and w0 + F*lr + i for a row-contiguous one.
+template <class O, bool KC, int F>
+__device__ __forceinline__ void staged_fragments(float (&f)[F][4], const char* s, int w0, int lr, int lg, int h) {
+    if constexpr (KC) {
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+            const fv4 v = *reinterpret_cast<const fv4*>(s + (w0 + 16 * i + lr) * O::LROW + (16 * h + 4 * lg) * 4);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) f[i][q] = v[q];
+        }
+    } else {
+        typedef float fvF __attribute__((ext_vector_type(F)));
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const int e = t + 256 * q;
-            // A: element (row, kk) of op(A); stored (row, kk) at row + kk*lda (N) or kk + row*lda (T)
-            int r, kk;
-            if (!ta) { r = e & 63; kk = e >> 6; } else { kk = e & 15; r = e >> 4; }
-            int64_t gr = m0 + r, gk = k0 + kk;
-            As[kk][r] = (gr < P.m && gk < P.k) ? (ta ? P.a[gk + gr * P.lda] : P.a[gr + gk * P.lda]) : 0.f;
-            // B: element (kk, col) of op(B); stored at kk + col*ldb (N) or col + kk*ldb (T)
-            if (!tb) { kk = e & 15; r = e >> 4; } else { r = e & 63; kk = e >> 6; }
-            gr = n0 + r; gk = k0 + kk;
-            Bs[kk][r] = (gr < P.n && gk < P.k) ? (tb ? P.b[gr + gk * P.ldb] : P.b[gk + gr * P.ldb]) : 0.f;
-        }
-        __syncthreads();
+            const fvF v = *reinterpret_cast<const fvF*>(s + (16 * h + 4 * lg + q) * O::LROW + (w0 + F * lr) * 4);
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][tx + 16 * i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][ty + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int64_t m = m0 + tx + 16 * i;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t n = n0 + ty + 16 * j;
-            if (m >= P.m || n >= P.n) continue;
-            float* cp = P.c + m + n * P.ldc;
-            float val = P.alpha * acc[i][j];
-            if (P.beta != 0.f) val = fmaf(P.beta, *cp, val);
-            *cp = val;
+            for (int i = 0; i < F; ++i) f[i][q] = v[i];
         }
     }
+}
+
+template <class C, bool AK, bool BKC>
+__global__ __launch_bounds__(256, C::OCC) void sgemm_kernel(SgemmArgs P) {
+    constexpr int T = C::T, BK = C::BK, F = C::F, H = C::H;
+    using OA = Staged<float, AK, T, BK>;
+    using OB = Staged<float, BKC, T, BK>;
+    constexpr int STAGE = OA::BYTES + OB::BYTES;
+    __shared__ __attribute__((aligned(16))) char lds[2 * STAGE];
+    const int64_t bid = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+    if (bid >= P.tiles_m * P.tiles_n) return;
+    const int tile = xcd_remap((int)bid, P.tiles_m * P.tiles_n);
+    const int per_group = sk::GROUP_M * P.tiles_n;
+    const int group = tile / per_group;
+    const int first_m = group * sk::GROUP_M;
+    const int gsize = min(P.tiles_m - first_m, sk::GROUP_M);
+    const int in_group = tile - group * per_group;
+    const int64_t m0 = (int64_t)(first_m + in_group % gsize) * T;
+    const int64_t n0 = (int64_t)(in_group / gsize) * T;
+    const int rows = (int)min(P.m - m0, (int64_t)T), cols = (int)min(P.n - n0, (int64_t)T);
+
+    const int lane = threadIdx.x & 63;
+    const int wave = threadIdx.x >> 6;
+    const int wm = (wave >> 1) * C::W, wn = (wave & 1) * C::W;
+    const int lr = lane & 15, lg = lane >> 4;
+
+    OA oa;
+    OB ob;
+    oa.start(P.a, P.lda, m0, rows);
+    ob.start(P.b, P.ldb, n0, cols);
+    int64_t left = P.k;  // k from the next stage to read on (0 or less: past the end)
+    fv4 va[2][OA::NL], vb[2][OB::NL];
+    auto read = [&](int d) {
+        if (left <= 0) return;
+        if (!P.by_elements && left > BK) {
+            oa.read(va[d]);
+            ob.read(vb[d]);
+        } else {
+            const int real = (int)min(left, (int64_t)BK);
+            oa.read_last(va[d], real, rows);
+            ob.read_last(vb[d], real, cols);
+        }
+        left -= BK;
+    };
+    auto store = [&](char* buf, int d) {
+        OA::store(buf, va[d]);
+        OB::store(buf + OA::BYTES, vb[d]);
+    };
+    float fa[2][F][4], fb[2][F][4];
+    auto fragments = [&](const char* buf, int h) {
+        staged_fragments<OA, AK>(fa[h & 1], buf, wm, lr, lg, h);
+        staged_fragments<OB, BKC>(fb[h & 1], buf + OA::BYTES, wn, lr, lg, h);
+    };
+    fv4 acc[F][F];
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = fv4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int h, int half) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int q = 2 * half; q < 2 * half + 2; ++q)
+#pragma unroll
+            for (int i = 0; i < F; ++i)
+#pragma unroll
+                for (int j = 0; j < F; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[h & 1][i][q], fb[h & 1][j][q], acc[i][j], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    const int64_t ns = (P.k + BK - 1) / BK;
+    read(0);
+    read(1);
+    store(lds, 0);
+    read(0);
+    __syncthreads();
+    char* const bufs[2] = {lds, lds + STAGE};
+    fragments(lds, 0);
+    // Two stages a turn: s, even, in buffer 0, and s + 1; stage s + 1 waits in
+    // register set (s + 1) % 2.  Turns that read only whole stages run without
+    // conditions.
+    const int64_t turns = !P.by_elements && left > 0 ? (left - 1) / (2 * BK) : 0;
+    for (int64_t i = 0; i < turns; ++i) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                if (h < H - 1) {
+                    fragments(bufs[u], h + 1);
+                } else {
+                    __syncthreads();
+                    fragments(bufs[u ^ 1], 0);
+                }
+                multiply(h, 0);
+                if (h == H - 2) {
+                    store(bufs[u ^ 1], u ^ 1);
+                    oa.read(va[u ^ 1]);
+                    ob.read(vb[u ^ 1]);
+                }
+                multiply(h, 1);
+            }
+    }
+    left -= 2 * BK * turns;
+    for (int64_t s = 2 * turns; s < ns;) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u, ++s) {
+            if (s >= ns) break;
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+                if (h < H - 1) {
+                    fragments(bufs[u], h + 1);
+                } else if (s + 1 < ns) {
+                    __syncthreads();
+                    fragments(bufs[u ^ 1], 0);
+                }
+                multiply(h, 0);
+                if (h == H - 2 && s + 1 < ns) {
+                    store(bufs[u ^ 1], u ^ 1);
+                    read(u ^ 1);
+                }
+                multiply(h, 1);
+            }
+        }
+    }
+
+    // acc[i][j][v] = sum for C(m0 + wm + row(i, 4lg + v), n0 + wn + row(j, lr)),
+    // row(i, r) = 16i + r for a k-contiguous operand and F*r + i for a
+    // row-contiguous one: for each column a lane holds 4F rows, in runs of four
+    // consecutive ones (one 16-byte store at any alignment each).  The old
+    // values are requested together before the first is used.
+    const float alpha = P.alpha, beta = P.beta;
+    typedef __attribute__((address_space(1))) float gf;
+    typedef __attribute__((address_space(1))) Vec16<float>::any gf4;
+    const bool inside = rows == T && cols == T;
+    const int64_t nc = n0 + wn, mc = m0 + wm;
+    auto row_of = [&](int b) { return mc + (AK ? 16 * b + 4 * lg : 4 * F * lg + 4 * b); };  // of run b
+    auto col_of = [&](int j) { return nc + (BKC ? 16 * j + lr : F * lr + j); };
+    auto sum_of = [&](int b, int j, int v) {
+        if constexpr (AK) return acc[b][j][v];
+        else return acc[(4 * b + v) % F][j][(4 * b + v) / F];
+    };
+    fv4 old[F][F];
+    if (beta != 0.f) {
+#pragma unroll
+        for (int j = 0; j < F; ++j)
+#pragma unroll
+            for (int b = 0; b < F; ++b) {
+                const int64_t m = row_of(b), n = col_of(j);
+                if (inside) {
+                    old[b][j] = *(gf4*)(P.c + m + n * P.ldc);
+                } else {
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        old[b][j][v] = *(gf*)(P.c + (m + v < P.m ? m + v : P.m - 1) + (n < P.n ? n : P.n - 1) * P.ldc);
+                }
+            }
+    }
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+        for (int b = 0; b < F; ++b) {
+            const int64_t m = row_of(b), n = col_of(j);
+            fv4 val;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                val[v] = alpha * sum_of(b, j, v);
+                if (beta != 0.f) val[v] = fmaf(beta, old[b][j][v], val[v]);
+            }
+            if (inside) {
+                *(gf4*)(P.c + m + n * P.ldc) = val;
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                    if (m + v < P.m && n < P.n) *(gf*)(P.c + m + v + n * P.ldc) = val[v];
+            }
+        }
 }
 
 __global__ void sgemm_scale_kernel(int64_t m, int64_t n, float beta, float* __restrict__ C, int64_t ldc) {
@@ -584,38 +758,80 @@ void launch_sgemm_dma(bool edge, const SgemmArgs& a, int tiles, hipStream_t st) 
         hipLaunchKernelGGL((sgemm_dma_kernel<AK, BKC, false>), dim3(tiles), dim3(256), sk::LDS_BYTES, st, a);
 }
 
-// One direct-to-LDS problem.  With a k-contiguous operand, whole even
-// k-steps and at least 8 whole interior tiles, an uneven problem is cut into
-// its interior block (register-operand kernel) and the strips after it (rows
-// past the interior, then the columns past it beside the interior rows),
-// which run the edge kernel: the cut adds no tiles, and since both kernels
-// sum every element in the same order it changes no result bit.
+template <class C, bool AK, bool BKC>
+void launch_sgemm(SgemmArgs a, hipStream_t st) {
+    a.tiles_m = (int)((a.m + C::T - 1) / C::T);
+    a.tiles_n = (int)((a.n + C::T - 1) / C::T);
+    a.by_elements = !Staged<float, AK, C::T, C::BK>::takes(a.a, a.lda) || !Staged<float, BKC, C::T, C::BK>::takes(a.b, a.ldb);
+    hipLaunchKernelGGL((sgemm_kernel<C, AK, BKC>), tile_grid(a.tiles_m * a.tiles_n), dim3(256), 0, st, a);
+}
+
+// Time (us) of one launch, to choose between the tiles: the fullest CU's c
+// tiles at the rate that as many reach (eff), plus 4 us of prologue and
+// epilogue per round of `conc` resident tiles.  Measured rates, share of 157.3
+// TFLOP/s: 128x128 direct to LDS 0.83 with one tile per CU, 0.92 with more
+// (0.90 with no operand in registers: opA = N, opB = T); 64x64 0.74, 0.84, 0.87,
+// 0.89 with one to four, 0.94 with more, 0.915 past 128, where its operands
+// come from beyond the L2; 32x32 0.62, 0.69, 0.73, 0.75, 0.80.  So 64x64 wins at
+// long K (4096^3: 941 us against 967), 128x128 at short K (8192 x 8192 x 256:
+// 273 us against 302) and in the largest NN products (16384^3: 60.9 ms against
+// 61.2), 32x32 where it fills CUs that 64x64 leaves idle (512^3: 7.3 us against
+// 13.3).
+double sgemm_time(int64_t m, int64_t n, int64_t k, int t, int conc, const double* eff) {
+    const int64_t c = (((m + t - 1) / t) * ((n + t - 1) / t) + 255) / 256;
+    const double u = 2.0 * t * t * (double)k / (157.3e6 / 256);
+    return (double)c * u / eff[c >= 128 ? 5 : c >= 8 ? 4 : std::min<int64_t>(c, 4) - 1] + 4.0 * std::max(1.0, (double)c / conc);
+}
+constexpr double kEffDma[2][6] = {{0.83, 0.90, 0.90, 0.90, 0.90, 0.90}, {0.83, 0.90, 0.91, 0.92, 0.92, 0.92}};
+constexpr double kEff64[6] = {0.74, 0.84, 0.87, 0.89, 0.94, 0.915}, kEff32[6] = {0.62, 0.69, 0.73, 0.75, 0.80, 0.78};
+
+// One problem.  The direct-to-LDS kernels take it when `dma`: cut, with a
+// k-contiguous operand, whole even k-steps and at least 8 whole interior
+// tiles, into its interior block (register-operand kernel) and strips after
+// it (rows past the interior, then the columns past it beside the interior
+// rows), which the register-staged kernel runs; else whole on the edge kernel.
+// The register-staged kernel takes the others, and those whose estimated time
+// on 64x64 or 32x32 tiles is less: 128x128 tiles leave CUs idle until there
+// are a few hundred of them.  Every kernel sums an element in the same order:
+// neither the cut nor the tile changes a result bit.  DG_GEMM_TILE forces a
+// choice.
 template <bool AK, bool BKC>
-void run_sgemm_dma(const SgemmArgs& a, hipStream_t st) {
-    auto one = [&](SgemmArgs p) {
+void run_sgemm(const SgemmArgs& a, bool dma, hipStream_t st) {
+    static const std::string forced = [] { const char* e = getenv("DG_GEMM_TILE"); return std::string(e ? e : ""); }();
+    static const bool no_areg = getenv("DG_GEMM_NO_AREG") != nullptr;
+    auto direct = [&](SgemmArgs p) {
         p.tiles_m = (int)((p.m + sk::BM - 1) / sk::BM);
         p.tiles_n = (int)((p.n + sk::BN - 1) / sk::BN);
         const int64_t steps = (p.k + sk::BK - 1) / sk::BK;
         const bool edge = p.m % sk::BM || p.n % sk::BN || p.k % sk::BK || (steps & 1);
         launch_sgemm_dma<AK, BKC>(edge, p, p.tiles_m * p.tiles_n, st);
     };
-    static const bool no_areg = getenv("DG_GEMM_NO_AREG") != nullptr;
+    auto staged = [&](const SgemmArgs& p) {
+        const bool small = forced == "32x32" || (forced != "64x64" && sgemm_time(p.m, p.n, p.k, 32, 4, kEff32) < sgemm_time(p.m, p.n, p.k, 64, 4, kEff64));
+        if (small) launch_sgemm<Sgemm32, AK, BKC>(p, st); else launch_sgemm<Sgemm64, AK, BKC>(p, st);
+    };
     const int64_t mi = a.m / sk::BM * sk::BM, ni = a.n / sk::BN * sk::BN;
     const bool k_ok = a.k % sk::BK == 0 && !((a.k / sk::BK) & 1);
-    if (!(AK || BKC) || no_areg || !k_ok || (mi == a.m && ni == a.n) || mi * ni < 8 * sk::BM * sk::BN) {
-        one(a);
-        return;
+    const bool cut = (AK || BKC) && !no_areg && k_ok && (mi != a.m || ni != a.n) && mi * ni >= 8 * sk::BM * sk::BN;
+    if (dma && forced != "128x128") {
+        auto least = [&](int64_t m, int64_t n) { return std::min(sgemm_time(m, n, a.k, 64, 4, kEff64), sgemm_time(m, n, a.k, 32, 4, kEff32)); };
+        double t = sgemm_time(cut ? mi : a.m, cut ? ni : a.n, a.k, 128, 2, kEffDma[AK || BKC]);
+        if (cut && mi < a.m) t += least(a.m - mi, a.n);
+        if (cut && ni < a.n) t += least(mi, a.n - ni);
+        dma = forced.empty() && t <= least(a.m, a.n);
     }
+    if (!dma) return staged(a);
+    if (!cut) return direct(a);
     SgemmArgs in = a;
     in.m = mi;
     in.n = ni;
-    one(in);
+    direct(in);
     if (mi < a.m) {
         SgemmArgs s = a;  // rows mi .. m of every column
         s.a = AK ? a.a + mi * a.lda : a.a + mi;
         s.c = a.c + mi;
         s.m = a.m - mi;
-        one(s);
+        staged(s);
     }
     if (ni < a.n) {
         SgemmArgs s = a;  // columns ni .. n of rows 0 .. mi
@@ -623,7 +839,7 @@ void run_sgemm_dma(const SgemmArgs& a, hipStream_t st) {
         s.c = a.c + ni * a.ldc;
         s.m = mi;
         s.n = a.n - ni;
-        one(s);
+        staged(s);
     }
 }
 
@@ -663,18 +879,13 @@ extern "C" int dg_sgemm(char opA, char opB, int64_t m, int64_t n, int64_t k, flo
     const int64_t tm = (m + sk::BM - 1) / sk::BM, tn = (n + sk::BN - 1) / sk::BN;
     if (tm * tn > INT32_MAX || (m + 63) / 64 > INT32_MAX || (n + 63) / 64 > 65535)
         return fail(DG_ERR_INVALID, "dg_sgemm: %lld x %lld output is too large", (long long)m, (long long)n);
-    SgemmArgs a{A, B, C, lda, ldb, ldc, m, n, k, alpha, beta, (int)tm, (int)tn, 0};
+    SgemmArgs a{A, B, C, lda, ldb, ldc, m, n, k, alpha, beta, 0, 0, 0, 0};
     a.cvec = aligned16(C) && ldc % 4 == 0;
     const bool dma = aligned16(A) && aligned16(B) && lda % 4 == 0 && ldb % 4 == 0 && (!(ak || bkc) || k % 4 == 0);
-    if (dma) {
-        if (ak && bkc) run_sgemm_dma<true, true>(a, st);
-        else if (ak) run_sgemm_dma<true, false>(a, st);
-        else if (bkc) run_sgemm_dma<false, true>(a, st);
-        else run_sgemm_dma<false, false>(a, st);
-    } else {
-        hipLaunchKernelGGL(sgemm_generic_kernel, dim3((unsigned)((m + 63) / 64), (unsigned)((n + 63) / 64)), dim3(256),
-                           0, st, (int)ak, (int)(ob == 'T'), a);
-    }
+    if (ak && bkc) run_sgemm<true, true>(a, dma, st);
+    else if (ak) run_sgemm<true, false>(a, dma, st);
+    else if (bkc) run_sgemm<false, true>(a, dma, st);
+    else run_sgemm<false, false>(a, dma, st);
     DG_LAUNCH_CHECK();
     return DG_OK;
 }

@@ -34,25 +34,19 @@
 #include <string>
 
 #include "dg_internal.hpp"
+#include "staged.hpp"
 
 namespace dg {
 
 namespace {
 
-typedef double dv2 __attribute__((ext_vector_type(2)));
 typedef double dv4 __attribute__((ext_vector_type(4)));
 
 // Global-address-space views: loads through them compile to global_load_*
 // (counted by vmcnt only), not flat_load_*, whose lgkmcnt share would make
 // every LDS wait also wait for the prefetch of the next k-step.
-typedef __attribute__((address_space(1))) const double gdouble;
 typedef __attribute__((address_space(1))) const dv2 gdv2;
-__device__ __forceinline__ double gld(const double* p) { return *(gdouble*)p; }
 __device__ __forceinline__ dv2 gld2(const double* p) { return *(gdv2*)p; }
-// a pair at any element alignment: one 16-byte load all the same
-typedef dv2 dv2u __attribute__((aligned(8)));
-typedef __attribute__((address_space(1))) const dv2u gdv2u;
-__device__ __forceinline__ dv2 gld2u(const double* p) { return *(gdv2u*)p; }
 
 constexpr int GROUP_M = 8;   // tile rows per raster group
 
@@ -70,7 +64,6 @@ struct TileCfg {
 };
 using Cfg64 = TileCfg<64, 64, 32, 32, 16, 2, 4>;
 using Cfg32 = TileCfg<32, 32, 16, 16, 32, 2, 3>;
-constexpr int64_t kMaxPairLd = (1 << 22) - 64;  // 8 * (127 ld + BK) stays below 2^32
 constexpr int64_t kNarrowMax = 32;  // problems and strips up to this many rows or columns wide take the 32 x 32 tiles
 
 // Block id -> tile id so that each XCD (blocks are dealt round-robin to the
@@ -83,111 +76,27 @@ __device__ __forceinline__ int xcd_remap(int bid, int total) {
     return x * q + min(x, r) + slot;
 }
 
-// One operand of the register-staged kernel: BK-deep stages of ROWS rows,
-// loaded in 16-byte pairs at whatever alignment the matrix has (the hardware
-// takes unaligned global loads; a pair per load instead of two elements is
-// what lets odd leading dimensions run like even ones), stored to LDS in the
-// direction memory has so that both the store and the fragment reads are
-// conflict-free runs.
-//  * KC, element (row, k) at base[k + row*ld]: a thread takes the k pair
-//    kt = 2*(t % CH) of rows t/CH + RPP*q; LDS [row][k], rows padded by one
-//    pair.
-//  * else, element (row, k) at base[row + k*ld]: a thread takes the row pair
-//    2*(t % HP) of k kt + KPP*q, kt = t/HP; LDS [k][row], k-rows padded by 64
-//    bytes.
-// Rows past the end are read from the last row; they feed only outputs that
-// are never stored.  A segment's last stage is read by elements (read_last),
-// with k past the end turned into zeros; in the stages before it every pair
-// is inside the matrix: a pair that starts at the last row ends at the next
-// k's first row or in the columns' padding.
-// An FP64 MFMA runs on the vector ALU's own pipes, so every vector
-// instruction of the loop is time taken from the product (1.4 to 3.7 of them
-// per MFMA cost a fifth of the rate): a whole stage uses none but the memory
-// instructions, with a scalar base that moves and 32-bit lane offsets that
-// stay.  The compiler counts loads in flight only along straight code, so
-// whole stages also have no branch around their loads (with one it waited
-// for all of them every stage).
-template <bool KC, int ROWS, int BK>
-struct Staged {
-    static constexpr int CH = BK / 2, RPP = 256 / CH;          // KC
-    static constexpr int HP = ROWS / 2, KPP = 256 / HP;        // else
-    static constexpr int NL = ROWS * BK / 512;                 // loads per thread and stage
-    static constexpr int LROW = KC ? (BK + 2) * 8 : ROWS * 8 + 64;  // bytes
-    static constexpr int BYTES = KC ? ROWS * LROW : BK * LROW;
-
-    const double* base;   // the tile's first row at the next stage's first k (uniform)
-    int64_t ld;
-    uint32_t off[NL];     // bytes from it to this thread's pairs
-
-    // row of this thread's pair q within the tile, k of it within the stage
-    static __device__ __forceinline__ int row(int q) { return KC ? (int)threadIdx.x / CH + RPP * q : 2 * ((int)threadIdx.x % HP); }
-    static __device__ __forceinline__ int kk(int q) { return KC ? 2 * ((int)threadIdx.x % CH) : (int)threadIdx.x / HP + KPP * q; }
-
-    // At a segment's first k; the tile has `rows` rows from row0 on.
-    __device__ __forceinline__ void start(const double* x, int64_t ld_, int64_t row0, int rows) {
-        ld = ld_;
-        base = x + row0 * (KC ? ld : 1);
+// f[i][q] = X(row w0 + 16i + lr, k = 8h + 2lg + q) of a stage of operand O.
+template <class O, bool KC, int F>
+__device__ __forceinline__ void staged_fragments(double (&f)[F][2], const char* s, int w0, int lr, int lg, int h) {
 #pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            const uint32_t r = min(row(q), rows - 1), k = kk(q);
-            off[q] = 8u * (KC ? r * (uint32_t)ld + k : k * (uint32_t)ld + r);
+    for (int i = 0; i < F; ++i) {
+        if constexpr (KC) {
+            const dv2 v = *reinterpret_cast<const dv2*>(s + (w0 + 16 * i + lr) * O::LROW + (8 * h + 2 * lg) * 8);
+            f[i][0] = v.x;
+            f[i][1] = v.y;
+        } else {
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                f[i][q] = *reinterpret_cast<const double*>(s + (8 * h + 2 * lg + q) * O::LROW + (w0 + 16 * i + lr) * 8);
         }
     }
-    __device__ __forceinline__ void advance() {
-        base += KC ? BK : BK * ld;
-        asm volatile("" : "+s"(base));  // stays a scalar: not folded into vector address increments
-    }
-    __device__ __forceinline__ void read(dv2 (&v)[NL]) {
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            asm volatile("" : "+v"(off[q]));  // stays 32 bits: the load adds it to the scalar base itself
-            v[q] = gld2u((const double*)((const char*)base + off[q]));
-        }
-        advance();
-    }
-    // The segment's last stage, `left` <= BK of its k real (or any stage of a
-    // matrix that read() does not take).
-    __device__ __forceinline__ void read_last(dv2 (&v)[NL], int left, int rows) {
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            const int r = min(row(q), rows - 1), k = min(kk(q), left - 1);
-            const double* x = base + (KC ? r * ld + k : k * ld + r);
-            v[q] = dv2{gld(x), gld(x + (KC ? k + 1 < left : r + 1 < rows))};
-        }
-#pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            const int k = kk(q);
-            v[q] = dv2{k < left ? v[q].x : 0.0, (KC ? k + 1 : k) < left ? v[q].y : 0.0};
-        }
-        advance();
-    }
-    static __device__ __forceinline__ void store(char* s, const dv2 (&v)[NL]) {
-#pragma unroll
-        for (int q = 0; q < NL; ++q)
-            *reinterpret_cast<dv2*>(s + (KC ? row(q) * LROW + kk(q) * 8 : kk(q) * LROW + row(q) * 8)) = v[q];
-    }
-    // f[i][q] = X(row w0 + 16i + lr, k = 8h + 2lg + q)
-    template <int F>
-    static __device__ __forceinline__ void fragments(double (&f)[F][2], const char* s, int w0, int lr, int lg, int h) {
-#pragma unroll
-        for (int i = 0; i < F; ++i) {
-            if constexpr (KC) {
-                const dv2 v = *reinterpret_cast<const dv2*>(s + (w0 + 16 * i + lr) * LROW + (8 * h + 2 * lg) * 8);
-                f[i][0] = v.x;
-                f[i][1] = v.y;
-            } else {
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-                    f[i][q] = *reinterpret_cast<const double*>(s + (8 * h + 2 * lg + q) * LROW + (w0 + 16 * i + lr) * 8);
-            }
-        }
-    }
-};
+}
 
 template <class C, bool TA, bool TB>
 struct TileLds {
-    using OA = Staged<TA, C::BM, C::BK>;    // op(A) is k-contiguous when A is transposed
-    using OB = Staged<!TB, C::BN, C::BK>;   // op(B) when B is not
+    using OA = Staged<double, TA, C::BM, C::BK>;    // op(A) is k-contiguous when A is transposed
+    using OB = Staged<double, !TB, C::BN, C::BK>;   // op(B) when B is not
     static constexpr int STAGE = OA::BYTES + OB::BYTES;
 };
 
@@ -288,8 +197,8 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     static_assert(H % 2 == 0, "fragment set of part h: h & 1");
     double fa[2][FM][2], fb[2][FN][2];
     auto fragments = [&](const char* buf, int h) {
-        OA::template fragments<FM>(fa[h & 1], buf, wm, lr, lg, h);
-        OB::template fragments<FN>(fb[h & 1], buf + OA::BYTES, wn, lr, lg, h);
+        staged_fragments<OA, TA>(fa[h & 1], buf, wm, lr, lg, h);
+        staged_fragments<OB, !TB>(fb[h & 1], buf + OA::BYTES, wn, lr, lg, h);
     };
     auto multiply = [&](int h, int q) {
         __builtin_amdgcn_sched_barrier(0);
@@ -403,10 +312,9 @@ __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_kernel(const Prob* __
         const Prob P = probs[lo];
         gemm_tile<C, TA, TB>(P, segs, tile - P.tile0, lds);
     };
-    if (MODE == 0) {
-        run(blockIdx.x);
-    } else if (MODE == 1) {
-        run(xcd_remap(blockIdx.x, total_tiles));
+    if (MODE == 0 || MODE == 1) {
+        const int64_t bid = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+        if (bid < total_tiles) run(MODE == 0 ? (int)bid : xcd_remap((int)bid, total_tiles));
     } else {
         __shared__ int next;
         while (true) {
@@ -1031,9 +939,9 @@ template <class C, bool TA, bool TB>
 void launch_mode(int mode, const Prob* dp, int np, const Seg* ds, int tiles, int grid, int* counter,
                  hipStream_t st) {
     if (mode == DG_GEMM_MODE_ROUND_ROBIN)
-        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 0>), dim3(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
+        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 0>), tile_grid(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
     else if (mode == DG_GEMM_MODE_XCD)
-        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 1>), dim3(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
+        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 1>), tile_grid(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
     else
         hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 2>), dim3(grid), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
 }
@@ -1060,13 +968,13 @@ int launch_scale(int64_t m, int64_t n, double beta, double* C, int64_t ldc, hipS
     return DG_OK;
 }
 
-// Whether the register-staged kernel must load a problem by single elements:
-// bases off 8-byte alignment, or rows so far apart that a tile's offsets
-// leave 32 bits.
-static bool by_elements(const Prob& p, const std::vector<Seg>& segs) {
+// Whether the register-staged kernel must load a problem by single elements.
+static bool by_elements(const Prob& p, const std::vector<Seg>& segs, bool ak, bool bkc) {
+    using KC = Staged<double, true, 64, 16>;
+    using RC = Staged<double, false, 64, 16>;
     for (int s = p.seg0; s < p.seg0 + p.nseg; ++s) {
         const Seg& g = segs[s];
-        if (((reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b)) & 7) || g.lda > kMaxPairLd || g.ldb > kMaxPairLd)
+        if (!(ak ? KC::takes(g.a, g.lda) : RC::takes(g.a, g.lda)) || !(bkc ? KC::takes(g.b, g.ldb) : RC::takes(g.b, g.ldb)))
             return true;
     }
     return false;
@@ -1126,7 +1034,7 @@ static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, c
     auto add_gen = [&](Prob q) {
         const int w = tile == DG_GEMM_TILE_32x32 || q.m <= kNarrowMax || q.n <= kNarrowMax ? 1 : 0;
         const int64_t e = w ? 32 : 64;
-        q.shift = by_elements(q, out.segs) ? kByElements : 0;
+        q.shift = by_elements(q, out.segs, ak, bkc) ? kByElements : 0;
         q.tile0 = (int32_t)tgen[w];
         const int64_t n = ((q.m + e - 1) / e) * ((q.n + e - 1) / e);
         tgen[w] += n;

@@ -1,0 +1,127 @@
+// One operand of a register-staged GEMM tile (gemm_f64_kernel,
+// sgemm_kernel): global memory -> registers -> LDS.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <cstdint>
+
+namespace dg {
+
+typedef double dv2 __attribute__((ext_vector_type(2)));
+typedef float fv4 __attribute__((ext_vector_type(4)));
+
+// 16 bytes of a matrix at whatever alignment its elements have: one load all
+// the same (the hardware takes unaligned global loads).
+template <typename T> struct Vec16;
+template <> struct Vec16<double> {
+    typedef dv2 type;
+    typedef dv2 any __attribute__((aligned(8)));
+};
+template <> struct Vec16<float> {
+    typedef fv4 type;
+    typedef fv4 any __attribute__((aligned(4)));
+};
+
+// Grid of one workgroup of 256 threads per tile: a launch dimension holds
+// less than 2^32 threads, so tiles past 2^22 go on a second one (the last row
+// may run over `tiles`).
+inline dim3 tile_grid(int tiles) {
+    const unsigned x = tiles < (1 << 22) ? (unsigned)tiles : 1u << 22;
+    return dim3(x, ((unsigned)tiles + x - 1) / x);
+}
+
+// BK-deep stages of ROWS rows for a workgroup of 256 threads, loaded in runs
+// of E elements (16 bytes) at any alignment -- a run per load instead of
+// single elements is what lets odd leading dimensions run like even ones --
+// and stored to LDS in the direction memory has, so that both the stores and
+// the fragment reads are conflict-free.
+//  * KC, element (row, k) at base[k + row*ld]: a thread takes the run at
+//    k = E*(t % CH) of rows t/CH + RPP*q; LDS [row][k], rows padded by a run.
+//  * else, element (row, k) at base[row + k*ld]: a thread takes the run at row
+//    E*(t % HP) of k t/HP + KPP*q; LDS [k][row], k-rows padded by 128/E bytes
+//    (the k-rows that one MFMA reads, E apart, then fall in different halves
+//    of the banks).
+// Rows past the end are read from the last row; they feed only outputs that
+// are never stored.  A segment's last stage is read by elements (read_last),
+// with k past the end turned into zeros; in the stages before it every run
+// is inside the matrix: one that starts at the last row ends in the next k's
+// first rows or in the columns' padding (ld >= E - 1).
+// A whole stage uses no vector instruction but the memory ones: a scalar base
+// that moves and 32-bit lane offsets that stay.  An FP64 MFMA runs on the
+// vector ALU's own pipes, and 1.4 to 3.7 vector instructions per MFMA cost a
+// fifth of the rate.  The compiler counts loads in flight only along straight
+// code, so whole stages also have no branch around their loads (with one it
+// waited for all of them every stage).
+template <typename T, bool KC, int ROWS, int BK>
+struct Staged {
+    static constexpr int E = 16 / sizeof(T), S = sizeof(T);
+    static constexpr int CH = BK / E, RPP = 256 / CH;          // KC
+    static constexpr int HP = ROWS / E, KPP = 256 / HP;        // else
+    static constexpr int NL = ROWS * BK / (256 * E);           // loads per thread and stage
+    static constexpr int LROW = KC ? (BK + E) * S : ROWS * S + 128 / E;  // bytes
+    static constexpr int BYTES = KC ? ROWS * LROW : BK * LROW;
+    static_assert(256 % CH == 0 && 256 % HP == 0 && NL * 256 * E == ROWS * BK, "whole loads");
+    typedef typename Vec16<T>::type vec;
+    typedef __attribute__((address_space(1))) const typename Vec16<T>::any gvec;
+    typedef __attribute__((address_space(1))) const T gelem;
+
+    const T* base;     // the tile's first row at the next stage's first k (uniform)
+    int64_t ld;
+    uint32_t off[NL];  // bytes from it to this thread's runs
+
+    // row of this thread's run q within the tile, k of it within the stage
+    static __device__ __forceinline__ int row(int q) { return KC ? (int)threadIdx.x / CH + RPP * q : E * ((int)threadIdx.x % HP); }
+    static __device__ __forceinline__ int kk(int q) { return KC ? E * ((int)threadIdx.x % CH) : (int)threadIdx.x / HP + KPP * q; }
+
+    // At a segment's first k; the tile has `rows` rows from row0 on.
+    __device__ __forceinline__ void start(const T* x, int64_t ld_, int64_t row0, int rows) {
+        ld = ld_;
+        base = x + row0 * (KC ? ld : 1);
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            const uint32_t r = min(row(q), rows - 1), k = kk(q);
+            off[q] = (uint32_t)S * (KC ? r * (uint32_t)ld + k : k * (uint32_t)ld + r);
+        }
+    }
+    __device__ __forceinline__ void advance() {
+        base += KC ? BK : BK * ld;
+        asm volatile("" : "+s"(base));  // stays a scalar: not folded into vector address increments
+    }
+    __device__ __forceinline__ void read(vec (&v)[NL]) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q) {
+            asm volatile("" : "+v"(off[q]));  // stays 32 bits: the load adds it to the scalar base itself
+            v[q] = *(gvec*)((const char*)base + off[q]);
+        }
+        advance();
+    }
+    // The segment's last stage, `left` <= BK of its k real (or any stage of a
+    // matrix that read() does not take).
+    __device__ __forceinline__ void read_last(vec (&v)[NL], int left, int rows) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                const int64_t r = min(row(q) + (KC ? 0 : e), rows - 1), k = min(kk(q) + (KC ? e : 0), left - 1);
+                v[q][e] = *(gelem*)(base + (KC ? r * ld + k : k * ld + r));
+            }
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[q][e] = kk(q) + (KC ? e : 0) < left ? v[q][e] : T(0);
+        advance();
+    }
+    static __device__ __forceinline__ void store(char* s, const vec (&v)[NL]) {
+#pragma unroll
+        for (int q = 0; q < NL; ++q)
+            *reinterpret_cast<vec*>(s + (KC ? row(q) * LROW + kk(q) * S : kk(q) * LROW + row(q) * S)) = v[q];
+    }
+    // Whether read() takes a matrix: elements on their own alignment, and rows
+    // neither so far apart that a tile's offsets leave 32 bits nor so close
+    // that a run at the last row would pass the matrix's end.
+    static bool takes(const T* x, int64_t ld) {
+        return !(reinterpret_cast<uintptr_t>(x) & (S - 1)) && ld <= ((int64_t)1 << 32) / (128 * S) - 128 && (KC || ld >= E - 1);
+    }
+};
+
+}  // namespace dg

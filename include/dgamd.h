@@ -61,10 +61,8 @@ int dg_dgemm(char opA, char opB, int64_t m, int64_t n, int64_t k,
 
 /* C = alpha*op(A)*op(B) + beta*C in FP32 on the FP32 matrix cores
  * (v_mfma_f32_16x16x4_f32; FP32 products and sums), same conventions as
- * dg_dgemm (column-major, 'N'/'T'/'C', beta == 0 does not read C).
- * 16-byte aligned A and B with lda, ldb multiples of 4 (and K a multiple of
- * 4 when an operand is stored contiguous along k) take the direct-to-LDS
- * kernel; other layouts a slower LDS-tiled FMA kernel.
+ * dg_dgemm (column-major, 'N'/'T'/'C', beta == 0 does not read C).  Any
+ * alignment and leading dimension runs on the matrix cores.
  * Replaces: the FP32 instantiations of the reference's GEMM entry points,
  *           slateGEMM<float> (src/Wrappers/Slate/slateWrapped.cpp:334-335)
  *           and cosmaPreDistributedOptimalGemm<float>
