@@ -519,7 +519,8 @@ __global__ __launch_bounds__(256, 2) void sgemm_dma_xr_kernel(SgemmArgs P) {
 // to fill the chip with 128x128 tiles: T x T tiles of four waves of T/2 x T/2,
 // BK-deep stages, two in flight in registers, two LDS buffers and one barrier
 // per stage, placed as in gemm_f64_kernel (a 16-deep part's fragments are
-// read while the part before it is multiplied).  The k order of an element
+// read while the part before it is multiplied, memory instructions one per
+// MFMA: 1024 x 1024 x 8192, one tile per CU, 147 -> 129 us, 2048^3 127 -> 124).  The k order of an element
 // is sgemm_dma_kernel's: lane group lg supplies k = 4lg + s of a 16-deep step
 // to MFMA s, A the first operand, so the tile choice changes no bit (but the
 // sign of an exactly zero sum).
@@ -611,17 +612,17 @@ __global__ __launch_bounds__(256, C::OCC) void sgemm_kernel(SgemmArgs P) {
     for (int i = 0; i < F; ++i)
 #pragma unroll
         for (int j = 0; j < F; ++j) acc[i][j] = fv4{0.f, 0.f, 0.f, 0.f};
-    auto multiply = [&](int h, int half) {
-        __builtin_amdgcn_sched_barrier(0);
+    auto products = [&](int h) {
 #pragma unroll
-        for (int q = 2 * half; q < 2 * half + 2; ++q)
+        for (int q = 0; q < 4; ++q)
 #pragma unroll
             for (int i = 0; i < F; ++i)
 #pragma unroll
                 for (int j = 0; j < F; ++j)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[h & 1][i][q], fb[h & 1][j][q], acc[i][j], 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
     };
+    // loads and stores of a stage, MFMAs of a part, LDS instructions of its fragments
+    constexpr int NL = OA::NL + OB::NL, NM = 4 * F * F, NF = (AK ? F : 4) + (BKC ? F : 4);
 
     const int64_t ns = (P.k + BK - 1) / BK;
     read(0);
@@ -635,26 +636,54 @@ __global__ __launch_bounds__(256, C::OCC) void sgemm_kernel(SgemmArgs P) {
     // register set (s + 1) % 2.  Turns that read only whole stages run without
     // conditions.
     const int64_t turns = !P.by_elements && left > 0 ? (left - 1) / (2 * BK) : 0;
-    for (int64_t i = 0; i < turns; ++i) {
+    auto turn = [&]() {
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int h = 0; h < H; ++h) {
+                __builtin_amdgcn_sched_barrier(0);
                 if (h < H - 1) {
                     fragments(bufs[u], h + 1);
+#pragma unroll
+                    for (int q = h * NL / (H - 1); q < (h + 1) * NL / (H - 1); ++q) {
+                        if (q < OA::NL) {
+                            OA::store(bufs[u ^ 1], va[u ^ 1], q);
+                            oa.read(va[u ^ 1], q);
+                        } else {
+                            OB::store(bufs[u ^ 1] + OA::BYTES, vb[u ^ 1], q - OA::NL);
+                            ob.read(vb[u ^ 1], q - OA::NL);
+                        }
+                    }
                 } else {
+                    oa.advance();
+                    ob.advance();
                     __syncthreads();
+                    __builtin_amdgcn_sched_barrier(0);
                     fragments(bufs[u ^ 1], 0);
                 }
-                multiply(h, 0);
-                if (h == H - 2) {
-                    store(bufs[u ^ 1], u ^ 1);
-                    oa.read(va[u ^ 1]);
-                    ob.read(vb[u ^ 1]);
+                products(h);
+                // one memory instruction per MFMA: the fragments' first, then the stage's
+                constexpr int R = NF < NM / 2 ? NF : NM / 2, X = (NL / (H - 1) + NM - R - 1) / (NM - R);
+#pragma unroll
+                for (int g = 0; g < R; ++g) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, NF / R, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
                 }
-                multiply(h, 1);
+                if (h < H - 1) {
+#pragma unroll
+                    for (int g = R; g < NM; ++g) {
+                        __builtin_amdgcn_sched_group_barrier(0x200, X, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x020, X, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
             }
-    }
+    };
+    // the first turn apart: its waits are for whatever loads came before,
+    // those of the loop for its own
+    if (turns > 0) turn();
+    for (int64_t i = 1; i < turns; ++i) turn();
     left -= 2 * BK * turns;
     for (int64_t s = 2 * turns; s < ns;) {
 #pragma unroll
@@ -668,12 +697,11 @@ __global__ __launch_bounds__(256, C::OCC) void sgemm_kernel(SgemmArgs P) {
                     __syncthreads();
                     fragments(bufs[u ^ 1], 0);
                 }
-                multiply(h, 0);
                 if (h == H - 2 && s + 1 < ns) {
                     store(bufs[u ^ 1], u ^ 1);
                     read(u ^ 1);
                 }
-                multiply(h, 1);
+                products(h);
             }
         }
     }
@@ -770,20 +798,20 @@ void launch_sgemm(SgemmArgs a, hipStream_t st) {
 // tiles at the rate that as many reach (eff), plus 4 us of prologue and
 // epilogue per round of `conc` resident tiles.  Measured rates, share of 157.3
 // TFLOP/s: 128x128 direct to LDS 0.83 with one tile per CU, 0.92 with more
-// (0.90 with no operand in registers: opA = N, opB = T); 64x64 0.74, 0.84, 0.87,
-// 0.89 with one to four, 0.94 with more, 0.915 past 128, where its operands
-// come from beyond the L2; 32x32 0.62, 0.69, 0.73, 0.75, 0.80.  So 64x64 wins at
-// long K (4096^3: 941 us against 967), 128x128 at short K (8192 x 8192 x 256:
+// (0.90 with no operand in registers: opA = N, opB = T); 64x64 0.87 to 0.91 with
+// one to four, 0.945 with more, 0.915 past 128, where its operands come from
+// beyond the L2; 32x32 0.64, 0.70, 0.75, 0.77, 0.81.  So 64x64 wins at
+// long K (4096^3: 938 us against 967), 128x128 at short K (8192 x 8192 x 256:
 // 273 us against 302) and in the largest NN products (16384^3: 60.9 ms against
-// 61.2), 32x32 where it fills CUs that 64x64 leaves idle (512^3: 7.3 us against
-// 13.3).
+// 61.2), 32x32 where it fills CUs that 64x64 leaves idle (512^3: 7.1 us against
+// 12.4).
 double sgemm_time(int64_t m, int64_t n, int64_t k, int t, int conc, const double* eff) {
     const int64_t c = (((m + t - 1) / t) * ((n + t - 1) / t) + 255) / 256;
     const double u = 2.0 * t * t * (double)k / (157.3e6 / 256);
     return (double)c * u / eff[c >= 128 ? 5 : c >= 8 ? 4 : std::min<int64_t>(c, 4) - 1] + 4.0 * std::max(1.0, (double)c / conc);
 }
 constexpr double kEffDma[2][6] = {{0.83, 0.90, 0.90, 0.90, 0.90, 0.90}, {0.83, 0.90, 0.91, 0.92, 0.92, 0.92}};
-constexpr double kEff64[6] = {0.74, 0.84, 0.87, 0.89, 0.94, 0.915}, kEff32[6] = {0.62, 0.69, 0.73, 0.75, 0.80, 0.78};
+constexpr double kEff64[6] = {0.87, 0.89, 0.90, 0.91, 0.945, 0.915}, kEff32[6] = {0.64, 0.70, 0.75, 0.77, 0.81, 0.79};
 
 // One problem.  The direct-to-LDS kernels take it when `dma`: cut, with a
 // k-contiguous operand, whole even k-steps and at least 8 whole interior

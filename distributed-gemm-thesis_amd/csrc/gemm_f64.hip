@@ -102,8 +102,11 @@ struct TileLds {
 
 // Computes one output tile of problem P.  Two LDS buffers, one barrier per
 // stage: while stage s is multiplied, stages s+1 .. s+D are in flight to
-// registers; s+1 is stored to the other buffer and s+1+D requested before the
-// stage's last MFMAs.
+// registers; s+1 is stored to the other buffer and s+1+D requested among the
+// MFMAs before the last part's, one memory instruction per MFMA: issued
+// together they take longer than the MFMA that runs meanwhile, and a CU with
+// few resident workgroups waits (one 64x64 tile per CU, K = 4096: 148 -> 122
+// us; 2048^3 249 -> 241 us).
 template <class C, bool TA, bool TB>
 __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__ segs, int local, char* lds) {
     constexpr int BM = C::BM, BN = C::BN, BK = C::BK, D = C::D;
@@ -200,15 +203,19 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
         staged_fragments<OA, TA>(fa[h & 1], buf, wm, lr, lg, h);
         staged_fragments<OB, !TB>(fb[h & 1], buf + OA::BYTES, wn, lr, lg, h);
     };
-    auto multiply = [&](int h, int q) {
-        __builtin_amdgcn_sched_barrier(0);
+    auto products = [&](int h, int q) {
 #pragma unroll
         for (int i = 0; i < FM; ++i)
 #pragma unroll
             for (int j = 0; j < FN; ++j)
                 acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[h & 1][j][q], fa[h & 1][i][q], acc[i][j], 0, 0, 0);
+    };
+    auto multiply = [&](int h, int q) {
+        __builtin_amdgcn_sched_barrier(0);
+        products(h, q);
         __builtin_amdgcn_sched_barrier(0);
     };
+    constexpr int NL = OA::NL + OB::NL, NM = 2 * FM * FN;  // loads and stores of a stage, MFMAs of a part
     // Two stages a turn: s, even, in buffer 0, and s + 1; stage s + 1 waits in
     // register set (s + 1) % D.  Turns that read only whole stages of one
     // segment run without conditions.
@@ -217,28 +224,68 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     fragments(lds, 0);
     for (int64_t s = 0; s < ns;) {
         const int64_t turns = pairs && left > 0 ? (left - 1) / (2 * BK) : 0;
-        for (int64_t i = 0; i < turns; ++i) {
+        auto turn = [&]() {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
                 const int nx = (u + 1) % D;
 #pragma unroll
                 for (int h = 0; h < H; ++h) {
+                    __builtin_amdgcn_sched_barrier(0);
                     if (h < H - 1) {
                         fragments(bufs[u], h + 1);
+#pragma unroll
+                        for (int q = h * NL / (H - 1); q < (h + 1) * NL / (H - 1); ++q) {
+                            if (q < OA::NL) {
+                                OA::store(bufs[u ^ 1], va[nx], q);
+                                oa.read(va[nx], q);
+                            } else {
+                                OB::store(bufs[u ^ 1] + OA::BYTES, vb[nx], q - OA::NL);
+                                ob.read(vb[nx], q - OA::NL);
+                            }
+                        }
                     } else {
+                        oa.advance();
+                        ob.advance();
                         __syncthreads();
+                        __builtin_amdgcn_sched_barrier(0);
                         fragments(bufs[u ^ 1], 0);
                     }
-                    multiply(h, 0);
-                    if (h == H - 2) {
-                        store(bufs[u ^ 1], nx);
-                        oa.read(va[nx]);
-                        ob.read(vb[nx]);
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) products(h, q);
+                    if (h < H - 1) {
+                        constexpr int R = FM + FN < NM ? FM + FN : NM;      // MFMAs that follow a fragment read
+                        constexpr int W = (NL / (H - 1) + NM - 1) / NM;
+#pragma unroll
+                        for (int g = 0; g < R; ++g) {
+                            __builtin_amdgcn_sched_group_barrier(0x100, (FM + FN) / R, 0);
+                            if (R == NM) {
+                                __builtin_amdgcn_sched_group_barrier(0x200, W, 0);
+                                __builtin_amdgcn_sched_group_barrier(0x020, W, 0);
+                            }
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        }
+                        constexpr int X = NM > R ? (NL / (H - 1) + NM - R - 1) / (NM - R) : 1;
+#pragma unroll
+                        for (int g = R; g < NM; ++g) {
+                            __builtin_amdgcn_sched_group_barrier(0x200, X, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x020, X, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        }
+                    } else {
+#pragma unroll
+                        for (int g = 0; g < FM + FN; ++g) {
+                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                        }
                     }
-                    multiply(h, 1);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
             }
-        }
+        };
+        // the first turn apart: its waits are for whatever loads came before,
+        // those of the loop for its own
+        if (turns > 0) turn();
+        for (int64_t i = 1; i < turns; ++i) turn();
         s += 2 * turns;
         left -= 2 * BK * turns;
 #pragma unroll
@@ -312,9 +359,21 @@ __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_kernel(const Prob* __
         const Prob P = probs[lo];
         gemm_tile<C, TA, TB>(P, segs, tile - P.tile0, lds);
     };
-    if (MODE == 0 || MODE == 1) {
+    if (MODE == 0) {
         const int64_t bid = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
-        if (bid < total_tiles) run(MODE == 0 ? (int)bid : xcd_remap((int)bid, total_tiles));
+        if (bid < total_tiles) run((int)bid);
+    } else if (MODE == 1) {
+        // the workgroups of XCD x walk its contiguous tile range side by side (one
+        // tile each when the grid has them all)
+        constexpr int X = 8;
+        const int x = blockIdx.x % X, slot = blockIdx.x / X;
+        const int q = total_tiles / X, r = total_tiles % X;
+        const int first = x * q + min(x, r), count = q + (x < r ? 1 : 0);
+        const int slots = gridDim.x / X + (x < (int)(gridDim.x % X) ? 1 : 0);
+        for (int t = slot; t < count; t += slots) {
+            run(first + t);
+            __syncthreads();  // the next tile's first stage goes where this one's last may still be read
+        }
     } else {
         __shared__ int next;
         while (true) {
@@ -941,7 +1000,7 @@ void launch_mode(int mode, const Prob* dp, int np, const Seg* ds, int tiles, int
     if (mode == DG_GEMM_MODE_ROUND_ROBIN)
         hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 0>), tile_grid(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
     else if (mode == DG_GEMM_MODE_XCD)
-        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 1>), tile_grid(tiles), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
+        hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 1>), dim3(std::min(grid, 1 << 22)), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
     else
         hipLaunchKernelGGL((gemm_f64_kernel<C, TA, TB, 2>), dim3(grid), dim3(C::NTH), 0, st, dp, np, ds, tiles, counter);
 }
@@ -981,11 +1040,12 @@ static bool by_elements(const Prob& p, const std::vector<Seg>& segs, bool ak, bo
 }
 
 // Time (us) of one list's launch, to choose between the tile shapes: the
-// fullest CU's tiles at the rate that `conc` resident workgroups reach (eff,
-// by how many there are), plus 4 us of prologue and epilogue per round of
-// resident tiles.  Measured rates, share of 78.6 TFLOP/s: 128x128 direct to
-// LDS 0.91 (256 tiles, one workgroup per CU) and 0.95 (two); 64x64 0.74, 0.83,
-// 0.865, 0.895 with one to four; 32x32 0.58, 0.68, 0.72, 0.76.
+// fullest CU's c tiles at the rate that so many reach (eff), plus 4 us of
+// prologue and epilogue per round of `conc` resident tiles.  Measured rates,
+// share of 78.6 TFLOP/s: 128x128 direct to LDS 0.91 (one tile per CU) and 0.95
+// (more); 64x64 0.92, 0.88 from 25 tiles per CU on and 0.85 from 64 on, where
+// its operands come from beyond the L2; 32x32 0.67, 0.72, 0.76, 0.78 with one to
+// four, 0.80 with more.
 struct ListCost {
     int64_t tiles = 0;
     double sum = 0, most = 0, least = 1e300;  // us of CU time: all tiles, the longest, the shortest
@@ -1000,11 +1060,12 @@ struct ListCost {
         if (!tiles) return 0;
         const int64_t c = (tiles + 255) / 256;
         const double load = most == least ? (double)c * most : std::max(sum / 256 + most / 2, most);
-        return load / eff[std::min<int64_t>(c, conc) - 1] + 4.0 * std::max(1.0, (double)c / conc);
+        return load / eff[c >= 64 ? 6 : c >= 25 ? 5 : std::min<int64_t>(c, 5) - 1] + 4.0 * std::max(1.0, (double)c / conc);
     }
 };
-constexpr double kEffInterior[2] = {0.91, 0.95}, kEffEdge[2] = {0.85, 0.93};
-constexpr double kEff64[4] = {0.74, 0.83, 0.865, 0.895}, kEff32[4] = {0.58, 0.68, 0.72, 0.76};
+constexpr double kEffInterior[7] = {0.91, 0.95, 0.95, 0.95, 0.95, 0.95, 0.95};
+constexpr double kEffEdge[7] = {0.85, 0.93, 0.93, 0.93, 0.93, 0.93, 0.93};
+constexpr double kEff64[7] = {0.92, 0.92, 0.92, 0.92, 0.91, 0.88, 0.85}, kEff32[7] = {0.67, 0.72, 0.76, 0.78, 0.80, 0.80, 0.78};
 
 // prepare_gemm for one tile choice; *time receives the estimate (us).
 static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, const std::vector<Seg>& segs,
@@ -1183,7 +1244,15 @@ int launch_gemm_f64_dev(char opA, char opB, int mode, const GemmBatchDev& b, int
     for (int w = 0; w < 2; ++w) {  // 64x64 tiles, then 32x32
         const int t = b.tiles_gen[w];
         if (t <= 0) continue;
-        const int grid = grid_of(t, w ? Cfg32::OCC : Cfg64::OCC);
+        int grid = grid_of(t, w ? Cfg32::OCC : Cfg64::OCC);
+        // Little more than one or two rounds of resident workgroups: the tiles
+        // left over land on the few CUs that drain first, several on each.
+        // Workgroups that walk the tiles in fixed steps keep them apart (2050^3,
+        // 1.06 rounds: 354 -> 305 us; 3072^3, 2.25: 853 -> 824).  With more left
+        // over, or more rounds, the order of completion balances better (4096^3:
+        // 1945 us against 1987).
+        const int slots = persistent_grid(Cfg64::OCC);
+        if (w == 0 && mode == DG_GEMM_MODE_XCD && t > slots && t < 3 * slots && t % slots <= slots / 4) grid = slots;
         if (w == 0) launch_cfg<Cfg64>(opA, opB, mode, b.gen[0], b.ngen[0], b.segs, t, grid, counter, stream);
         else launch_cfg<Cfg32>(opA, opB, mode, b.gen[1], b.ngen[1], b.segs, t, grid, counter, stream);
         DG_LAUNCH_CHECK();

@@ -87,12 +87,14 @@ struct Staged {
         base += KC ? BK : BK * ld;
         asm volatile("" : "+s"(base));  // stays a scalar: not folded into vector address increments
     }
+    // Run q of a whole stage (all of them, then advance).
+    __device__ __forceinline__ void read(vec (&v)[NL], int q) {
+        asm volatile("" : "+v"(off[q]));  // stays 32 bits: the load adds it to the scalar base itself
+        v[q] = *(gvec*)((const char*)base + off[q]);
+    }
     __device__ __forceinline__ void read(vec (&v)[NL]) {
 #pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            asm volatile("" : "+v"(off[q]));  // stays 32 bits: the load adds it to the scalar base itself
-            v[q] = *(gvec*)((const char*)base + off[q]);
-        }
+        for (int q = 0; q < NL; ++q) read(v, q);
         advance();
     }
     // The segment's last stage, `left` <= BK of its k real (or any stage of a
@@ -111,10 +113,12 @@ struct Staged {
             for (int e = 0; e < E; ++e) v[q][e] = kk(q) + (KC ? e : 0) < left ? v[q][e] : T(0);
         advance();
     }
+    static __device__ __forceinline__ void store(char* s, const vec (&v)[NL], int q) {
+        *reinterpret_cast<vec*>(s + (KC ? row(q) * LROW + kk(q) * S : kk(q) * LROW + row(q) * S)) = v[q];
+    }
     static __device__ __forceinline__ void store(char* s, const vec (&v)[NL]) {
 #pragma unroll
-        for (int q = 0; q < NL; ++q)
-            *reinterpret_cast<vec*>(s + (KC ? row(q) * LROW + kk(q) * S : kk(q) * LROW + row(q) * S)) = v[q];
+        for (int q = 0; q < NL; ++q) store(s, v, q);
     }
     // Whether read() takes a matrix: elements on their own alignment, and rows
     // neither so far apart that a tile's offsets leave 32 bits nor so close
