@@ -129,13 +129,15 @@ enum {
     DG_GEMM_MODE_PERSISTENT = 2,   // CU-count workgroups pull tiles from an atomic counter
 };
 
-// Output tiles of an FP64 GEMM batch.
+// Tile choices of an FP64 GEMM batch.
 enum {
-    DG_GEMM_TILE_AUTO = -1,    // the one whose estimated time is least
-    DG_GEMM_TILE_128x128 = 0,  // direct-to-LDS kernels where they apply, 64x64 register-staged elsewhere
-    DG_GEMM_TILE_64x64 = 1,    // register-staged kernel
-    DG_GEMM_TILE_32x32 = 2,    // register-staged kernel
-    DG_GEMM_TILES = 3,
+    DG_GEMM_TILE_AUTO = -1,          // the one whose estimated time is least
+    DG_GEMM_TILE_DIRECT = 0,         // direct-to-LDS kernels where they apply, as 128x128 elsewhere
+    DG_GEMM_TILE_128x128 = 1,        // register-staged kernel, uneven problems cut into whole tiles and strips
+    DG_GEMM_TILE_128x128_WHOLE = 2,  // the same, uncut
+    DG_GEMM_TILE_64x64 = 3,          // register-staged kernel
+    DG_GEMM_TILE_32x32 = 4,          // register-staged kernel
+    DG_GEMM_TILES = 5,
 };
 
 // Launches the FP64 MFMA GEMM over `probs` (host vector; uploaded through
@@ -143,19 +145,19 @@ enum {
 int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs,
                     const std::vector<Seg>& segs, hipStream_t stream, int mode);
 
-// A batch split by kernel.  With DG_GEMM_TILE_128x128, the direct-to-LDS
+// A batch split by kernel.  With DG_GEMM_TILE_DIRECT, the direct-to-LDS
 // kernels take a problem when every segment has K > 0 and even leading
 // dimensions, its k-contiguous operand (A with opA = T, B with opB = N) has
 // 16-byte aligned bases and even K, and its row-contiguous operand (A with
 // opA = N, B with opB = T) has 8-byte aligned bases with the same offset
 // within 16 bytes in every segment; the register-staged kernel takes the
-// others, and all of them with the other tiles.  DG_GEMM_TILE_AUTO estimates
-// each choice's time from its tiles and takes the least: 128x128 tiles keep
-// the matrix cores busiest but leave CUs idle until there are a few hundred
-// of them (DG_GEMM_TILE forces a choice, DG_GEMM_NO_DMA routes everything to
-// the register-staged kernel).  Every kernel and tile sums an element in the
-// same order, so a problem gives the same bits alone, in any batch and on any
-// tile.
+// others, and all of them with the other choices.  DG_GEMM_TILE_AUTO estimates
+// each choice's time from its tiles and takes the least: the larger the
+// tiles, the less operand traffic, but the more CUs stay idle and the more of
+// the work is padding (DG_GEMM_TILE forces a choice, DG_GEMM_NO_DMA routes
+// everything to the register-staged kernel).  Every kernel and tile sums an
+// element in the same order, so a problem gives the same bits alone, in any
+// batch and on any tile.
 // Direct-to-LDS problems whose tiles are all interior (no row shift, m and n
 // multiples of 128, whole k-steps, an even step count) go to `dma`, which
 // the A-in-registers kernel runs; the others go to `dmae` (the edge-handling
@@ -165,29 +167,30 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs,
 // around it on the register-staged kernel (on `dmae` under
 // DG_GEMM_NO_NARROW).  The sub-problems' segments are appended to `segs`
 // (which starts as a copy of the input segments).
-// Register-staged problems and strips go to gen[0] (64x64 tiles), or gen[1]
-// (32x32) when 32x32 is the choice or they are at most 32 rows or columns.
+// Register-staged problems and strips go to gen[0] (128x128 tiles), gen[1]
+// (64x64) or gen[2] (32x32): the choice's own, or a smaller one where they are
+// at most 96 or 32 rows or columns.
 struct GemmBatch {
-    std::vector<Prob> dma, dmae, gen[2];  // tile ranges assigned per list
-    int tiles_dma = 0, tiles_dmae = 0, tiles_gen[2] = {0, 0};
+    std::vector<Prob> dma, dmae, gen[3];  // tile ranges assigned per list
+    int tiles_dma = 0, tiles_dmae = 0, tiles_gen[3] = {0, 0, 0};
     std::vector<Seg> segs;                // the segment table all lists index
-    bool empty() const { return dma.empty() && dmae.empty() && gen[0].empty() && gen[1].empty(); }
+    bool empty() const { return dma.empty() && dmae.empty() && gen[0].empty() && gen[1].empty() && gen[2].empty(); }
 };
 int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, const std::vector<Seg>& segs, GemmBatch& out,
                  bool split_edges = true, int tile = DG_GEMM_TILE_AUTO);
 
 // The same batch with its tables resident on the device.
 struct GemmBatchDev {
-    const Prob *dma = nullptr, *dmae = nullptr, *gen[2] = {nullptr, nullptr};
-    int ndma = 0, ndmae = 0, ngen[2] = {0, 0};
-    int tiles_dma = 0, tiles_dmae = 0, tiles_gen[2] = {0, 0};
+    const Prob *dma = nullptr, *dmae = nullptr, *gen[3] = {nullptr, nullptr, nullptr};
+    int ndma = 0, ndmae = 0, ngen[3] = {0, 0, 0};
+    int tiles_dma = 0, tiles_dmae = 0, tiles_gen[3] = {0, 0, 0};
     const Seg* segs = nullptr;
     void set_counts(const GemmBatch& h) {
         ndma = (int)h.dma.size();
         ndmae = (int)h.dmae.size();
         tiles_dma = h.tiles_dma;
         tiles_dmae = h.tiles_dmae;
-        for (int w = 0; w < 2; ++w) {
+        for (int w = 0; w < 3; ++w) {
             ngen[w] = (int)h.gen[w].size();
             tiles_gen[w] = h.tiles_gen[w];
         }

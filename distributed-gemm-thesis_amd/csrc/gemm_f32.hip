@@ -585,10 +585,12 @@ __global__ __launch_bounds__(256, C::OCC) void sgemm_kernel(SgemmArgs P) {
     oa.start(P.a, P.lda, m0, rows);
     ob.start(P.b, P.ldb, n0, cols);
     int64_t left = P.k;  // k from the next stage to read on (0 or less: past the end)
+    // whether the last k can be read in runs too: none passes a last row (or all go along k)
+    const int last = (AK || rows == T) && (BKC || cols == T) ? 0 : 1;
     fv4 va[2][OA::NL], vb[2][OB::NL];
     auto read = [&](int d) {
         if (left <= 0) return;
-        if (!P.by_elements && left > BK) {
+        if (!P.by_elements && left >= BK + last) {
             oa.read(va[d]);
             ob.read(vb[d]);
         } else {
@@ -635,7 +637,7 @@ __global__ __launch_bounds__(256, C::OCC) void sgemm_kernel(SgemmArgs P) {
     // Two stages a turn: s, even, in buffer 0, and s + 1; stage s + 1 waits in
     // register set (s + 1) % 2.  Turns that read only whole stages run without
     // conditions.
-    const int64_t turns = !P.by_elements && left > 0 ? (left - 1) / (2 * BK) : 0;
+    const int64_t turns = !P.by_elements && left > 0 ? (left - last) / (2 * BK) : 0;
     auto turn = [&]() {
 #pragma unroll
         for (int u = 0; u < 2; ++u)
@@ -841,7 +843,7 @@ void run_sgemm(const SgemmArgs& a, bool dma, hipStream_t st) {
     const int64_t mi = a.m / sk::BM * sk::BM, ni = a.n / sk::BN * sk::BN;
     const bool k_ok = a.k % sk::BK == 0 && !((a.k / sk::BK) & 1);
     const bool cut = (AK || BKC) && !no_areg && k_ok && (mi != a.m || ni != a.n) && mi * ni >= 8 * sk::BM * sk::BN;
-    if (dma && forced != "128x128") {
+    if (dma && forced != "direct" && forced != "128x128") {
         auto least = [&](int64_t m, int64_t n) { return std::min(sgemm_time(m, n, a.k, 64, 4, kEff64), sgemm_time(m, n, a.k, 32, 4, kEff32)); };
         double t = sgemm_time(cut ? mi : a.m, cut ? ni : a.n, a.k, 128, 2, kEffDma[AK || BKC]);
         if (cut && mi < a.m) t += least(a.m - mi, a.n);

@@ -62,9 +62,9 @@ struct TileCfg {
     static constexpr int FM = WM / 16, FN = WN / 16;
     static_assert((BM / WM) * (BN / WN) * 64 == NTH, "one wave per WM x WN sub-tile");
 };
+using Cfg128 = TileCfg<128, 128, 64, 64, 16, 1, 2>;
 using Cfg64 = TileCfg<64, 64, 32, 32, 16, 2, 4>;
 using Cfg32 = TileCfg<32, 32, 16, 16, 32, 2, 3>;
-constexpr int64_t kNarrowMax = 32;  // problems and strips up to this many rows or columns wide take the 32 x 32 tiles
 
 // Block id -> tile id so that each XCD (blocks are dealt round-robin to the
 // 8 XCDs) receives one contiguous range of tiles, which the grouped raster
@@ -144,6 +144,9 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     // load cursor over the problem's segments, one stage at a time
     const int rows = (int)min(P.m - m0, (int64_t)BM), cols = (int)min(P.n - n0, (int64_t)BN);
     const bool pairs = !(P.shift & kByElements);
+    // whether the last k of a segment can be read in pairs too: no pair starts
+    // at a last row (or all go along k)
+    const int last = (TA || rows == BM) && (!TB || cols == BN) ? 0 : 1;
     int sg = P.seg0;
     const int sg_last = P.seg0 + P.nseg - 1;
     int64_t left;  // k of the segment from the next stage on (0 or less: past the last segment)
@@ -158,7 +161,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     dv2 va[D][OA::NL], vb[D][OB::NL];
     auto read = [&](int d) {
         if (left <= 0) return;
-        if (pairs && left > BK) {
+        if (pairs && left >= BK + last) {
             oa.read(va[d]);
             ob.read(vb[d]);
         } else {
@@ -223,7 +226,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     char* const bufs[2] = {lds, lds + L::STAGE};
     fragments(lds, 0);
     for (int64_t s = 0; s < ns;) {
-        const int64_t turns = pairs && left > 0 ? (left - 1) / (2 * BK) : 0;
+        const int64_t turns = pairs && left > 0 ? (left - last) / (2 * BK) : 0;
         auto turn = [&]() {
 #pragma unroll
             for (int u = 0; u < 2; ++u) {
@@ -288,6 +291,10 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
         for (int64_t i = 1; i < turns; ++i) turn();
         s += 2 * turns;
         left -= 2 * BK * turns;
+        if (turns > 0 && left == 0 && sg < sg_last) {
+            ++sg;
+            enter();
+        }
 #pragma unroll
         for (int u = 0; u < 2; ++u, ++s) {
             if (s >= ns) break;
@@ -1039,13 +1046,27 @@ static bool by_elements(const Prob& p, const std::vector<Seg>& segs, bool ak, bo
     return false;
 }
 
-// Time (us) of one list's launch, to choose between the tile shapes: the
-// fullest CU's c tiles at the rate that so many reach (eff), plus 4 us of
-// prologue and epilogue per round of `conc` resident tiles.  Measured rates,
-// share of 78.6 TFLOP/s: 128x128 direct to LDS 0.91 (one tile per CU) and 0.95
-// (more); 64x64 0.92, 0.88 from 25 tiles per CU on and 0.85 from 64 on, where
-// its operands come from beyond the L2; 32x32 0.67, 0.72, 0.76, 0.78 with one to
-// four, 0.80 with more.
+// Time (us) of one list's launch, to choose between the tiles: the fullest
+// CU's c tiles at the rate that so many reach, share of 78.6 TFLOP/s, plus
+// `round` us of prologue and epilogue per round of `conc` resident tiles.
+// Measured: A in registers 0.91 with one tile per CU, 0.95 with more (both
+// operands in LDS 0.85, 0.93); register-staged 128x128 0.95 with one, 0.965 up
+// to 15 (4096^3: 1812 us against 1838 with A in registers), then less, 0.89
+// from 32 on: its matrix cores are 99 % busy, but its workgroups drift apart,
+// fetch their operands from beyond the L2 (16384^3: 374 GB against 101) and
+// the clock falls; 64x64 0.92, 0.88 from 25 tiles per CU on, 0.85 from 64 on;
+// 32x32 0.67, 0.72, 0.76, 0.78 with one to four, 0.80 with more.
+struct Rate {
+    int conc;
+    double round;
+    struct { int64_t from; double eff; } at[5];  // ascending; the last whose `from` c reaches
+};
+constexpr Rate kAreg = {2, 4, {{1, 0.91}, {2, 0.95}}}, kEdge = {2, 4, {{1, 0.85}, {2, 0.93}}};
+constexpr Rate kGen[3] = {{2, 8, {{1, 0.95}, {2, 0.965}, {16, 0.93}, {32, 0.89}}},
+                          {4, 4, {{1, 0.92}, {5, 0.91}, {25, 0.88}, {64, 0.85}}},
+                          {4, 4, {{1, 0.67}, {2, 0.72}, {3, 0.76}, {4, 0.78}, {5, 0.80}}}};
+constexpr int64_t kEdgeOf[3] = {Cfg128::BM, Cfg64::BM, Cfg32::BM};  // tile edge of gen[w]
+
 struct ListCost {
     int64_t tiles = 0;
     double sum = 0, most = 0, least = 1e300;  // us of CU time: all tiles, the longest, the shortest
@@ -1056,16 +1077,16 @@ struct ListCost {
         most = std::max(most, u);
         least = std::min(least, u);
     }
-    double time(int conc, const double* eff) const {
+    double time(const Rate& r) const {
         if (!tiles) return 0;
         const int64_t c = (tiles + 255) / 256;
+        double eff = 0;
+        for (const auto& x : r.at)
+            if (x.from > 0 && x.from <= c) eff = x.eff;
         const double load = most == least ? (double)c * most : std::max(sum / 256 + most / 2, most);
-        return load / eff[c >= 64 ? 6 : c >= 25 ? 5 : std::min<int64_t>(c, 5) - 1] + 4.0 * std::max(1.0, (double)c / conc);
+        return load / eff + r.round * std::max(1.0, (double)c / r.conc);
     }
 };
-constexpr double kEffInterior[7] = {0.91, 0.95, 0.95, 0.95, 0.95, 0.95, 0.95};
-constexpr double kEffEdge[7] = {0.85, 0.93, 0.93, 0.93, 0.93, 0.93, 0.93};
-constexpr double kEff64[7] = {0.92, 0.92, 0.92, 0.92, 0.91, 0.88, 0.85}, kEff32[7] = {0.67, 0.72, 0.76, 0.78, 0.80, 0.80, 0.78};
 
 // prepare_gemm for one tile choice; *time receives the estimate (us).
 static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, const std::vector<Seg>& segs,
@@ -1073,8 +1094,8 @@ static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, c
     out = GemmBatch{};
     out.segs = segs;
     const bool ak = opA == 'T', bkc = opB != 'T';  // k-contiguous operands
-    int64_t tdma = 0, tdmae = 0, tgen[2] = {0, 0};
-    ListCost cdma, cdmae, cgen[2];
+    int64_t tdma = 0, tdmae = 0, tgen[3] = {0, 0, 0};
+    ListCost cdma, cdmae, cgen[3];
     constexpr int64_t TM = dmak::DBM, TN = dmak::DBN;
     auto depth = [&](const Prob& p) {
         int64_t k = 0;
@@ -1091,10 +1112,13 @@ static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, c
         (interior ? cdma : cdmae).add(n, TM * TN, depth(p));
         (interior ? out.dma : out.dmae).push_back(p);
     };
-    // a problem, or a strip of one, onto the register-staged kernel's list
+    // a problem, or a part of one, onto a list of the register-staged kernel:
+    // the choice's own, or the smaller tiles that a narrow one fills better
     auto add_gen = [&](Prob q) {
-        const int w = tile == DG_GEMM_TILE_32x32 || q.m <= kNarrowMax || q.n <= kNarrowMax ? 1 : 0;
-        const int64_t e = w ? 32 : 64;
+        int w = tile == DG_GEMM_TILE_32x32 ? 2 : tile == DG_GEMM_TILE_64x64 ? 1 : 0;
+        const int64_t narrow = std::min(q.m, q.n);
+        w = std::max(w, narrow <= 32 ? 2 : narrow <= 96 ? 1 : 0);
+        const int64_t e = kEdgeOf[w];
         q.shift = by_elements(q, out.segs, ak, bkc) ? kByElements : 0;
         q.tile0 = (int32_t)tgen[w];
         const int64_t n = ((q.m + e - 1) / e) * ((q.n + e - 1) / e);
@@ -1123,9 +1147,28 @@ static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, c
         return q;
     };
     static const bool no_narrow = getenv("DG_GEMM_NO_NARROW") != nullptr;
+    // the strips of p around rows [r0, r0 + mi) x columns [c0, c0 + ni)
+    auto add_strips = [&](const Prob& p, int64_t r0, int64_t mi, int64_t c0, int64_t ni, bool edge) {
+        auto strip = [&](const Prob& q) { if (edge) add_dma(q, false); else add_gen(q); };
+        if (r0 > 0) strip(sub(p, 0, r0, 0, p.n));                                    // rows before it
+        if (r0 + mi < p.m) strip(sub(p, r0 + mi, p.m - r0 - mi, 0, p.n));            // rows after it
+        if (c0 > 0) strip(sub(p, r0, mi, 0, c0));                                    // columns before it
+        if (c0 + ni < p.n) strip(sub(p, r0, mi, c0 + ni, p.n - c0 - ni));            // columns after it
+    };
+    // whole, or cut into whole 128x128 tiles and strips (a strip that nearly
+    // fills its tiles stays with them)
+    auto add_staged = [&](const Prob& p) {
+        auto inside = [](int64_t x) { return x % 128 > 96 ? x : x / 128 * 128; };
+        const int64_t mi = inside(p.m), ni = inside(p.n);
+        if (tile == DG_GEMM_TILE_64x64 || tile == DG_GEMM_TILE_32x32 || tile == DG_GEMM_TILE_128x128_WHOLE ||
+            !split_edges || (mi == p.m && ni == p.n) || mi * ni < 8 * 128 * 128)
+            return add_gen(p);
+        add_gen(sub(p, 0, mi, 0, ni));
+        add_strips(p, 0, mi, 0, ni, false);
+    };
     for (const Prob& p0 : probs_in) {
         if (p0.m <= 0 || p0.n <= 0 || p0.nseg <= 0) continue;
-        bool d = tile == DG_GEMM_TILE_128x128;
+        bool d = tile == DG_GEMM_TILE_DIRECT;
         int off_a = -1, off_b = -1;  // byte offset within 16 of a row-contiguous A / B
         for (int s = p0.seg0; d && s < p0.seg0 + p0.nseg; ++s) {
             const Seg& g = segs[s];
@@ -1138,7 +1181,7 @@ static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, c
         }
         Prob p = p0;
         if (!d) {
-            add_gen(p);
+            add_staged(p);
             continue;
         }
         const int sa = off_a == 8, sb = off_b == 8;
@@ -1163,20 +1206,19 @@ static int prepare_tile(char opA, char opB, const std::vector<Prob>& probs_in, c
             add_dma(p, false);
             continue;
         }
-        auto strip = [&](const Prob& q) { if (no_narrow) add_dma(q, false); else add_gen(q); };
-        add_dma(sub(p, r0, mi, c0, ni), true);                                       // interior
-        if (r0 > 0) strip(sub(p, 0, r0, 0, p.n));                                    // rows before it
-        if (r0 + mi < p.m) strip(sub(p, r0 + mi, p.m - r0 - mi, 0, p.n));            // rows after it
-        if (c0 > 0) strip(sub(p, r0, mi, 0, c0));                                    // columns before it
-        if (c0 + ni < p.n) strip(sub(p, r0, mi, c0 + ni, p.n - c0 - ni));            // columns after it
+        add_dma(sub(p, r0, mi, c0, ni), true);
+        add_strips(p, r0, mi, c0, ni, no_narrow);
     }
-    if (tdma > INT32_MAX || tdmae > INT32_MAX || tgen[0] > INT32_MAX || tgen[1] > INT32_MAX ||
+    if (tdma > INT32_MAX || tdmae > INT32_MAX || std::max({tgen[0], tgen[1], tgen[2]}) > INT32_MAX ||
         out.segs.size() > (size_t)INT32_MAX)
         return fail(DG_ERR_INVALID, "gemm: output tiles exceed one launch");
     out.tiles_dma = (int)tdma;
     out.tiles_dmae = (int)tdmae;
-    for (int w = 0; w < 2; ++w) out.tiles_gen[w] = (int)tgen[w];
-    *time = cdma.time(2, kEffInterior) + cdmae.time(2, kEffEdge) + cgen[0].time(4, kEff64) + cgen[1].time(4, kEff32);
+    *time = cdma.time(kAreg) + cdmae.time(kEdge);
+    for (int w = 0; w < 3; ++w) {
+        out.tiles_gen[w] = (int)tgen[w];
+        *time += cgen[w].time(kGen[w]);
+    }
     return DG_OK;
 }
 
@@ -1186,6 +1228,7 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, const std::
     static const int forced = [] {
         const char* e = getenv("DG_GEMM_TILE");
         const std::string v = e ? e : "";
+        if (v == "direct") return (int)DG_GEMM_TILE_DIRECT;
         if (v == "128x128") return (int)DG_GEMM_TILE_128x128;
         if (v == "64x64") return (int)DG_GEMM_TILE_64x64;
         if (v == "32x32") return (int)DG_GEMM_TILE_32x32;
@@ -1193,12 +1236,12 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, const std::
     }();
     static const bool no_dma = getenv("DG_GEMM_NO_DMA") != nullptr;
     if (forced != DG_GEMM_TILE_AUTO) tile = forced;
-    if (no_dma && tile == DG_GEMM_TILE_128x128) tile = DG_GEMM_TILE_64x64;
+    if (no_dma && tile == DG_GEMM_TILE_DIRECT) tile = DG_GEMM_TILE_128x128;
     double t = 0;
     if (tile != DG_GEMM_TILE_AUTO) return prepare_tile(opA, opB, probs, segs, out, split_edges, tile, &t);
     double best = 0;
     int rc_best = DG_ERR_INVALID;
-    for (int c = no_dma ? DG_GEMM_TILE_64x64 : DG_GEMM_TILE_128x128; c < DG_GEMM_TILES; ++c) {
+    for (int c = no_dma ? DG_GEMM_TILE_128x128 : DG_GEMM_TILE_DIRECT; c < DG_GEMM_TILES; ++c) {
         GemmBatch b;
         const int rc = prepare_tile(opA, opB, probs, segs, b, split_edges, c, &t);
         if (rc == DG_OK && (rc_best != DG_OK || t < best)) {
@@ -1241,20 +1284,22 @@ int launch_gemm_f64_dev(char opA, char opB, int mode, const GemmBatchDev& b, int
         else launch_dma<false, false>(edge, mode, dp, np, b.segs, t0, grid, counter, stream);
         DG_LAUNCH_CHECK();
     }
-    for (int w = 0; w < 2; ++w) {  // 64x64 tiles, then 32x32
+    const int occ[3] = {Cfg128::OCC, Cfg64::OCC, Cfg32::OCC};
+    for (int w = 0; w < 3; ++w) {  // 128x128 tiles, 64x64, 32x32
         const int t = b.tiles_gen[w];
         if (t <= 0) continue;
-        int grid = grid_of(t, w ? Cfg32::OCC : Cfg64::OCC);
+        int grid = grid_of(t, occ[w]);
         // Little more than one or two rounds of resident workgroups: the tiles
         // left over land on the few CUs that drain first, several on each.
-        // Workgroups that walk the tiles in fixed steps keep them apart (2050^3,
-        // 1.06 rounds: 354 -> 305 us; 3072^3, 2.25: 853 -> 824).  With more left
-        // over, or more rounds, the order of completion balances better (4096^3:
-        // 1945 us against 1987).
-        const int slots = persistent_grid(Cfg64::OCC);
-        if (w == 0 && mode == DG_GEMM_MODE_XCD && t > slots && t < 3 * slots && t % slots <= slots / 4) grid = slots;
-        if (w == 0) launch_cfg<Cfg64>(opA, opB, mode, b.gen[0], b.ngen[0], b.segs, t, grid, counter, stream);
-        else launch_cfg<Cfg32>(opA, opB, mode, b.gen[1], b.ngen[1], b.segs, t, grid, counter, stream);
+        // Workgroups that walk the tiles in fixed steps keep them apart (2050^3 on
+        // 64x64 tiles, 1.06 rounds: 354 -> 305 us; 3072^3, 2.25: 853 -> 824).  With
+        // more left over, or more rounds, the order of completion balances better
+        // (4096^3: 1945 us against 1987).
+        const int slots = persistent_grid(occ[w]);
+        if (w < 2 && mode == DG_GEMM_MODE_XCD && t > slots && t < 3 * slots && t % slots <= slots / 4) grid = slots;
+        if (w == 0) launch_cfg<Cfg128>(opA, opB, mode, b.gen[0], b.ngen[0], b.segs, t, grid, counter, stream);
+        else if (w == 1) launch_cfg<Cfg64>(opA, opB, mode, b.gen[1], b.ngen[1], b.segs, t, grid, counter, stream);
+        else launch_cfg<Cfg32>(opA, opB, mode, b.gen[2], b.ngen[2], b.segs, t, grid, counter, stream);
         DG_LAUNCH_CHECK();
     }
     return DG_OK;
@@ -1276,7 +1321,7 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs_in, const
         return *dst != nullptr;
     };
     if (!table(hb.dma, &b.dma) || !table(hb.dmae, &b.dmae) || !table(hb.gen[0], &b.gen[0]) ||
-        !table(hb.gen[1], &b.gen[1]) || !table(hb.segs, &b.segs))
+        !table(hb.gen[1], &b.gen[1]) || !table(hb.gen[2], &b.gen[2]) || !table(hb.segs, &b.segs))
         return DG_ERR_ALLOC;
     b.set_counts(hb);
     if (mode == DG_GEMM_MODE_PERSISTENT) mode = DG_GEMM_MODE_XCD;  // needs a counter: plans only

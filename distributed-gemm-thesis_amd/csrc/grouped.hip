@@ -300,7 +300,7 @@ int build_groups(dg_grouped_plan* p, const dg_gemm_desc* descs, int count, const
             GemmBatchDev& b = p->groups[t].back().b;
             put(hb.dma, &b.dma);
             put(hb.dmae, &b.dmae);
-            for (int w = 0; w < 2; ++w) put(hb.gen[w], &b.gen[w]);
+            for (int w = 0; w < 3; ++w) put(hb.gen[w], &b.gen[w]);
             put(hb.segs, &b.segs);
             b.set_counts(hb);
         }
@@ -589,7 +589,7 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
     // Lay out every op group's tables (problems routed to each kernel, then
     // segments) in one host image, 256-byte aligned pieces, and check the size
     // before anything is launched.
-    struct Piece { char opA, opB; GemmBatch hb; size_t off_dma, off_dmae, off_gen[2], off_seg; };
+    struct Piece { char opA, opB; GemmBatch hb; size_t off_dma, off_dmae, off_gen[3], off_seg; };
     std::vector<Piece> pieces;
     size_t total = 0;
     auto take = [&](size_t bytes) { const size_t o = total; total = (total + bytes + 255) / 256 * 256; return o; };
@@ -598,13 +598,13 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
         std::vector<Seg> segs;
         build_group(descs, kv.second, probs, segs);
         if (probs.empty()) continue;
-        Piece pc{kv.first.first, kv.first.second, GemmBatch{}, 0, 0, {0, 0}, 0};
+        Piece pc{kv.first.first, kv.first.second, GemmBatch{}, 0, 0, {0, 0, 0}, 0};
         // no sub-problems here: the tables stay within the documented capacity
         rc = prepare_gemm(pc.opA, pc.opB, probs, segs, pc.hb, false);
         if (rc) return rc;
         pc.off_dma = take(pc.hb.dma.size() * sizeof(Prob));
         pc.off_dmae = take(pc.hb.dmae.size() * sizeof(Prob));
-        for (int w = 0; w < 2; ++w) pc.off_gen[w] = take(pc.hb.gen[w].size() * sizeof(Prob));
+        for (int w = 0; w < 3; ++w) pc.off_gen[w] = take(pc.hb.gen[w].size() * sizeof(Prob));
         pc.off_seg = take(pc.hb.segs.size() * sizeof(Seg));
         pieces.push_back(std::move(pc));
     }
@@ -621,7 +621,7 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
         auto copy = [&](const auto& v, size_t off) { if (!v.empty()) memcpy(image.data() + off, v.data(), v.size() * sizeof(v[0])); };
         copy(pc.hb.dma, pc.off_dma);
         copy(pc.hb.dmae, pc.off_dmae);
-        for (int w = 0; w < 2; ++w) copy(pc.hb.gen[w], pc.off_gen[w]);
+        for (int w = 0; w < 3; ++w) copy(pc.hb.gen[w], pc.off_gen[w]);
         copy(pc.hb.segs, pc.off_seg);
     }
     rc = store_bytes(base, image, st);
@@ -631,7 +631,7 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
         GemmBatchDev d;
         d.dma = reinterpret_cast<const Prob*>(b + pc.off_dma);
         d.dmae = reinterpret_cast<const Prob*>(b + pc.off_dmae);
-        for (int w = 0; w < 2; ++w) d.gen[w] = reinterpret_cast<const Prob*>(b + pc.off_gen[w]);
+        for (int w = 0; w < 3; ++w) d.gen[w] = reinterpret_cast<const Prob*>(b + pc.off_gen[w]);
         d.segs = reinterpret_cast<const Seg*>(b + pc.off_seg);
         d.set_counts(pc.hb);
         rc = launch_gemm_f64_dev(pc.opA, pc.opB, DG_GEMM_MODE_ROUND_ROBIN, d, nullptr, st);
@@ -688,7 +688,7 @@ int dg_grouped_plan_create_form(const dg_gemm_desc* descs, int count, int mode, 
     p->form = form;
     p->moduli_req = moduli;
     (void)hipGetDevice(&p->device);
-    p->shape_key = "t3:" + shape_class(descs, count);  // three tile choices: entries of other choices stay unread
+    p->shape_key = "t5:" + shape_class(descs, count);  // five tile choices: entries of other choices stay unread
     if (form == DG_FORM_OZAKI_INT8) p->shape_key = "oz" + std::to_string(moduli) + ":" + p->shape_key;
     if (mode == DG_PLAN_NONPERSISTENT) p->variant = DG_GEMM_MODE_ROUND_ROBIN;
     if (mode == DG_PLAN_PERSISTENT) p->variant = DG_GEMM_MODE_PERSISTENT;

@@ -42,10 +42,11 @@ inline dim3 tile_grid(int tiles) {
 //    (the k-rows that one MFMA reads, E apart, then fall in different halves
 //    of the banks).
 // Rows past the end are read from the last row; they feed only outputs that
-// are never stored.  A segment's last stage is read by elements (read_last),
-// with k past the end turned into zeros; in the stages before it every run
+// are never stored.  In a whole stage that is not a segment's last, every run
 // is inside the matrix: one that starts at the last row ends in the next k's
-// first rows or in the columns' padding (ld >= E - 1).
+// first rows or in the columns' padding (ld >= E - 1).  A segment's last stage
+// is read by elements (read_last), with k past the end turned into zeros,
+// unless it is whole and no run can start at a last row (KC, or a full tile).
 // A whole stage uses no vector instruction but the memory ones: a scalar base
 // that moves and 32-bit lane offsets that stay.  An FP64 MFMA runs on the
 // vector ALU's own pipes, and 1.4 to 3.7 vector instructions per MFMA cost a

@@ -2,8 +2,8 @@
 every edge of the rule (one tile to several per CU, strips up to and past 32
 wide, odd sizes and leading dimensions, single rows and columns, shifted
 bases, short and partial k-stages) give the same result as in child processes
-that force 128x128 tiles (direct-to-LDS kernels), 64x64 and 32x32
-(register-staged kernels), in FP64 and in FP32, and all are within a
+that force the direct-to-LDS kernels and the register-staged ones' 128x128
+(cut into whole tiles and strips), 64x64 and 32x32 tiles, in FP64 and in FP32, and all are within a
 rounding bound of the product (FP64 1e-13; FP32 the a-priori 2^-24 (k + 2) per
 element on |A||B|)."""
 import os
@@ -25,7 +25,7 @@ SHAPES = [
     ("N", "N", 64, 64, 16, 0, 0), ("T", "N", 65, 63, 33, 0, 0), ("N", "T", 33, 31, 15, 1, 1), ("T", "T", 1, 70, 17, 0, 0),
     ("N", "N", 70, 1, 1, 0, 0), ("N", "T", 1, 1, 40, 0, 1), ("N", "N", 512, 512, 512, 0, 0), ("T", "N", 511, 513, 1000, 1, 1),
     ("N", "T", 1031, 777, 272, 1, 0), ("T", "T", 1040, 1056, 256, 0, 0), ("N", "N", 1089, 833, 256, 2, 1),
-    ("N", "N", 2048, 2048, 48, 0, 0), ("T", "N", 3000, 40, 128, 0, 0), ("N", "N", 31, 3000, 96, 0, 0),
+    ("N", "N", 2048, 2048, 48, 0, 0), ("T", "N", 1281, 1125, 80, 1, 0), ("N", "T", 1125, 1058, 96, 0, 1), ("T", "N", 3000, 40, 128, 0, 0), ("N", "N", 31, 3000, 96, 0, 0),
 ]
 
 
@@ -63,7 +63,7 @@ def test_same_bits_on_every_tile(dev, tmp_path, dtype):
             assert np.linalg.norm(c - ref) <= 1e-13 * np.linalg.norm(ref)
         else:
             assert np.all(np.abs(c - ref) <= 2.0 ** -24 * (k + 2) * (1.5 * np.abs(a) @ np.abs(b) + 0.5 * np.abs(c0)))
-    for tile in ("128x128", "64x64", "32x32"):
+    for tile in ("direct", "128x128", "64x64", "32x32"):
         path = str(tmp_path / tile)
         subprocess.run([sys.executable, os.path.abspath(__file__), path, str(dtype)], check=True, timeout=100,
                        env=dict(os.environ, DG_GEMM_TILE=tile))

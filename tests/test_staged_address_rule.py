@@ -8,11 +8,11 @@ import numpy as np
 import pytest
 
 # (rows of the operand's tile, k of a stage) the kernels are built with
-SHAPES = {2: [(64, 16), (32, 32)], 4: [(64, 32), (32, 64)]}  # by elements of a 16-byte load: FP64, FP32
+SHAPES = {2: [(128, 16), (64, 16), (32, 32)], 4: [(64, 32), (32, 64)]}  # by elements of a 16-byte load: FP64, FP32
 ZERO = -1
 
 
-def stages(E, ROWS, BK, rows, ld, klen, row0, kc):
+def stages(E, ROWS, BK, rows, ld, klen, row0, kc, last):
     """(stage, tile rows, k within it, offsets loaded, offsets stored) for element e of every run."""
     t = np.arange(256)
     CH, HP = BK // E, ROWS // E
@@ -24,10 +24,10 @@ def stages(E, ROWS, BK, rows, ld, klen, row0, kc):
             for e in range(E):
                 er, ek = (0, e) if kc else (e, 0)
                 at = lambda r, k: r * ld + k + s * BK if kc else r + (k + s * BK) * ld
-                if left > BK:  # read
+                if left >= BK + last:  # read
                     x = at(np.minimum(row0 + row, rows - 1), kk) + e
                     yield s, row + er, kk + ek, x, x
-                else:          # read_last
+                else:                  # read_last
                     x = at(np.minimum(row0 + row + er, rows - 1), np.minimum(kk + ek, left - 1))
                     yield s, row + er, kk + ek, x, np.where(kk + ek < left, x, ZERO)
 
@@ -43,11 +43,12 @@ def test_loads_inside_and_at_their_places(E, ROWS, BK, kc):
                 ns = (klen + BK - 1) // BK
                 end = (rows - 1) * ld + klen if kc else rows + (klen - 1) * ld
                 for row0 in range(0, rows, ROWS):
+                    inside = min(ROWS, rows - row0)
                     got = np.full((ROWS, ns * BK), -2, np.int64)
-                    for s, row, k, loaded, stored in stages(E, ROWS, BK, rows, ld, klen, row0, kc):
+                    for s, row, k, loaded, stored in stages(E, ROWS, BK, rows, ld, klen, row0, kc,
+                                                            0 if kc or inside == ROWS else 1):
                         assert np.all((loaded >= 0) & (loaded < end))
                         got[row, s * BK + k] = stored
-                    inside = min(ROWS, rows - row0)
                     r, kk = np.meshgrid(np.arange(inside), np.arange(klen), indexing="ij")
                     assert np.array_equal(got[:inside, :klen], (row0 + r) * ld + kk if kc else row0 + r + kk * ld)
                     assert np.all(got[:inside, klen:] == ZERO)
