@@ -9,7 +9,9 @@
 // 256-thread workgroups, against 5.5-5.8 TB/s for four columns or two
 // vectors per thread and 4.4-4.9 TB/s for grid-stride loops; nontemporal
 // accesses and one-wave workgroups then took the kernels from 73-78 % to
-// 78-83 % of the 8 TB/s peak (a plain 2 GiB copy: 79 -> 83.5 %).
+// 78-83 % of the 8 TB/s peak (a plain 2 GiB copy: 79 -> 83.5 %).  Runs off
+// 16-byte alignment: 5003 x 7001 at 4.9-6.2 TB/s (element by element
+// 3.8-5.2 TB/s).
 #include "dg_internal.hpp"
 
 #include <algorithm>
@@ -25,38 +27,41 @@ typedef __attribute__((address_space(1))) const double gcdouble;
 typedef __attribute__((address_space(1))) double gdouble;
 typedef double dv2 __attribute__((ext_vector_type(2)));
 
-// Every byte these kernels move is read once and written once, so loads and
-// stores carry the nontemporal hint.
+// Every byte these kernels move is read once and written once.
 template <typename G>
 __device__ __forceinline__ void move_nt(const G* src, G* dst) {
     __builtin_nontemporal_store(__builtin_nontemporal_load(src), dst);
 }
 
 // Copies one chunk of `len` <= lanes*E elements (E = 16/sizeof(T)) with the
-// calling thread's `lane` of `lanes`.  When source and destination share
-// their offset within 16 bytes, the first elements up to a 16-byte boundary
-// are copied singly, then one 16-byte vector per lane, then the tail
-// elements; otherwise element by element.
-template <typename T>
+// calling thread's `lane` of `lanes`: the first elements up to a 16-byte
+// boundary of the destination singly, then one 16-byte vector per lane, then
+// the tail elements.  The vector loads take any element's alignment, so only
+// the stores have to be aligned.  LINES: every run starts and ends on a
+// 128-byte line of both buffers; only then does a load carry the nontemporal
+// hint (16384^2: 1-3 % faster), because two workgroups read a line that two
+// runs share (5003 x 7001, runs of 112-715 rows, with the hint 113-140 us,
+// without 90-119 us; element by element, nontemporal, 107-146 us).
+template <bool LINES, typename T>
 __device__ __forceinline__ void copy_chunk(const T* src, T* dst, int64_t len, int lane, int lanes) {
     typedef __attribute__((address_space(1))) const T gcT;
     typedef __attribute__((address_space(1))) T gT;
     typedef T vT __attribute__((ext_vector_type(16 / sizeof(T))));
-    typedef __attribute__((address_space(1))) const vT gcV;
+    typedef vT uT __attribute__((aligned(sizeof(T))));
+    typedef __attribute__((address_space(1))) const uT gcV;
     typedef __attribute__((address_space(1))) vT gV;
     constexpr int E = 16 / sizeof(T);
-    const uintptr_t as = reinterpret_cast<uintptr_t>(src), ad = reinterpret_cast<uintptr_t>(dst);
-    if (!((as ^ ad) & 15)) {
-        int64_t p = (int64_t)(((16 - (as & 15)) & 15) / sizeof(T));
-        if (p > len) p = len;
-        const int64_t nv = (len - p) / E;
-        const int64_t t0 = p + nv * E;
-        if (lane < nv) move_nt((gcV*)(src + p) + lane, (gV*)(dst + p) + lane);
-        if (lane < p) move_nt((gcT*)src + lane, (gT*)dst + lane);
-        if (lane < len - t0) move_nt((gcT*)src + t0 + lane, (gT*)dst + t0 + lane);
-    } else {
-        for (int64_t x = lane; x < len; x += lanes) move_nt((gcT*)src + x, (gT*)dst + x);
+    int64_t p = (int64_t)(((16 - (reinterpret_cast<uintptr_t>(dst) & 15)) & 15) / sizeof(T));
+    if (p > len) p = len;
+    const int64_t nv = (len - p) / E;
+    const int64_t t0 = p + nv * E;
+    if (lane < nv) {
+        gcV* x = (gcV*)(src + p) + lane;
+        const vT v = LINES ? __builtin_nontemporal_load(x) : *x;
+        __builtin_nontemporal_store(v, (gV*)(dst + p) + lane);
     }
+    if (lane < p) move_nt((gcT*)src + lane, (gT*)dst + lane);
+    if (lane < len - t0) move_nt((gcT*)src + t0 + lane, (gT*)dst + t0 + lane);
 }
 
 // Workgroup shape for runs of `run` elements: `lanes` threads (a power of
@@ -87,6 +92,18 @@ unsigned col_groups(int64_t cols, int cols_per_wg) {
     return (unsigned)(g < 1 ? 1 : g);
 }
 
+// Workgroups of `chunks` run chunks (x, spilling into z, so that a dimension
+// stays below 2^32 threads) by `cols` column groups.
+dim3 run_grid(int64_t chunks, unsigned cols) {
+    const int64_t z = (chunks + (1 << 25) - 1) >> 25;
+    return dim3((unsigned)((chunks + z - 1) / z), cols, (unsigned)z);
+}
+
+// Whether two addresses and a length in bytes are whole lines.
+bool whole_lines(const void* a, const void* b, int64_t bytes) {
+    return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)bytes) & 127) == 0;
+}
+
 struct Bands {
     int64_t off[kMaxParts + 1];
     int32_t cpre[kMaxParts + 1];  // first chunk of each band (prefix of its chunk counts)
@@ -96,29 +113,32 @@ struct Bands {
 // Row band b (rows [off[b], off[b+1])) of every column: the packed index of
 // global (r, c) in band b is off[b]*cols + (r - off[b]) + c*rows_b (tiles of
 // one band are contiguous in rank order and share ld = rows_b).  The grid
-// walks the source in memory order: packing reads global columns top to
-// bottom (blockIdx.x = chunk of the column across the bands, blockIdx.y =
-// column group); unpacking reads each band's packed region front to back
-// (blockIdx.x = chunk of the band's column run, blockIdx.y = column group,
-// blockIdx.z = band).
-template <bool PACK>
+// walks global columns top to bottom (blockIdx.x, blockIdx.z = chunk of the
+// column across the bands, blockIdx.y = column group), so that the two bands
+// that share a line of the global matrix are in flight together: unpacking
+// band by band took 129 us for 5003 x 7001 in 7 bands, this order 111 us
+// (5000 x 7000 in 5: 120 -> 88 us).  Where no line is shared (LINES),
+// unpacking reads each band's packed region front to back (blockIdx.x = chunk
+// of the band's column run, blockIdx.z = band; 16384^2 in 4: 667 us, global
+// order 684 us).
+template <bool PACK, bool LINES>
 __global__ __launch_bounds__(kThreads) void block2d_kernel(const double* __restrict__ src, double* __restrict__ dst,
                                                            int64_t ldg, int64_t cols, Bands bands, int lanes_log2) {
-    const int x = blockIdx.x;
     int b;
     int64_t q0;  // first row of the chunk within its band
     const int64_t chunk = (int64_t)2 << lanes_log2;
-    if (PACK) {
+    if (PACK || !LINES) {
+        const int64_t x = (int64_t)blockIdx.z * gridDim.x + blockIdx.x;
         int lo = 0, hi = bands.n - 1;  // band b with cpre[b] <= x < cpre[b+1]
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
             if (bands.cpre[mid] <= x) lo = mid; else hi = mid - 1;
         }
         b = lo;
-        q0 = (int64_t)(x - bands.cpre[b]) * chunk;
+        q0 = (x - bands.cpre[b]) * chunk;
     } else {
         b = blockIdx.z;
-        q0 = (int64_t)x * chunk;
+        q0 = (int64_t)blockIdx.x * chunk;
     }
     const int64_t r0 = bands.off[b];
     const int64_t rb = bands.off[b + 1] - r0;
@@ -130,7 +150,7 @@ __global__ __launch_bounds__(kThreads) void block2d_kernel(const double* __restr
     for (int64_t c = (int64_t)blockIdx.y * cpw + (threadIdx.x >> lanes_log2); c < cols; c += (int64_t)gridDim.y * cpw) {
         const int64_t g = r0 + q0 + c * ldg;
         const int64_t p = band_base + q0 + c * rb;
-        copy_chunk(PACK ? src + g : src + p, PACK ? dst + p : dst + g, len, lane, 1 << lanes_log2);
+        copy_chunk<LINES>(PACK ? src + g : src + p, PACK ? dst + p : dst + g, len, lane, 1 << lanes_log2);
     }
 }
 
@@ -166,56 +186,40 @@ struct Cyclic {
 // ib % P at local row (ib / P)*mb; column c to process column (c/nb) % Q at
 // local column ((c/nb)/Q)*nb + c % nb.  The local matrix of rank (pr, pc)
 // (column-major, ld = its local rows) starts at rowpre(pr)*cols +
-// lrows(pr)*colpre(pc) in the packed buffer.  Packing walks the global
-// columns top to bottom (blockIdx.x = row block * chunks + chunk,
-// blockIdx.y = column group); unpacking walks every rank's local matrix in
-// memory order (blockIdx.x = local row block * chunks + chunk, blockIdx.y =
-// local column group, blockIdx.z = rank pr*Q + pc, looping past 65535).
-template <bool PACK>
+// lrows(pr)*colpre(pc) in the packed buffer.  Both directions walk the global
+// columns top to bottom (blockIdx.x, blockIdx.z = row block * chunks + chunk,
+// blockIdx.y = column group).  Unpacking in this order, against each rank's
+// local matrix front to back: 5003 x 7001 on 3 x 2 in blocks of 128 x 96
+// 110 -> 106 us, 11003 x 12000 on 3 x 4 in 32 x 32 913 -> 806 us, 16384^2 on
+// 4 x 4 in 512 x 512 649 -> 651 us.
+template <bool PACK, bool LINES>
 __global__ __launch_bounds__(kThreads) void cyclic_kernel(const double* __restrict__ src, double* __restrict__ dst,
                                                           Cyclic g, int lanes_log2) {
     const uint32_t chunk = 2u << lanes_log2;
-    const uint32_t blk = fdiv(blockIdx.x, g.dchunks);
-    const uint32_t q0 = (blockIdx.x - blk * g.dchunks.d) * chunk;  // first row of the chunk within its row block
+    const uint32_t x = blockIdx.z * gridDim.x + blockIdx.x;
+    const uint32_t blk = fdiv(x, g.dchunks);
+    const uint32_t q0 = (x - blk * g.dchunks.d) * chunk;  // first row of the chunk within its row block
     const int lane = threadIdx.x & ((1 << lanes_log2) - 1);
     const uint32_t cpw = kThreads >> lanes_log2;
-    if (PACK) {
-        const uint32_t row0 = blk * g.mb + q0;
-        if (row0 >= g.rows || q0 >= g.mb) return;
-        uint32_t len = g.mb - q0 < chunk ? g.mb - q0 : chunk;
-        if (g.rows - row0 < len) len = g.rows - row0;
-        const uint32_t bq = fdiv(blk, g.dP), pr = blk - bq * g.P;
-        const uint32_t lrows = local_extent(g.nr, pr);
-        const int64_t rbase = (int64_t)local_prefix(g.nr, pr) * g.cols + bq * g.mb + q0;
-        for (uint32_t c = blockIdx.y * cpw + (threadIdx.x >> lanes_log2); c < g.cols; c += gridDim.y * cpw) {
-            const uint32_t jb = fdiv(c, g.dnb);
-            const uint32_t jq = fdiv(jb, g.dQ), pc = jb - jq * g.Q;
-            const uint32_t lcol = jq * g.nb + (c - jb * g.nb);
-            const int64_t p = rbase + (int64_t)lrows * (local_prefix(g.nc, pc) + lcol);
-            copy_chunk(src + row0 + c * g.ldg, dst + p, len, lane, 1 << lanes_log2);
-        }
-    } else {
-        for (uint32_t rank = blockIdx.z; rank < g.P * g.Q; rank += gridDim.z) {
-            const uint32_t pr = fdiv(rank, g.dQ), pc = rank - pr * g.Q;
-            const uint32_t lrows = local_extent(g.nr, pr);
-            const uint32_t lr0 = blk * g.mb + q0;  // first local row of the chunk
-            if (lr0 >= lrows || q0 >= g.mb) continue;
-            uint32_t len = g.mb - q0 < chunk ? g.mb - q0 : chunk;
-            if (lrows - lr0 < len) len = lrows - lr0;
-            const uint32_t lcols = local_extent(g.nc, pc);
-            const int64_t base = (int64_t)local_prefix(g.nr, pr) * g.cols + (int64_t)lrows * local_prefix(g.nc, pc) + lr0;
-            const int64_t row0 = (int64_t)(blk * g.P + pr) * g.mb + q0;
-            for (uint32_t lc = blockIdx.y * cpw + (threadIdx.x >> lanes_log2); lc < lcols; lc += gridDim.y * cpw) {
-                const uint32_t lb = fdiv(lc, g.dnb);
-                const int64_t c = (int64_t)(lb * g.Q + pc) * g.nb + (lc - lb * g.nb);
-                copy_chunk(src + base + (int64_t)lc * lrows, dst + row0 + c * g.ldg, len, lane, 1 << lanes_log2);
-            }
-        }
+    if ((uint64_t)blk * g.mb + q0 >= g.rows || q0 >= g.mb) return;
+    const uint32_t row0 = blk * g.mb + q0;
+    uint32_t len = g.mb - q0 < chunk ? g.mb - q0 : chunk;
+    if (g.rows - row0 < len) len = g.rows - row0;
+    const uint32_t bq = fdiv(blk, g.dP), pr = blk - bq * g.P;
+    const uint32_t lrows = local_extent(g.nr, pr);
+    const int64_t rbase = (int64_t)local_prefix(g.nr, pr) * g.cols + bq * g.mb + q0;
+    for (uint32_t c = blockIdx.y * cpw + (threadIdx.x >> lanes_log2); c < g.cols; c += gridDim.y * cpw) {
+        const uint32_t jb = fdiv(c, g.dnb);
+        const uint32_t jq = fdiv(jb, g.dQ), pc = jb - jq * g.Q;
+        const uint32_t lcol = jq * g.nb + (c - jb * g.nb);
+        const int64_t p = rbase + (int64_t)lrows * (local_prefix(g.nc, pc) + lcol);
+        const int64_t at = row0 + c * g.ldg;
+        copy_chunk<LINES>(PACK ? src + at : src + p, PACK ? dst + p : dst + at, len, lane, 1 << lanes_log2);
     }
 }
 
 // blockIdx.x = chunk of a column, blockIdx.y = column group.
-template <typename T>
+template <bool LINES, typename T>
 __global__ __launch_bounds__(kThreads) void copy_block_kernel(int64_t rows, int64_t cols, const T* __restrict__ src,
                                                               int64_t lds, T* __restrict__ dst, int64_t ldd,
                                                               int lanes_log2) {
@@ -227,37 +231,40 @@ __global__ __launch_bounds__(kThreads) void copy_block_kernel(int64_t rows, int6
     const int lane = threadIdx.x & ((1 << lanes_log2) - 1);
     const int cpw = kThreads >> lanes_log2;
     for (int64_t c = (int64_t)blockIdx.y * cpw + (threadIdx.x >> lanes_log2); c < cols; c += (int64_t)gridDim.y * cpw)
-        copy_chunk(src + r0 + c * lds, dst + r0 + c * ldd, len, lane, 1 << lanes_log2);
+        copy_chunk<LINES>(src + r0 + c * lds, dst + r0 + c * ldd, len, lane, 1 << lanes_log2);
 }
 
-// C[x] += partial[0*n + x] + partial[1*n + x] + ... in layer order.  The
-// 128-bit path needs n even so that every layer starts 16-byte aligned; one
-// vector (or element) per thread, the grid covering n.
-template <bool VEC>
+// C[x] += partial[0*n + x] + partial[1*n + x] + ... in layer order, one pair
+// per thread, the grid covering n.  With n odd every second layer starts off
+// 16-byte alignment, and C may: the pair accesses take any element's
+// alignment.  With n odd (ODD) the layers' loads are plain ones, since a line
+// may then serve two workgroups: 35026003 elements and one layer 121 us, with
+// the nontemporal hint 123 us, single elements 142 us; 3 layers 225, 229 and
+// 225 us.  With n even the hint stays (70052006 elements, one layer: 249 us,
+// without 253 us).
+template <bool ODD>
 __global__ __launch_bounds__(kThreads) void layer_reduce_kernel(double* __restrict__ C,
                                                                 const double* __restrict__ partial, int64_t n,
                                                                 int nlayers) {
+    typedef dv2 uv2 __attribute__((aligned(8)));
+    typedef __attribute__((address_space(1))) uv2 guv2;
+    typedef __attribute__((address_space(1))) const uv2 gcuv2;
     gdouble* c = (gdouble*)C;
     gcdouble* p = (gcdouble*)partial;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    if (VEC) {
-        typedef __attribute__((address_space(1))) dv2 gdv2;
-        typedef __attribute__((address_space(1))) const dv2 gcdv2;
-        const int64_t nv = n / 2;
-        for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < nv; x += stride) {
-            dv2 acc = __builtin_nontemporal_load((gdv2*)(c + 2 * x));
+    const int64_t nv = n / 2;
+    for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < nv + (n & 1); x += stride) {
+        if (x < nv) {
+            dv2 acc = __builtin_nontemporal_load((guv2*)(c + 2 * x));
             for (int l = 0; l < nlayers; ++l) {
-                const dv2 v = __builtin_nontemporal_load((gcdv2*)(p + (int64_t)l * n + 2 * x));
-                acc.x += v.x;
-                acc.y += v.y;
+                gcuv2* y = (gcuv2*)(p + (int64_t)l * n + 2 * x);
+                acc += ODD ? *y : __builtin_nontemporal_load(y);
             }
-            __builtin_nontemporal_store(acc, (gdv2*)(c + 2 * x));
-        }
-    } else {
-        for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < n; x += stride) {
-            double acc = __builtin_nontemporal_load(c + x);
-            for (int l = 0; l < nlayers; ++l) acc += __builtin_nontemporal_load(p + (int64_t)l * n + x);
-            __builtin_nontemporal_store(acc, c + x);
+            __builtin_nontemporal_store(acc, (guv2*)(c + 2 * x));
+        } else {
+            double acc = __builtin_nontemporal_load(c + n - 1);
+            for (int l = 0; l < nlayers; ++l) acc += __builtin_nontemporal_load(p + (int64_t)l * n + n - 1);
+            __builtin_nontemporal_store(acc, c + n - 1);
         }
     }
 }
@@ -298,11 +305,12 @@ int block2d(const char* who, const double* src, double* dst, int64_t ldg, int64_
         if (chunks > INT32_MAX) return fail(DG_ERR_INVALID, "%s: too many row chunks", who);
     }
     b.cpre[nrb] = (int32_t)chunks;
-    // packing: chunks of whole global columns; unpacking: chunks of the tallest band, one z per band
-    dim3 grid(PACK ? (unsigned)chunks : (unsigned)((tallest + rs.chunk - 1) / rs.chunk),
-              col_groups(cols, rs.cols_per_wg), PACK ? 1u : (unsigned)nrb);
-    hipLaunchKernelGGL(block2d_kernel<PACK>, grid, dim3(kThreads), 0, as_stream(stream), src, dst, ldg, cols, b,
-                       rs.lanes_log2);
+    bool lines = whole_lines(src, dst, 8 * ldg);
+    for (int i = 1; i <= nrb; ++i) lines = lines && row_off[i] % 16 == 0;
+    dim3 grid = run_grid(chunks, col_groups(cols, rs.cols_per_wg));
+    if (!PACK && lines) grid = dim3((unsigned)((tallest + rs.chunk - 1) / rs.chunk), grid.y, (unsigned)nrb);
+    const auto kernel = lines ? block2d_kernel<PACK, true> : block2d_kernel<PACK, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, as_stream(stream), src, dst, ldg, cols, b, rs.lanes_log2);
     DG_LAUNCH_CHECK();
     return DG_OK;
 }
@@ -330,15 +338,12 @@ int cyclic(const char* who, const double* src, double* dst, int64_t ldg, int64_t
     const RunShape rs = run_shape(mb < rows ? mb : rows, 2);
     g.dP = make_fastdiv(g.P); g.dQ = make_fastdiv(g.Q); g.dnb = make_fastdiv(g.nb);
     g.dchunks = make_fastdiv((uint32_t)rs.chunks);
-    // packing: every global row block; unpacking: process row 0's local row
-    // blocks (the most) and process column 0's local columns (the most)
-    const int64_t row_blocks = PACK ? (rows + mb - 1) / mb : (dg_numroc(rows, mb, 0, 0, P) + mb - 1) / mb;
-    const int64_t ncols = PACK ? cols : dg_numroc(cols, nb, 0, 0, Q);
+    const int64_t row_blocks = (rows + mb - 1) / mb;
     if (row_blocks > INT32_MAX / rs.chunks) return fail(DG_ERR_INVALID, "%s: too many row chunks", who);
-    const int ranks = P * Q;
-    dim3 grid((unsigned)(row_blocks * rs.chunks), col_groups(ncols, rs.cols_per_wg),
-              PACK ? 1u : (unsigned)(ranks < 65535 ? ranks : 65535));
-    hipLaunchKernelGGL(cyclic_kernel<PACK>, grid, dim3(kThreads), 0, as_stream(stream), src, dst, g, rs.lanes_log2);
+    const dim3 grid = run_grid(row_blocks * rs.chunks, col_groups(cols, rs.cols_per_wg));
+    const bool lines = whole_lines(src, dst, 8 * (ldg | rows | std::min(mb, rows)));
+    const auto kernel = lines ? cyclic_kernel<PACK, true> : cyclic_kernel<PACK, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, as_stream(stream), src, dst, g, rs.lanes_log2);
     DG_LAUNCH_CHECK();
     return DG_OK;
 }
@@ -423,7 +428,9 @@ int copy_block(const char* name, int64_t rows, int64_t cols, const T* src, int64
     if (rc) return rc;
     const RunShape rs = run_shape(rows, 16 / (int)sizeof(T));
     if (rs.chunks > INT32_MAX) return fail(DG_ERR_INVALID, "%s: too many rows", name);
-    hipLaunchKernelGGL(copy_block_kernel<T>, dim3((unsigned)rs.chunks, col_groups(cols, rs.cols_per_wg)),
+    const bool lines = whole_lines(src, dst, (lds | ldd | rows) * (int64_t)sizeof(T));
+    const auto kernel = lines ? copy_block_kernel<true, T> : copy_block_kernel<false, T>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)rs.chunks, col_groups(cols, rs.cols_per_wg)),
                        dim3(kThreads), 0, as_stream(stream), rows, cols, src, lds, dst, ldd, rs.lanes_log2);
     DG_LAUNCH_CHECK();
     return DG_OK;
@@ -452,15 +459,10 @@ int dg_layer_reduce(double* C, const double* partial, int64_t n, int nlayers, vo
         return fail(DG_ERR_INVALID, "dg_layer_reduce: buffers must be 16-byte aligned");
     int rc = require_device();
     if (rc) return rc;
-    const bool vec = (n % 2) == 0;
-    int64_t blocks = ((vec ? n / 2 : n) + kThreads - 1) / kThreads;
+    int64_t blocks = ((n + 1) / 2 + kThreads - 1) / kThreads;
     if (blocks > (1 << 30)) blocks = 1 << 30;  // beyond that the kernel loops
-    if (vec)
-        hipLaunchKernelGGL(layer_reduce_kernel<true>, dim3((unsigned)blocks), dim3(kThreads), 0, as_stream(stream), C,
-                           partial, n, nlayers);
-    else
-        hipLaunchKernelGGL(layer_reduce_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, as_stream(stream),
-                           C, partial, n, nlayers);
+    hipLaunchKernelGGL((n & 1) ? layer_reduce_kernel<true> : layer_reduce_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, as_stream(stream), C, partial, n,
+                       nlayers);
     DG_LAUNCH_CHECK();
     return DG_OK;
 }
