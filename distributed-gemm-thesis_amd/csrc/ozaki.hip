@@ -30,6 +30,7 @@
 // would make.
 #include "dg_internal.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 // Every FP64 operation of the recombination is rounded on its own (no fused
@@ -510,23 +511,28 @@ __global__ __launch_bounds__(CNT, OCC) void crt_gemm_kernel(CrtArgs g) {
 // against slices u0 - p of B for p < count, one level, one k range) add up
 // to one long-K product, so a group's k-steps run back to back through the
 // scheme II pipeline above.  Workgroup b computes tile b % tiles of the
-// launch's group b / tiles and stores its 32-bit sums (INT32 for INT8
-// slices, FP32 for BF16 slices) as a plane, [Np][Mp] column-major;
-// oz_combine_kernel then adds the planes into FP64 in group order.
+// launch's job b / tiles (a group) and stores its 32-bit sums (INT32 for
+// INT8 slices, FP32 for BF16 slices) as a plane, [Np][Mp] column-major;
+// oz_combine_kernel then adds the planes into FP64 in group order.  One
+// workgroup has a CU to itself, a launch has a few hundred of them and the
+// groups differ up to 8-fold in length, so the jobs run longest first: in
+// schedule order (counts 1, 2, ... 8) the longest tiles began last and left
+// most CUs idle for their whole length (8 INT8 slices of 3000 x 2000 x 5000:
+// 1115 us a call, longest first 978; 11 BF16 slices of 2048^3: 972 and 833).
 struct OzGroup {
     int32_t t0, u0;   // 0-based slices of the first product
     int32_t count;    // products
     int32_t level;    // t + u + 2 (t, u 1-based) of every product
     int32_t kb;       // byte offset of the k range within a slice row
     FastDiv nks;      // 128-byte k-steps per product (nks.d), as a divisor
+    int32_t plane;    // plane of its launch that takes the sums
 };
 
 struct OzPlaneArgs {
     const int8_t* a;             // A slices, [s][Mp] rows of rb bytes
     const int8_t* b;             // B slices, [s][Np] rows of rb bytes
     int32_t* planes;             // one [Np][Mp] plane per group of the launch
-    const OzGroup* groups;
-    int32_t g0;                  // first group of the launch
+    const OzGroup* jobs;         // the launch's groups, longest first
     int32_t tiles_m, tiles_n;
     int64_t Mp, rb;
     int64_t a_slice, b_slice;    // bytes per slice
@@ -552,7 +558,7 @@ __global__ __launch_bounds__(CNT, OCC) void oz_plane_kernel(OzPlaneArgs g) {
     const int gi = blockIdx.x / tiles;
     int64_t m0, n0;
     tile_origin(blockIdx.x - gi * tiles, tiles, g.tiles_m, g.tiles_n, m0, n0);
-    const OzGroup gr = g.groups[g.g0 + gi];
+    const OzGroup gr = g.jobs[gi];
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -616,7 +622,7 @@ __global__ __launch_bounds__(CNT, OCC) void oz_plane_kernel(OzPlaneArgs g) {
     }
     wait_vmcnt<0>();
     // acc[i][j][v] = sum at (m0 + wm + 16i + 4lg + v, n0 + wn + 16j + lr): one 16-byte store
-    int32_t* out = g.planes + (int64_t)gi * g.plane;
+    int32_t* out = g.planes + (int64_t)gr.plane * g.plane;
 #pragma unroll
     for (int j = 0; j < FN; ++j) {
         const int64_t n = n0 + wn + 16 * j + lr;
@@ -1342,7 +1348,7 @@ bool make_groups(const std::vector<OzSeg>& sched, int64_t esz, std::vector<OzGro
         }
         if ((f.klen * esz) % CK2 != 0 || (f.k0 * esz) % CK2 != 0 || f.klen <= 0) return false;
         out.push_back(OzGroup{f.t, f.u, (int32_t)(j - i + 1), f.level, (int32_t)(f.k0 * esz),
-                              make_fastdiv((uint32_t)(f.klen * esz / CK2))});
+                              make_fastdiv((uint32_t)(f.klen * esz / CK2)), 0});
         if ((int64_t)out.back().count * out.back().nks.d > INT32_MAX) return false;
         i = j + 1;
     }
@@ -1582,23 +1588,33 @@ int dg_ozaki_dgemm(char opA, char opB, int64_t m, int64_t n, int64_t k, double a
     std::vector<OzGroup> groups;
     if (!make_groups(sched, p.esz, groups))
         return fail(DG_ERR_INVALID, "dg_ozaki_dgemm: internal error: product schedule without group form");
+    const int ng = (int)groups.size();
+    const int batch = (int)p.plane_batch;
+    for (int i = 0; i < ng; ++i) groups[i].plane = i % batch;
+    // entries ng.. : the same groups in launch order, each batch's longest first
+    groups.reserve(2 * (size_t)ng);
+    groups.insert(groups.end(), groups.begin(), groups.begin() + ng);
+    for (int g0 = 0; g0 < ng; g0 += batch)
+        std::stable_sort(groups.begin() + ng + g0, groups.begin() + ng + std::min(ng, g0 + batch),
+                         [](const OzGroup& a, const OzGroup& b) {
+                             return (int64_t)a.count * a.nks.d > (int64_t)b.count * b.nks.d;
+                         });
     TableUseScope uses{st};  // after the launches below return
     const OzGroup* dgroups = static_cast<const OzGroup*>(cached_table(groups.data(), groups.size() * sizeof(OzGroup), st));
     if (!dgroups) return DG_ERR_ALLOC;
-    const int ng = (int)groups.size();
     const int64_t tiles = (p.Mp / BM) * (p.Np / BN);
     if (tiles * p.plane_batch > INT32_MAX || (p.Mp / 4) * p.Np > UINT32_MAX)
         return fail(DG_ERR_INVALID, "dg_ozaki_dgemm: too many tiles");
     OzPlaneArgs g{};
-    g.a = sa; g.b = sb; g.planes = reinterpret_cast<int32_t*>(ws + p.off_planes); g.groups = dgroups;
+    g.a = sa; g.b = sb; g.planes = reinterpret_cast<int32_t*>(ws + p.off_planes);
     g.tiles_m = (int32_t)(p.Mp / BM); g.tiles_n = (int32_t)(p.Np / BN);
     g.Mp = p.Mp; g.rb = p.Kp * p.esz; g.a_slice = p.a_slice; g.b_slice = p.b_slice; g.plane = p.Mp * p.Np;
     double* W = reinterpret_cast<double*>(ws + p.off_w);
     const uint32_t total = (uint32_t)((p.Mp / 4) * p.Np);
     const FastDiv dqm = make_fastdiv((uint32_t)(p.Mp / 4));
-    for (int g0 = 0; g0 < ng; g0 += (int)p.plane_batch) {
-        const int cnt = ng - g0 < (int)p.plane_batch ? ng - g0 : (int)p.plane_batch;
-        g.g0 = g0;
+    for (int g0 = 0; g0 < ng; g0 += batch) {
+        const int cnt = std::min(batch, ng - g0);
+        g.jobs = dgroups + ng + g0;
         const dim3 grid((unsigned)(tiles * cnt));
         const dim3 cgrid((total + 255) / 256);
         if (bf16) {
