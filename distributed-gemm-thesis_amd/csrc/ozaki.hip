@@ -806,6 +806,7 @@ __global__ __launch_bounds__(256) void crt_reconstruct_kernel(const uint8_t* __r
 }
 
 typedef double pdv2 __attribute__((ext_vector_type(2)));
+typedef pdv2 udv2 __attribute__((aligned(8)));
 
 // Rows contiguous in k whose every row starts 16-byte aligned: the scans read
 // them in 16-byte pairs, 16 lanes per row (host and device take the same test).
@@ -813,77 +814,92 @@ __host__ __device__ inline bool pair_rows(const double* x, int64_t rs) {
     return !(rs & 1) && !(reinterpret_cast<uintptr_t>(x) & 15);
 }
 
-// Row maxima of op(X): partial max |x| over a k-chunk for every row.
-// Element (row, k) of op(X) is at x[row*rs + k*ks].
-__global__ void oz_partial_max_kernel(const double* __restrict__ x, int64_t rows, int64_t K, int64_t rs, int64_t ks,
-                                      int64_t kchunk, double* __restrict__ part) {
-    // blockIdx.y: k-chunk.  Rows strided in memory (ks != 1): a thread per
-    // row, consecutive lanes on consecutive rows, four loads in flight.
-    // Rows contiguous in k (ks == 1): a wave per row, lanes along k, then a
-    // wave reduction.
-    const int64_t k0 = blockIdx.y * kchunk;
-    const int64_t k1 = min(K, k0 + kchunk);
-    if (ks != 1) {
-        for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < rows; r += (int64_t)gridDim.x * blockDim.x) {
-            const double* xr = x + r * rs;
-            double m0 = 0.0, m1 = 0.0, m2 = 0.0, m3 = 0.0;
-            int64_t k = k0;
-            for (; k + 4 <= k1; k += 4) {
-                m0 = fmax(m0, fabs(xr[k * ks]));
-                m1 = fmax(m1, fabs(xr[(k + 1) * ks]));
-                m2 = fmax(m2, fabs(xr[(k + 2) * ks]));
-                m3 = fmax(m3, fabs(xr[(k + 3) * ks]));
-            }
-            for (; k < k1; ++k) m0 = fmax(m0, fabs(xr[k * ks]));
-            part[blockIdx.y * rows + r] = fmax(fmax(m0, m1), fmax(m2, m3));
-        }
-    } else if (pair_rows(x, rs)) {
-        // 16 lanes per row, k pairs 32 apart: a load of the wave reads 256
-        // contiguous bytes of each of its four rows
-        const int l16 = threadIdx.x & 15;
-        const int64_t groups = (int64_t)gridDim.x * (blockDim.x >> 4);
-        for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 4) + (threadIdx.x >> 4); r < rows; r += groups) {
-            const double* xr = x + r * rs;
-            double mx = 0.0;
-            for (int64_t k = k0 + 2 * l16; k < k1; k += 32) {
-                if (k + 1 < k1) {
-                    const pdv2 v = *reinterpret_cast<const pdv2*>(xr + k);
-                    mx = fmax(mx, fmax(fabs(v.x), fabs(v.y)));
-                } else {
-                    mx = fmax(mx, fabs(xr[k]));
-                }
-            }
+// One operand of scheme I: op(X)(row, k) at x[row*rs + k*ks].
+struct OzSide {
+    const double* x;
+    int64_t rows, rs, ks;
+    double* part;         // chunk maxima, [nchunk][rows], in the place of the slices (written after them)
+    int64_t kchunk;
+    uint32_t nchunk, groups;  // k-chunks and row groups of the maxima pass
+    int32_t* e;           // exponents, zeros in the padding
+    int8_t* out;          // slices
+    int64_t rows_p, slice_bytes;
+};
+
+// Row maxima of both operands in one launch (the first `na` workgroups take
+// op(A)): max |x| over a k-chunk for every row.  Rows strided in memory
+// (ks != 1): a thread per row, consecutive lanes on consecutive rows, 16
+// loads in flight, consecutive workgroups down the columns.  Rows
+// contiguous in k: 16 lanes per row in pairs of any alignment, eight in
+// flight, consecutive workgroups along the rows.  Both operands of 3000 x
+// 2000 x 5000, transposed and plain: 44 us (4.6 TB/s; a launch each with 256
+// k and four loads in flight per thread: 53 us), of 2048^3: 14 us (37 us).
+__global__ __launch_bounds__(NT) void oz_partial_max_kernel(OzSide A, OzSide B, int64_t K, uint32_t na) {
+    const bool first = blockIdx.x < na;
+    const OzSide o = first ? A : B;
+    const uint32_t b = first ? blockIdx.x : blockIdx.x - na;
+    if (o.ks != 1) {
+        const uint32_t c = b / o.groups;
+        const int64_t r = (int64_t)(b - c * o.groups) * NT + threadIdx.x;
+        if (r >= o.rows) return;
+        const int64_t k0 = c * o.kchunk, k1 = min(K, k0 + o.kchunk);
+        const double* xr = o.x + r * o.rs;
+        double mx = 0.0;
+        for (int64_t k = k0; k < k1; k += 16) {
+            double v[16];  // past the end: the last entry again
 #pragma unroll
-            for (int off = 8; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
-            if (l16 == 0) part[blockIdx.y * rows + r] = mx;
+            for (int i = 0; i < 16; ++i) v[i] = xr[min(k + i, k1 - 1) * o.ks];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mx = fmax(mx, fabs(v[i]));
         }
+        o.part[c * o.rows + r] = mx;
     } else {
-        const int lane = threadIdx.x & 63;
-        const int64_t waves = (int64_t)gridDim.x * (blockDim.x >> 6);
-        for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); r < rows; r += waves) {
-            const double* xr = x + r * rs;
-            double mx = 0.0;
-            for (int64_t k = k0 + lane; k < k1; k += 64) mx = fmax(mx, fabs(xr[k]));
+        const uint32_t grp = b / o.nchunk, c = b - grp * o.nchunk;
+        const int l16 = threadIdx.x & 15;
+        const int64_t r = (int64_t)grp * (NT / 16) + (threadIdx.x >> 4);
+        if (r >= o.rows) return;  // whole 16-lane groups leave together
+        const int64_t k0 = c * o.kchunk, k1 = min(K, k0 + o.kchunk);
+        const double* xr = o.x + r * o.rs;
+        double mx = 0.0;
+        for (int64_t k = k0; k < k1; k += 256) {
+            if (k + 256 <= k1) {
+                udv2 v[8];
 #pragma unroll
-            for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
-            if (lane == 0) part[blockIdx.y * rows + r] = mx;
+                for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const udv2*>(xr + k + 32 * i + 2 * l16);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) mx = fmax(mx, fmax(fabs(v[i].x), fabs(v[i].y)));
+            } else {
+                for (int64_t kk = k + l16; kk < k1; kk += 16) mx = fmax(mx, fabs(xr[kk]));
+            }
         }
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
+        if (l16 == 0) o.part[c * o.rows + r] = mx;
     }
 }
 
-// Reduces the chunk maxima and writes the frexp exponent (0 for zero rows,
-// and for the padding rows beyond `rows`).
-__global__ void oz_exponent_kernel(const double* __restrict__ part, int64_t rows, int64_t rows_p, int nchunk,
-                                   int32_t* __restrict__ e) {
-    for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < rows_p; r += (int64_t)gridDim.x * blockDim.x) {
-        int ex = 0;
-        if (r < rows) {
-            double mx = 0.0;
-            for (int c = 0; c < nchunk; ++c) mx = fmax(mx, part[(int64_t)c * rows + r]);
-            if (mx != 0.0) frexp(mx, &ex);
-        }
-        e[r] = ex;
+// Reduces the chunk maxima of both operands and writes the frexp exponents
+// (0 for zero rows, and for the padding rows beyond `rows`): 64 rows per
+// workgroup (rows_p is a multiple of 256), its waves splitting the chunks.
+__global__ __launch_bounds__(NT) void oz_exponent_kernel(OzSide A, OzSide B) {
+    __shared__ double red[NT / 64][64];
+    const uint32_t na = (uint32_t)(A.rows_p / 64);
+    const bool first = blockIdx.x < na;
+    const OzSide o = first ? A : B;
+    const int64_t r = (int64_t)(first ? blockIdx.x : blockIdx.x - na) * 64 + (threadIdx.x & 63);
+    double mx = 0.0;
+    if (r < o.rows) {
+#pragma unroll 4
+        for (uint32_t c = threadIdx.x >> 6; c < o.nchunk; c += NT / 64) mx = fmax(mx, o.part[c * o.rows + r]);
     }
+    red[threadIdx.x >> 6][threadIdx.x & 63] = mx;
+    __syncthreads();
+    if (threadIdx.x >= 64) return;
+#pragma unroll
+    for (int w = 1; w < NT / 64; ++w) mx = fmax(mx, red[w][threadIdx.x]);
+    int ex = 0;
+    if (mx != 0.0) frexp(mx, &ex);
+    o.e[r] = ex;
 }
 
 // Ozaki scheme II scaling (Cauchy-Schwarz bound).  Entry bound: |x| = m 2^ex
@@ -1081,61 +1097,112 @@ __global__ __launch_bounds__(256) void crt_shift_kernel(const uint64_t* __restri
 }
 
 // Writes the s digits of op(X)(row, k) into slices[t][row][Kp] (zeros in the
-// padding).  A 64x64 tile goes through LDS so that both the read of op(X)
-// and the k-contiguous slice writes are coalesced whatever op(X)'s layout.
+// padding), both operands in one launch.  A workgroup takes OS_R rows by
+// OS_K k, a thread four consecutive k of every 8th row: one store per row
+// and slice, 128 (INT8) or 256 (BF16) contiguous bytes per row.  Rows
+// contiguous in k are read straight into registers, 16 bytes at any
+// alignment; rows strided in memory go through LDS, loaded along the rows
+// (quads of k rotated by 2 (k / 32) places, so that the reads of four
+// consecutive k per lane spread over the banks).  Bound by memory: the
+// arithmetic (six operations per element and slice) takes less than half of
+// the time of reading op(X) and writing the slices.  3000 x 2000 x 5000 into
+// 8 INT8 slices: 74 us (5.5 TB/s; 64 x 64 tiles through LDS, one launch per
+// operand: 146 us), 2048^3 into 11 BF16 slices: 41 us (56 us).
+constexpr int OS_R = 32, OS_K = 128;
+
+__device__ __forceinline__ int os_pos(int k) { return (k & ~3) | ((k + 2 * (k >> 5)) & 3); }
+
 template <bool BF16>
-__global__ void oz_slice_kernel(const double* __restrict__ x, int64_t rows, int64_t K, int64_t rs, int64_t ks,
-                                const int32_t* __restrict__ e, int s, int bits, int8_t* __restrict__ out,
-                                int64_t Kp, int64_t slice_bytes) {
-    __shared__ double tile[64][65];
-    const int64_t r0 = (int64_t)blockIdx.y * 64;
-    const int64_t k0 = (int64_t)blockIdx.x * 64;
-    const int tx = threadIdx.x & 63;
-    const int ty = threadIdx.x >> 6;  // 0..3
-    // load: along the contiguous direction of op(X)
-    if (ks == 1) {
-        for (int rr = ty; rr < 64; rr += 4) {
-            const int64_t r = r0 + rr, k = k0 + tx;
-            tile[rr][tx] = (r < rows && k < K) ? x[r * rs + k] : 0.0;
-        }
-    } else {
-        for (int kk = ty; kk < 64; kk += 4) {
-            const int64_t r = r0 + tx, k = k0 + kk;
-            tile[tx][kk] = (r < rows && k < K) ? x[r * rs + k * ks] : 0.0;
-        }
-    }
-    __syncthreads();
-    const double scale = ldexp(1.0, bits);
-    // thread: row t/4 of the tile, 16 consecutive k -> 16 (INT8) or 32 (BF16) bytes per slice
-    const int rr = threadIdx.x >> 2;
-    const int kq = (threadIdx.x & 3) * 16;
-    const int64_t r = r0 + rr;
-    double v[16];
-    const int sh = r < rows ? -e[r] : 0;
+__global__ __launch_bounds__(NT) void oz_slice_kernel(OzSide A, OzSide B, int64_t K, int64_t Kp, int s, int bits,
+                                                      uint32_t nkt, uint32_t na, uint32_t tiles) {
+    __shared__ double tile[OS_R][OS_K + 1];
+    uint32_t b = blockIdx.y * gridDim.x + blockIdx.x;
+    if (b >= tiles) return;
+    const bool first = b < na;
+    const OzSide o = first ? A : B;
+    if (!first) b -= na;
+    const int t = threadIdx.x;
+    const int kq = 4 * (t & 31);
+    int64_t r0, k0;
+    double v[4][4];
+    if (o.ks == 1) {  // tiles along k
+        r0 = (int64_t)(b / nkt) * OS_R;
+        k0 = (int64_t)(b % nkt) * OS_K;
+        const int64_t k = k0 + kq;
+        if (r0 + OS_R <= o.rows && k0 + OS_K <= K) {
+            udv2 w[4][2];
 #pragma unroll
-    for (int c = 0; c < 16; ++c) v[c] = r < rows ? ldexp(tile[rr][kq + c], sh) : 0.0;
-    int8_t* dst = out + (r * Kp + k0 + kq) * (BF16 ? 2 : 1);
-    for (int t = 0; t < s; ++t) {
-        uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+            for (int i = 0; i < 4; ++i) {
+                const double* xr = o.x + (r0 + (t >> 5) + 8 * i) * o.rs + k;
+                w[i][0] = *reinterpret_cast<const udv2*>(xr);
+                w[i][1] = *reinterpret_cast<const udv2*>(xr + 2);
+            }
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-            v[c] = v[c] * scale;
-            const double d = trunc(v[c]);
-            v[c] = v[c] - d;
-            if (BF16) {
-                const float f = (float)d;  // |d| <= 31: exact, low mantissa bits zero
-                w[c >> 1] |= (__float_as_uint(f) >> 16) << (16 * (c & 1));
-            } else {
-                w[c >> 2] |= (uint32_t)(uint8_t)(int8_t)(int)d << (8 * (c & 3));
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[i][c] = w[i][c >> 1][c & 1];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int64_t r = r0 + (t >> 5) + 8 * i;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[i][c] = r < o.rows && k + c < K ? o.x[r * o.rs + k + c] : 0.0;
             }
         }
-        iv4* o = reinterpret_cast<iv4*>(dst + t * slice_bytes);
-        o[0] = iv4{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
-        if (BF16) o[1] = iv4{(int)w[4], (int)w[5], (int)w[6], (int)w[7]};
+    } else {  // tiles down the rows
+        const uint32_t nrt = (uint32_t)(o.rows_p / OS_R);
+        r0 = (int64_t)(b % nrt) * OS_R;
+        k0 = (int64_t)(b / nrt) * OS_K;
+        const int64_t r = r0 + (t & 31);
+        const double* xr = o.x + min(r, o.rows - 1) * o.rs;
+        double w[16];  // past the edges: the last row or entry again
+#pragma unroll
+        for (int i = 0; i < 16; ++i) w[i] = xr[min(k0 + (t >> 5) + 8 * i, K - 1) * o.ks];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int kk = (t >> 5) + 8 * i;
+            tile[t & 31][os_pos(kk)] = r < o.rows && k0 + kk < K ? w[i] : 0.0;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) v[i][c] = tile[(t >> 5) + 8 * i][os_pos(kq + c)];
+    }
+    if (k0 + kq >= Kp) return;  // Kp is a multiple of 64
+    const double scale = ldexp(1.0, bits);
+    int8_t* dst = o.out + ((r0 + (t >> 5)) * Kp + k0 + kq) * (BF16 ? 2 : 1);
+    const int64_t step = 8 * Kp * (BF16 ? 2 : 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int sh = -o.e[r0 + (t >> 5) + 8 * i];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[i][c] = ldexp(v[i][c], sh);
+    }
+    for (int l = 0; l < s; ++l) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t w[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                v[i][c] = v[i][c] * scale;
+                const double d = trunc(v[i][c]);
+                v[i][c] = v[i][c] - d;
+                // BF16: |d| <= 31 is exact, its low mantissa bits are zero
+                w[c] = BF16 ? __float_as_uint((float)d) : (uint32_t)(int)d;
+            }
+            int8_t* q = dst + l * o.slice_bytes + i * step;
+            if (BF16) {
+                *reinterpret_cast<u32x2*>(q) = u32x2{__builtin_amdgcn_perm(w[1], w[0], 0x07060302u),
+                                                     __builtin_amdgcn_perm(w[3], w[2], 0x07060302u)};
+            } else {
+                *reinterpret_cast<uint32_t*>(q) =
+                    __builtin_amdgcn_perm(__builtin_amdgcn_perm(w[3], w[2], 0x0c0c0400u),
+                                          __builtin_amdgcn_perm(w[1], w[0], 0x0c0c0400u), 0x05040100u);
+            }
+        }
     }
 }
-
-constexpr int64_t kMaxChunk = 256;  // k-chunk of the max reduction
 
 int64_t round_up(int64_t x, int64_t m) { return (x + m - 1) / m * m; }
 
@@ -1166,7 +1233,7 @@ namespace {
 constexpr int kPlaneBatch = 8;
 
 struct Plan {
-    int64_t Mp, Np, Kp, esz, a_slice, b_slice, res_plane, nchunk_a, nchunk_b, kchunk_max;
+    int64_t Mp, Np, Kp, esz, a_slice, b_slice, res_plane;
     int64_t plane_batch;  // scheme I: groups per product launch
     size_t off_a, off_b, off_ea, off_eb, off_part, off_w, off_planes, total;
 };
@@ -1236,10 +1303,6 @@ Plan make_crt_plan(int64_t m, int64_t n, int64_t k, int nmod) {
     p.a_slice = p.Mp * p.Kp;
     p.b_slice = p.Np * p.Kp;
     p.res_plane = p.Mp * p.Np;
-    p.kchunk_max = CRT_KC;  // the line scan's k-chunk (k < 2^17 keeps grid.y below 2^11)
-    p.nchunk_a = (k + CRT_KC - 1) / CRT_KC;
-    if (p.nchunk_a < 1) p.nchunk_a = 1;
-    p.nchunk_b = p.nchunk_a;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off = (off + bytes + 255) / 256 * 256; return o; };
     p.off_a = take((size_t)crt_operand_bytes(m, k, nmod));
@@ -1260,18 +1323,12 @@ Plan make_plan(int64_t m, int64_t n, int64_t k, int s, bool bf16) {
     p.Kp = round_up(k > 0 ? k : 1, KSB / p.esz);
     p.a_slice = p.Mp * p.Kp * p.esz;
     p.b_slice = p.Np * p.Kp * p.esz;
-    p.kchunk_max = kMaxChunk;
-    while ((k + p.kchunk_max - 1) / p.kchunk_max > 4096) p.kchunk_max *= 2;  // keep grid.y small
-    p.nchunk_a = (k + p.kchunk_max - 1) / p.kchunk_max;
-    if (p.nchunk_a < 1) p.nchunk_a = 1;
-    p.nchunk_b = p.nchunk_a;
     size_t off = 0;
     auto take = [&](size_t bytes) { size_t o = off; off = (off + bytes + 255) / 256 * 256; return o; };
     p.off_a = take((size_t)s * p.a_slice);
     p.off_b = take((size_t)s * p.b_slice);
     p.off_ea = take((size_t)p.Mp * 4);
     p.off_eb = take((size_t)p.Np * 4);
-    p.off_part = take((size_t)p.nchunk_a * (size_t)(m > n ? m : n) * 8);
     p.off_w = take((size_t)p.Mp * (size_t)p.Np * 8);
     {  // group planes
         int err = 0;
@@ -1529,13 +1586,10 @@ int dg_ozaki_dgemm(char opA, char opB, int64_t m, int64_t n, int64_t k, double a
     int8_t* sb = reinterpret_cast<int8_t*>(ws + p.off_b);
     int32_t* ea = reinterpret_cast<int32_t*>(ws + p.off_ea);
     int32_t* eb = reinterpret_cast<int32_t*>(ws + p.off_eb);
-    double* part = reinterpret_cast<double*>(ws + p.off_part);
 
     // op(A)(i, k) at A[i*rs + k*ks]; op(B) as the rows of its transpose: B^T(j, k).
     const int64_t a_rs = oa == 'N' ? 1 : lda, a_ks = oa == 'N' ? lda : 1;
     const int64_t b_rs = ob == 'N' ? ldb : 1, b_ks = ob == 'N' ? 1 : ldb;
-    const int nchunk = (int)p.nchunk_a;
-    const unsigned gy = (unsigned)nchunk;
 
     if (crt) {
         // op(A)'s rows and op(B)'s columns prepared in the workspace, then their product
@@ -1544,45 +1598,36 @@ int dg_ozaki_dgemm(char opA, char opB, int64_t m, int64_t n, int64_t k, double a
         if (!rc) rc = crt_multiply(m, n, k, slices, alpha, ws + p.off_a, ws + p.off_b, beta, C, ldc, ws + p.off_w, st);
         return rc;
     }
-    {
-        // Row exponents of op(A), column exponents of op(B).
-        // ks == 1: 16 lanes per row when the rows pair up (NT/16 rows per block), else
-        // a wave per row (NT/64); otherwise a thread per row
-        auto pm_grid = [](int64_t rows, int64_t ks, const double* x, int64_t rs) {
-            const int64_t per = ks == 1 ? (pair_rows(x, rs) ? NT / 16 : NT / 64) : NT;
-            const int64_t g = (rows + per - 1) / per;
-            return (unsigned)(g < 65535 ? g : 65535);
-        };
-        unsigned gx = pm_grid(m, a_ks, A, a_rs);
-        hipLaunchKernelGGL(oz_partial_max_kernel, dim3(gx, gy), dim3(NT), 0, st, A, m, k, a_rs, a_ks, p.kchunk_max, part);
-        DG_LAUNCH_CHECK();
-        hipLaunchKernelGGL(oz_exponent_kernel, dim3((unsigned)((p.Mp + NT - 1) / NT)), dim3(NT), 0, st, part, m, p.Mp,
-                           nchunk, ea);
-        DG_LAUNCH_CHECK();
-        gx = pm_grid(n, b_ks, B, b_rs);
-        hipLaunchKernelGGL(oz_partial_max_kernel, dim3(gx, gy), dim3(NT), 0, st, B, n, k, b_rs, b_ks, p.kchunk_max, part);
-        DG_LAUNCH_CHECK();
-        hipLaunchKernelGGL(oz_exponent_kernel, dim3((unsigned)((p.Np + NT - 1) / NT)), dim3(NT), 0, st, part, n, p.Np,
-                           nchunk, eb);
-        DG_LAUNCH_CHECK();
-    }
-    // Slices (the padding is written as zeros by the same kernels).
-    {
-        dim3 ga((unsigned)(p.Kp / 64), (unsigned)(p.Mp / 64));
-        dim3 gb((unsigned)(p.Kp / 64), (unsigned)(p.Np / 64));
-        if (bf16) {
-            hipLaunchKernelGGL(oz_slice_kernel<true>, ga, dim3(NT), 0, st, A, m, k, a_rs, a_ks, ea, slices, bits, sa,
-                               p.Kp, p.a_slice);
-            hipLaunchKernelGGL(oz_slice_kernel<true>, gb, dim3(NT), 0, st, B, n, k, b_rs, b_ks, eb, slices, bits, sb,
-                               p.Kp, p.b_slice);
-        } else {
-            hipLaunchKernelGGL(oz_slice_kernel<false>, ga, dim3(NT), 0, st, A, m, k, a_rs, a_ks, ea, slices, bits, sa,
-                               p.Kp, p.a_slice);
-            hipLaunchKernelGGL(oz_slice_kernel<false>, gb, dim3(NT), 0, st, B, n, k, b_rs, b_ks, eb, slices, bits, sb,
-                               p.Kp, p.b_slice);
-        }
-        DG_LAUNCH_CHECK();
-    }
+    // Row exponents of op(A), column exponents of op(B), then the slices (the
+    // padding is written as zeros by the same kernels).  The chunk maxima lie
+    // where the slices go: a chunk has at least 32 k, 8 bytes of maximum
+    // against 32 bytes of the smallest slice.
+    const auto side = [&](const double* x, int64_t rows, int64_t rs, int64_t ks, int8_t* out, int32_t* e,
+                          int64_t rows_p, int64_t slice_bytes) {
+        OzSide o{x, rows, rs, ks, reinterpret_cast<double*>(out), ks == 1 ? 256 : 32, 0, 0, e, out, rows_p, slice_bytes};
+        while ((k + o.kchunk - 1) / o.kchunk > 4096) o.kchunk *= 2;  // bounds the grid and the reduction
+        o.nchunk = (uint32_t)((k + o.kchunk - 1) / o.kchunk);
+        const int64_t per = ks == 1 ? NT / 16 : NT;
+        o.groups = (uint32_t)((rows + per - 1) / per);
+        return o;
+    };
+    const OzSide da = side(A, m, a_rs, a_ks, sa, ea, p.Mp, p.a_slice);
+    const OzSide db = side(B, n, b_rs, b_ks, sb, eb, p.Np, p.b_slice);
+    const int64_t max_a = (int64_t)da.groups * da.nchunk, max_b = (int64_t)db.groups * db.nchunk;
+    const uint32_t nkt = (uint32_t)((p.Kp + OS_K - 1) / OS_K);
+    const int64_t sl_a = p.Mp / OS_R * nkt, sl = sl_a + p.Np / OS_R * nkt;
+    const int64_t sl_y = (sl >> 23) + 1;  // keeps a dimension below 2^32 threads
+    if (max_a + max_b >= (int64_t)1 << 24 || sl > INT32_MAX)
+        return fail(DG_ERR_UNSUPPORTED, "dg_ozaki_dgemm: matrix too large for one slicing launch");
+    hipLaunchKernelGGL(oz_partial_max_kernel, dim3((unsigned)(max_a + max_b)), dim3(NT), 0, st, da, db, k,
+                       (uint32_t)max_a);
+    DG_LAUNCH_CHECK();
+    hipLaunchKernelGGL(oz_exponent_kernel, dim3((unsigned)((p.Mp + p.Np) / 64)), dim3(NT), 0, st, da, db);
+    DG_LAUNCH_CHECK();
+    hipLaunchKernelGGL(bf16 ? oz_slice_kernel<true> : oz_slice_kernel<false>,
+                       dim3((unsigned)((sl + sl_y - 1) / sl_y), (unsigned)sl_y), dim3(NT), 0, st, da, db, k, p.Kp,
+                       slices, bits, nkt, (uint32_t)sl_a, (uint32_t)sl);
+    DG_LAUNCH_CHECK();
     // INT8 products: each launch computes up to plane_batch groups into
     // planes, then the combine adds them into W (or, after the last group, C).
     std::vector<OzGroup> groups;
