@@ -45,7 +45,10 @@ typedef int iv4 __attribute__((ext_vector_type(4)));
 typedef float fv4 __attribute__((ext_vector_type(4)));
 typedef double dv4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+typedef double pdv2 __attribute__((ext_vector_type(2)));
+typedef pdv2 udv2 __attribute__((aligned(8)));  // a pair at any alignment
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
 
 constexpr int PAD = 256;     // row padding of the slices and residues (a multiple of BM and BN)
 constexpr int KSB = 128;     // K padding granule of the slices and residues, bytes
@@ -160,21 +163,25 @@ __host__ __device__ constexpr int crt_modulus(int t) {
 
 // Balanced residues of A' = rint(op(X)(row, k) * 2^(q - e_row)) for every
 // modulus, [t][row][Kp] int8 (zeros in the padding).  A workgroup stages a
-// 16-row x 128-k tile of op(X) through LDS (loaded along whichever direction
-// is contiguous in memory; 16.5 KB, so eight workgroups share a CU and the
-// load and arithmetic phases of different workgroups overlap); each thread
-// then turns 8 consecutive k of one row into one 8-byte store per modulus,
-// so a wave writes whole 128-byte lines.  Residues in [-floor(p/2),
-// ceil(p/2) - 1] from an exact split of A' (below), five FP64 operations
-// per element and modulus.
-constexpr int RT_R = 16, RT_K = 128, RT_T = 256 / RT_R, RT_KPT = RT_K / RT_T;  // threads per row, k per thread
-// Per-modulus constants of the residue pass, passed as kernel arguments so
-// that they sit in scalar registers (a VOP3 FMA takes them directly; gfx9
-// VOP3 encodings take no 64-bit literals).
+// tile of op(X) through LDS, loaded along whichever direction is contiguous
+// in memory (16.5 KB, so eight workgroups share a CU and the load and store
+// phases of different workgroups overlap); each thread then turns 8
+// consecutive k of one row into one 8-byte store per modulus, so a wave
+// writes whole 128-byte lines.  One FP64 operation and one packed 16-bit one
+// per two elements make a residue (below), which leaves the pass bound by
+// its memory traffic, two thirds of it stores to as many places as there are
+// moduli.  8192^2 and 14 moduli (1.48 GB): contiguous lines 285 -> 273 us from
+// tiles of 16 x 128 to 8 x 256 (straight from registers, without LDS: 297),
+// strided lines 335 -> 285 us from nontemporal to plain stores (plain ones
+// cost the contiguous form 25 us).
+constexpr int RT_R = 16, RT_K = 128;  // tile of strided lines
+constexpr int RC_R = 8, RC_K = 256;   // tile of lines contiguous in k
+
+// fl(1/p) of each modulus, passed as a kernel argument so that it sits in
+// scalar registers (a VOP3 FMA takes it directly; gfx9 VOP3 encodings take no
+// 64-bit literals).
 struct ResidueConsts {
-    double c24[kMaxModuli];   // 2^24 mod p
-    double inv_p[kMaxModuli]; // fl(1/p)
-    double pd[kMaxModuli];    // p
+    double inv_p[kMaxModuli];
 };
 
 // Tile order of the residue pass (blockIdx.x -> row tile, k tile): lines
@@ -189,89 +196,96 @@ __global__ __launch_bounds__(256) void crt_residue_kernel(const double* __restri
                                                           int64_t rs, int64_t ks, const int32_t* __restrict__ e, int q,
                                                           int8_t* __restrict__ out, int64_t Kp, int64_t slice_bytes,
                                                           ResidueConsts rc, uint32_t nkt, uint32_t nrt) {
-    __shared__ double tile[RT_R][RT_K + 1];
-    uint32_t kt, rt;
+    __shared__ double tile[RT_R * (RT_K + 1)];
+    static_assert(RC_R * (RC_K + 1) <= RT_R * (RT_K + 1), "either tile fits");
+    constexpr int KPT = 8;
+    const int t = threadIdx.x;
+    int64_t r, k0;
+    const double* row;  // the thread's eight k in the tile
+    double w[KPT];
+    // Eight loads per thread, all issued before the first wait: addresses
+    // outside op(X) are clamped onto its last row / k (in bounds) and the
+    // loaded value replaced by zero.  op(X) is read for the last time here.
     if (ks == 1) {
-        rt = blockIdx.x / nkt;
-        kt = blockIdx.x - rt * nkt;
+        const uint32_t rt = blockIdx.x / nkt;
+        const int64_t r0 = (int64_t)rt * RC_R;
+        k0 = (int64_t)(blockIdx.x - rt * nkt) * RC_K;
+        const int64_t k = k0 + t;
+        const int64_t kc = k < K ? k : K - 1;
+#pragma unroll
+        for (int i = 0; i < RC_R; ++i)
+            w[i] = __builtin_nontemporal_load(x + (r0 + i < rows ? r0 + i : rows - 1) * rs + kc);
+#pragma unroll
+        for (int i = 0; i < RC_R; ++i) tile[i * (RC_K + 1) + t] = k < K ? w[i] : 0.0;
+        r = r0 + t / (RC_K / KPT);
+        k0 += KPT * (t % (RC_K / KPT));
+        row = tile + t / (RC_K / KPT) * (RC_K + 1) + KPT * (t % (RC_K / KPT));
     } else {
         const uint32_t grp = blockIdx.x / (RT_KG * nrt);
         const uint32_t first = grp * RT_KG;
         const uint32_t gk = nkt - first < RT_KG ? nkt - first : RT_KG;
         const uint32_t in = blockIdx.x - grp * RT_KG * nrt;
-        rt = in / gk;
-        kt = first + (in - rt * gk);
-    }
-    const int64_t r0 = (int64_t)rt * RT_R;
-    const int64_t k0 = (int64_t)kt * RT_K;
-    const int t = threadIdx.x;
-    // Eight loads per thread, all issued before the first wait: addresses
-    // outside op(X) are clamped onto its last row / k (in bounds) and the
-    // loaded value replaced by zero.  op(X) is read once here and the
-    // residues written once, so both go nontemporal.
-    if (ks == 1) {
-        const int64_t k = k0 + (t & 127);
-        const int64_t kc = k < K ? k : K - 1;
-        double v[RT_R / 2];
+        const uint32_t rt = in / gk;
+        const int64_t r0 = (int64_t)rt * RT_R;
+        k0 = (int64_t)(first + (in - rt * gk)) * RT_K;
+        const int64_t lr = r0 + t % RT_R;
+        const double* xr = x + (lr < rows ? lr : rows - 1) * rs;
 #pragma unroll
-        for (int i = 0; i < RT_R / 2; ++i) {
-            const int64_t r = r0 + (t >> 7) + 2 * i;
-            v[i] = __builtin_nontemporal_load(x + (r < rows ? r : rows - 1) * rs + kc);
-        }
-#pragma unroll
-        for (int i = 0; i < RT_R / 2; ++i) {
-            const int rr = (t >> 7) + 2 * i;
-            tile[rr][t & 127] = (r0 + rr < rows && k < K) ? v[i] : 0.0;
-        }
-    } else {
-        const int64_t r = r0 + (t % RT_R);
-        const int64_t rc = r < rows ? r : rows - 1;
-        double v[RT_K * RT_R / 256];
-#pragma unroll
-        for (int i = 0; i < RT_K * RT_R / 256; ++i) {
+        for (int i = 0; i < KPT; ++i) {
             const int64_t k = k0 + t / RT_R + (256 / RT_R) * i;
-            v[i] = __builtin_nontemporal_load(x + rc * rs + (k < K ? k : K - 1) * ks);
+            w[i] = __builtin_nontemporal_load(xr + (k < K ? k : K - 1) * ks);
         }
 #pragma unroll
-        for (int i = 0; i < RT_K * RT_R / 256; ++i) {
+        for (int i = 0; i < KPT; ++i) {
             const int kk = t / RT_R + (256 / RT_R) * i;
-            tile[t % RT_R][kk] = (r < rows && k0 + kk < K) ? v[i] : 0.0;
+            tile[t % RT_R * (RT_K + 1) + kk] = k0 + kk < K ? w[i] : 0.0;
         }
+        r = r0 + t / (RT_K / KPT);
+        k0 += KPT * (t % (RT_K / KPT));
+        row = tile + t / (RT_K / KPT) * (RT_K + 1) + KPT * (t % (RT_K / KPT));
     }
     __syncthreads();
-    const int rr = t / RT_T;
-    const int kq = (t % RT_T) * RT_KPT;
-    const int64_t r = r0 + rr;
-    // a = ah 2^24 + al exactly (al in [0, 2^24)), so for each modulus
-    // y = ah (2^24 mod p) + al = a (mod p) with |y| < 2^38, whose quotient
-    // estimate fma(y, fl(1/p), 1/2) is within 2^-22 of y/p + 1/2 (never closer
-    // than 1/(2p) to an integer for odd p; exact for p = 256, where y = al):
-    // r = y - p floor(y/p + 1/2) is the balanced residue, computed exactly.
-    double ah[RT_KPT], al[RT_KPT];
+    if (k0 >= Kp) return;  // Kp is a multiple of 128
+    // |a| <= 2^53 and |fl(1/p) - 1/p| <= 2^-61, so t = fma(a, fl(1/p), 1.5 2^52)
+    // is 1.5 2^52 + q with an integer q within 1/2 + 2^-8 of a/p, and r = a - q p
+    // is at most p/2 + p/256 in magnitude: at most 127 for p <= 253, for p = 255
+    // too (fl(1/255) is within 2^-63), and 128 = -128 (mod 256) for p = 256.  Its
+    // low byte, which is r, needs a and q modulo 256 only: a + q (256 - p) on the
+    // low half words of t, two elements at a time.  Not-a-numbers and infinities
+    // count as zeros.
+    double a[KPT];
+    u16x2 ab[KPT / 2];
     const int sh = r < rows ? q - e[r] : 0;
 #pragma unroll
-    for (int c = 0; c < RT_KPT; ++c) {
-        const double a = r < rows ? rint(ldexp(tile[rr][kq + c], sh)) : 0.0;
-        ah[c] = floor(a * 0x1p-24);
-        al[c] = fma(-ah[c], 0x1p24, a);
+    for (int c = 0; c < KPT; ++c) {
+        const double y = rint(ldexp(row[c], sh));
+        a[c] = r < rows && fabs(y) <= 0x1p53 ? y : 0.0;
+        const double f = a[c] * 0x1p-8;
+        ab[c / 2][c % 2] = (unsigned short)(int)((f - floor(f)) * 256.0);
     }
-    int8_t* dst = out + r * Kp + k0 + kq;
+    int8_t* dst = out + r * Kp + k0;
 #pragma unroll
     for (int m = 0; m < NMOD; ++m) {
-        static_assert(RT_KPT == 8, "one 8-byte store per modulus");
-        uint32_t v[RT_KPT];
+        uint32_t rb[KPT / 2];
 #pragma unroll
-        for (int c = 0; c < RT_KPT; ++c) {
-            const double y = m == 0 ? al[c] : fma(ah[c], rc.c24[m], al[c]);
-            const double qd = floor(fma(y, rc.inv_p[m], 0.5));
-            v[c] = (uint32_t)(int)fma(-qd, rc.pd[m], y);
+        for (int c = 0; c < KPT / 2; ++c) {
+            if (m == 0) {  // p = 256
+                rb[c] = __builtin_bit_cast(uint32_t, ab[c]);
+                continue;
+            }
+            const uint32_t t0 = (uint32_t)__double_as_longlong(fma(a[2 * c], rc.inv_p[m], 0x1.8p52));
+            const uint32_t t1 = (uint32_t)__double_as_longlong(fma(a[2 * c + 1], rc.inv_p[m], 0x1.8p52));
+            const u16x2 qw = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(t1, t0, 0x05040100u));
+            const unsigned short d = (unsigned short)(256 - crt_modulus(m));
+            rb[c] = __builtin_bit_cast(uint32_t, qw * u16x2{d, d} + ab[c]);
         }
-        // bytes 0 of four words into one word: two selections of two bytes, then one of the two halves
-        const uint32_t w0 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(v[3], v[2], 0x0c0c0400u),
-                                                  __builtin_amdgcn_perm(v[1], v[0], 0x0c0c0400u), 0x05040100u);
-        const uint32_t w1 = __builtin_amdgcn_perm(__builtin_amdgcn_perm(v[7], v[6], 0x0c0c0400u),
-                                                  __builtin_amdgcn_perm(v[5], v[4], 0x0c0c0400u), 0x05040100u);
-        __builtin_nontemporal_store(u32x2{w0, w1}, reinterpret_cast<u32x2*>(dst + m * slice_bytes));
+        const uint32_t w0 = __builtin_amdgcn_perm(rb[1], rb[0], 0x06040200u);
+        const uint32_t w1 = __builtin_amdgcn_perm(rb[3], rb[2], 0x06040200u);
+        u32x2* o = reinterpret_cast<u32x2*>(dst + m * slice_bytes);
+        if (ks == 1)
+            __builtin_nontemporal_store(u32x2{w0, w1}, o);
+        else
+            *o = u32x2{w0, w1};
     }
 }
 
@@ -694,44 +708,29 @@ __global__ __launch_bounds__(256) void oz_combine_kernel(const int32_t* __restri
 // Since |V| <= P/4 (the scaling bound), S/P lies within 1/4 of the integer j
 // and j = rint(fl(S) fl(1/P)) exactly (the estimate errs by ~2^-47).  Then
 // in FP64, every step exact: D_l = L_l - j P_l (|D_l| < 2^52), and two carries
-// bring D0, D1 into [0, 2^40), so V = D2 2^80 + D1 2^40 + D0 with D2 signed.
-// The three limbs split into 32-bit words that make V in 128-bit two's
-// complement, whose magnitude is rounded to double once: the top 64 bits
-// with a sticky bit for everything below, converted with one rounding.
+// bring D0, D1 into [-2^39, 2^39], so V = D2 2^80 + D1 2^40 + D0.  With
+// s = fl(D2 2^80 + D1 2^40) and its exact error e, V = s + (e + D0): one
+// rounding if e = 0.  Otherwise |s| >= 2^93, and s + e and every point halfway
+// between two doubles there are multiples of 2^40 > |D0|, so that only D0's
+// sign matters: +-2^30 in its place makes e + D0 exact (|e| <= 2^71).  About 30
+// operations in all, none on 64-bit integers.
 __host__ __device__ inline double crt_value(double L0, double L1, double L2, const CrtTables& tb) {
     const double Sd = fma(L2, 0x1p80, fma(L1, 0x1p40, L0));
     const double jd = rint(Sd * tb.invPd);
     double D0 = fma(-jd, tb.Pl[0], L0);
     double D1 = fma(-jd, tb.Pl[1], L1);
     double D2 = fma(-jd, tb.Pl[2], L2);
-    double c = floor(D0 * 0x1p-40);
+    double c = rint(D0 * 0x1p-40);
     D0 = fma(-c, 0x1p40, D0);
     D1 = D1 + c;
-    c = floor(D1 * 0x1p-40);
+    c = rint(D1 * 0x1p-40);
     D1 = fma(-c, 0x1p40, D1);
     D2 = D2 + c;
-    // 32-bit halves: D0, D1 in [0, 2^40) (high halves below 2^8), D2 signed below 2^44
-    const double h0 = floor(D0 * 0x1p-32), h1 = floor(D1 * 0x1p-32), h2 = floor(D2 * 0x1p-32);
-    const uint32_t lo0 = (uint32_t)fma(-h0, 0x1p32, D0), lo1 = (uint32_t)fma(-h1, 0x1p32, D1);
-    const uint32_t lo2 = (uint32_t)fma(-h2, 0x1p32, D2);
-    const uint32_t hi0 = (uint32_t)h0, hi1 = (uint32_t)h1, hi2 = (uint32_t)(int32_t)h2;
-    const uint32_t w0 = lo0;
-    const uint32_t w1 = hi0 | (lo1 << 8);
-    const uint32_t w2 = (lo1 >> 24) | (hi1 << 8) | (lo2 << 16);
-    const uint32_t w3 = (lo2 >> 16) | (hi2 << 16);
-    uint64_t hi = ((uint64_t)w3 << 32) | w2;
-    uint64_t lo = ((uint64_t)w1 << 32) | w0;
-    const bool neg = (int64_t)hi < 0;
-    // magnitude
-    const uint64_t nlo = ~lo + 1;
-    const uint64_t nhi = ~hi + (nlo == 0 ? 1u : 0u);
-    lo = neg ? nlo : lo;
-    hi = neg ? nhi : hi;
-    const int z = hi ? __builtin_clzll(hi) : 64;
-    const uint64_t top = z == 64 ? lo : (z ? (hi << z) | (lo >> (64 - z)) : hi);
-    const uint64_t rest = z == 64 ? 0 : (z ? (lo << z) : lo);
-    const double v = ldexp((double)(top | (rest != 0 ? 1ull : 0ull)), z == 64 ? 0 : 64 - z);
-    return neg ? -v : v;
+    const double mid = D1 * 0x1p40;
+    const double s = fma(D2, 0x1p80, mid);
+    const double e = mid - fma(-D2, 0x1p80, s);
+    const double low = e != 0.0 ? fmin(fmax(D0, -1.0), 1.0) * 0x1p30 : D0;
+    return s + (e + low);
 }
 
 // Four consecutive rows per thread (one 32-bit load of CRT digits per modulus).
@@ -805,8 +804,6 @@ __global__ __launch_bounds__(256) void crt_reconstruct_kernel(const uint8_t* __r
     }
 }
 
-typedef double pdv2 __attribute__((ext_vector_type(2)));
-typedef pdv2 udv2 __attribute__((aligned(8)));
 
 // Rows contiguous in k whose every row starts 16-byte aligned: the scans read
 // them in 16-byte pairs, 16 lanes per row (host and device take the same test).
@@ -1058,34 +1055,43 @@ __global__ __launch_bounds__(256) void crt_scan_rows_kernel(const double* __rest
 // 2^(2(sigma + e)) S <= 2^(2Q + 32) (sigma = Q + 16 - e - ceil(log4 S)),
 // capped at 53 - e; an all-zero line keeps sigma = 0.  Stored as
 // e' = Q - sigma, the form the residue and reconstruction kernels take.
-// A workgroup takes 64 lines; its four waves split the chunks (lanes on
-// consecutive lines, so every load is coalesced) and combine through LDS.
+// A workgroup takes 16 lines (a 128-byte line of words); 16 lanes a line split
+// the chunks, eight loads in flight, and combine through LDS.
+constexpr int CS_L = 16, CS_W = 256 / CS_L;
+
 __global__ __launch_bounds__(256) void crt_shift_kernel(const uint64_t* __restrict__ part, int64_t rows, int64_t rows_p,
                                                         int nchunk, int Q, int32_t* __restrict__ e) {
-    __shared__ uint64_t red[4][64];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int64_t r = (int64_t)blockIdx.x * 64 + lane;
+    __shared__ uint64_t red[CS_W][CS_L];
+    const int lane = threadIdx.x % CS_L, w = threadIdx.x / CS_L;
+    const int64_t r = (int64_t)blockIdx.x * CS_L + lane;
     const bool valid = r < rows;
     uint64_t top = 0;
-    if (valid)
-        for (int c = w; c < nchunk; c += 4) top = max(top, part[(int64_t)c * rows + r] >> 48);
+    if (valid) {
+#pragma unroll 8
+        for (int c = w; c < nchunk; c += CS_W) top = max(top, part[(int64_t)c * rows + r] >> 48);
+    }
     red[w][lane] = top;
     __syncthreads();
-    top = max(max(red[0][lane], red[1][lane]), max(red[2][lane], red[3][lane]));
+#pragma unroll
+    for (int i = 0; i < CS_W; ++i) top = max(top, red[i][lane]);
     __syncthreads();
     uint64_t S = 0;
-    if (valid && top != 0)
-        for (int c = w; c < nchunk; c += 4) {
+    if (valid && top != 0) {
+#pragma unroll 8
+        for (int c = w; c < nchunk; c += CS_W) {
             const uint64_t wd = part[(int64_t)c * rows + r];
-            if (wd == 0) continue;
             const uint64_t sc = wd & ((1ull << 48) - 1);
             const int d2 = 2 * (int)(top - (wd >> 48));
-            S += d2 >= 62 ? 1 : (sc + (1ull << d2) - 1) >> d2;
+            const uint64_t v = d2 >= 62 ? 1 : (sc + (1ull << d2) - 1) >> d2;
+            S += wd == 0 ? 0 : v;
         }
+    }
     red[w][lane] = S;
     __syncthreads();
     if (w != 0 || r >= rows_p) return;
-    S = (red[0][lane] + red[1][lane]) + (red[2][lane] + red[3][lane]);
+    S = 0;
+#pragma unroll
+    for (int i = 0; i < CS_W; ++i) S += red[i][lane];
     int sig = 0;
     if (valid && top != 0) {
         const int bl = S > 1 ? 64 - __builtin_clzll(S - 1) : 0;  // bit length of S - 1
@@ -1444,8 +1450,9 @@ int crt_prepare(const double* x, int64_t rows, int64_t k, int64_t rs, int64_t ks
         hipLaunchKernelGGL(crt_scan_rows_kernel, dim3((unsigned)blocks), dim3(NT), 0, st, x, rows, k, rs,
                            (uint32_t)nchunk, bp);
     }
-    hipLaunchKernelGGL(crt_shift_kernel, dim3((unsigned)((rp + 63) / 64)), dim3(NT), 0, st, bp, rows, rp, nchunk, q, e);
-    const uint32_t nkt = (uint32_t)(kp / RT_K), nrt = (uint32_t)(rp / RT_R);
+    hipLaunchKernelGGL(crt_shift_kernel, dim3((unsigned)(rp / CS_L)), dim3(NT), 0, st, bp, rows, rp, nchunk, q, e);
+    const uint32_t nkt = (uint32_t)(ks == 1 ? (kp + RC_K - 1) / RC_K : kp / RT_K);
+    const uint32_t nrt = (uint32_t)(ks == 1 ? rp / RC_R : rp / RT_R);
     if ((int64_t)nkt * nrt > INT32_MAX) return fail(DG_ERR_UNSUPPORTED, "dg_ozaki_dgemm: too many residue tiles");
     decltype(&crt_residue_kernel<16>) rsk = crt_residue_kernel<16>;
     switch (nmod) {
@@ -1458,10 +1465,7 @@ int crt_prepare(const double* x, int64_t rows, int64_t k, int64_t rs, int64_t ks
     }
     ResidueConsts rcs{};
     for (int t = 0; t < kMaxModuli; ++t) {
-        const int pm = crt_modulus(t);
-        rcs.c24[t] = (double)((1 << 24) % pm);
-        rcs.inv_p[t] = 1.0 / (double)pm;
-        rcs.pd[t] = (double)pm;
+        rcs.inv_p[t] = 1.0 / (double)crt_modulus(t);
     }
     hipLaunchKernelGGL(rsk, dim3(nkt * nrt), dim3(256), 0, st, x, rows, k, rs, ks, e, q, slices, kp, rp * kp, rcs, nkt,
                        nrt);
