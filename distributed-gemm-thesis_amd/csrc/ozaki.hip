@@ -108,6 +108,7 @@ __device__ __forceinline__ const int8_t* wave_uniform(const int8_t* p) {
 // distinct operand slices per k-step, as for 8 x 4) while the A panels all
 // XCDs revisit stay at half the size, which keeps them in the last-level
 // cache (measured on the 16384^3 CRT product: 4.8% faster than 8 x 4).
+template <int TILE>
 __device__ __forceinline__ void tile_origin(int bid, int tiles, int tiles_m, int tiles_n, int64_t& m0, int64_t& n0) {
     const int tile = xcd_remap(bid, tiles);
     const int per_group = GROUP_M * tiles_n;
@@ -115,8 +116,8 @@ __device__ __forceinline__ void tile_origin(int bid, int tiles, int tiles_m, int
     const int first_m = group * GROUP_M;
     const int gsize = min(tiles_m - first_m, GROUP_M);
     const int in_group = tile - group * per_group;
-    m0 = (int64_t)(first_m + in_group % gsize) * BM;
-    n0 = (int64_t)(in_group / gsize) * BN;
+    m0 = (int64_t)(first_m + in_group % gsize) * TILE;
+    n0 = (int64_t)(in_group / gsize) * TILE;
 }
 
 // ------------------------------------------------------------ Ozaki scheme II
@@ -347,24 +348,24 @@ __device__ __forceinline__ void mfma64(fv4& acc, const iv4& a, const iv4& b) {
 
 // One MFMA half-step on fa / cb, reading the fragments of the following
 // half-step meanwhile: fa[i] right after its last use, B into nb.
-template <class ACC>
-__device__ __forceinline__ void crt_half(ACC (&acc)[FM][FN], iv4 (&fa)[FM], const iv4 (&cb)[FN], iv4 (&nb)[FN],
+template <class ACC, int M, int N>
+__device__ __forceinline__ void crt_half(ACC (&acc)[M][N], iv4 (&fa)[M], const iv4 (&cb)[N], iv4 (&nb)[N],
                                          const int8_t* nas, const int8_t* nbs) {
 #pragma unroll
-    for (int i = 0; i < FM; ++i) {
+    for (int i = 0; i < M; ++i) {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) mfma64(acc[i][j], fa[i], cb[j]);
+        for (int j = 0; j < N; ++j) mfma64(acc[i][j], fa[i], cb[j]);
         if (i == 0) {
 #pragma unroll
-            for (int j = 0; j < FN; ++j) nb[j] = *reinterpret_cast<const iv4*>(nbs + 2048 * j);
+            for (int j = 0; j < N; ++j) nb[j] = *reinterpret_cast<const iv4*>(nbs + 2048 * j);
         }
         fa[i] = *reinterpret_cast<const iv4*>(nas + 2048 * i);
     }
-    __builtin_amdgcn_sched_group_barrier(0x008, FN, 0);
-    __builtin_amdgcn_sched_group_barrier(0x100, FN + 1, 0);
+    __builtin_amdgcn_sched_group_barrier(0x008, N, 0);
+    __builtin_amdgcn_sched_group_barrier(0x100, N + 1, 0);
 #pragma unroll
-    for (int g = 1; g < FM; ++g) {
-        __builtin_amdgcn_sched_group_barrier(0x008, FN, 0);
+    for (int g = 1; g < M; ++g) {
+        __builtin_amdgcn_sched_group_barrier(0x008, N, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
 }
@@ -410,6 +411,132 @@ __device__ __forceinline__ void crt_half_ld(ACC (&acc)[FM][FN], iv4 (&fa)[FM], c
     }
 }
 
+// The digits of a wave's sums: acc[i][j][v] = V_t(m0 + 16i + v, n0 + 16j),
+// four consecutive rows of one column, stored as one 32-bit word of digits.
+// x = acc * cinv is exact (|x| < 2^39) and floor(fl(x fl(1/p) + 2^-10)) is
+// floor(x/p) exactly (the estimate errs by < 2^-20 and the fractional
+// part of x/p lies in [0, 1 - 1/p]), so x - p floor(x/p) is the digit.
+template <int M, int N>
+__device__ __forceinline__ void store_digits(const iv4 (&acc)[M][N], const CrtArgs& g, int tmod, int64_t m0,
+                                             int64_t n0) {
+    const int p = c_moduli[tmod];
+    const double pd = p, inv_p = 1.0 / p, cinv = g.cinv[tmod];
+    uint8_t* out = g.res + (int64_t)tmod * g.res_plane;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int i = 0; i < M; ++i) {
+            uint32_t w = 0;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const double x = (double)acc[i][j][v] * cinv;
+                const double qd = floor(fma(x, inv_p, 0x1p-10));
+                w |= (uint32_t)(int)fma(-qd, pd, x) << (8 * v);
+            }
+            *reinterpret_cast<uint32_t*>(out + (n0 + 16 * j) * g.Mp + m0 + 16 * i) = w;
+        }
+}
+
+// ------------------------------------------------------------ 128 x 128 tiles
+// The same pipeline for products with too few 256 x 256 tiles to fill the
+// chip: four waves of 64 x 64, a ring of five whole steps (160 KB, one
+// workgroup per CU).  A step's MFMAs take a quarter of the time here, so the
+// loads run five steps ahead instead of two and a half.
+constexpr int ST = 128, SNW = 4, SCNT = SNW * 64, SFM = 4, SFN = 4, SDEPTH = 5;
+constexpr int SSTEP = 2 * ST * CK2;  // A's and B's rows of one step
+static_assert(SDEPTH * SSTEP == (int)kCrtLds, "the ring fills the LDS");
+
+// Sums of k-steps 0..last into acc; a_at(s), b_at(s): this wave's 32 rows of
+// step s, `ld` bytes apart (steps past the end clamped to the last one).
+template <class ACC, class At, class Bt>
+__device__ __forceinline__ void small_product(ACC (&acc)[SFM][SFN], int8_t* lds, const At& a_at, const Bt& b_at,
+                                              uint32_t last, int64_t ld, int wave, int lane, int wm, int wn) {
+    const uint32_t loff = (uint32_t)((lane >> 3) * ld + 16 * ((lane & 7) ^ (lane >> 3)));
+    const int lr = lane & 15, lg = lane >> 4;
+    const int a0 = (wm + lr) * CK2 + 16 * (lg ^ (lr & 7)), a1 = (wm + lr) * CK2 + 16 * ((4 + lg) ^ (lr & 7));
+    const int ab = ST * CK2 + (wn - wm) * CK2;  // from A's fragment rows to B's
+    const auto load = [&](const int8_t* g, int8_t* d, int i) {
+        __builtin_amdgcn_global_load_lds((gvoid_t*)(wave_uniform(g + (int64_t)(8 * i) * ld) + loff),
+                                         (lds_void_t*)(d + wave * 4096 + 1024 * i), 16, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < SDEPTH; ++s) {
+        const int8_t *ga = a_at(s), *gb = b_at(s);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) load(ga, lds + s * SSTEP, i);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) load(gb, lds + s * SSTEP + ST * CK2, i);
+    }
+    wait_vmcnt<8 * (SDEPTH - 1)>();  // step 0 landed
+    __builtin_amdgcn_s_barrier();
+    iv4 fa[SFM], cb[SFN], nb[SFN];
+#pragma unroll
+    for (int j = 0; j < SFN; ++j) cb[j] = *reinterpret_cast<const iv4*>(lds + a0 + ab + 2048 * j);
+#pragma unroll
+    for (int i = 0; i < SFM; ++i) fa[i] = *reinterpret_cast<const iv4*>(lds + a0 + 2048 * i);
+    int8_t* cur = lds;  // ring position of step s
+    for (uint32_t s = 0; s < last; ++s) {
+        int8_t* next = cur == lds + (SDEPTH - 1) * SSTEP ? lds : cur + SSTEP;
+        crt_half(acc, fa, cb, nb, cur + a1, cur + a1 + ab);
+        // this wave's reads of step s are done; its part of step s + 1 landed
+        // with three steps pending
+        __builtin_amdgcn_s_waitcnt((0xF) | (0x3 << 14) | (0x7 << 4));  // lgkmcnt(0)
+        wait_vmcnt<8 * (SDEPTH - 2)>();
+        __builtin_amdgcn_s_barrier();
+        const int8_t *ga = a_at(s + SDEPTH), *gb = b_at(s + SDEPTH);
+#pragma unroll
+        for (int i = 0; i < SFM; ++i) {
+#pragma unroll
+            for (int j = 0; j < SFN; ++j) mfma64(acc[i][j], fa[i], nb[j]);
+            if (i == 0) {
+#pragma unroll
+                for (int j = 0; j < SFN; ++j) cb[j] = *reinterpret_cast<const iv4*>(next + a0 + ab + 2048 * j);
+            }
+            fa[i] = *reinterpret_cast<const iv4*>(next + a0 + 2048 * i);
+            load(ga, cur, i);
+            load(gb, cur + ST * CK2, i);
+        }
+        __builtin_amdgcn_sched_group_barrier(0x008, SFN, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, SFN + 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+#pragma unroll
+        for (int i = 1; i < SFM; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, SFN, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+        }
+        cur = next;
+    }
+    // last step: no loads; the reads of a following one are in bounds and unused
+    int8_t* next = cur == lds + (SDEPTH - 1) * SSTEP ? lds : cur + SSTEP;
+    crt_half(acc, fa, cb, nb, cur + a1, cur + a1 + ab);
+    crt_half(acc, fa, nb, cb, next + a0, next + a0 + ab);
+    wait_vmcnt<0>();  // the loads past the end land before the workgroup's LDS is released
+}
+
+__global__ __launch_bounds__(SCNT, 2) void crt_gemm_small_kernel(CrtArgs g) {
+    extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+    const int tiles = g.tiles_m * g.tiles_n;
+    const int tmod = blockIdx.x / tiles;
+    int64_t m0, n0;
+    tile_origin<ST>(blockIdx.x - tmod * tiles, tiles, g.tiles_m, g.tiles_n, m0, n0);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const int8_t* ga = g.a + tmod * g.a_slice + (m0 + 32 * wave) * g.Kp;
+    const int8_t* gb = g.b + tmod * g.b_slice + (n0 + 32 * wave) * g.Kp;
+    const uint32_t last = (uint32_t)(g.Kp / CK2) - 1;
+    iv4 acc[SFM][SFN];
+#pragma unroll
+    for (int i = 0; i < SFM; ++i)
+#pragma unroll
+        for (int j = 0; j < SFN; ++j) acc[i][j] = iv4{0, 0, 0, 0};
+    small_product(
+        acc, lds, [&](uint32_t s) { return ga + (int64_t)(s < last ? s : last) * CK2; },
+        [&](uint32_t s) { return gb + (int64_t)(s < last ? s : last) * CK2; }, last, g.Kp, wave, lane, wm, wn);
+    store_digits(acc, g, tmod, m0 + wm + 4 * (lane >> 4), n0 + wn + (lane & 15));
+}
+
 // One INT8 GEMM per modulus in one launch: workgroup b computes tile
 // b % tiles of modulus b / tiles and stores the CRT digit
 // x_t = ((A'_t B'_t) mod p_t) * ((P / p_t)^-1 mod p_t) mod p_t as a byte.
@@ -418,7 +545,7 @@ __global__ __launch_bounds__(CNT, OCC) void crt_gemm_kernel(CrtArgs g) {
     const int tiles = g.tiles_m * g.tiles_n;
     const int tmod = blockIdx.x / tiles;
     int64_t m0, n0;
-    tile_origin(blockIdx.x - tmod * tiles, tiles, g.tiles_m, g.tiles_n, m0, n0);
+    tile_origin<BM>(blockIdx.x - tmod * tiles, tiles, g.tiles_m, g.tiles_n, m0, n0);
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -494,30 +621,7 @@ __global__ __launch_bounds__(CNT, OCC) void crt_gemm_kernel(CrtArgs g) {
         crt_half(acc, fa, nb, cb, lds + asl1 * CSLOT + wm * CK2 + roff0, lds + bsl1 * CSLOT + wn * CK2 + roff0);
     }
     wait_vmcnt<0>();  // the reloads past the end land before the workgroup's LDS is released
-    // acc[i][j][v] = V_t(m0 + wm + 16i + 4lg + v, n0 + wn + 16j + lr): four
-    // consecutive rows of one column, stored as one 32-bit word of digits.
-    // x = acc * cinv is exact (|x| < 2^39) and floor(fl(x fl(1/p) + 2^-10)) is
-    // floor(x/p) exactly (the estimate errs by < 2^-20 and the fractional
-    // part of x/p lies in [0, 1 - 1/p]), so x - p floor(x/p) is the digit.
-    const int p = c_moduli[tmod];
-    const double pd = p, inv_p = 1.0 / p, cinv = g.cinv[tmod];
-    uint8_t* out = g.res + (int64_t)tmod * g.res_plane;
-#pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        const int64_t n = n0 + wn + 16 * j + lr;
-#pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const int64_t m = m0 + wm + 16 * i + 4 * lg;
-            uint32_t w = 0;
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const double x = (double)acc[i][j][v] * cinv;
-                const double qd = floor(fma(x, inv_p, 0x1p-10));
-                w |= (uint32_t)(int)fma(-qd, pd, x) << (8 * v);
-            }
-            *reinterpret_cast<uint32_t*>(out + n * g.Mp + m) = w;
-        }
-    }
+    store_digits(acc, g, tmod, m0 + wm + 4 * lg, n0 + wn + lr);
 }
 
 // ---------------------------------------------- scheme I on the scheme II pipeline
@@ -564,6 +668,17 @@ __device__ __forceinline__ const int8_t* group_step(const int8_t* first, int64_t
     return first + (int64_t)p * stride + (int64_t)(sc - p * nks.d) * CK2;
 }
 
+// acc[i][j][v] = sum at (m0 + 16i + v, n0 + 16j): one 16-byte store each.
+template <class ACC, int M, int N>
+__device__ __forceinline__ void store_plane(const ACC (&acc)[M][N], int32_t* out, int64_t Mp, int64_t m0, int64_t n0) {
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+#pragma unroll
+        for (int i = 0; i < M; ++i)
+            __builtin_nontemporal_store(__builtin_bit_cast(iv4, acc[i][j]),
+                                        reinterpret_cast<iv4*>(out + (n0 + 16 * j) * Mp + m0 + 16 * i));
+}
+
 template <bool BF16>
 __global__ __launch_bounds__(CNT, OCC) void oz_plane_kernel(OzPlaneArgs g) {
     typedef typename std::conditional<BF16, fv4, iv4>::type acc_t;
@@ -571,7 +686,7 @@ __global__ __launch_bounds__(CNT, OCC) void oz_plane_kernel(OzPlaneArgs g) {
     const int tiles = g.tiles_m * g.tiles_n;
     const int gi = blockIdx.x / tiles;
     int64_t m0, n0;
-    tile_origin(blockIdx.x - gi * tiles, tiles, g.tiles_m, g.tiles_n, m0, n0);
+    tile_origin<BM>(blockIdx.x - gi * tiles, tiles, g.tiles_m, g.tiles_n, m0, n0);
     const OzGroup gr = g.jobs[gi];
 
     const int lane = threadIdx.x & 63;
@@ -635,17 +750,34 @@ __global__ __launch_bounds__(CNT, OCC) void oz_plane_kernel(OzPlaneArgs g) {
         crt_half(acc, fa, nb, fb, lds + asl1 * CSLOT + wm * CK2 + roff0, lds + bsl1 * CSLOT + wn * CK2 + roff0);
     }
     wait_vmcnt<0>();
-    // acc[i][j][v] = sum at (m0 + wm + 16i + 4lg + v, n0 + wn + 16j + lr): one 16-byte store
-    int32_t* out = g.planes + (int64_t)gr.plane * g.plane;
+    store_plane(acc, g.planes + (int64_t)gr.plane * g.plane, g.Mp, m0 + wm + 4 * lg, n0 + wn + lr);
+}
+
+// oz_plane_kernel on 128 x 128 tiles.
+template <bool BF16>
+__global__ __launch_bounds__(SCNT, 2) void oz_plane_small_kernel(OzPlaneArgs g) {
+    typedef typename std::conditional<BF16, fv4, iv4>::type acc_t;
+    extern __shared__ __attribute__((aligned(1024))) int8_t lds[];
+    const int tiles = g.tiles_m * g.tiles_n;
+    const int gi = blockIdx.x / tiles;
+    int64_t m0, n0;
+    tile_origin<ST>(blockIdx.x - gi * tiles, tiles, g.tiles_m, g.tiles_n, m0, n0);
+    const OzGroup gr = g.jobs[gi];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+    const uint32_t last = (uint32_t)gr.count * gr.nks.d - 1;
+    const int8_t* ga = g.a + gr.t0 * g.a_slice + (m0 + 32 * wave) * g.rb + gr.kb;
+    const int8_t* gb = g.b + gr.u0 * g.b_slice + (n0 + 32 * wave) * g.rb + gr.kb;
+    acc_t acc[SFM][SFN];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) {
-        const int64_t n = n0 + wn + 16 * j + lr;
+    for (int i = 0; i < SFM; ++i)
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            const int64_t m = m0 + wm + 16 * i + 4 * lg;
-            __builtin_nontemporal_store(__builtin_bit_cast(iv4, acc[i][j]), reinterpret_cast<iv4*>(out + n * g.Mp + m));
-        }
-    }
+        for (int j = 0; j < SFN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    small_product(
+        acc, lds, [&](uint32_t s) { return group_step(ga, g.a_slice, s, last, gr.nks); },
+        [&](uint32_t s) { return group_step(gb, -g.b_slice, s, last, gr.nks); }, last, g.rb, wave, lane, wm, wn);
+    store_plane(acc, g.planes + (int64_t)gr.plane * g.plane, g.Mp, m0 + wm + 4 * (lane >> 4), n0 + wn + (lane & 15));
 }
 
 // The FP64 recombination of scheme I from the planes of groups [gb, ge) of
@@ -805,12 +937,6 @@ __global__ __launch_bounds__(256) void crt_reconstruct_kernel(const uint8_t* __r
 }
 
 
-// Rows contiguous in k whose every row starts 16-byte aligned: the scans read
-// them in 16-byte pairs, 16 lanes per row (host and device take the same test).
-__host__ __device__ inline bool pair_rows(const double* x, int64_t rs) {
-    return !(rs & 1) && !(reinterpret_cast<uintptr_t>(x) & 15);
-}
-
 // One operand of scheme I: op(X)(row, k) at x[row*rs + k*ks].
 struct OzSide {
     const double* x;
@@ -920,9 +1046,9 @@ __device__ __forceinline__ double crt_bound_term(double x, int e) {
 // e_c) (at most CRT_KC * 2^32 = 2^38), stored as one word
 // ((e_c + 2048) << 48) | S_c, or 0 for an all-zero chunk.  crt_shift_kernel
 // rescales the chunk bounds to the line's max exponent.  Rows strided in
-// memory (ks != 1): a 64-line x 64-k tile through LDS, loaded along the
-// lines.  Lines contiguous in k: 16 lanes per line with 16-byte pair loads
-// when every line starts 16-byte aligned, else a wave per line.  Every term
+// memory (ks != 1): 4 threads per line; lines contiguous in k: 16 lanes per
+// line.  Either is bound by the one read of op(X): 8192^2 strided 81 us (6.6
+// TB/s; a thread per line with 64 loads: 110 us), contiguous 88 us.  Every term
 // and chunk sum is an integer below 2^39, so the sums are exact in any order.
 constexpr int CRT_KC = 64;
 
@@ -939,115 +1065,96 @@ __device__ __forceinline__ int crt_chunk_exp(double amax) {
     return ec;
 }
 
-// Lines contiguous in k: 16 lanes per line with 16-byte pair loads when every
-// line starts 16-byte aligned, else a wave per line.
-__device__ __forceinline__ void scan_contiguous(const double* __restrict__ x, int64_t rows, int64_t K, int64_t rs,
-                                                int64_t tile, int64_t chunk, uint64_t* __restrict__ part) {
-    const int64_t k0 = chunk * CRT_KC;
-    if (pair_rows(x, rs)) {
-        // 16 lanes per line, two 16-byte pairs each (k0 + 2 l16 and 32 further)
-        const int l16 = threadIdx.x & 15;
-        const int64_t r = tile * (int64_t)(blockDim.x >> 4) + (threadIdx.x >> 4);
-        if (r >= rows) return;  // whole 16-lane groups leave together
-        const double* xr = x + r * rs;
-        double v[4];
-        if (k0 + CRT_KC <= K) {  // the whole chunk inside the line: both loads in flight together
-            const pdv2 w0 = __builtin_nontemporal_load(reinterpret_cast<const pdv2*>(xr + k0 + 2 * l16));
-            const pdv2 w1 = __builtin_nontemporal_load(reinterpret_cast<const pdv2*>(xr + k0 + 32 + 2 * l16));
-            v[0] = w0.x; v[1] = w0.y; v[2] = w1.x; v[3] = w1.y;
-        } else {
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int64_t k = k0 + 32 * h + 2 * l16;
-                if (k + 1 < K) {
-                    const pdv2 w = *reinterpret_cast<const pdv2*>(xr + k);
-                    v[2 * h] = w.x;
-                    v[2 * h + 1] = w.y;
-                } else {
-                    v[2 * h] = k < K ? xr[k] : 0.0;
-                    v[2 * h + 1] = 0.0;
-                }
-            }
-        }
-        double mx = fmax(fmax(fabs(v[0]), fabs(v[1])), fmax(fabs(v[2]), fabs(v[3])));
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
-        const int ec = crt_chunk_exp(mx);
-        double sum = (crt_bound_term(v[0], ec) + crt_bound_term(v[1], ec)) +
-                     (crt_bound_term(v[2], ec) + crt_bound_term(v[3], ec));
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-        if (l16 == 0) part[chunk * rows + r] = crt_chunk_word(mx, (uint64_t)sum);
-    } else {
-        const int lane = threadIdx.x & 63;
-        const int64_t r = tile * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6);
-        if (r >= rows) return;
-        const double* xr = x + r * rs;
-        const double v = k0 + lane < K ? xr[k0 + lane] : 0.0;
-        double mx = fabs(v);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
-        const int ec = crt_chunk_exp(mx);
-        double sum = crt_bound_term(v, ec);
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
-        if (lane == 0) part[chunk * rows + r] = crt_chunk_word(mx, (uint64_t)sum);
-    }
-}
-
-// Lines strided in memory (ks != 1): a thread per line, consecutive lanes on
-// consecutive lines (a wave's load reads 512 contiguous bytes when rs == 1),
-// every load of the chunk in flight at once.  Each entry is kept as its
+// Lines strided in memory (ks != 1): a workgroup takes CSL_L lines of one
+// chunk, CSL_P threads a line with CRT_KC / CSL_P entries each, consecutive
+// lanes on consecutive lines (a load of CSL_L lanes is contiguous when
+// rs == 1), every load in flight at once.  Each entry is kept as its
 // exponent ex and mantissa bound M = ceil(256 m) (|x| = m 2^ex, M in
 // [128, 256], 0 for a zero entry) packed as ((ex + 2048) << 9) | M, so the
 // largest packed word of the chunk carries the exponent e of its largest
 // entry, and the terms of crt_bound_term follow from (M, ex).  blockIdx.x =
 // line tile, blockIdx.y = chunk (the grid walks down the columns).
+constexpr int CSL_P = 4, CSL_L = 256 / CSL_P, CSL_K = CRT_KC / CSL_P;
+
 __global__ __launch_bounds__(256) void crt_scan_lines_kernel(const double* __restrict__ x, int64_t rows, int64_t K,
                                                              int64_t rs, int64_t ks, uint64_t* __restrict__ part) {
-    const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (r >= rows) return;
-    const int64_t k0 = (int64_t)blockIdx.y * CRT_KC;
-    const int64_t kn = K - k0 < CRT_KC ? K - k0 : CRT_KC;
-    const double* xr = x + r * rs + k0 * ks;
-    // every load unconditional (a clamped, in-bounds address past the end
-    // of the line), so that all of them issue before the first wait
-    double raw[CRT_KC];
+    __shared__ uint32_t tops[CSL_P][CSL_L];
+    __shared__ double sums[CSL_P][CSL_L];
+    const int line = threadIdx.x % CSL_L, w = threadIdx.x / CSL_L;
+    const int64_t r = (int64_t)blockIdx.x * CSL_L + line;
+    const int64_t k0 = (int64_t)blockIdx.y * CRT_KC + w * CSL_K;
+    // every load unconditional (the last entry or line again past the end),
+    // so that all of them issue before the first wait
+    const double* xr = x + min(r, rows - 1) * rs;
+    double raw[CSL_K];
 #pragma unroll
-    for (int i = 0; i < CRT_KC; ++i) raw[i] = __builtin_nontemporal_load(xr + (i < kn ? i : kn - 1) * ks);
-    uint32_t wd[CRT_KC];
+    for (int i = 0; i < CSL_K; ++i) raw[i] = __builtin_nontemporal_load(xr + min(k0 + i, K - 1) * ks);
+    uint32_t wd[CSL_K];
     uint32_t top = 0;
 #pragma unroll
-    for (int i = 0; i < CRT_KC; ++i) {
-        const double v = i < kn ? raw[i] : 0.0;
+    for (int i = 0; i < CSL_K; ++i) {
+        const double v = k0 + i < K ? raw[i] : 0.0;
         int ex;
         const double m = frexp(fabs(v), &ex);
         const uint32_t M = (uint32_t)ceil(m * 256.0);
         wd[i] = M ? ((uint32_t)(ex + 2048) << 9) | M : 0u;
         top = top > wd[i] ? top : wd[i];
     }
-    uint64_t word = 0;
-    if (top) {
-        const int ec = (int)(top >> 9) - 2048;
-        double sum = 0.0;
+    tops[w][line] = top;
+    __syncthreads();
 #pragma unroll
-        for (int i = 0; i < CRT_KC; ++i) {
+    for (int p = 0; p < CSL_P; ++p) top = max(top, tops[p][line]);
+    const int ec = (int)(top >> 9) - 2048;
+    double sum = 0.0;
+    if (top) {
+#pragma unroll
+        for (int i = 0; i < CSL_K; ++i) {
             const double M = (double)(wd[i] & 511u);
             const int ex = (int)(wd[i] >> 9) - 2048;
             sum += wd[i] ? ceil(ldexp(M * M, -min(2 * (ec - ex) - 16, 64))) : 0.0;
         }
-        word = ((uint64_t)(ec + 2048) << 48) | (uint64_t)sum;
     }
-    part[(int64_t)blockIdx.y * rows + r] = word;
+    sums[w][line] = sum;
+    __syncthreads();
+    if (w != 0 || r >= rows) return;
+#pragma unroll
+    for (int p = 1; p < CSL_P; ++p) sum += sums[p][line];
+    part[(int64_t)blockIdx.y * rows + r] = top ? ((uint64_t)(ec + 2048) << 48) | (uint64_t)sum : 0;
 }
 
-// Lines contiguous in k: blockIdx.x = line tile * nchunk + chunk, so the grid
-// walks along the lines (consecutive workgroups read consecutive chunks of
-// the same lines).
+// Lines contiguous in k: 16 lanes per line, two pairs of any alignment each.
+// blockIdx.x = line tile * nchunk + chunk, so the grid walks along the lines
+// (consecutive workgroups read consecutive chunks of the same lines).
 __global__ __launch_bounds__(256) void crt_scan_rows_kernel(const double* __restrict__ x, int64_t rows, int64_t K,
                                                             int64_t rs, uint32_t nchunk, uint64_t* __restrict__ part) {
     const uint32_t tile = blockIdx.x / nchunk;
-    scan_contiguous(x, rows, K, rs, tile, blockIdx.x - tile * nchunk, part);
+    const uint32_t chunk = blockIdx.x - tile * nchunk;
+    const int64_t k0 = (int64_t)chunk * CRT_KC;
+    const int l16 = threadIdx.x & 15;
+    const int64_t r = (int64_t)tile * (NT / 16) + (threadIdx.x >> 4);
+    if (r >= rows) return;  // whole 16-lane groups leave together
+    const double* xr = x + r * rs;
+    double v[4];
+    if (k0 + CRT_KC <= K) {  // the whole chunk inside the line: both loads in flight together
+        const pdv2 w0 = __builtin_nontemporal_load(reinterpret_cast<const udv2*>(xr + k0 + 2 * l16));
+        const pdv2 w1 = __builtin_nontemporal_load(reinterpret_cast<const udv2*>(xr + k0 + 32 + 2 * l16));
+        v[0] = w0.x; v[1] = w0.y; v[2] = w1.x; v[3] = w1.y;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t k = k0 + 32 * (i >> 1) + 2 * l16 + (i & 1);
+            v[i] = k < K ? xr[k] : 0.0;
+        }
+    }
+    double mx = fmax(fmax(fabs(v[0]), fabs(v[1])), fmax(fabs(v[2]), fabs(v[3])));
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off));
+    const int ec = crt_chunk_exp(mx);
+    double sum = (crt_bound_term(v[0], ec) + crt_bound_term(v[1], ec)) +
+                 (crt_bound_term(v[2], ec) + crt_bound_term(v[3], ec));
+#pragma unroll
+    for (int off = 8; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
+    if (l16 == 0) part[chunk * rows + r] = crt_chunk_word(mx, (uint64_t)sum);
 }
 
 // Line shifts: e = the largest chunk exponent, S = sum over the nonzero
@@ -1244,6 +1351,25 @@ struct Plan {
     size_t off_a, off_b, off_ea, off_eb, off_part, off_w, off_planes, total;
 };
 
+// Whether a launch of `wgs` 256 x 256 tiles, the longest of `longest` k-steps,
+// `total` k-steps in all, takes 128 x 128 tiles instead: the launch lasts
+// about as long as its longest tile or its work spread over the CUs (whole
+// rounds of equal tiles), and a k-step of a quarter tile takes kSmallStep of
+// a whole one's time (0.37 with every CU busy, 0.42 with few: the LDS bounds
+// it, whose reads per MFMA grow by a third).  8 INT8 slices, 512^3: 41 us a
+// call with 128 x 128 tiles, 67 with 256 x 256; 300 x 700 x 4000: 137 and
+// 294; 2048^3: 411 and 319.  14 moduli, 512^3: 39 and 43; 1024^3: 74 and 61.
+constexpr double kSmallStep = 0.4;
+
+bool small_tiles(int64_t wgs, int64_t longest, int64_t total) {
+    constexpr int kCus = 256;
+    const auto spread = [&](int64_t n) {
+        if (total == wgs * longest) return (double)((n + kCus - 1) / kCus * longest);
+        return std::max((double)longest, (double)total * (double)(n / wgs) / kCus);
+    };
+    return kSmallStep * spread(4 * wgs) < spread(wgs);
+}
+
 // Host side of the CRT form: q and the reconstruction tables for n moduli.
 int crt_setup(int64_t k, int nmod, CrtTables* tb, int* q_out) {
     unsigned __int128 P = 1;
@@ -1437,15 +1563,12 @@ int crt_prepare(const double* x, int64_t rows, int64_t k, int64_t rs, int64_t ks
     int32_t* e = reinterpret_cast<int32_t*>(static_cast<char*>(operand) + round_up((int64_t)nmod * rp * kp, 256));
     uint64_t* bp = static_cast<uint64_t*>(scan);
     // Line exponents and Cauchy-Schwarz shifts: one scan (chunk exponents
-    // and chunk bounds), then the per-line combination.  Strided lines: a
-    // thread per line; contiguous lines: 16 lanes per line when the lines
-    // pair up in 16-byte loads, else a wave per line.
+    // and chunk bounds), then the per-line combination.
     if (ks != 1) {
-        hipLaunchKernelGGL(crt_scan_lines_kernel, dim3((unsigned)((rows + 255) / 256), (unsigned)nchunk), dim3(NT), 0,
-                           st, x, rows, k, rs, ks, bp);
+        hipLaunchKernelGGL(crt_scan_lines_kernel, dim3((unsigned)((rows + CSL_L - 1) / CSL_L), (unsigned)nchunk), dim3(NT),
+                           0, st, x, rows, k, rs, ks, bp);
     } else {
-        const int64_t per = pair_rows(x, rs) ? NT / 16 : NT / 64;
-        const int64_t blocks = (rows + per - 1) / per * nchunk;
+        const int64_t blocks = (rows + NT / 16 - 1) / (NT / 16) * nchunk;
         if (blocks > INT32_MAX) return fail(DG_ERR_UNSUPPORTED, "dg_ozaki_dgemm: too many lines for one scan");
         hipLaunchKernelGGL(crt_scan_rows_kernel, dim3((unsigned)blocks), dim3(NT), 0, st, x, rows, k, rs,
                            (uint32_t)nchunk, bp);
@@ -1494,12 +1617,22 @@ int crt_multiply(int64_t m, int64_t n, int64_t k, int nmod, double alpha, const 
     for (int t = 0; t < kMaxModuli; ++t) cg.cinv[t] = tables.cinv[t];
     const int32_t* ea = reinterpret_cast<const int32_t*>(static_cast<const char*>(a_op) + round_up((int64_t)nmod * mp * kp, 256));
     const int32_t* eb = reinterpret_cast<const int32_t*>(static_cast<const char*>(b_op) + round_up((int64_t)nmod * np * kp, 256));
-    const int64_t grid = (int64_t)cg.tiles_m * cg.tiles_n * nmod;
+    int64_t grid = (int64_t)cg.tiles_m * cg.tiles_n * nmod;
+    const int64_t steps = kp / CK2;
+    const bool small = small_tiles(grid, steps, grid * steps);
+    if (small) {
+        cg.tiles_m *= BM / ST;
+        cg.tiles_n *= BN / ST;
+        grid *= (BM / ST) * (BN / ST);
+    }
     if (grid > INT32_MAX) return fail(DG_ERR_INVALID, "dg_ozaki_dgemm: too many tiles");
     const int64_t quads = ((m + 3) / 4) * n;
     if (quads > (int64_t)UINT32_MAX - 255)
         return fail(DG_ERR_UNSUPPORTED, "dg_ozaki_dgemm: too many output elements for one reconstruction");
-    hipLaunchKernelGGL(crt_gemm_kernel, dim3((unsigned)grid), dim3(CNT), kCrtLds, st, cg);
+    if (small)
+        hipLaunchKernelGGL(crt_gemm_small_kernel, dim3((unsigned)grid), dim3(SCNT), kCrtLds, st, cg);
+    else
+        hipLaunchKernelGGL(crt_gemm_kernel, dim3((unsigned)grid), dim3(CNT), kCrtLds, st, cg);
     DG_LAUNCH_CHECK();
     decltype(&crt_reconstruct_kernel<16>) rk = crt_reconstruct_kernel<16>;
     switch (nmod) {
@@ -1656,7 +1789,6 @@ int dg_ozaki_dgemm(char opA, char opB, int64_t m, int64_t n, int64_t k, double a
         return fail(DG_ERR_INVALID, "dg_ozaki_dgemm: too many tiles");
     OzPlaneArgs g{};
     g.a = sa; g.b = sb; g.planes = reinterpret_cast<int32_t*>(ws + p.off_planes);
-    g.tiles_m = (int32_t)(p.Mp / BM); g.tiles_n = (int32_t)(p.Np / BN);
     g.Mp = p.Mp; g.rb = p.Kp * p.esz; g.a_slice = p.a_slice; g.b_slice = p.b_slice; g.plane = p.Mp * p.Np;
     double* W = reinterpret_cast<double*>(ws + p.off_w);
     const uint32_t total = (uint32_t)((p.Mp / 4) * p.Np);
@@ -1664,14 +1796,23 @@ int dg_ozaki_dgemm(char opA, char opB, int64_t m, int64_t n, int64_t k, double a
     for (int g0 = 0; g0 < ng; g0 += batch) {
         const int cnt = std::min(batch, ng - g0);
         g.jobs = dgroups + ng + g0;
-        const dim3 grid((unsigned)(tiles * cnt));
+        int64_t longest = 0, sum = 0;
+        for (int i = g0; i < g0 + cnt; ++i) {
+            const int64_t steps = (int64_t)groups[i].count * groups[i].nks.d;
+            longest = std::max(longest, steps);
+            sum += steps;
+        }
+        const bool small = small_tiles(tiles * cnt, longest, tiles * sum);
+        const int split = small ? BM / ST : 1;
+        g.tiles_m = (int32_t)(p.Mp / BM) * split; g.tiles_n = (int32_t)(p.Np / BN) * split;
+        const dim3 grid((unsigned)(tiles * cnt * split * split)), wg(small ? SCNT : CNT);
         const dim3 cgrid((total + 255) / 256);
         if (bf16) {
-            hipLaunchKernelGGL(oz_plane_kernel<true>, grid, dim3(CNT), kCrtLds, st, g);
+            hipLaunchKernelGGL(small ? oz_plane_small_kernel<true> : oz_plane_kernel<true>, grid, wg, kCrtLds, st, g);
             hipLaunchKernelGGL(oz_combine_kernel<true>, cgrid, dim3(256), 0, st, g.planes, g.plane, dgroups, g0,
                                g0 + cnt, ng, bits, W, p.Mp, m, n, ea, eb, alpha, beta, C, ldc, dqm, total);
         } else {
-            hipLaunchKernelGGL(oz_plane_kernel<false>, grid, dim3(CNT), kCrtLds, st, g);
+            hipLaunchKernelGGL(small ? oz_plane_small_kernel<false> : oz_plane_kernel<false>, grid, wg, kCrtLds, st, g);
             hipLaunchKernelGGL(oz_combine_kernel<false>, cgrid, dim3(256), 0, st, g.planes, g.plane, dgroups, g0,
                                g0 + cnt, ng, bits, W, p.Mp, m, n, ea, eb, alpha, beta, C, ldc, dqm, total);
         }
