@@ -121,8 +121,8 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     const int first_m = group * GROUP_M;
     const int gsize = min(tiles_m - first_m, GROUP_M);
     const int in_group = local - group * per_group;
-    const int tm = first_m + in_group % gsize;
-    const int tn = in_group / gsize;
+    const int tm = __builtin_amdgcn_readfirstlane(first_m + in_group % gsize);
+    const int tn = __builtin_amdgcn_readfirstlane(in_group / gsize);
 
     const int64_t m0 = (int64_t)tm * BM;
     const int64_t n0 = (int64_t)tn * BN;
@@ -347,6 +347,22 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     }
 }
 
+// Tiles of this workgroup when each XCD takes one contiguous range: the
+// workgroups of XCD x walk its range side by side (one tile each when the grid
+// has them all).
+template <class F>
+__device__ __forceinline__ void walk_xcd(int total_tiles, const F& run) {
+    constexpr int X = 8;
+    const int x = blockIdx.x % X, slot = blockIdx.x / X;
+    const int q = total_tiles / X, r = total_tiles % X;
+    const int first = x * q + min(x, r), count = q + (x < r ? 1 : 0);
+    const int slots = gridDim.x / X + (x < (int)(gridDim.x % X) ? 1 : 0);
+    for (int t = slot; t < count; t += slots) {
+        run(first + t);
+        __syncthreads();  // the next tile's first stage goes where this one's last may still be read
+    }
+}
+
 // MODE 0: one workgroup per tile, tile = blockIdx.x (round-robin over XCDs);
 // MODE 1: one workgroup per tile, XCD-contiguous tile ranges (xcd_remap);
 // MODE 2: persistent: every workgroup takes tiles from `counter` (zeroed
@@ -370,17 +386,7 @@ __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_kernel(const Prob* __
         const int64_t bid = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
         if (bid < total_tiles) run((int)bid);
     } else if (MODE == 1) {
-        // the workgroups of XCD x walk its contiguous tile range side by side (one
-        // tile each when the grid has them all)
-        constexpr int X = 8;
-        const int x = blockIdx.x % X, slot = blockIdx.x / X;
-        const int q = total_tiles / X, r = total_tiles % X;
-        const int first = x * q + min(x, r), count = q + (x < r ? 1 : 0);
-        const int slots = gridDim.x / X + (x < (int)(gridDim.x % X) ? 1 : 0);
-        for (int t = slot; t < count; t += slots) {
-            run(first + t);
-            __syncthreads();  // the next tile's first stage goes where this one's last may still be read
-        }
+        walk_xcd(total_tiles, run);
     } else {
         __shared__ int next;
         while (true) {
@@ -392,6 +398,19 @@ __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_kernel(const Prob* __
             run(tile);
         }
     }
+}
+
+// One problem of one segment, passed by value: nothing is uploaded on the
+// first call with new buffers, and a workgroup's first loads wait on no table
+// reads (512^3: 9.3 -> 8.4 us a call, 7.9 of them on the GPU).  One workgroup
+// per tile, XCD-contiguous ranges; the walk of several tiles per workgroup
+// would spill registers here and stays with the tables.
+template <class C, bool TA, bool TB>
+__global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_one_kernel(Prob P, Seg S) {
+    __shared__ __attribute__((aligned(16))) char lds[2 * TileLds<C, TA, TB>::STAGE];
+    P.seg0 = 0;
+    P.nseg = 1;
+    gemm_tile<C, TA, TB>(P, &S, xcd_remap(blockIdx.x, gridDim.x), lds);
 }
 
 // ---------------------------------------------------------------------------
@@ -1013,6 +1032,14 @@ void launch_mode(int mode, const Prob* dp, int np, const Seg* ds, int tiles, int
 }
 
 template <class C>
+void launch_one(char opA, char opB, const Prob& p, const Seg& s, int tiles, hipStream_t st) {
+    const bool ta = opA == 'T', tb = opB == 'T';
+    const auto kernel = !ta && !tb ? gemm_f64_one_kernel<C, false, false> : !ta ? gemm_f64_one_kernel<C, false, true>
+                      : !tb        ? gemm_f64_one_kernel<C, true, false>  : gemm_f64_one_kernel<C, true, true>;
+    hipLaunchKernelGGL(kernel, dim3(tiles), dim3(C::NTH), 0, st, p, s);
+}
+
+template <class C>
 void launch_cfg(char opA, char opB, int mode, const Prob* dp, int np, const Seg* ds, int tiles, int grid, int* counter,
                 hipStream_t st) {
     const bool ta = opA == 'T', tb = opB == 'T';
@@ -1261,6 +1288,19 @@ int persistent_grid(int occ) {
     return cus * occ;
 }
 
+static constexpr int kOcc[3] = {Cfg128::OCC, Cfg64::OCC, Cfg32::OCC};
+
+// Workgroups of a register-staged launch in XCD ranges.  Little more than one
+// or two rounds of resident workgroups: the tiles left over land on the few
+// CUs that drain first, several on each.  Workgroups that walk the tiles in
+// fixed steps keep them apart (2050^3 on 64x64 tiles, 1.06 rounds: 354 -> 305
+// us; 3072^3, 2.25: 853 -> 824).  With more left over, or more rounds, the
+// order of completion balances better (4096^3: 1945 us against 1987).
+static int xcd_grid(int w, int t) {
+    const int slots = persistent_grid(kOcc[w]);
+    return w < 2 && t > slots && t < 3 * slots && t % slots <= slots / 4 ? slots : t;
+}
+
 int launch_gemm_f64_dev(char opA, char opB, int mode, const GemmBatchDev& b, int* counter, hipStream_t stream) {
     if (mode == DG_GEMM_MODE_PERSISTENT && !counter)
         return fail(DG_ERR_INVALID, "gemm: persistent launch without a work counter");
@@ -1284,19 +1324,11 @@ int launch_gemm_f64_dev(char opA, char opB, int mode, const GemmBatchDev& b, int
         else launch_dma<false, false>(edge, mode, dp, np, b.segs, t0, grid, counter, stream);
         DG_LAUNCH_CHECK();
     }
-    const int occ[3] = {Cfg128::OCC, Cfg64::OCC, Cfg32::OCC};
     for (int w = 0; w < 3; ++w) {  // 128x128 tiles, 64x64, 32x32
         const int t = b.tiles_gen[w];
         if (t <= 0) continue;
-        int grid = grid_of(t, occ[w]);
-        // Little more than one or two rounds of resident workgroups: the tiles
-        // left over land on the few CUs that drain first, several on each.
-        // Workgroups that walk the tiles in fixed steps keep them apart (2050^3 on
-        // 64x64 tiles, 1.06 rounds: 354 -> 305 us; 3072^3, 2.25: 853 -> 824).  With
-        // more left over, or more rounds, the order of completion balances better
-        // (4096^3: 1945 us against 1987).
-        const int slots = persistent_grid(occ[w]);
-        if (w < 2 && mode == DG_GEMM_MODE_XCD && t > slots && t < 3 * slots && t % slots <= slots / 4) grid = slots;
+        int grid = grid_of(t, kOcc[w]);
+        if (mode == DG_GEMM_MODE_XCD) grid = xcd_grid(w, t);
         if (w == 0) launch_cfg<Cfg128>(opA, opB, mode, b.gen[0], b.ngen[0], b.segs, t, grid, counter, stream);
         else if (w == 1) launch_cfg<Cfg64>(opA, opB, mode, b.gen[1], b.ngen[1], b.segs, t, grid, counter, stream);
         else launch_cfg<Cfg32>(opA, opB, mode, b.gen[2], b.ngen[2], b.segs, t, grid, counter, stream);
@@ -1311,6 +1343,21 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs_in, const
     int rc = prepare_gemm(opA, opB, probs_in, segs, hb);
     if (rc) return rc;
     if (hb.empty()) return DG_OK;
+    if (mode == DG_GEMM_MODE_PERSISTENT) mode = DG_GEMM_MODE_XCD;  // needs a counter: plans only
+    if (mode == DG_GEMM_MODE_XCD && hb.dma.empty() && hb.dmae.empty() &&
+        hb.gen[0].size() + hb.gen[1].size() + hb.gen[2].size() == 1) {
+        const int w = hb.gen[0].size() ? 0 : hb.gen[1].size() ? 1 : 2;
+        const Prob& p = hb.gen[w][0];
+        const int t = hb.tiles_gen[w];
+        if (p.nseg == 1 && t <= (1 << 22) && xcd_grid(w, t) == t) {
+            const Seg& s = hb.segs[p.seg0];
+            if (w == 0) launch_one<Cfg128>(opA, opB, p, s, t, stream);
+            else if (w == 1) launch_one<Cfg64>(opA, opB, p, s, t, stream);
+            else launch_one<Cfg32>(opA, opB, p, s, t, stream);
+            DG_LAUNCH_CHECK();
+            return DG_OK;
+        }
+    }
     GemmBatchDev b;
     TableUseScope uses{stream};  // after the launch below returns
     auto table = [&](const auto& v, auto** dst) -> bool {
@@ -1324,7 +1371,6 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs_in, const
         !table(hb.gen[1], &b.gen[1]) || !table(hb.gen[2], &b.gen[2]) || !table(hb.segs, &b.segs))
         return DG_ERR_ALLOC;
     b.set_counts(hb);
-    if (mode == DG_GEMM_MODE_PERSISTENT) mode = DG_GEMM_MODE_XCD;  // needs a counter: plans only
     return launch_gemm_f64_dev(opA, opB, mode, b, nullptr, stream);
 }
 
