@@ -53,7 +53,7 @@ struct dg_grouped_plan {
     std::vector<OzOperand> oz_ops;
     std::vector<int> oz_a, oz_b;   // per entry of oz_idx: its op(A) rows and op(B) columns in oz_ops
     void* oz_shared = nullptr;
-    int64_t oz_scan_off = 0, oz_digit_off = 0;
+    int64_t oz_digit_off = 0;
 };
 
 namespace dg {
@@ -174,8 +174,15 @@ int plan_launch(dg_grouped_plan* p, int variant, int cfg, hipStream_t st, bool w
     if (!with_ozaki) return DG_OK;
     if (p->oz_shared) {
         char* base = static_cast<char*>(p->oz_shared);
-        for (const auto& o : p->oz_ops) {
-            int rc = crt_prepare(o.x, o.rows, o.k, o.rs, o.ks, o.nmod, base + o.off, base + p->oz_scan_off, st);
+        for (size_t t = 0; t < p->oz_ops.size();) {  // neighbours of one k and moduli count in pairs
+            const auto& o = p->oz_ops[t];
+            CrtLines ops[2];
+            int count = 0;
+            while (count < 2 && t < p->oz_ops.size() && p->oz_ops[t].k == o.k && p->oz_ops[t].nmod == o.nmod) {
+                const auto& x = p->oz_ops[t++];
+                ops[count++] = CrtLines{x.x, x.rows, x.rs, x.ks, base + x.off};
+            }
+            const int rc = crt_prepare(ops, count, o.k, o.nmod, st);
             if (rc) return rc;
         }
         for (size_t t = 0; t < p->oz_idx.size(); ++t) {
@@ -197,15 +204,15 @@ int plan_launch(dg_grouped_plan* p, int variant, int cfg, hipStream_t st, bool w
 // Finds the operands that several Ozaki problems read (same lines: pointer,
 // line count, k, strides, moduli) and, when any repeats, no emulated
 // problem's C overlaps an operand and the prepared copies fit in half of the
-// free device memory, allocates one buffer for all of them plus one scan and
-// one digit buffer; otherwise leaves the per-problem path in place.  The products are bit for bit those of
+// free device memory, allocates one buffer for all of them plus one digit
+// buffer; otherwise leaves the per-problem path in place.  The products are bit for bit those of
 // dg_ozaki_dgemm: a prepared operand depends only on its own lines.
 int share_operands(dg_grouped_plan* p) {
     p->oz_ops.clear();
     p->oz_a.clear();
     p->oz_b.clear();
     std::map<std::tuple<uintptr_t, int64_t, int64_t, int64_t, int64_t, int>, int> index;
-    int64_t off = 0, scan = 0, digits = 0;
+    int64_t off = 0, digits = 0;
     auto add = [&](const double* x, int64_t rows, int64_t k, int64_t rs, int64_t ks, int nmod) {
         const auto key = std::make_tuple(reinterpret_cast<uintptr_t>(x), rows, k, rs, ks, nmod);
         auto it = index.find(key);
@@ -213,7 +220,6 @@ int share_operands(dg_grouped_plan* p) {
         const int id = (int)p->oz_ops.size();
         p->oz_ops.push_back({x, rows, k, rs, ks, nmod, off});
         off += (crt_operand_bytes(rows, k, nmod) + 255) / 256 * 256;
-        scan = std::max(scan, crt_scan_bytes(rows, k));
         index[key] = id;
         return id;
     };
@@ -241,7 +247,7 @@ int share_operands(dg_grouped_plan* p) {
         }
     }
     size_t free_b = 0, total_b = 0;
-    const int64_t bytes = off + (scan + 255) / 256 * 256 + digits;
+    const int64_t bytes = off + digits;
     const bool repeats = p->oz_ops.size() < 2 * p->oz_idx.size();
     if (!repeats || !disjoint || hipMemGetInfo(&free_b, &total_b) != hipSuccess || bytes > (int64_t)(free_b / 2) ||
         hipMalloc(&p->oz_shared, (size_t)bytes) != hipSuccess) {
@@ -252,8 +258,7 @@ int share_operands(dg_grouped_plan* p) {
         p->oz_b.clear();
         return DG_OK;
     }
-    p->oz_scan_off = off;
-    p->oz_digit_off = off + (scan + 255) / 256 * 256;
+    p->oz_digit_off = off;
     if (p->oz_ws) {  // the per-problem workspace served the form trials only
         (void)hipFree(p->oz_ws);
         p->oz_ws = nullptr;
