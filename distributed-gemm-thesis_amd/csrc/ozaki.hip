@@ -795,6 +795,28 @@ __global__ __launch_bounds__(SCNT, 2) void oz_plane_small_kernel(OzPlaneArgs g) 
     store_plane(acc, g.planes + (int64_t)gr.plane * g.plane, g.Mp, m0 + wm + 4 * (lane >> 4), n0 + wn + (lane & 15));
 }
 
+// C = val + beta C on up to four rows of a column (`left` of them in C), in
+// 32-byte accesses where C allows it (the combination of 8 planes of 3000 x
+// 2000: 52 -> 44 us against single elements).
+__device__ __forceinline__ void store_c(double (&val)[4], double* cp, int64_t left, double beta) {
+    if (left >= 4 && (reinterpret_cast<uintptr_t>(cp) & 31) == 0) {
+        dv4* c4 = reinterpret_cast<dv4*>(cp);
+        if (beta != 0.0) {
+            const dv4 old = __builtin_nontemporal_load(c4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) val[e] = __dadd_rn(val[e], __dmul_rn(beta, old[e]));
+        }
+        __builtin_nontemporal_store(dv4{val[0], val[1], val[2], val[3]}, c4);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (e >= left) break;
+            if (beta != 0.0) val[e] = __dadd_rn(val[e], __dmul_rn(beta, cp[e]));
+            cp[e] = val[e];
+        }
+    }
+}
+
 // The FP64 recombination of scheme I from the planes of groups [gb, ge) of
 // ng, for one thread's 4 rows of one column of the padded Mp x Np extent:
 // each group's x = sum * 2^-(bits*level) (exact) is added in group order,
@@ -839,14 +861,8 @@ __global__ __launch_bounds__(256) void oz_combine_kernel(const int32_t* __restri
     if ((int64_t)j >= n) return;
     const int jf = eb[j];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int64_t i = i0 + e;
-        if (i >= m) break;
-        double* cp = C + i + (int64_t)j * ldc;
-        double val = __dmul_rn(alpha, ldexp(cur[e], ea[i] + jf));
-        if (beta != 0.0) val = __dadd_rn(val, __dmul_rn(beta, *cp));
-        *cp = val;
-    }
+    for (int e = 0; e < 4; ++e) cur[e] = __dmul_rn(alpha, ldexp(cur[e], ea[i0 + e] + jf));  // ea is padded
+    store_c(cur, C + i0 + (int64_t)j * ldc, m - i0, beta);
 }
 
 // The balanced CRT value V of one element, correctly rounded to double, from
@@ -930,24 +946,7 @@ __global__ __launch_bounds__(256) void crt_reconstruct_kernel(const uint8_t* __r
             const int64_t i = i0 + e < m ? i0 + e : m - 1;  // rows past m are computed but never stored
             val[e] = __dmul_rn(alpha, ldexp(crt_value(L[e][0], L[e][1], L[e][2], tb), ea[i] + jf - 2 * q));
         }
-        double* cp = C + i0 + j * ldc;
-        if (i0 + 3 < m && (reinterpret_cast<uintptr_t>(cp) & 31) == 0) {
-            dv4* c4 = reinterpret_cast<dv4*>(cp);
-            if (beta != 0.0) {
-                const dv4 old = __builtin_nontemporal_load(c4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) val[e] = __dadd_rn(val[e], __dmul_rn(beta, old[e]));
-            }
-            __builtin_nontemporal_store(dv4{val[0], val[1], val[2], val[3]}, c4);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (i0 + e >= m) break;
-                double v = val[e];
-                if (beta != 0.0) v = __dadd_rn(v, __dmul_rn(beta, cp[e]));
-                cp[e] = v;
-            }
-        }
+        store_c(val, C + i0 + j * ldc, m - i0, beta);
     }
 }
 
