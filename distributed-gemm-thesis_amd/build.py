@@ -53,7 +53,7 @@ def _run(cmd):
 # outstanding loads and place their waits by hand; a register spill would put
 # scratch traffic between those loads and the waits (and has gone with wrong
 # results), so any spill in them fails the build.
-NO_SPILL = ("_dma_", "crt_gemm_kernel", "oz_plane_kernel")
+NO_SPILL = ("_dma_", "crt_gemm_kernel", "crt_gemm_small_kernel", "oz_plane_kernel", "oz_plane_small_kernel")
 
 
 def _check_spills(src, remarks):
