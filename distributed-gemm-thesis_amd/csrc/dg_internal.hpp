@@ -142,8 +142,8 @@ enum {
 
 // Launches the FP64 MFMA GEMM over `probs` (host vector; uploaded through
 // the table cache).  All problems share opA/opB.
-int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs,
-                    const std::vector<Seg>& segs, hipStream_t stream, int mode);
+int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs, std::vector<Seg> segs, hipStream_t stream,
+                    int mode);
 
 // A batch split by kernel.  With DG_GEMM_TILE_DIRECT, the direct-to-LDS
 // kernels take a problem when every segment has K > 0 and even leading
@@ -166,7 +166,7 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs,
 // `dma` (a row-shifted problem's interior starts at its row 127), and strips
 // around it on the register-staged kernel (on `dmae` under
 // DG_GEMM_NO_NARROW).  The sub-problems' segments are appended to `segs`
-// (which starts as a copy of the input segments).
+// (which starts with the input segments).
 // Register-staged problems and strips go to gen[0] (128x128 tiles), gen[1]
 // (64x64) or gen[2] (32x32): the choice's own, or a smaller one where they are
 // at most 96 or 32 rows or columns.
@@ -176,7 +176,7 @@ struct GemmBatch {
     std::vector<Seg> segs;                // the segment table all lists index
     bool empty() const { return dma.empty() && dmae.empty() && gen[0].empty() && gen[1].empty() && gen[2].empty(); }
 };
-int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, const std::vector<Seg>& segs, GemmBatch& out,
+int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector<Seg> segs, GemmBatch& out,
                  bool split_edges = true, int tile = DG_GEMM_TILE_AUTO);
 
 // The same batch with its tables resident on the device.

@@ -146,7 +146,7 @@ int dg_cannon25d(char opA, char opB, int64_t M, int64_t N, int64_t K, double alp
                 }
                 probs.push_back(pr);
             }
-    rc = launch_gemm_f64(oa, ob, probs, segs, st, DG_GEMM_MODE_XCD);
+    rc = launch_gemm_f64(oa, ob, probs, std::move(segs), st, DG_GEMM_MODE_XCD);
     if (rc) return rc;
     if (c > 1) return dg_layer_reduce(C_packed, workspace, M * N, c - 1, stream);
     return DG_OK;
@@ -260,7 +260,7 @@ int dg_summa(char opA, char opB, int64_t M, int64_t N, int64_t K, double alpha, 
         }
     if (probs.size() > (size_t)INT32_MAX || segs.size() > (size_t)INT32_MAX)
         return fail(DG_ERR_UNSUPPORTED, "dg_summa: too many blocks");
-    return launch_gemm_f64(oa, ob, probs, segs, st, DG_GEMM_MODE_XCD);
+    return launch_gemm_f64(oa, ob, probs, std::move(segs), st, DG_GEMM_MODE_XCD);
 }
 
 }  // extern "C"

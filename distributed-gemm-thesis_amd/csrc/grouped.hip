@@ -298,7 +298,7 @@ int build_groups(dg_grouped_plan* p, const dg_gemm_desc* descs, int count, const
             std::vector<Seg> segs;
             build_group(sel.data(), kv.second, probs0, segs);
             GemmBatch hb;
-            int rc = prepare_gemm(kv.first.first, kv.first.second, probs0, segs, hb, true, tune ? t : (int)DG_GEMM_TILE_AUTO);
+            int rc = prepare_gemm(kv.first.first, kv.first.second, probs0, std::move(segs), hb, true, tune ? t : (int)DG_GEMM_TILE_AUTO);
             if (rc) return rc;
             if (hb.empty()) continue;
             p->groups[t].push_back({kv.first.first, kv.first.second, GemmBatchDev{}});
@@ -605,7 +605,7 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
         if (probs.empty()) continue;
         Piece pc{kv.first.first, kv.first.second, GemmBatch{}, 0, 0, {0, 0, 0}, 0};
         // no sub-problems here: the tables stay within the documented capacity
-        rc = prepare_gemm(pc.opA, pc.opB, probs, segs, pc.hb, false);
+        rc = prepare_gemm(pc.opA, pc.opB, probs, std::move(segs), pc.hb, false);
         if (rc) return rc;
         pc.off_dma = take(pc.hb.dma.size() * sizeof(Prob));
         pc.off_dmae = take(pc.hb.dmae.size() * sizeof(Prob));
@@ -660,7 +660,7 @@ int dg_grouped_dgemm(const dg_gemm_desc* descs, int count, void* stream) {
         std::vector<Seg> segs;
         build_group(descs, kv.second, probs, segs);
         if (probs.empty()) continue;
-        rc = launch_gemm_f64(kv.first.first, kv.first.second, probs, segs, st, DG_GEMM_MODE_ROUND_ROBIN);
+        rc = launch_gemm_f64(kv.first.first, kv.first.second, probs, std::move(segs), st, DG_GEMM_MODE_ROUND_ROBIN);
         if (rc) return rc;
     }
     return DG_OK;

@@ -1,0 +1,147 @@
+// CPU-only checks of the FP64 GEMM's routing (prepare_gemm of libdgamd.so),
+// built and run by tests/test_host_route.py.  No GPU call is made and no
+// operand is read: the matrices are addresses only.
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <new>
+#include <random>
+#include <string>
+
+static inline uint32_t __umulhi(uint32_t a, uint32_t b) { return (uint32_t)((uint64_t)a * b >> 32); }  // no device pass here
+#include "dg_internal.hpp"
+
+static size_t allocated = 0;  // bytes asked of operator new so far, the library's included
+void* operator new(size_t n) {
+    allocated += n;
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
+
+using dg::Prob;
+using dg::Seg;
+
+static int failures = 0;
+#define CHECK(c)                                                                                        \
+    do {                                                                                                \
+        if (!(c)) { std::fprintf(stderr, "FAILED: %s (line %d)\n", #c, __LINE__); ++failures; }         \
+    } while (0)
+
+static double* at(uintptr_t x) { return reinterpret_cast<double*>(x); }
+
+// The host cost of a batch of many segments: its tables are copied once.
+static void check_bytes() {
+    std::vector<Prob> probs;
+    std::vector<Seg> segs;
+    for (int i = 0; i < 1024; ++i) {
+        Prob p{};
+        p.m = p.n = 64;
+        p.c = at(0x100000000 + 32768 * (uintptr_t)i);
+        p.ldc = 64;
+        p.alpha = 1.0;
+        p.seg0 = (int32_t)segs.size();
+        p.nseg = 64;
+        for (int s = 0; s < 64; ++s) segs.push_back(Seg{at(0x200000000), at(0x300000000), 2048, 2048, 64});
+        probs.push_back(p);
+    }
+    for (char oa : {'N', 'T'}) {
+        dg::GemmBatch b;
+        const size_t before = allocated;
+        CHECK(dg::prepare_gemm(oa, 'T', probs, segs, b) == DG_OK);
+        const size_t spent = allocated - before, tables = segs.size() * sizeof(Seg) + probs.size() * sizeof(Prob);
+        std::printf("prepared %zu bytes of tables with %zu bytes\n", tables, spent);
+        CHECK(spent <= tables + tables / 2);
+    }
+}
+
+// Every choice covers each element of each problem once, each part at the
+// operands' right places, with tile numbers that follow one another.
+static void check_parts() {
+    std::mt19937_64 rng(7);
+    auto pick = [&](int64_t lo, int64_t hi) { return lo + (int64_t)(rng() % (uint64_t)(hi - lo + 1)); };
+    const int64_t edges[5] = {128, 128, 128, 64, 32};
+    for (int trial = 0; trial < 60; ++trial) {
+        const char oa = "NT"[trial & 1], ob = "NT"[(trial >> 1) & 1];
+        const bool ak = oa == 'T', bkc = ob == 'N', even = trial % 3 != 0;
+        std::vector<Prob> probs;
+        std::vector<Seg> segs;
+        const int count = (int)pick(1, 3);
+        for (int i = 0; i < count; ++i) {
+            Prob p{};
+            p.m = pick(1, trial % 5 ? 3000 : 300);
+            p.n = pick(1, trial % 5 ? 3000 : 300);
+            if (trial % 7 == 0) { p.m = (p.m + 127) / 128 * 128; p.n = (p.n + 127) / 128 * 128; }
+            p.ldc = p.m + pick(0, 5);
+            p.c = at(0x1000000000 * (uintptr_t)(i + 1));
+            p.alpha = 1.0;
+            p.seg0 = (int32_t)segs.size();
+            p.nseg = (int32_t)pick(1, 4);
+            const uintptr_t sa = even ? 8 * pick(0, 1) : 0, sb = even ? 8 * pick(0, 1) : 0;
+            for (int s = 0; s < p.nseg; ++s) {
+                const int64_t k = even ? 16 * pick(1, 20) : pick(1, 300);
+                Seg g{at(0x20000000000 + sa * !ak), at(0x30000000000 + sb * !bkc), (ak ? k : p.m) + pick(0, 9), (bkc ? k : p.n) + pick(0, 9), k};
+                if (even) { g.lda += g.lda & 1; g.ldb += g.ldb & 1; }
+                segs.push_back(g);
+            }
+            probs.push_back(p);
+        }
+        for (int tile = dg::DG_GEMM_TILE_AUTO; tile < dg::DG_GEMM_TILES; ++tile)
+            for (bool split : {true, false}) {
+                dg::GemmBatch b;
+                CHECK(dg::prepare_gemm(oa, ob, probs, segs, b, split, tile) == DG_OK);
+                CHECK(b.segs.size() >= segs.size() && !memcmp(b.segs.data(), segs.data(), segs.size() * sizeof(Seg)));
+                const std::vector<Prob>* lists[5] = {&b.dma, &b.dmae, &b.gen[0], &b.gen[1], &b.gen[2]};
+                const int tiles[5] = {b.tiles_dma, b.tiles_dmae, b.tiles_gen[0], b.tiles_gen[1], b.tiles_gen[2]};
+                std::vector<std::vector<unsigned char>> seen(count);
+                for (int i = 0; i < count; ++i) seen[i].assign((size_t)(probs[i].m * probs[i].n), 0);
+                for (int l = 0; l < 5; ++l) {
+                    int64_t next = 0;
+                    for (const Prob& q : *lists[l]) {
+                        const int i = (int)(reinterpret_cast<uintptr_t>(q.c) / 0x1000000000) - 1;
+                        CHECK(i >= 0 && i < count);
+                        const Prob& p = probs[i];
+                        const int64_t off = q.c - p.c, r0 = off % p.ldc, c0 = off / p.ldc;
+                        CHECK(q.ldc == p.ldc && q.nseg == p.nseg && r0 + q.m <= p.m && c0 + q.n <= p.n);
+                        CHECK(q.tile0 == next);
+                        int sa = 0, sb = 0;
+                        for (int s = 0; s < q.nseg; ++s) {
+                            const Seg &g = b.segs[q.seg0 + s], &h = segs[p.seg0 + s];
+                            CHECK(g.lda == h.lda && g.ldb == h.ldb && g.klen == h.klen);
+                            CHECK(g.a == h.a + (ak ? r0 * h.lda : r0) && g.b == h.b + (bkc ? c0 * h.ldb : c0));
+                            sa = !ak && (reinterpret_cast<uintptr_t>(g.a) & 15);
+                            sb = !bkc && (reinterpret_cast<uintptr_t>(g.b) & 15);
+                            if (l < 2) CHECK(!(g.lda & 1) && !(g.ldb & 1) && (!ak || !(reinterpret_cast<uintptr_t>(g.a) & 15)));
+                            if (l == 0) CHECK(g.klen % 8 == 0 && !sa && !sb);
+                        }
+                        if (l == 0) CHECK(q.m % 128 == 0 && q.n % 128 == 0);
+                        if (l < 2) CHECK(q.shift == (sa | sb << 1)); else { CHECK(q.shift == 0); sa = sb = 0; }
+                        next += ((q.m + sa + edges[l] - 1) / edges[l]) * ((q.n + sb + edges[l] - 1) / edges[l]);
+                        for (int64_t c = c0; c < c0 + q.n; ++c)
+                            for (int64_t r = r0; r < r0 + q.m; ++r) ++seen[i][(size_t)(r + c * p.m)];
+                    }
+                    CHECK(tiles[l] == next);
+                }
+                for (int i = 0; i < count; ++i) {
+                    bool once = true;
+                    for (unsigned char x : seen[i]) once = once && x == 1;
+                    CHECK(once);
+                }
+                if (failures) {
+                    std::fprintf(stderr, "trial %d, choice %d, split %d\n", trial, tile, (int)split);
+                    return;
+                }
+            }
+    }
+}
+
+int main(int argc, char** argv) {
+    const std::string what = argc > 1 ? argv[1] : "";
+    if (what == "bytes") check_bytes();
+    else if (what == "parts") check_parts();
+    else { std::fprintf(stderr, "unknown check '%s'\n", what.c_str()); return 2; }
+    if (!failures) std::printf("%s: ok\n", what.c_str());
+    return failures ? 1 : 0;
+}

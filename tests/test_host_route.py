@@ -1,0 +1,47 @@
+"""The FP64 GEMM's host-side routing on the CPU: tests/host_route/check.cpp,
+built against libdgamd.so, looks at the lists that prepare_gemm makes of a
+batch.  No GPU call is made."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+PKG = os.path.join(ROOT, "distributed-gemm-thesis_amd")
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no host C++ compiler")
+
+
+@pytest.fixture(scope="module")
+def check(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("route") / "check")
+    cmd = ["g++", "-O2", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I" + os.path.join(ROOT, "include"),
+           "-I" + os.path.join(PKG, "csrc"), "-I" + os.path.join(ROCM, "include"),
+           os.path.join(ROOT, "tests", "host_route", "check.cpp"), "-o", exe, "-L" + PKG, "-ldgamd",
+           "-L" + os.path.join(ROCM, "lib"), "-lamdhip64", "-Wl,-rpath," + PKG,
+           "-Wl,-rpath," + os.path.join(ROCM, "lib")]
+    b = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
+    assert b.returncode == 0, b.stderr[-3000:]
+
+    def run(what):
+        env = {k: v for k, v in os.environ.items() if not k.startswith("DG_GEMM_")}
+        r = subprocess.run([exe, what], capture_output=True, text=True, timeout=300, env=env)
+        assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-3000:])
+        assert what + ": ok" in r.stdout
+    return run
+
+
+def test_tables_are_copied_once(check):
+    """A batch of many segments costs the host one copy of its tables,
+    whatever the number of tile choices that are compared."""
+    check("bytes")
+
+
+def test_parts_cover_each_problem_once(check):
+    """Under every tile choice, cut or not: each element of each problem is
+    in one part, each part's operands start at its rows and columns, the
+    tile numbers of a list follow one another, and the kernels get only what
+    they take."""
+    check("parts")
