@@ -789,10 +789,15 @@ void launch_sgemm_dma(bool edge, const SgemmArgs& a, int tiles, hipStream_t st) 
 }
 
 template <class C, bool AK, bool BKC>
+bool by_elements(const SgemmArgs& a) {
+    return !Staged<float, AK, C::T, C::BK>::takes(a.a, a.lda) || !Staged<float, BKC, C::T, C::BK>::takes(a.b, a.ldb);
+}
+
+template <class C, bool AK, bool BKC>
 void launch_sgemm(SgemmArgs a, hipStream_t st) {
     a.tiles_m = (int)((a.m + C::T - 1) / C::T);
     a.tiles_n = (int)((a.n + C::T - 1) / C::T);
-    a.by_elements = !Staged<float, AK, C::T, C::BK>::takes(a.a, a.lda) || !Staged<float, BKC, C::T, C::BK>::takes(a.b, a.ldb);
+    a.by_elements = by_elements<C, AK, BKC>(a);
     hipLaunchKernelGGL((sgemm_kernel<C, AK, BKC>), tile_grid(a.tiles_m * a.tiles_n), dim3(256), 0, st, a);
 }
 
@@ -806,10 +811,12 @@ void launch_sgemm(SgemmArgs a, hipStream_t st) {
 // long K (4096^3: 938 us against 967), 128x128 at short K (8192 x 8192 x 256:
 // 273 us against 302) and in the largest NN products (16384^3: 60.9 ms against
 // 61.2), 32x32 where it fills CUs that 64x64 leaves idle (512^3: 7.1 us against
-// 12.4).
-double sgemm_time(int64_t m, int64_t n, int64_t k, int t, int conc, const double* eff) {
+// 12.4).  Loads by elements: kElementRate of these (NN 2048 x 2048 x 480 with
+// 2^23 + 4 rows to a column: 77 us, 42 with whole runs).
+constexpr double kElementRate = 0.55;
+double sgemm_time(int64_t m, int64_t n, int64_t k, int t, int conc, const double* eff, bool elements) {
     const int64_t c = (((m + t - 1) / t) * ((n + t - 1) / t) + 255) / 256;
-    const double u = 2.0 * t * t * (double)k / (157.3e6 / 256);
+    const double u = 2.0 * t * t * (double)k / (157.3e6 / 256) / (elements ? kElementRate : 1.0);
     return (double)c * u / eff[c >= 128 ? 5 : c >= 8 ? 4 : std::min<int64_t>(c, 4) - 1] + 4.0 * std::max(1.0, (double)c / conc);
 }
 constexpr double kEffDma[2][6] = {{0.83, 0.90, 0.90, 0.90, 0.90, 0.90}, {0.83, 0.90, 0.91, 0.92, 0.92, 0.92}};
@@ -836,16 +843,19 @@ void run_sgemm(const SgemmArgs& a, bool dma, hipStream_t st) {
         const bool edge = p.m % sk::BM || p.n % sk::BN || p.k % sk::BK || (steps & 1);
         launch_sgemm_dma<AK, BKC>(edge, p, p.tiles_m * p.tiles_n, st);
     };
+    const bool el64 = by_elements<Sgemm64, AK, BKC>(a), el32 = by_elements<Sgemm32, AK, BKC>(a);
+    auto time64 = [&](int64_t m, int64_t n) { return sgemm_time(m, n, a.k, 64, 4, kEff64, el64); };
+    auto time32 = [&](int64_t m, int64_t n) { return sgemm_time(m, n, a.k, 32, 4, kEff32, el32); };
     auto staged = [&](const SgemmArgs& p) {
-        const bool small = forced == "32x32" || (forced != "64x64" && sgemm_time(p.m, p.n, p.k, 32, 4, kEff32) < sgemm_time(p.m, p.n, p.k, 64, 4, kEff64));
+        const bool small = forced == "32x32" || (forced != "64x64" && time32(p.m, p.n) < time64(p.m, p.n));
         if (small) launch_sgemm<Sgemm32, AK, BKC>(p, st); else launch_sgemm<Sgemm64, AK, BKC>(p, st);
     };
     const int64_t mi = a.m / sk::BM * sk::BM, ni = a.n / sk::BN * sk::BN;
     const bool k_ok = a.k % sk::BK == 0 && !((a.k / sk::BK) & 1);
     const bool cut = (AK || BKC) && !no_areg && k_ok && (mi != a.m || ni != a.n) && mi * ni >= 8 * sk::BM * sk::BN;
     if (dma && forced != "direct" && forced != "128x128") {
-        auto least = [&](int64_t m, int64_t n) { return std::min(sgemm_time(m, n, a.k, 64, 4, kEff64), sgemm_time(m, n, a.k, 32, 4, kEff32)); };
-        double t = sgemm_time(cut ? mi : a.m, cut ? ni : a.n, a.k, 128, 2, kEffDma[AK || BKC]);
+        auto least = [&](int64_t m, int64_t n) { return std::min(time64(m, n), time32(m, n)); };
+        double t = sgemm_time(cut ? mi : a.m, cut ? ni : a.n, a.k, 128, 2, kEffDma[AK || BKC], false);
         if (cut && mi < a.m) t += least(a.m - mi, a.n);
         if (cut && ni < a.n) t += least(mi, a.n - ni);
         dma = forced.empty() && t <= least(a.m, a.n);

@@ -1067,13 +1067,22 @@ struct Route {
     bool direct = true;     // the direct-to-LDS kernels take it; then
     int sa = 0, sb = 0;     // whether its A (B) starts 8 bytes past a 16-byte boundary (k-contiguous: -1), and
     bool k_ok = false;      // its k is an even number of whole k-steps
-    bool elements = false;  // the register-staged kernel loads it by single elements
+    bool elements[3] = {};  // the register-staged kernel's tiles (gen[w]) load it by single elements
 };
 
+// Whether tiles of shape C load a problem's runs whole (`bits`: all its bases).
+template <class C>
+static bool takes(bool ak, bool bkc, uintptr_t bits, int64_t lda, int64_t ldb) {
+    using KC = Staged<double, true, C::BM, C::BK>;
+    using RC = Staged<double, false, C::BM, C::BK>;
+    const double* x = reinterpret_cast<const double*>(bits);
+    return (ak ? KC::takes(x, lda) : RC::takes(x, lda)) && (bkc ? KC::takes(x, ldb) : RC::takes(x, ldb));
+}
+
 static Route route_of(const Prob& p, const std::vector<Seg>& segs, bool ak, bool bkc) {
-    using KC = Staged<double, true, 64, 16>;
-    using RC = Staged<double, false, 64, 16>;
     Route r;
+    uintptr_t bits = 0;
+    int64_t lda = 1, ldb = 1;  // the longest
     int off_a = -1, off_b = -1;  // byte offset within 16 of a row-contiguous A / B
     int64_t steps = 0;
     bool whole = true;  // every segment a whole number of k-steps
@@ -1082,8 +1091,9 @@ static Route route_of(const Prob& p, const std::vector<Seg>& segs, bool ak, bool
         r.depth += g.klen;
         steps += (g.klen + dmak::DBK - 1) / dmak::DBK;
         if (g.klen % dmak::DBK) whole = false;
-        if (!(ak ? KC::takes(g.a, g.lda) : RC::takes(g.a, g.lda)) || !(bkc ? KC::takes(g.b, g.ldb) : RC::takes(g.b, g.ldb)))
-            r.elements = true;
+        bits |= reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b);
+        lda = std::max(lda, g.lda);
+        ldb = std::max(ldb, g.ldb);
         const int oa = (int)(reinterpret_cast<uintptr_t>(g.a) & 15), ob = (int)(reinterpret_cast<uintptr_t>(g.b) & 15);
         if ((g.lda & 1) || (g.ldb & 1) || g.klen <= 0) r.direct = false;
         if (ak) { if (oa || (g.klen & 1)) r.direct = false; }   // k pairs, 16-byte aligned
@@ -1094,6 +1104,9 @@ static Route route_of(const Prob& p, const std::vector<Seg>& segs, bool ak, bool
     r.sa = ak ? -1 : off_a == 8;
     r.sb = bkc ? -1 : off_b == 8;
     r.k_ok = whole && !(steps & 1);
+    r.elements[0] = !takes<Cfg128>(ak, bkc, bits, lda, ldb);
+    r.elements[1] = !takes<Cfg64>(ak, bkc, bits, lda, ldb);
+    r.elements[2] = !takes<Cfg32>(ak, bkc, bits, lda, ldb);
     return r;
 }
 
@@ -1112,7 +1125,11 @@ static_assert(dmak::DBM == dmak::DBN, "one edge per list");
 // from 32 on: its matrix cores are 99 % busy, but its workgroups drift apart,
 // fetch their operands from beyond the L2 (16384^3: 374 GB against 101) and
 // the clock falls; 64x64 0.92, 0.88 from 25 tiles per CU on, 0.85 from 64 on;
-// 32x32 0.67, 0.72, 0.76, 0.78 with one to four, 0.80 with more.
+// 32x32 0.67, 0.72, 0.76, 0.78 with one to four, 0.80 with more.  Loads by
+// elements: kElementRate of these (TN 500 x 4096 x 4096 with 2^22 + 2 rows to a
+// column, 64x64 tiles: 403 us, 257 with whole runs; NN 4096 x 4096 x 480, odd:
+// 319 us against 251).
+constexpr double kElementRate = 0.65;
 struct Rate {
     int conc;
     double round;
@@ -1127,8 +1144,8 @@ constexpr Rate kRate[kLists] = {{2, 4, {{1, 0.91}, {2, 0.95}}},
 struct ListCost {
     int64_t tiles = 0;
     double sum = 0, most = 0, least = 1e300;  // us of CU time: all tiles, the longest, the shortest
-    void add(int64_t n, int64_t area, int64_t k) {
-        const double u = 2.0 * (double)area * (double)k / (78.6e6 / 256);
+    void add(int64_t n, int64_t area, int64_t k, bool elements) {
+        const double u = 2.0 * (double)area * (double)k / (78.6e6 / 256) / (elements ? kElementRate : 1.0);
         tiles += n;
         sum += (double)n * u;
         most = std::max(most, u);
@@ -1192,7 +1209,7 @@ static void split_problem(const Prob& p, const Route& r, int tile, bool split_ed
 
 // Shift bits and tiles of a part of a problem on a list.
 static int shift_of(const Route& r, int list, int64_t r0, int64_t c0) {
-    if (list >= kListGen) return r.elements ? kByElements : 0;
+    if (list >= kListGen) return r.elements[list - kListGen] ? kByElements : 0;
     // k-contiguous operands have no shift, wherever their part starts
     return (r.sa >= 0 ? (int)((r.sa + r0) & 1) : 0) | (r.sb >= 0 ? (int)((r.sb + c0) & 1) : 0) << 1;
 }
@@ -1218,7 +1235,8 @@ static Estimate estimate(const std::vector<Prob>& probs, const std::vector<Route
         const Route& r = routes[i];
         if (p.m <= 0 || p.n <= 0 || p.nseg <= 0) continue;
         split_problem(p, r, tile, split_edges, [&](int list, int64_t r0, int64_t nr, int64_t c0, int64_t nc) {
-            cost[list].add(tiles_of(list, shift_of(r, list, r0, c0), nr, nc), kTileOf[list] * kTileOf[list], r.depth);
+            const int shift = shift_of(r, list, r0, c0);
+            cost[list].add(tiles_of(list, shift, nr, nc), kTileOf[list] * kTileOf[list], r.depth, shift & kByElements);
             if (nr < p.m || nc < p.n) x.segs += p.nseg;
         });
     }

@@ -70,19 +70,27 @@ struct Staged {
     int64_t ld;
     uint32_t off[NL];  // bytes from it to this thread's runs
 
-    // row of this thread's run q within the tile, k of it within the stage
-    static __device__ __forceinline__ int row(int q) { return KC ? (int)threadIdx.x / CH + RPP * q : E * ((int)threadIdx.x % HP); }
-    static __device__ __forceinline__ int kk(int q) { return KC ? E * ((int)threadIdx.x % CH) : (int)threadIdx.x / HP + KPP * q; }
+    // Run q of thread t: its row within the tile, its k within the stage, and
+    // its place in a whole stage, bytes from the stage's first element.
+    static constexpr __host__ __device__ __forceinline__ int row(int t, int q) { return KC ? t / CH + RPP * q : E * (t % HP); }
+    static constexpr __host__ __device__ __forceinline__ int kk(int t, int q) { return KC ? E * (t % CH) : t / HP + KPP * q; }
+    static __host__ __device__ __forceinline__ uint32_t offset(int t, int q, int64_t ld, int rows) {
+        const uint32_t r = row(t, q) < rows ? row(t, q) : rows - 1, k = kk(t, q);
+        return (uint32_t)S * (KC ? r * (uint32_t)ld + k : k * (uint32_t)ld + r);
+    }
+    // Where element e of it is read in a stage of `left` real k, in elements.
+    static __host__ __device__ __forceinline__ int64_t last_offset(int t, int q, int e, int64_t ld, int rows, int left) {
+        const int r0 = row(t, q) + (KC ? 0 : e), k0 = kk(t, q) + (KC ? e : 0);
+        const int64_t r = r0 < rows ? r0 : rows - 1, k = k0 < left ? k0 : left - 1;
+        return KC ? r * ld + k : k * ld + r;
+    }
 
     // At a segment's first k; the tile has `rows` rows from row0 on.
     __device__ __forceinline__ void start(const T* x, int64_t ld_, int64_t row0, int rows) {
         ld = ld_;
         base = x + row0 * (KC ? ld : 1);
 #pragma unroll
-        for (int q = 0; q < NL; ++q) {
-            const uint32_t r = min(row(q), rows - 1), k = kk(q);
-            off[q] = (uint32_t)S * (KC ? r * (uint32_t)ld + k : k * (uint32_t)ld + r);
-        }
+        for (int q = 0; q < NL; ++q) off[q] = offset(threadIdx.x, q, ld, rows);
     }
     __device__ __forceinline__ void advance() {
         base += KC ? BK : BK * ld;
@@ -104,28 +112,29 @@ struct Staged {
 #pragma unroll
         for (int q = 0; q < NL; ++q)
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                const int64_t r = min(row(q) + (KC ? 0 : e), rows - 1), k = min(kk(q) + (KC ? e : 0), left - 1);
-                v[q][e] = *(gelem*)(base + (KC ? r * ld + k : k * ld + r));
-            }
+            for (int e = 0; e < E; ++e) v[q][e] = *(gelem*)(base + last_offset(threadIdx.x, q, e, ld, rows, left));
 #pragma unroll
         for (int q = 0; q < NL; ++q)
 #pragma unroll
-            for (int e = 0; e < E; ++e) v[q][e] = kk(q) + (KC ? e : 0) < left ? v[q][e] : T(0);
+            for (int e = 0; e < E; ++e) v[q][e] = kk(threadIdx.x, q) + (KC ? e : 0) < left ? v[q][e] : T(0);
         advance();
     }
     static __device__ __forceinline__ void store(char* s, const vec (&v)[NL], int q) {
-        *reinterpret_cast<vec*>(s + (KC ? row(q) * LROW + kk(q) * S : kk(q) * LROW + row(q) * S)) = v[q];
+        const int r = row(threadIdx.x, q), k = kk(threadIdx.x, q);
+        *reinterpret_cast<vec*>(s + (KC ? r * LROW + k * S : k * LROW + r * S)) = v[q];
     }
     static __device__ __forceinline__ void store(char* s, const vec (&v)[NL]) {
 #pragma unroll
         for (int q = 0; q < NL; ++q) store(s, v, q);
     }
     // Whether read() takes a matrix: elements on their own alignment, and rows
-    // neither so far apart that a tile's offsets leave 32 bits nor so close
-    // that a run at the last row would pass the matrix's end.
+    // (or k) neither so far apart that a lane's offset leaves 32 bits nor so
+    // close that a run at the last row would pass the matrix's end.  Others are
+    // read by elements throughout, at 0.65 (FP64) or 0.55 (FP32) of the rate.
+    static constexpr int64_t kMaxLd =
+        ((((int64_t)1 << 32) - 1) / S - ((KC ? BK : ROWS) - E)) / ((KC ? ROWS : BK) - 1);
     static bool takes(const T* x, int64_t ld) {
-        return !(reinterpret_cast<uintptr_t>(x) & (S - 1)) && ld <= ((int64_t)1 << 32) / (128 * S) - 128 && (KC || ld >= E - 1);
+        return !(reinterpret_cast<uintptr_t>(x) & (S - 1)) && ld <= kMaxLd && (KC || ld >= E - 1);
     }
 };
 

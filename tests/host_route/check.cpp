@@ -137,10 +137,56 @@ static void check_parts() {
     }
 }
 
+// Leading dimensions of millions: the direct-to-LDS kernels keep the problems
+// that they take, and the register-staged ones load by elements only where a
+// lane's offset would leave 32 bits.
+static void check_long() {
+    struct { char oa, ob; int64_t m, n, k, lda, ldb; int direct, elements; } cases[] = {
+        {'T', 'N', 2048, 2048, 5000000, 5000000, 5000000, -1, 0},
+        {'T', 'N', 4096, 4096, 5000000, 5000000, 5000000, -1, 0},
+        {'N', 'N', 4096, 4096, 4096, 8000000, 4096, -1, 0},
+        {'N', 'N', 4096, 4096, 4096, 8000001, 4096, 0, 0},
+        {'T', 'N', 2048, 2048, 4096, 4227000, 4096, -1, 0},
+        {'T', 'N', 2048, 2048, 4096, 8000001, 4096, 0, 0},   // 128x128 tiles past their limit, 64x64 within it
+        {'T', 'N', 2048, 2048, 4096, 18000000, 4096, 1, 0},  // past every tile's
+        {'T', 'T', 4096, 4096, 4096, 18000000, 4096, 1, 0},
+        {'T', 'N', 2048, 2048, 4096, 18000001, 4096, 0, 1},
+        {'N', 'T', 2048, 2048, 512, 35000000, 2048, -1, 0},
+        {'N', 'T', 2048, 2048, 512, 36000000, 2048, 1, 0},
+        {'N', 'T', 2048, 2048, 512, 36000001, 2048, 0, 1},
+    };
+    const int64_t edges[3] = {128, 64, 32}, depths[3] = {16, 16, 32};
+    for (const auto& c : cases) {
+        const bool ak = c.oa == 'T', bkc = c.ob == 'N';
+        std::vector<Seg> segs{Seg{at(0x10000), at(0x20000), c.lda, c.ldb, c.k}};
+        Prob p{};
+        p.m = c.m; p.n = c.n; p.ldc = c.m; p.c = at(0x30000); p.alpha = 1.0; p.nseg = 1;
+        dg::GemmBatch b;
+        CHECK(dg::prepare_gemm(c.oa, c.ob, {p}, segs, b) == DG_OK);
+        const bool direct = !b.dma.empty() || !b.dmae.empty();
+        bool any = false;
+        for (int w = 0; w < 3; ++w)
+            for (const Prob& q : b.gen[w]) {
+                const bool elements = q.shift & dg::kByElements;
+                auto most = [&](bool kc, int64_t ld) { return 8 * (kc ? (edges[w] - 1) * ld : (depths[w] - 1) * ld + edges[w]); };
+                const bool leaves = std::max(most(ak, c.lda), most(bkc, c.ldb)) >= (int64_t)1 << 32;
+                CHECK(elements == leaves);
+                any = any || elements;
+            }
+        CHECK(any == (c.elements != 0));
+        CHECK(c.direct < 0 || direct == (c.direct != 0));
+        if (failures) {
+            std::fprintf(stderr, "%c%c %lld %lld %lld lda %lld\n", c.oa, c.ob, (long long)c.m, (long long)c.n, (long long)c.k, (long long)c.lda);
+            return;
+        }
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") check_bytes();
     else if (what == "parts") check_parts();
+    else if (what == "long") check_long();
     else { std::fprintf(stderr, "unknown check '%s'\n", what.c_str()); return 2; }
     if (!failures) std::printf("%s: ok\n", what.c_str());
     return failures ? 1 : 0;

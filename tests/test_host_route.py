@@ -1,6 +1,7 @@
-"""The FP64 GEMM's host-side routing on the CPU: tests/host_route/check.cpp,
-built against libdgamd.so, looks at the lists that prepare_gemm makes of a
-batch.  No GPU call is made."""
+"""The GEMMs' host-side routing on the CPU: tests/host_route/check.cpp, built
+against libdgamd.so, looks at the lists that prepare_gemm makes of a batch,
+and tests/host_route/staged.cpp at the addresses of csrc/staged.hpp, compiled
+for the host.  No GPU call is made."""
 import os
 import shutil
 import subprocess
@@ -45,3 +46,25 @@ def test_parts_cover_each_problem_once(check):
     tile numbers of a list follow one another, and the kernels get only what
     they take."""
     check("parts")
+
+
+def test_long_columns(check):
+    """Leading dimensions of millions of elements: no problem that the
+    direct-to-LDS kernels take goes to loads by elements instead, and only
+    offsets that leave 32 bits do."""
+    check("long")
+
+
+def test_staged_addresses(tmp_path):
+    """Every element that the register-staged kernels load lies inside its
+    operand and arrives at its own place, and 32-bit lane offsets are the
+    true ones up to the longest leading dimension that takes them."""
+    exe = str(tmp_path / "staged")
+    hipcc = os.environ.get("HIPCC", os.path.join(ROCM, "bin", "hipcc"))
+    b = subprocess.run([hipcc, "-x", "hip", "--offload-host-only", "-O1", "-std=c++17", "-I" + os.path.join(PKG, "csrc"),
+                        os.path.join(ROOT, "tests", "host_route", "staged.cpp"), "-o", exe],
+                       capture_output=True, text=True, timeout=300)
+    assert b.returncode == 0, b.stderr[-3000:]
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-3000:])
+    assert "staged: ok" in r.stdout
