@@ -7,6 +7,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <algorithm>
 #include <vector>
 
 #include "dgamd.h"
@@ -178,6 +179,40 @@ struct GemmBatch {
 };
 int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector<Seg> segs, GemmBatch& out,
                  bool split_edges = true, int tile = DG_GEMM_TILE_AUTO);
+
+// Whether two tile choices of one batch came out alike: the same lists of the
+// same problems.
+bool same_lists(const GemmBatch& a, const GemmBatch& b);
+
+// Times the scheduling modes of each tile choice in `choices` and keeps the
+// fastest: trial(choice, mode, &ms) runs one and returns a status.  The middle
+// of three runs counts (some variants have a fast and a slow state, and their
+// best run says little about the next: 4 x 2048^3 on 64x64 tiles, 0.92 and
+// 0.97 ms); a variant whose first run is already a twentieth and 0.2 ms slower
+// than the best so far gets no second one.
+template <class F>
+int fastest_variant(const std::vector<int>& choices, const F& trial, int* choice, int* mode) {
+    float best = 1e30f;
+    for (int c : choices)
+        for (int v : {(int)DG_GEMM_MODE_XCD, (int)DG_GEMM_MODE_ROUND_ROBIN, (int)DG_GEMM_MODE_PERSISTENT}) {
+            float ms[3];
+            int runs = 0;
+            while (runs < 3) {
+                const int rc = trial(c, v, &ms[runs]);
+                if (rc) return rc;
+                ++runs;
+                if (runs == 1 && ms[0] > 1.05f * best && ms[0] > best + 0.2f) break;
+            }
+            if (runs < 3) continue;
+            std::sort(ms, ms + 3);
+            if (ms[1] < best) {
+                best = ms[1];
+                *choice = c;
+                *mode = v;
+            }
+        }
+    return DG_OK;
+}
 
 // The same batch with its tables resident on the device.
 struct GemmBatchDev {

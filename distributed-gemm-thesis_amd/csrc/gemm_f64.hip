@@ -1325,6 +1325,15 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector
     return DG_OK;
 }
 
+bool same_lists(const GemmBatch& a, const GemmBatch& b) {
+    static_assert(sizeof(Prob) == 64 && sizeof(Seg) == 40, "no padding: compared as bytes");
+    auto same = [](const auto& x, const auto& y) {
+        return x.size() == y.size() && (x.empty() || memcmp(x.data(), y.data(), x.size() * sizeof(x[0])) == 0);
+    };
+    return same(a.dma, b.dma) && same(a.dmae, b.dmae) && same(a.gen[0], b.gen[0]) && same(a.gen[1], b.gen[1]) &&
+           same(a.gen[2], b.gen[2]) && same(a.segs, b.segs);
+}
+
 int persistent_grid(int occ) {
     int dev = 0, cus = 0;
     if (hipGetDevice(&dev) != hipSuccess ||

@@ -18,6 +18,7 @@ struct dg_grouped_plan {
         dg::GemmBatchDev b;
     };
     std::vector<Group> groups[dg::DG_GEMM_TILES];  // per tile choice; [0] alone unless autotuned
+    int same_as[dg::DG_GEMM_TILES] = {};           // the choice that has its tables: the first that came out alike
     void* tables = nullptr;                        // the tables of all of them
     int mode = DG_PLAN_AUTOTUNE;   // requested
     int variant = -1;              // DG_GEMM_MODE_* in use (-1: not tuned yet)
@@ -269,7 +270,7 @@ int share_operands(dg_grouped_plan* p) {
 
 // Device tables of the FP64 problems listed in `use` (all when null), one
 // allocation and one copy for all: with the autotuner a set per tile choice
-// for it to time, else the estimated best.
+// that differs from those before it, else the estimated best.
 int build_groups(dg_grouped_plan* p, const dg_gemm_desc* descs, int count, const std::vector<char>* use) {
     std::vector<dg_gemm_desc> sel;
     sel.reserve(count);
@@ -291,8 +292,8 @@ int build_groups(dg_grouped_plan* p, const dg_gemm_desc* descs, int count, const
     p->tables = nullptr;
     const bool tune = p->mode == DG_PLAN_AUTOTUNE;
     const auto kinds = by_ops(sel.data(), (int)sel.size());
+    std::vector<GemmBatch> built[DG_GEMM_TILES];  // per choice, in the order of `kinds`
     for (int t = 0; t < (tune ? (int)DG_GEMM_TILES : 1); ++t) {
-        p->groups[t].reserve(kinds.size());  // `puts` points into it
         for (auto& kv : kinds) {
             std::vector<Prob> probs0;
             std::vector<Seg> segs;
@@ -300,6 +301,17 @@ int build_groups(dg_grouped_plan* p, const dg_gemm_desc* descs, int count, const
             GemmBatch hb;
             int rc = prepare_gemm(kv.first.first, kv.first.second, probs0, std::move(segs), hb, true, tune ? t : (int)DG_GEMM_TILE_AUTO);
             if (rc) return rc;
+            built[t].push_back(std::move(hb));
+        }
+        p->same_as[t] = t;
+        for (int u = t - 1; u >= 0; --u)
+            if (p->same_as[u] == u && std::equal(built[t].begin(), built[t].end(), built[u].begin(), same_lists))
+                p->same_as[t] = u;
+        if (p->same_as[t] != t) continue;
+        p->groups[t].reserve(kinds.size());  // `puts` points into it
+        size_t i = 0;
+        for (auto& kv : kinds) {
+            const GemmBatch& hb = built[t][i++];
             if (hb.empty()) continue;
             p->groups[t].push_back({kv.first.first, kv.first.second, GemmBatchDev{}});
             GemmBatchDev& b = p->groups[t].back().b;
@@ -470,9 +482,9 @@ int choose_forms(dg_grouped_plan* p, hipStream_t st) {
     return DG_OK;
 }
 
-// Times each tile choice and scheduling variant (best of three) on the plan's own operands
-// and keeps the fastest.  The outputs are saved before the trials and
-// restored after them, also when a trial fails, so tuning leaves C as it
+// Times the tile choices that differ and their scheduling modes on the plan's
+// own operands and keeps the fastest.  The outputs are saved before the trials
+// and restored after them, also when a trial fails, so tuning leaves C as it
 // found it.
 int autotune(dg_grouped_plan* p, hipStream_t st) {
     TuneCache& c = tune_cache();
@@ -482,38 +494,34 @@ int autotune(dg_grouped_plan* p, hipStream_t st) {
         auto it = c.best.find(p->shape_key);
         if (it != c.best.end() && it->second >= 0 && it->second / 4 < DG_GEMM_TILES && it->second % 4 < 3) {
             p->variant = it->second % 4;
-            p->cfg = it->second / 4;
+            p->cfg = p->same_as[it->second / 4];
             return DG_OK;
         }
     }
-    const int variants[3] = {DG_GEMM_MODE_XCD, DG_GEMM_MODE_ROUND_ROBIN, DG_GEMM_MODE_PERSISTENT};
-    float best_ms = 1e30f;
-    int best = DG_GEMM_MODE_XCD;  // encoded tile choice * 4 + scheduling mode
+    std::vector<int> choices;
+    for (int t = 0; t < DG_GEMM_TILES; ++t)
+        if (p->same_as[t] == t) choices.push_back(t);
+    int choice = 0, mode = DG_GEMM_MODE_XCD;
     {
         // the outputs are restored when `trial` ends, whether or not the trials succeed
         TrialScope trial;
         int rc = trial.save(st, p->c_spans);
         if (rc) return rc;
-        for (int cfg = 0; cfg < DG_GEMM_TILES; ++cfg)
-            for (int v : variants) {
-                float vbest = 1e30f;
-                for (int rep = 0; rep < 3; ++rep) {
-                    DG_HIP(hipEventRecord(trial.e0, st));
-                    rc = plan_launch(p, v, cfg, st, false);
-                    if (rc) return rc;
-                    DG_HIP(hipEventRecord(trial.e1, st));
-                    DG_HIP(hipEventSynchronize(trial.e1));
-                    float ms = 0.f;
-                    DG_HIP(hipEventElapsedTime(&ms, trial.e0, trial.e1));
-                    vbest = std::min(vbest, ms);
-                }
-                if (vbest < best_ms) { best_ms = vbest; best = cfg * 4 + v; }
-            }
+        rc = fastest_variant(choices, [&](int cfg, int v, float* ms) -> int {
+            DG_HIP(hipEventRecord(trial.e0, st));
+            const int rc = plan_launch(p, v, cfg, st, false);
+            if (rc) return rc;
+            DG_HIP(hipEventRecord(trial.e1, st));
+            DG_HIP(hipEventSynchronize(trial.e1));
+            DG_HIP(hipEventElapsedTime(ms, trial.e0, trial.e1));
+            return DG_OK;
+        }, &choice, &mode);
+        if (rc) return rc;
     }
-    p->variant = best % 4;
-    p->cfg = best / 4;
+    p->variant = mode;
+    p->cfg = choice;
     std::lock_guard<std::mutex> lock(c.mu);
-    tune_store_locked(c, p->shape_key, best);
+    tune_store_locked(c, p->shape_key, choice * 4 + mode);
     return DG_OK;
 }
 

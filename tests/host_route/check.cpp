@@ -182,11 +182,58 @@ static void check_long() {
     }
 }
 
+// An autotuned plan's first use: choices that come out alike are timed once,
+// and slow variants once.
+static void check_trials() {
+    auto distinct = [](char oa, char ob, int64_t m, int64_t n, int64_t k) {
+        std::vector<Seg> segs{Seg{at(0x10000), at(0x20000), oa == 'T' ? k : m, ob == 'N' ? k : n, k}};
+        Prob p{};
+        p.m = m; p.n = n; p.ldc = m; p.c = at(0x30000); p.alpha = 1.0; p.nseg = 1;
+        std::vector<dg::GemmBatch> b(dg::DG_GEMM_TILES);
+        std::vector<int> out;
+        for (int t = 0; t < dg::DG_GEMM_TILES; ++t) {
+            CHECK(dg::prepare_gemm(oa, ob, {p}, segs, b[t], true, t) == DG_OK);
+            bool seen = false;
+            for (int u : out) seen = seen || dg::same_lists(b[t], b[u]);
+            if (!seen) out.push_back(t);
+        }
+        return out;
+    };
+    CHECK((distinct('N', 'N', 2048, 2048, 2048) == std::vector<int>{0, 1, 3, 4}));     // nothing to cut
+    CHECK((distinct('N', 'N', 2047, 2049, 2049) == std::vector<int>{0, 2, 3, 4}));     // odd: not direct
+    CHECK((distinct('T', 'N', 5000, 5000, 5000) == std::vector<int>{0, 1, 2, 3, 4}));
+    CHECK((distinct('T', 'T', 90, 2000, 333) == std::vector<int>{0, 4}));              // narrow: 64x64 at most
+    // the fastest, found with one run of what is clearly slower and three of the others
+    const std::vector<int> choices{0, 1, 3, 4};
+    const float ms[4][3] = {{6.0f, 6.1f, 6.9f}, {5.5f, 5.4f, 5.6f}, {0, 0, 0}, {7.0f, 7.1f, 7.2f}};
+    int runs = 0, choice = -1, mode = -1;
+    auto trial = [&](int c, int v, float* t) {
+        ++runs;
+        const int row = c == 0 ? 0 : c == 1 ? 1 : 3;
+        *t = c == 3 ? 5.45f : ms[row][v == dg::DG_GEMM_MODE_XCD ? 0 : v == dg::DG_GEMM_MODE_ROUND_ROBIN ? 1 : 2];
+        return DG_OK;
+    };
+    CHECK(dg::fastest_variant(choices, trial, &choice, &mode) == DG_OK);
+    CHECK(choice == 1 && mode == dg::DG_GEMM_MODE_ROUND_ROBIN);
+    CHECK(runs == 3 + 3 + 1 + 9 + 9 + 3);
+    // runs so short that a launch's gap decides keep all three
+    runs = 0;
+    CHECK(dg::fastest_variant(choices, [&](int c, int v, float* t) { trial(c, v, t); *t *= 0.01f; return DG_OK; }, &choice, &mode) == DG_OK);
+    CHECK(choice == 1 && runs == 36);
+    // one lucky run of three does not win
+    runs = 0;
+    CHECK(dg::fastest_variant({0, 1}, [&](int c, int, float* t) { *t = c == 0 ? 5.0f : runs++ % 3 == 1 ? 4.5f : 5.1f; return DG_OK; }, &choice, &mode) == DG_OK);
+    CHECK(choice == 0);
+    // a failing trial ends it
+    CHECK(dg::fastest_variant(choices, [&](int, int, float*) { return DG_ERR_HIP; }, &choice, &mode) == DG_ERR_HIP);
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") check_bytes();
     else if (what == "parts") check_parts();
     else if (what == "long") check_long();
+    else if (what == "trials") check_trials();
     else { std::fprintf(stderr, "unknown check '%s'\n", what.c_str()); return 2; }
     if (!failures) std::printf("%s: ok\n", what.c_str());
     return failures ? 1 : 0;

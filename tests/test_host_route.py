@@ -55,6 +55,12 @@ def test_long_columns(check):
     check("long")
 
 
+def test_first_use_times_distinct_choices(check):
+    """An autotuned plan's first use times each distinct tile choice, and
+    what is clearly slower only once."""
+    check("trials")
+
+
 def test_staged_addresses(tmp_path):
     """Every element that the register-staged kernels load lies inside its
     operand and arrives at its own place, and 32-bit lane offsets are the
