@@ -38,10 +38,10 @@ inline char norm_op(char op) {
 // error on failure.  Uploading while `stream` is being captured into a HIP
 // graph is refused: tables must be built before capture; a table looked up
 // during a capture stays resident for the life of the process (the graph
-// holds its address), and so do the first 128 of a device.  Beyond 256 tables
-// per device, a new table reuses the buffer of the least recently used of the
-// others whose last use has completed on the device, found by event queries
-// (nothing waits, nothing is freed).
+// holds its address), and so do the first 128 of at most 64 KiB of a device.
+// Beyond 256 others per device, a new table reuses the buffer of the least
+// recently used of them whose last use has completed on the device, found by
+// event queries (nothing waits, nothing is freed).
 const void* cached_table(const void* host, size_t bytes, hipStream_t stream);
 
 // Marks the kernels that read this thread's tables looked up since the last

@@ -57,10 +57,12 @@ uint64_t hash_bytes(const void* p, size_t n) {
 //  * done: recorded on the stream of the last use after that call's kernels
 //    were enqueued (table_uses_enqueued); an entry is retired only when it is
 //    complete, so no retirement waits on the device.
-//  * kept: made while the cache held fewer than kKeptEntries; never retired,
-//    so its uses record no event.  An event is a packet of its own behind the
-//    kernel (a 64^3 dg_dgemm, two tables: 23.3 us a call with the events, 15.5
-//    without), and a program that never fills the cache needs none.
+//  * kept: one of the first kKeptEntries tables of at most kKeptBytes; never
+//    retired, so its uses record no event.  An event is a packet of its own
+//    behind the kernel (a 64^3 dg_dgemm, two tables: 23.3 us a call with the
+//    events, 15.5 without).  Kept tables hold 8 MiB at most and take nothing
+//    from the room of the others; larger tables belong to calls long enough not
+//    to notice an event.
 struct TableEntry {
     std::vector<unsigned char> bytes;  // host copy, compared on every hit
     void* dev = nullptr;
@@ -79,7 +81,7 @@ struct TableCache {
     std::unordered_map<uint64_t, std::vector<std::unique_ptr<TableEntry>>> map[64];  // per device: hash -> entries
     std::vector<void*> free_bufs[64][40];                                            // per device and size class
     uint64_t clock = 0;
-    size_t entries[64] = {};
+    size_t entries[64] = {}, kept[64] = {};  // per device: kept ones apart
 };
 
 TableCache& cache() {
@@ -87,10 +89,10 @@ TableCache& cache() {
     return *c;
 }
 
-// Soft cap on the resident entries per device: beyond it, a new table first
-// retires the least recently used retirable entry.
+// Soft cap on the resident entries per device that are not kept: beyond it, a
+// new table first retires the least recently used retirable entry.
 constexpr size_t kMaxEntries = 256;
-constexpr size_t kKeptEntries = 128;
+constexpr size_t kKeptEntries = 128, kKeptBytes = 64 * 1024;
 
 thread_local std::vector<TableEntry*> t_pending;  // this thread's lookups since its last enqueue mark
 
@@ -159,7 +161,8 @@ const void* cached_table(const void* host, size_t bytes, hipStream_t stream) {
         return nullptr;
     }
     // Retiring may erase any hash bucket, this one included: look it up again after.
-    if (tc.entries[dev] >= kMaxEntries) retire_one(tc, dev);
+    const bool kept = tc.kept[dev] < kKeptEntries && bytes <= kKeptBytes;
+    if (!kept && tc.entries[dev] >= kMaxEntries) retire_one(tc, dev);
     auto& slot = tc.map[dev][h];
     auto e = std::make_unique<TableEntry>();
     e->bytes.assign(static_cast<const unsigned char*>(host), static_cast<const unsigned char*>(host) + bytes);
@@ -188,14 +191,14 @@ const void* cached_table(const void* host, size_t bytes, hipStream_t stream) {
         return nullptr;
     }
     e->last_use = ++tc.clock;
-    e->kept = tc.entries[dev] < kKeptEntries;
-    if (!e->kept) {
+    e->kept = kept;
+    if (!kept) {
         e->pending = 1;
         t_pending.push_back(e.get());
     }
     void* d = e->dev;
     slot.push_back(std::move(e));
-    ++tc.entries[dev];
+    ++(kept ? tc.kept : tc.entries)[dev];
     return d;
 }
 
