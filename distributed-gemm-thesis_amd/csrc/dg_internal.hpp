@@ -123,6 +123,20 @@ __device__ __forceinline__ uint32_t fdiv(uint32_t n, const FastDiv& f) {
     return (t + ((n - t) >> f.s1)) >> f.s2;
 }
 
+// A launch dimension holds less than 2^32 threads (a launch past that is
+// refused).  Workgroups for `items` threads' work in a kernel that loops over
+// what they leave:
+inline unsigned looped_blocks(int64_t items, int threads) {
+    const int64_t blocks = (items + threads - 1) / threads, most = (((int64_t)1 << 32) - 1) / threads;
+    return (unsigned)std::max<int64_t>(1, std::min(blocks, most));
+}
+// Workgroups of at most 64 threads for `chunks` run chunks (x, spilling into
+// z; at most 2^31) by `cols` column groups:
+inline dim3 run_grid(int64_t chunks, unsigned cols) {
+    const int64_t z = (chunks + (1 << 25) - 1) >> 25;
+    return dim3((unsigned)((chunks + z - 1) / z), cols, (unsigned)z);
+}
+
 // Tile scheduling of the FP64 GEMM launch.
 enum {
     DG_GEMM_MODE_ROUND_ROBIN = 0,  // tile = workgroup id (tiles dealt round-robin over XCDs)

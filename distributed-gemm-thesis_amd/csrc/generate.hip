@@ -91,14 +91,12 @@ static int dg_generate_common(uint64_t seed, int dist, T* ptr, int64_t n, void* 
     int peel = vec ? (int)(((16 - (addr & 15)) & 15) / sizeof(T)) : 0;
     if (peel > n) peel = (int)n;
     const int64_t per = vec ? 16 / sizeof(T) : 1;
-    int64_t blocks = ((n - peel) / per + 255) / 256;
-    if (blocks > (1 << 30)) blocks = 1 << 30;  // beyond that the kernel loops
-    if (blocks < 1) blocks = 1;
+    const dim3 blocks(looped_blocks((n - peel) / per, 256));
     if (vec)
-        hipLaunchKernelGGL((generate_kernel<T, true>), dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), seed,
+        hipLaunchKernelGGL((generate_kernel<T, true>), blocks, dim3(256), 0, as_stream(stream), seed,
                            dist, ptr, n, peel);
     else
-        hipLaunchKernelGGL((generate_kernel<T, false>), dim3((unsigned)blocks), dim3(256), 0, as_stream(stream), seed,
+        hipLaunchKernelGGL((generate_kernel<T, false>), blocks, dim3(256), 0, as_stream(stream), seed,
                            dist, ptr, n, 0);
     DG_LAUNCH_CHECK();
     return DG_OK;

@@ -92,13 +92,6 @@ unsigned col_groups(int64_t cols, int cols_per_wg) {
     return (unsigned)(g < 1 ? 1 : g);
 }
 
-// Workgroups of `chunks` run chunks (x, spilling into z, so that a dimension
-// stays below 2^32 threads) by `cols` column groups.
-dim3 run_grid(int64_t chunks, unsigned cols) {
-    const int64_t z = (chunks + (1 << 25) - 1) >> 25;
-    return dim3((unsigned)((chunks + z - 1) / z), cols, (unsigned)z);
-}
-
 // Whether two addresses and a length in bytes are whole lines.
 bool whole_lines(const void* a, const void* b, int64_t bytes) {
     return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)bytes) & 127) == 0;
@@ -218,14 +211,14 @@ __global__ __launch_bounds__(kThreads) void cyclic_kernel(const double* __restri
     }
 }
 
-// blockIdx.x = chunk of a column, blockIdx.y = column group.
+// blockIdx.x, blockIdx.z = chunk of a column, blockIdx.y = column group.
 template <bool LINES, typename T>
 __global__ __launch_bounds__(kThreads) void copy_block_kernel(int64_t rows, int64_t cols, const T* __restrict__ src,
                                                               int64_t lds, T* __restrict__ dst, int64_t ldd,
                                                               int lanes_log2) {
     constexpr int E = 16 / sizeof(T);
     const int64_t chunk = (int64_t)E << lanes_log2;
-    const int64_t r0 = (int64_t)blockIdx.x * chunk;
+    const int64_t r0 = ((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * chunk;
     const int64_t len = rows - r0 < chunk ? rows - r0 : chunk;
     if (len <= 0) return;
     const int lane = threadIdx.x & ((1 << lanes_log2) - 1);
@@ -235,9 +228,9 @@ __global__ __launch_bounds__(kThreads) void copy_block_kernel(int64_t rows, int6
 }
 
 // C[x] += partial[0*n + x] + partial[1*n + x] + ... in layer order, one pair
-// per thread, the grid covering n.  With n odd every second layer starts off
-// 16-byte alignment, and C may: the pair accesses take any element's
-// alignment.  With n odd (ODD) the layers' loads are plain ones, since a line
+// per thread, the grid covering n (past 2^33 the kernel loops).  With n odd
+// every second layer starts off 16-byte alignment: the pair accesses take any
+// element's alignment.  With n odd (ODD) the layers' loads are plain ones, since a line
 // may then serve two workgroups: 35026003 elements and one layer 121 us, with
 // the nontemporal hint 123 us, single elements 142 us; 3 layers 225, 229 and
 // 225 us.  With n even the hint stays (70052006 elements, one layer: 249 us,
@@ -307,8 +300,10 @@ int block2d(const char* who, const double* src, double* dst, int64_t ldg, int64_
     b.cpre[nrb] = (int32_t)chunks;
     bool lines = whole_lines(src, dst, 8 * ldg);
     for (int i = 1; i <= nrb; ++i) lines = lines && row_off[i] % 16 == 0;
+    const int64_t tallest_chunks = (tallest + rs.chunk - 1) / rs.chunk;
+    lines = lines && (PACK || tallest_chunks <= 1 << 25);  // the band's own order has its chunks on x alone
     dim3 grid = run_grid(chunks, col_groups(cols, rs.cols_per_wg));
-    if (!PACK && lines) grid = dim3((unsigned)((tallest + rs.chunk - 1) / rs.chunk), grid.y, (unsigned)nrb);
+    if (!PACK && lines) grid = dim3((unsigned)tallest_chunks, grid.y, (unsigned)nrb);
     const auto kernel = lines ? block2d_kernel<PACK, true> : block2d_kernel<PACK, false>;
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, as_stream(stream), src, dst, ldg, cols, b, rs.lanes_log2);
     DG_LAUNCH_CHECK();
@@ -430,8 +425,8 @@ int copy_block(const char* name, int64_t rows, int64_t cols, const T* src, int64
     if (rs.chunks > INT32_MAX) return fail(DG_ERR_INVALID, "%s: too many rows", name);
     const bool lines = whole_lines(src, dst, (lds | ldd | rows) * (int64_t)sizeof(T));
     const auto kernel = lines ? copy_block_kernel<true, T> : copy_block_kernel<false, T>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)rs.chunks, col_groups(cols, rs.cols_per_wg)),
-                       dim3(kThreads), 0, as_stream(stream), rows, cols, src, lds, dst, ldd, rs.lanes_log2);
+    hipLaunchKernelGGL(kernel, run_grid(rs.chunks, col_groups(cols, rs.cols_per_wg)), dim3(kThreads), 0,
+                       as_stream(stream), rows, cols, src, lds, dst, ldd, rs.lanes_log2);
     DG_LAUNCH_CHECK();
     return DG_OK;
 }
@@ -459,9 +454,8 @@ int dg_layer_reduce(double* C, const double* partial, int64_t n, int nlayers, vo
         return fail(DG_ERR_INVALID, "dg_layer_reduce: buffers must be 16-byte aligned");
     int rc = require_device();
     if (rc) return rc;
-    int64_t blocks = ((n + 1) / 2 + kThreads - 1) / kThreads;
-    if (blocks > (1 << 30)) blocks = 1 << 30;  // beyond that the kernel loops
-    hipLaunchKernelGGL((n & 1) ? layer_reduce_kernel<true> : layer_reduce_kernel<false>, dim3((unsigned)blocks), dim3(kThreads), 0, as_stream(stream), C, partial, n,
+    hipLaunchKernelGGL((n & 1) ? layer_reduce_kernel<true> : layer_reduce_kernel<false>,
+                       dim3(looped_blocks((n + 1) / 2, kThreads)), dim3(kThreads), 0, as_stream(stream), C, partial, n,
                        nlayers);
     DG_LAUNCH_CHECK();
     return DG_OK;

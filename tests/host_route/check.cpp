@@ -228,12 +228,29 @@ static void check_trials() {
     CHECK(dg::fastest_variant(choices, [&](int, int, float*) { return DG_ERR_HIP; }, &choice, &mode) == DG_ERR_HIP);
 }
 
+// Launch dimensions stay below 2^32 threads and cover the work, or leave the
+// rest to the kernel's loop.
+static void check_grids() {
+    for (int64_t items : {(int64_t)0, (int64_t)1, (int64_t)64, (int64_t)65, ((int64_t)1 << 32) - 1, (int64_t)1 << 32, ((int64_t)1 << 32) + 1, (int64_t)1 << 40})
+        for (int threads : {64, 256}) {
+            const int64_t blocks = dg::looped_blocks(items, threads);
+            CHECK(blocks >= 1 && blocks * threads < (int64_t)1 << 32);
+            CHECK(blocks * threads >= items || (blocks + 1) * threads >= (int64_t)1 << 32);
+        }
+    for (int64_t chunks : {(int64_t)1, (int64_t)1000, (int64_t)1 << 25, ((int64_t)1 << 25) + 1, (int64_t)1 << 26, ((int64_t)1 << 26) + 12345, ((int64_t)1 << 31) - 1}) {
+        const dim3 g = dg::run_grid(chunks, 7);
+        CHECK((int64_t)g.x * 64 < (int64_t)1 << 32 && g.y == 7 && g.z < 65536);
+        CHECK((int64_t)g.x * g.z >= chunks && (int64_t)g.x * (g.z - 1) < chunks);
+    }
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") check_bytes();
     else if (what == "parts") check_parts();
     else if (what == "long") check_long();
     else if (what == "trials") check_trials();
+    else if (what == "grids") check_grids();
     else { std::fprintf(stderr, "unknown check '%s'\n", what.c_str()); return 2; }
     if (!failures) std::printf("%s: ok\n", what.c_str());
     return failures ? 1 : 0;

@@ -1,7 +1,7 @@
 """The GEMMs' host-side routing on the CPU: tests/host_route/check.cpp, built
-against libdgamd.so, looks at the lists that prepare_gemm makes of a batch,
-and tests/host_route/staged.cpp at the addresses of csrc/staged.hpp, compiled
-for the host.  No GPU call is made."""
+against libdgamd.so, looks at the lists that prepare_gemm makes of a batch
+and at launch sizes, and tests/host_route/staged.cpp at the addresses of
+csrc/staged.hpp, compiled for the host.  No GPU call is made."""
 import os
 import shutil
 import subprocess
@@ -59,6 +59,12 @@ def test_first_use_times_distinct_choices(check):
     """An autotuned plan's first use times each distinct tile choice, and
     what is clearly slower only once."""
     check("trials")
+
+
+def test_launch_dimensions(check):
+    """The grids of the copies, the layer reduction and the generator stay
+    below 2^32 threads a dimension at any size."""
+    check("grids")
 
 
 def test_staged_addresses(tmp_path):
