@@ -154,6 +154,10 @@ enum {
     DG_GEMM_TILE_32x32 = 4,          // register-staged kernel
     DG_GEMM_TILES = 5,
 };
+// The choice that DG_GEMM_TILE forces, FP32 included: "direct", "128x128",
+// "128x128whole", "64x64" or "32x32"; DG_GEMM_TILE_AUTO when it is unset or
+// anything else.
+int forced_tile();
 
 // Launches the FP64 MFMA GEMM over `probs` (host vector; uploaded through
 // the table cache).  All problems share opA/opB.

@@ -50,7 +50,6 @@
 // gets one zero step.
 #include <algorithm>
 #include <cstdlib>
-#include <string>
 
 #include "dg_internal.hpp"
 #include "staged.hpp"
@@ -831,10 +830,10 @@ constexpr double kEff64[6] = {0.87, 0.89, 0.90, 0.91, 0.945, 0.915}, kEff32[6] =
 // on 64x64 or 32x32 tiles is less: 128x128 tiles leave CUs idle until there
 // are a few hundred of them.  Every kernel sums an element in the same order:
 // neither the cut nor the tile changes a result bit.  DG_GEMM_TILE forces a
-// choice.
+// choice (both 128x128 ones are the direct-to-LDS kernels here).
 template <bool AK, bool BKC>
 void run_sgemm(const SgemmArgs& a, bool dma, hipStream_t st) {
-    static const std::string forced = [] { const char* e = getenv("DG_GEMM_TILE"); return std::string(e ? e : ""); }();
+    const int forced = forced_tile();
     static const bool no_areg = getenv("DG_GEMM_NO_AREG") != nullptr;
     auto direct = [&](SgemmArgs p) {
         p.tiles_m = (int)((p.m + sk::BM - 1) / sk::BM);
@@ -847,18 +846,19 @@ void run_sgemm(const SgemmArgs& a, bool dma, hipStream_t st) {
     auto time64 = [&](int64_t m, int64_t n) { return sgemm_time(m, n, a.k, 64, 4, kEff64, el64); };
     auto time32 = [&](int64_t m, int64_t n) { return sgemm_time(m, n, a.k, 32, 4, kEff32, el32); };
     auto staged = [&](const SgemmArgs& p) {
-        const bool small = forced == "32x32" || (forced != "64x64" && time32(p.m, p.n) < time64(p.m, p.n));
+        const bool small = forced == DG_GEMM_TILE_32x32 || (forced != DG_GEMM_TILE_64x64 && time32(p.m, p.n) < time64(p.m, p.n));
         if (small) launch_sgemm<Sgemm32, AK, BKC>(p, st); else launch_sgemm<Sgemm64, AK, BKC>(p, st);
     };
     const int64_t mi = a.m / sk::BM * sk::BM, ni = a.n / sk::BN * sk::BN;
     const bool k_ok = a.k % sk::BK == 0 && !((a.k / sk::BK) & 1);
     const bool cut = (AK || BKC) && !no_areg && k_ok && (mi != a.m || ni != a.n) && mi * ni >= 8 * sk::BM * sk::BN;
-    if (dma && forced != "direct" && forced != "128x128") {
+    if (forced == DG_GEMM_TILE_64x64 || forced == DG_GEMM_TILE_32x32) dma = false;
+    if (dma && forced == DG_GEMM_TILE_AUTO) {
         auto least = [&](int64_t m, int64_t n) { return std::min(time64(m, n), time32(m, n)); };
         double t = sgemm_time(cut ? mi : a.m, cut ? ni : a.n, a.k, 128, 2, kEffDma[AK || BKC], false);
         if (cut && mi < a.m) t += least(a.m - mi, a.n);
         if (cut && ni < a.n) t += least(mi, a.n - ni);
-        dma = forced.empty() && t <= least(a.m, a.n);
+        dma = t <= least(a.m, a.n);
     }
     if (!dma) return staged(a);
     if (!cut) return direct(a);

@@ -1286,23 +1286,25 @@ static void build_lists(bool ak, bool bkc, const std::vector<Prob>& probs, const
     for (int w = 0; w < 3; ++w) out.tiles_gen[w] = (int)tiles[kListGen + w];
 }
 
+int forced_tile() {
+    static const int forced = [] {
+        const char* const names[DG_GEMM_TILES] = {"direct", "128x128", "128x128whole", "64x64", "32x32"};
+        const char* e = getenv("DG_GEMM_TILE");
+        for (int t = 0; e && t < DG_GEMM_TILES; ++t)
+            if (!strcmp(e, names[t])) return t;
+        return (int)DG_GEMM_TILE_AUTO;
+    }();
+    return forced;
+}
+
 // The batch is looked at once and built once: the choices are compared by
 // their estimates.  SUMMA, both operands transposed, 8192^3 in blocks of 64
 // (2.1 million segments): 13 ms of host time, 290 with a build per choice.
 int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector<Seg> segs, GemmBatch& out,
                  bool split_edges, int tile) {
-    // DG_GEMM_TILE forces a shape; DG_GEMM_NO_DMA keeps everything on the register-staged kernel
-    static const int forced = [] {
-        const char* e = getenv("DG_GEMM_TILE");
-        const std::string v = e ? e : "";
-        if (v == "direct") return (int)DG_GEMM_TILE_DIRECT;
-        if (v == "128x128") return (int)DG_GEMM_TILE_128x128;
-        if (v == "64x64") return (int)DG_GEMM_TILE_64x64;
-        if (v == "32x32") return (int)DG_GEMM_TILE_32x32;
-        return (int)DG_GEMM_TILE_AUTO;
-    }();
+    // DG_GEMM_NO_DMA keeps everything on the register-staged kernel
     static const bool no_dma = getenv("DG_GEMM_NO_DMA") != nullptr;
-    if (forced != DG_GEMM_TILE_AUTO) tile = forced;
+    if (forced_tile() != DG_GEMM_TILE_AUTO) tile = forced_tile();
     if (no_dma && tile == DG_GEMM_TILE_DIRECT) tile = DG_GEMM_TILE_128x128;
     const bool ak = opA == 'T', bkc = opB != 'T';  // k-contiguous operands
     std::vector<Route> routes;

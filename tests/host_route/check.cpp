@@ -244,6 +244,19 @@ static void check_grids() {
     }
 }
 
+// The lists of one FP64 problem under DG_GEMM_TILE: sizes of the five.
+static void print_lists(char** v) {
+    const char oa = v[0][0], ob = v[1][0];
+    int64_t x[7];
+    for (int i = 0; i < 7; ++i) x[i] = std::atoll(v[2 + i]);  // m n k lda ldb, elements off a 16-byte boundary of A and B
+    std::vector<Seg> segs{Seg{at(0x10000) + x[5], at(0x20000) + x[6], x[3], x[4], x[2]}};
+    Prob p{};
+    p.m = x[0]; p.n = x[1]; p.ldc = x[0]; p.c = at(0x30000); p.alpha = 1.0; p.nseg = 1;
+    dg::GemmBatch b;
+    CHECK(dg::prepare_gemm(oa, ob, {p}, segs, b) == DG_OK);
+    std::printf("%zu %zu %zu %zu %zu\n", b.dma.size(), b.dmae.size(), b.gen[0].size(), b.gen[1].size(), b.gen[2].size());
+}
+
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "bytes") check_bytes();
@@ -251,6 +264,8 @@ int main(int argc, char** argv) {
     else if (what == "long") check_long();
     else if (what == "trials") check_trials();
     else if (what == "grids") check_grids();
+    else if (what == "forced") std::printf("%d\n", dg::forced_tile());
+    else if (what == "lists" && argc == 11) print_lists(argv + 2);
     else { std::fprintf(stderr, "unknown check '%s'\n", what.c_str()); return 2; }
     if (!failures) std::printf("%s: ok\n", what.c_str());
     return failures ? 1 : 0;

@@ -26,11 +26,12 @@ def check(tmp_path_factory):
     b = subprocess.run(cmd, capture_output=True, text=True, timeout=300)
     assert b.returncode == 0, b.stderr[-3000:]
 
-    def run(what):
+    def run(what, *args, **extra):
         env = {k: v for k, v in os.environ.items() if not k.startswith("DG_GEMM_")}
-        r = subprocess.run([exe, what], capture_output=True, text=True, timeout=300, env=env)
+        r = subprocess.run([exe, what, *map(str, args)], capture_output=True, text=True, timeout=300, env=dict(env, **extra))
         assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-3000:])
         assert what + ": ok" in r.stdout
+        return r.stdout.split()
     return run
 
 
@@ -65,6 +66,14 @@ def test_launch_dimensions(check):
     """The grids of the copies, the layer reduction and the generator stay
     below 2^32 threads a dimension at any size."""
     check("grids")
+
+
+@pytest.mark.parametrize("value,choice", [(None, -1), ("direct", 0), ("128x128", 1), ("128x128whole", 2), ("64x64", 3),
+                                          ("32x32", 4), ("256x128", -1), ("64", -1), ("", -1)])
+def test_forced_choice(check, value, choice):
+    """DG_GEMM_TILE: every choice by its name; anything else forces nothing,
+    in FP64 and in FP32."""
+    assert check("forced", **({} if value is None else {"DG_GEMM_TILE": value}))[0] == str(choice)
 
 
 def test_staged_addresses(tmp_path):
