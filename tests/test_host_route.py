@@ -89,3 +89,13 @@ def test_staged_addresses(tmp_path):
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0, (r.stdout[-2000:], r.stderr[-3000:])
     assert "staged: ok" in r.stdout
+
+
+def test_forced_shapes_reach_their_kernels(check):
+    """The FP64 shapes of the forced-kernel GPU test fall on the lists that
+    they stand for under the direct choice."""
+    from test_gpu_forced_kernels import EXPECT, SHAPES, geometry
+    for oa, ob, m, n, k, off_a, off_b, kind in SHAPES:
+        (_, _, lda), (_, _, ldb), _ = geometry(oa, ob, m, n, k, 2)
+        x = [int(v) for v in check("lists", oa, ob, m, n, k, lda, ldb, off_a, off_b, DG_GEMM_TILE="direct")[:5]]
+        assert EXPECT[kind](x[0], x[1], sum(x[2:])), (oa, ob, m, n, k, off_a, off_b, kind, x)
