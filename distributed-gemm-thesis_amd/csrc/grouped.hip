@@ -625,7 +625,7 @@ int dg_grouped_dgemm_noalloc(const dg_gemm_desc* descs, int count, void* stream)
         return fail(DG_ERR_WORKSPACE,
                     "dg_grouped_dgemm_noalloc: the batch's descriptor tables need %zu bytes, more than the %zu-byte "
                     "scratch array (about %zu problems of one segment each)",
-                    total, kScratchBytes, kScratchBytes / (2 * sizeof(Prob) + sizeof(Seg)));
+                    total, kScratchBytes, kScratchBytes / (sizeof(Prob) + sizeof(Seg)));
     rc = scale_only(descs, count, st);
     if (rc) return rc;
     if (pieces.empty()) return DG_OK;

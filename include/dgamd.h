@@ -256,7 +256,7 @@ int dg_grouped_dgemm(const dg_gemm_desc* descs, int count, void* stream);
  * into the library's static device scratch array (256 KiB per GPU, held
  * until the process ends) instead of the table cache, written by kernels
  * whose arguments carry them, so the call also records cleanly into a HIP
- * graph.  A batch whose tables exceed the array (about 1900 single-segment
+ * graph.  A batch whose tables exceed the array (about 2500 single-segment
  * problems) fails with DG_ERR_WORKSPACE before any launch.  Calls that
  * overlap on one GPU share the array and race.  No counterpart in the
  * reference: for callers that cannot allocate device memory (graph capture,
