@@ -1064,6 +1064,7 @@ int launch_scale(int64_t m, int64_t n, double beta, double* C, int64_t ldc, hipS
 // What the routing needs to know of a problem, from one pass over its segments.
 struct Route {
     int64_t depth = 0;      // k of all segments
+    int64_t staged[3];      // of several: k of the register-staged tiles' stages, each segment's last one whole
     bool direct = true;     // the direct-to-LDS kernels take it; then
     int sa = 0, sb = 0;     // whether its A (B) starts 8 bytes past a 16-byte boundary (k-contiguous: -1), and
     bool k_ok = false;      // its k is an even number of whole k-steps
@@ -1083,6 +1084,8 @@ static Route route_of(const Prob& p, const std::vector<Seg>& segs, bool ak, bool
     Route r;
     uintptr_t bits = 0;
     int64_t lda = 1, ldb = 1;  // the longest
+    int64_t s16 = 0, s32 = 0;  // stages 16 and 32 deep
+    static_assert(Cfg128::BK == 16 && Cfg64::BK == 16 && Cfg32::BK == 32, "stages counted below");
     int off_a = -1, off_b = -1;  // byte offset within 16 of a row-contiguous A / B
     int64_t steps = 0;
     bool whole = true;  // every segment a whole number of k-steps
@@ -1090,6 +1093,8 @@ static Route route_of(const Prob& p, const std::vector<Seg>& segs, bool ak, bool
         const Seg& g = segs[s];
         r.depth += g.klen;
         steps += (g.klen + dmak::DBK - 1) / dmak::DBK;
+        s16 += (g.klen + 15) / 16;
+        s32 += (g.klen + 31) / 32;
         if (g.klen % dmak::DBK) whole = false;
         bits |= reinterpret_cast<uintptr_t>(g.a) | reinterpret_cast<uintptr_t>(g.b);
         lda = std::max(lda, g.lda);
@@ -1104,6 +1109,8 @@ static Route route_of(const Prob& p, const std::vector<Seg>& segs, bool ak, bool
     r.sa = ak ? -1 : off_a == 8;
     r.sb = bkc ? -1 : off_b == 8;
     r.k_ok = whole && !(steps & 1);
+    r.staged[0] = r.staged[1] = p.nseg > 1 ? 16 * s16 : r.depth;
+    r.staged[2] = p.nseg > 1 ? 32 * s32 : r.depth;
     r.elements[0] = !takes<Cfg128>(ak, bkc, bits, lda, ldb);
     r.elements[1] = !takes<Cfg64>(ak, bkc, bits, lda, ldb);
     r.elements[2] = !takes<Cfg32>(ak, bkc, bits, lda, ldb);
@@ -1118,7 +1125,8 @@ static_assert(dmak::DBM == dmak::DBN, "one edge per list");
 
 // Time (us) of one list's launch, to choose between the tiles: the fullest
 // CU's c tiles at the rate that so many reach, share of 78.6 TFLOP/s, plus
-// `round` us of prologue and epilogue per round of `conc` resident tiles.
+// `round` us of prologue and epilogue, and `seg` us per segment after a tile's
+// first, per round of `conc` resident tiles.
 // Measured: A in registers 0.91 with one tile per CU, 0.95 with more (both
 // operands in LDS 0.85, 0.93); register-staged 128x128 0.95 with one, 0.965 up
 // to 15 (4096^3: 1812 us against 1838 with A in registers), then less, 0.89
@@ -1129,24 +1137,30 @@ static_assert(dmak::DBM == dmak::DBN, "one edge per list");
 // elements: kElementRate of these (TN 500 x 4096 x 4096 with 2^22 + 2 rows to a
 // column, 64x64 tiles: 403 us, 257 with whole runs; NN 4096 x 4096 x 480, odd:
 // 319 us against 251).
+// A register-staged kernel leaves its steady turns at every segment's end,
+// the direct-to-LDS kernels do not: SUMMA 2048^3 on 2 x 2 in panels of 512, 128,
+// 64 and 16: direct 251, 255, 259 and 287 us, 128x128 243, 260, 282 and 380,
+// 64x64 245, 255, 267 and 320, 32x32 297, 315, 346 and 963 (its stages are 32
+// deep).
 constexpr double kElementRate = 0.65;
 struct Rate {
     int conc;
-    double round;
+    double round, seg;
     struct { int64_t from; double eff; } at[5];  // ascending; the last whose `from` c reaches
 };
-constexpr Rate kRate[kLists] = {{2, 4, {{1, 0.91}, {2, 0.95}}},
-                                {2, 4, {{1, 0.85}, {2, 0.93}}},
-                                {2, 8, {{1, 0.95}, {2, 0.965}, {16, 0.93}, {32, 0.89}}},
-                                {4, 4, {{1, 0.92}, {5, 0.91}, {25, 0.88}, {64, 0.85}}},
-                                {4, 4, {{1, 0.67}, {2, 0.72}, {3, 0.76}, {4, 0.78}, {5, 0.80}}}};
+constexpr Rate kRate[kLists] = {{2, 4, 0.25, {{1, 0.91}, {2, 0.95}}},
+                                {2, 4, 0.25, {{1, 0.85}, {2, 0.93}}},
+                                {2, 8, 1.2, {{1, 0.95}, {2, 0.965}, {16, 0.93}, {32, 0.89}}},
+                                {4, 4, 0.6, {{1, 0.92}, {5, 0.91}, {25, 0.88}, {64, 0.85}}},
+                                {4, 4, 0.4, {{1, 0.67}, {2, 0.72}, {3, 0.76}, {4, 0.78}, {5, 0.80}}}};
 
 struct ListCost {
-    int64_t tiles = 0;
+    int64_t tiles = 0, seams = 0;  // seams: segments after a tile's first, of all tiles
     double sum = 0, most = 0, least = 1e300;  // us of CU time: all tiles, the longest, the shortest
-    void add(int64_t n, int64_t area, int64_t k, bool elements) {
+    void add(int64_t n, int64_t area, int64_t k, int nseg, bool elements) {
         const double u = 2.0 * (double)area * (double)k / (78.6e6 / 256) / (elements ? kElementRate : 1.0);
         tiles += n;
+        seams += n * (nseg - 1);
         sum += (double)n * u;
         most = std::max(most, u);
         least = std::min(least, u);
@@ -1158,7 +1172,7 @@ struct ListCost {
         for (const auto& x : r.at)
             if (x.from > 0 && x.from <= c) eff = x.eff;
         const double load = most == least ? (double)c * most : std::max(sum / 256 + most / 2, most);
-        return load / eff + r.round * std::max(1.0, (double)c / r.conc);
+        return load / eff + (r.round + r.seg * (double)seams / (double)tiles) * std::max(1.0, (double)c / r.conc);
     }
 };
 
@@ -1236,7 +1250,8 @@ static Estimate estimate(const std::vector<Prob>& probs, const std::vector<Route
         if (p.m <= 0 || p.n <= 0 || p.nseg <= 0) continue;
         split_problem(p, r, tile, split_edges, [&](int list, int64_t r0, int64_t nr, int64_t c0, int64_t nc) {
             const int shift = shift_of(r, list, r0, c0);
-            cost[list].add(tiles_of(list, shift, nr, nc), kTileOf[list] * kTileOf[list], r.depth, shift & kByElements);
+            cost[list].add(tiles_of(list, shift, nr, nc), kTileOf[list] * kTileOf[list],
+                           list < kListGen ? r.depth : r.staged[list - kListGen], p.nseg, shift & kByElements);
             if (nr < p.m || nc < p.n) x.segs += p.nseg;
         });
     }

@@ -182,6 +182,32 @@ static void check_long() {
     }
 }
 
+// Short segments: the direct-to-LDS kernels, which run through them, keep the
+// products whose register-staged tiles would start anew every few stages.
+static void check_short() {
+    struct { int64_t M; int nb, direct; } cases[] = {{2048, 16, 1}, {2048, 32, 1}, {2048, 64, 1}, {2048, 512, 0},
+                                                     {4096, 16, 1}, {4096, 64, 1}, {4096, 512, 0}, {1024, 64, 0}};
+    for (const auto& c : cases) {  // SUMMA of M^3 on 2 x 2 in panels of nb
+        std::vector<Prob> probs;
+        std::vector<Seg> segs;
+        for (int r = 0; r < 4; ++r) {
+            Prob p{};
+            p.m = p.n = p.ldc = c.M / 2;
+            p.c = at(0x100000000); p.alpha = 1.0;
+            p.seg0 = (int32_t)segs.size();
+            p.nseg = (int32_t)(c.M / c.nb);
+            for (int s = 0; s < p.nseg; ++s) segs.push_back(Seg{at(0x200000000), at(0x300000000), c.M / 2, c.M / 2, c.nb});
+            probs.push_back(p);
+        }
+        dg::GemmBatch b;
+        CHECK(dg::prepare_gemm('N', 'N', probs, segs, b) == DG_OK);
+        CHECK(b.dma.empty() == !c.direct);
+        // half-empty stages of the 32x32 tiles are no bargain
+        if (c.nb == 16) CHECK(b.gen[2].empty());
+        if (failures) { std::fprintf(stderr, "%lld in panels of %d\n", (long long)c.M, c.nb); return; }
+    }
+}
+
 // An autotuned plan's first use: choices that come out alike are timed once,
 // and slow variants once.
 static void check_trials() {
@@ -262,6 +288,7 @@ int main(int argc, char** argv) {
     if (what == "bytes") check_bytes();
     else if (what == "parts") check_parts();
     else if (what == "long") check_long();
+    else if (what == "short") check_short();
     else if (what == "trials") check_trials();
     else if (what == "grids") check_grids();
     else if (what == "forced") std::printf("%d\n", dg::forced_tile());

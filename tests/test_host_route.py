@@ -56,6 +56,12 @@ def test_long_columns(check):
     check("long")
 
 
+def test_short_segments(check):
+    """The choice between the kernels knows what a segment's end costs each:
+    SUMMA in panels of 16 to 64 stays on the direct-to-LDS kernels."""
+    check("short")
+
+
 def test_first_use_times_distinct_choices(check):
     """An autotuned plan's first use times each distinct tile choice, and
     what is clearly slower only once."""
