@@ -1120,8 +1120,8 @@ static Route route_of(const Prob& p, const std::vector<Seg>& segs, bool ak, bool
 // Lists of a batch: A in registers, edge-handling direct-to-LDS, then the
 // register-staged kernel's three tile edges.
 enum { kListAreg, kListEdge, kListGen, kLists = kListGen + 3 };
-constexpr int64_t kTileOf[kLists] = {dmak::DBM, dmak::DBM, Cfg128::BM, Cfg64::BM, Cfg32::BM};
-static_assert(dmak::DBM == dmak::DBN, "one edge per list");
+constexpr int kTileLog2[kLists] = {7, 7, 7, 6, 5};  // of their tiles' edges
+static_assert(dmak::DBM == 128 && dmak::DBN == 128 && Cfg128::BM == 128 && Cfg64::BM == 64 && Cfg32::BM == 32, "kTileLog2");
 
 // Time (us) of one list's launch, to choose between the tiles: the fullest
 // CU's c tiles at the rate that so many reach, share of 78.6 TFLOP/s, plus
@@ -1156,23 +1156,24 @@ constexpr Rate kRate[kLists] = {{2, 4, 0.25, {{1, 0.91}, {2, 0.95}}},
 
 struct ListCost {
     int64_t tiles = 0, seams = 0;  // seams: segments after a tile's first, of all tiles
-    double sum = 0, most = 0, least = 1e300;  // us of CU time: all tiles, the longest, the shortest
-    void add(int64_t n, int64_t area, int64_t k, int nseg, bool elements) {
-        const double u = 2.0 * (double)area * (double)k / (78.6e6 / 256) / (elements ? kElementRate : 1.0);
+    double sum = 0, most = 0, least = 1e300;  // k of all tiles, the longest, the shortest
+    void add(int64_t n, int64_t k, int nseg, bool elements) {
+        const double x = elements ? (double)k * (1.0 / kElementRate) : (double)k;
         tiles += n;
         seams += n * (nseg - 1);
-        sum += (double)n * u;
-        most = std::max(most, u);
-        least = std::min(least, u);
+        sum += (double)n * x;
+        most = std::max(most, x);
+        least = std::min(least, x);
     }
-    double time(const Rate& r) const {
+    double time(const Rate& r, int64_t edge) const {
         if (!tiles) return 0;
         const int64_t c = (tiles + 255) / 256;
         double eff = 0;
         for (const auto& x : r.at)
             if (x.from > 0 && x.from <= c) eff = x.eff;
         const double load = most == least ? (double)c * most : std::max(sum / 256 + most / 2, most);
-        return load / eff + (r.round + r.seg * (double)seams / (double)tiles) * std::max(1.0, (double)c / r.conc);
+        const double us = 2.0 * (double)(edge * edge) / (78.6e6 / 256);  // per k of a tile
+        return load * us / eff + (r.round + r.seg * (double)seams / (double)tiles) * std::max(1.0, (double)c / r.conc);
     }
 };
 
@@ -1228,15 +1229,17 @@ static int shift_of(const Route& r, int list, int64_t r0, int64_t c0) {
     return (r.sa >= 0 ? (int)((r.sa + r0) & 1) : 0) | (r.sb >= 0 ? (int)((r.sb + c0) & 1) : 0) << 1;
 }
 static int64_t tiles_of(int list, int shift, int64_t nr, int64_t nc) {
-    const int64_t e = kTileOf[list];
+    const int e = kTileLog2[list], round = (1 << e) - 1;
     const int sa = list < kListGen ? shift & 1 : 0, sb = list < kListGen ? (shift >> 1) & 1 : 0;
-    return ((nr + sa + e - 1) / e) * ((nc + sb + e - 1) / e);
+    return ((nr + sa + round) >> e) * ((nc + sb + round) >> e);
 }
 
 // One tile choice of a batch: the estimated time (us) of its launches, the
-// segments that cut parts add, and whether it fits one launch per list.
+// problems of each list, the segments that cut parts add, and whether it fits
+// one launch per list.
 struct Estimate {
     double time = 0;
+    size_t probs[kLists] = {};
     int64_t segs = 0;
     bool fits = true;
 };
@@ -1250,13 +1253,14 @@ static Estimate estimate(const std::vector<Prob>& probs, const std::vector<Route
         if (p.m <= 0 || p.n <= 0 || p.nseg <= 0) continue;
         split_problem(p, r, tile, split_edges, [&](int list, int64_t r0, int64_t nr, int64_t c0, int64_t nc) {
             const int shift = shift_of(r, list, r0, c0);
-            cost[list].add(tiles_of(list, shift, nr, nc), kTileOf[list] * kTileOf[list],
-                           list < kListGen ? r.depth : r.staged[list - kListGen], p.nseg, shift & kByElements);
+            cost[list].add(tiles_of(list, shift, nr, nc), list < kListGen ? r.depth : r.staged[list - kListGen], p.nseg,
+                           shift & kByElements);
+            ++x.probs[list];
             if (nr < p.m || nc < p.n) x.segs += p.nseg;
         });
     }
     for (int l = 0; l < kLists; ++l) {
-        x.time += cost[l].time(kRate[l]);
+        x.time += cost[l].time(kRate[l], (int64_t)1 << kTileLog2[l]);
         x.fits = x.fits && cost[l].tiles <= INT32_MAX;
     }
     x.fits = x.fits && (int64_t)nsegs + x.segs <= INT32_MAX;
@@ -1266,11 +1270,12 @@ static Estimate estimate(const std::vector<Prob>& probs, const std::vector<Route
 // Fills the lists of one tile choice.  A part of a problem becomes a problem
 // of its own, its segments re-based and appended.
 static void build_lists(bool ak, bool bkc, const std::vector<Prob>& probs, const std::vector<Route>& routes,
-                        std::vector<Seg>&& segs, int tile, bool split_edges, int64_t extra, GemmBatch& out) {
+                        std::vector<Seg>&& segs, int tile, bool split_edges, const Estimate& size, GemmBatch& out) {
     out = GemmBatch{};
     out.segs = std::move(segs);
-    if (extra) out.segs.reserve(out.segs.size() + (size_t)extra);
+    if (size.segs) out.segs.reserve(out.segs.size() + (size_t)size.segs);
     std::vector<Prob>* lists[kLists] = {&out.dma, &out.dmae, &out.gen[0], &out.gen[1], &out.gen[2]};
+    for (int l = 0; l < kLists; ++l) lists[l]->reserve(size.probs[l]);
     int64_t tiles[kLists] = {};
     for (size_t i = 0; i < probs.size(); ++i) {
         const Prob& p = probs[i];
@@ -1324,21 +1329,30 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector
     const bool ak = opA == 'T', bkc = opB != 'T';  // k-contiguous operands
     std::vector<Route> routes;
     routes.reserve(probs.size());
-    for (const Prob& p : probs) routes.push_back(route_of(p, segs, ak, bkc));
+    bool direct = false;
+    for (const Prob& p : probs) {
+        routes.push_back(route_of(p, segs, ak, bkc));
+        direct = direct || routes.back().direct;
+    }
     const bool any = tile == DG_GEMM_TILE_AUTO;
     Estimate best;
     best.fits = false;
-    const int first = !any ? tile : no_dma ? (int)DG_GEMM_TILE_128x128 : (int)DG_GEMM_TILE_DIRECT;
+    // without a problem for the direct-to-LDS kernels that choice is 128x128,
+    // and without one to cut the uncut choice is
+    const int first = !any ? tile : no_dma || !direct ? (int)DG_GEMM_TILE_128x128 : (int)DG_GEMM_TILE_DIRECT;
     const int end = any ? (int)DG_GEMM_TILES : tile + 1;
+    bool cuts = true;
     for (int c = first; c < end; ++c) {
+        if (any && c == DG_GEMM_TILE_128x128_WHOLE && !cuts) continue;
         const Estimate x = estimate(probs, routes, segs.size(), c, split_edges);
+        if (c == DG_GEMM_TILE_128x128) cuts = x.segs > 0;
         if (x.fits && (!best.fits || x.time < best.time)) {
             best = x;
             tile = c;
         }
     }
     if (!best.fits) return fail(DG_ERR_INVALID, "gemm: output tiles exceed one launch");
-    build_lists(ak, bkc, probs, routes, std::move(segs), tile, split_edges, best.segs, out);
+    build_lists(ak, bkc, probs, routes, std::move(segs), tile, split_edges, best, out);
     return DG_OK;
 }
 

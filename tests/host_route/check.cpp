@@ -55,6 +55,21 @@ static void check_bytes() {
         std::printf("prepared %zu bytes of tables with %zu bytes\n", tables, spent);
         CHECK(spent <= tables + tables / 2);
     }
+    // many problems of one segment: their lists are made in their final size
+    segs.assign(1000, Seg{at(0x200000000), at(0x300000000), 33, 17, 17});
+    probs.resize(1000);
+    for (int i = 0; i < 1000; ++i) {
+        probs[i].m = probs[i].ldc = 33;
+        probs[i].n = 65;
+        probs[i].seg0 = i;
+        probs[i].nseg = 1;
+    }
+    dg::GemmBatch b;
+    const size_t before = allocated;
+    CHECK(dg::prepare_gemm('N', 'N', probs, segs, b) == DG_OK);
+    const size_t spent = allocated - before, tables = segs.size() * sizeof(Seg) + probs.size() * sizeof(Prob);
+    std::printf("prepared %zu bytes of tables with %zu bytes\n", tables, spent);
+    CHECK(spent <= 2 * tables);
 }
 
 // Every choice covers each element of each problem once, each part at the
