@@ -683,17 +683,6 @@ __device__ __forceinline__ const int8_t* group_step(const int8_t* first, int64_t
     return first + (int64_t)p * stride + (int64_t)(sc - p * nks.d) * CK2;
 }
 
-// acc[i][j][v] = sum at (m0 + 16i + v, n0 + 16j): one 16-byte store each.
-template <class ACC, int M, int N>
-__device__ __forceinline__ void store_plane(const ACC (&acc)[M][N], int32_t* out, int64_t Mp, int64_t m0, int64_t n0) {
-#pragma unroll
-    for (int j = 0; j < N; ++j)
-#pragma unroll
-        for (int i = 0; i < M; ++i)
-            __builtin_nontemporal_store(__builtin_bit_cast(iv4, acc[i][j]),
-                                        reinterpret_cast<iv4*>(out + (n0 + 16 * j) * Mp + m0 + 16 * i));
-}
-
 template <bool BF16>
 __global__ __launch_bounds__(CNT, OCC) void oz_plane_kernel(OzPlaneArgs g) {
     typedef typename std::conditional<BF16, fv4, iv4>::type acc_t;
@@ -765,7 +754,22 @@ __global__ __launch_bounds__(CNT, OCC) void oz_plane_kernel(OzPlaneArgs g) {
         crt_half(acc, fa, nb, fb, lds + asl1 * CSLOT + wm * CK2 + roff0, lds + bsl1 * CSLOT + wn * CK2 + roff0);
     }
     wait_vmcnt<0>();
-    store_plane(acc, g.planes + (int64_t)gr.plane * g.plane, g.Mp, m0 + wm + 4 * lg, n0 + wn + lr);
+    // acc[i][j][v] = sum at (m0 + wm + 16i + 4lg + v, n0 + wn + 16j + lr): one
+    // 16-byte store each.  Written out here on purpose: the same loop in a
+    // function of its own comes out with its column addresses and stores in
+    // another order, and products of short K, which are bound by these stores,
+    // take 7 % longer (8192 x 8192 x 64 with 8 slices: 750 us against 653 for this
+    // kernel, 1205 against 1126 a call).
+    int32_t* out = g.planes + (int64_t)gr.plane * g.plane;
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const int64_t n = n0 + wn + 16 * j + lr;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int64_t m = m0 + wm + 16 * i + 4 * lg;
+            __builtin_nontemporal_store(__builtin_bit_cast(iv4, acc[i][j]), reinterpret_cast<iv4*>(out + n * g.Mp + m));
+        }
+    }
 }
 
 // oz_plane_kernel on 128 x 128 tiles.
@@ -792,7 +796,14 @@ __global__ __launch_bounds__(SCNT, 2) void oz_plane_small_kernel(OzPlaneArgs g) 
     small_product(
         acc, lds, [&](uint32_t s) { return group_step(ga, g.a_slice, s, last, gr.nks); },
         [&](uint32_t s) { return group_step(gb, -g.b_slice, s, last, gr.nks); }, last, g.rb, wave, lane, wm, wn);
-    store_plane(acc, g.planes + (int64_t)gr.plane * g.plane, g.Mp, m0 + wm + 4 * (lane >> 4), n0 + wn + (lane & 15));
+    int32_t* out = g.planes + (int64_t)gr.plane * g.plane + m0 + wm + 4 * (lane >> 4);
+    n0 += wn + (lane & 15);
+#pragma unroll
+    for (int j = 0; j < SFN; ++j)
+#pragma unroll
+        for (int i = 0; i < SFM; ++i)
+            __builtin_nontemporal_store(__builtin_bit_cast(iv4, acc[i][j]),
+                                        reinterpret_cast<iv4*>(out + (n0 + 16 * j) * g.Mp + 16 * i));
 }
 
 // C = val + beta C on up to four rows of a column (`left` of them in C), in
