@@ -230,11 +230,10 @@ __global__ __launch_bounds__(kThreads) void copy_block_kernel(int64_t rows, int6
 // C[x] += partial[0*n + x] + partial[1*n + x] + ... in layer order, one pair
 // per thread, the grid covering n (past 2^33 the kernel loops).  With n odd
 // every second layer starts off 16-byte alignment: the pair accesses take any
-// element's alignment.  With n odd (ODD) the layers' loads are plain ones, since a line
-// may then serve two workgroups: 35026003 elements and one layer 121 us, with
-// the nontemporal hint 123 us, single elements 142 us; 3 layers 225, 229 and
-// 225 us.  With n even the hint stays (70052006 elements, one layer: 249 us,
-// without 253 us).
+// element's alignment, and the layers' loads (ODD) are plain ones, since a line
+// may then serve two workgroups: 35026003 elements and one layer 119 us, with
+// the nontemporal hint 125 us.  With n even the hint stays (70052006 elements,
+// one layer: 249 us, without 253 us).
 template <bool ODD>
 __global__ __launch_bounds__(kThreads) void layer_reduce_kernel(double* __restrict__ C,
                                                                 const double* __restrict__ partial, int64_t n,
@@ -261,6 +260,25 @@ __global__ __launch_bounds__(kThreads) void layer_reduce_kernel(double* __restri
         }
     }
 }
+
+// The same with one element per thread.  Up to three odd layers that do not
+// stay in the caches run faster so, by all loads being nontemporal: 70000001
+// elements and 1, 2, 3 or 4 layers 243, 345, 446 and 555 us, in pairs 256, 357,
+// 457 and 555; 20000001 elements 72, 101, 130 and 160, in pairs 69, 95, 128 and
+// 157.
+__global__ __launch_bounds__(kThreads) void layer_reduce_single_kernel(double* __restrict__ C,
+                                                                       const double* __restrict__ partial, int64_t n,
+                                                                       int nlayers) {
+    gdouble* c = (gdouble*)C;
+    gcdouble* p = (gcdouble*)partial;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t x = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; x < n; x += stride) {
+        double acc = __builtin_nontemporal_load(c + x);
+        for (int l = 0; l < nlayers; ++l) acc += __builtin_nontemporal_load(p + (int64_t)l * n + x);
+        __builtin_nontemporal_store(acc, c + x);
+    }
+}
+constexpr double kSingleBytes = 600e6;  // of C and the layers; the two cross there (25000001 elements, two layers)
 
 int check_offsets(const char* who, const int64_t* off, int parts, int64_t total) {
     if (!off) return fail(DG_ERR_INVALID, "%s: null offsets", who);
@@ -454,9 +472,10 @@ int dg_layer_reduce(double* C, const double* partial, int64_t n, int nlayers, vo
         return fail(DG_ERR_INVALID, "dg_layer_reduce: buffers must be 16-byte aligned");
     int rc = require_device();
     if (rc) return rc;
-    hipLaunchKernelGGL((n & 1) ? layer_reduce_kernel<true> : layer_reduce_kernel<false>,
-                       dim3(looped_blocks((n + 1) / 2, kThreads)), dim3(kThreads), 0, as_stream(stream), C, partial, n,
-                       nlayers);
+    const bool single = (n & 1) && nlayers <= 3 && 8.0 * (double)n * (nlayers + 1) > kSingleBytes;
+    const auto kernel = single ? layer_reduce_single_kernel : (n & 1) ? layer_reduce_kernel<true> : layer_reduce_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3(looped_blocks(single ? n : (n + 1) / 2, kThreads)), dim3(kThreads), 0,
+                       as_stream(stream), C, partial, n, nlayers);
     DG_LAUNCH_CHECK();
     return DG_OK;
 }
