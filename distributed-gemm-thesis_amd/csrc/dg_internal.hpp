@@ -203,32 +203,46 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector
 bool same_lists(const GemmBatch& a, const GemmBatch& b);
 
 // Times the scheduling modes of each tile choice in `choices` and keeps the
-// fastest: trial(choice, mode, &ms) runs one and returns a status.  The middle
-// of three runs counts (some variants have a fast and a slow state, and their
-// best run says little about the next: 4 x 2048^3 on 64x64 tiles, 0.92 and
-// 0.97 ms); a variant whose first run is already a twentieth and 0.2 ms slower
-// than the best so far gets no second one.
+// fastest: trial(choice, mode, &ms) runs one and returns a status.  Every
+// variant runs once before any is timed, because a cold run takes up to 1.34
+// times the steady time (the 7 x 5 batch of 5000 with 256 products: 6.1 against
+// 5.5 ms for its best variant); what is then half as slow again as the least
+// drops out.  The others, the least first, run up to three times in a row.
+// The first run after another variant's is slower too (0.61 against 0.58 ms for
+// a batch of 2100 with 40 products): a fifth behind the best so far ends a
+// variant there, 3 % after two runs.  Of three the middle one counts: some
+// variants have a fast and a slow state, and their best run says little about
+// the next (4 x 2048^3 on 64x64 tiles, 0.92 and 0.97 ms).
 template <class F>
 int fastest_variant(const std::vector<int>& choices, const F& trial, int* choice, int* mode) {
-    float best = 1e30f;
+    struct Variant { int choice, mode; float cold; };
+    std::vector<Variant> all;
     for (int c : choices)
         for (int v : {(int)DG_GEMM_MODE_XCD, (int)DG_GEMM_MODE_ROUND_ROBIN, (int)DG_GEMM_MODE_PERSISTENT}) {
-            float ms[3];
-            int runs = 0;
-            while (runs < 3) {
-                const int rc = trial(c, v, &ms[runs]);
-                if (rc) return rc;
-                ++runs;
-                if (runs == 1 && ms[0] > 1.05f * best && ms[0] > best + 0.2f) break;
-            }
-            if (runs < 3) continue;
-            std::sort(ms, ms + 3);
-            if (ms[1] < best) {
-                best = ms[1];
-                *choice = c;
-                *mode = v;
-            }
+            float ms = 0.f;
+            const int rc = trial(c, v, &ms);
+            if (rc) return rc;
+            all.push_back({c, v, ms});
         }
+    std::stable_sort(all.begin(), all.end(), [](const Variant& a, const Variant& b) { return a.cold < b.cold; });
+    float best = 1e30f;
+    for (const Variant& x : all) {
+        if (x.cold > std::max(1.5f * all[0].cold, all[0].cold + 0.2f)) break;
+        const float most[2] = {std::max(1.2f * best, best + 0.05f), std::max(1.03f * best, best + 0.01f)};
+        float ms[3], least = 1e30f;
+        int runs = 0;
+        do {
+            const int rc = trial(x.choice, x.mode, &ms[runs]);
+            if (rc) return rc;
+            least = std::min(least, ms[runs]);
+        } while (++runs < 3 && least <= most[runs - 1]);
+        if (runs < 3) continue;
+        std::sort(ms, ms + 3);
+        if (ms[1] >= best) continue;
+        best = ms[1];
+        *choice = x.choice;
+        *mode = x.mode;
+    }
     return DG_OK;
 }
 
