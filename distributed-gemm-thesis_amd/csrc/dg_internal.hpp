@@ -203,46 +203,39 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector
 bool same_lists(const GemmBatch& a, const GemmBatch& b);
 
 // Times the scheduling modes of each tile choice in `choices` and keeps the
-// fastest: trial(choice, mode, &ms) runs one and returns a status.  Every
-// variant runs once before any is timed, because a cold run takes up to 1.34
-// times the steady time (the 7 x 5 batch of 5000 with 256 products: 6.1 against
-// 5.5 ms for its best variant); what is then half as slow again as the least
-// drops out.  The others, the least first, run up to three times in a row.
-// The first run after another variant's is slower too (0.61 against 0.58 ms for
-// a batch of 2100 with 40 products): a fifth behind the best so far ends a
-// variant there, 3 % after two runs.  Of three the middle one counts: some
-// variants have a fast and a slow state, and their best run says little about
-// the next (4 x 2048^3 on 64x64 tiles, 0.92 and 0.97 ms).
+// fastest: trial(choice, mode, &ms) runs one and returns a status.  The
+// variants run in turn, in rounds, because the clock moves by a tenth during
+// the first 60 ms of load.  The first round's runs are cold, up to 1.34 times
+// the steady time (a process's very first one more, it loads the code: run
+// twice); only what is half as slow again as the least drops out.  After the
+// second round, what is a tenth slower.  Two rounds of two runs then decide:
+// the first run after another variant's finds the caches as that one left
+// them (0.61 to 0.65 against 0.58 ms for a batch of 2100 with 40 products), so
+// the second one counts.
 template <class F>
 int fastest_variant(const std::vector<int>& choices, const F& trial, int* choice, int* mode) {
-    struct Variant { int choice, mode; float cold; };
-    std::vector<Variant> all;
+    struct Variant { int choice, mode; float sum, ms; };
+    std::vector<Variant> in;
     for (int c : choices)
-        for (int v : {(int)DG_GEMM_MODE_XCD, (int)DG_GEMM_MODE_ROUND_ROBIN, (int)DG_GEMM_MODE_PERSISTENT}) {
-            float ms = 0.f;
-            const int rc = trial(c, v, &ms);
-            if (rc) return rc;
-            all.push_back({c, v, ms});
+        for (int v : {(int)DG_GEMM_MODE_XCD, (int)DG_GEMM_MODE_ROUND_ROBIN, (int)DG_GEMM_MODE_PERSISTENT})
+            in.push_back({c, v, 0.f, 0.f});
+    const struct { int runs; float factor, gap; } rounds[4] = {{1, 1.5f, 0.2f}, {1, 1.1f, 0.03f}, {2, 1.05f, 0.02f}, {2, 1e30f, 0.f}};
+    for (int r = 0; r < 4; ++r) {
+        float least = 1e30f;
+        for (Variant& x : in) {
+            for (int n = r == 0 && &x == &in[0] ? 2 : rounds[r].runs; n > 0; --n) {
+                const int rc = trial(x.choice, x.mode, &x.ms);
+                if (rc) return rc;
+            }
+            if (r >= 2) x.sum += x.ms;
+            least = std::min(least, x.ms);
         }
-    std::stable_sort(all.begin(), all.end(), [](const Variant& a, const Variant& b) { return a.cold < b.cold; });
-    float best = 1e30f;
-    for (const Variant& x : all) {
-        if (x.cold > std::max(1.5f * all[0].cold, all[0].cold + 0.2f)) break;
-        const float most[2] = {std::max(1.2f * best, best + 0.05f), std::max(1.03f * best, best + 0.01f)};
-        float ms[3], least = 1e30f;
-        int runs = 0;
-        do {
-            const int rc = trial(x.choice, x.mode, &ms[runs]);
-            if (rc) return rc;
-            least = std::min(least, ms[runs]);
-        } while (++runs < 3 && least <= most[runs - 1]);
-        if (runs < 3) continue;
-        std::sort(ms, ms + 3);
-        if (ms[1] >= best) continue;
-        best = ms[1];
-        *choice = x.choice;
-        *mode = x.mode;
+        const float most = std::max(rounds[r].factor * least, least + rounds[r].gap);
+        in.erase(std::remove_if(in.begin(), in.end(), [&](const Variant& x) { return x.ms > most; }), in.end());
     }
+    const Variant best = *std::min_element(in.begin(), in.end(), [](const Variant& a, const Variant& b) { return a.sum < b.sum; });
+    *choice = best.choice;
+    *mode = best.mode;
     return DG_OK;
 }
 
