@@ -159,6 +159,14 @@ enum {
 // anything else.
 int forced_tile();
 
+// Whether an FP32 product of m rows on the register-staged kernels runs
+// sgemm_short_kernel: K less than one 32-deep stage of sgemm_kernel, or less
+// than two with few rows in tiles that are not whole.  Share of sgemm_kernel's
+// time over 15 outputs in all layouts: K = 1 0.73, 8 0.81, 16 0.80, none above
+// 1.04; K = 32 0.90, but 130 x 60000 1.07 and 2000 x 2001 1.04; 37 x 400000 x 48
+// 0.56.
+inline bool sgemm_is_short(int64_t m, int64_t k) { return k < 32 || (k < 64 && m < 128 && m % 64); }
+
 // Launches the FP64 MFMA GEMM over `probs` (host vector; uploaded through
 // the table cache).  All problems share opA/opB.
 int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs, std::vector<Seg> segs, hipStream_t stream,

@@ -170,7 +170,7 @@ struct SgemmArgs {
     float alpha, beta;
     int tiles_m, tiles_n;
     int cvec;  // C 16-byte aligned with ldc % 4 == 0: vector stores
-    int by_elements;  // sgemm_kernel: operands that Staged::read does not take
+    int by_elements;  // register-staged kernels: operands that Staged::read does not take
 };
 
 __device__ __forceinline__ int xcd_remap(int bid, int total) {
@@ -760,6 +760,120 @@ __global__ __launch_bounds__(256, C::OCC) void sgemm_kernel(SgemmArgs P) {
         }
 }
 
+// Products of short K (sgemm_is_short): bound by C and by the latency of a
+// tile's chain of loads, LDS and stores.  64x64 tiles, 16 k at a time through
+// one LDS buffer and 62 VGPRs, so that eight workgroups share a CU (four of
+// sgemm_kernel do), and C goes through LDS, so that a wave stores (and reads,
+// beta != 0) 64 rows of a column at a time instead of single elements 16 bytes
+// apart where a tile is not whole.  The sums are sgemm_kernel's, bit for bit.
+// NT, us (sgemm_kernel, this one, and the FMA kernel before both): 37 x 400000
+// x 4 59.0, 26.0, 24.6; 103 x 100000 x 8 with beta = 1 42.7, 20.7, 34.1; 4001 x
+// 4003 x 8 27.8, 20.0, 24.1.  The old C requested before the products instead
+// of after them takes 80 VGPRs, six workgroups, and 1 to 4 % longer.
+struct SgemmShort {
+    static constexpr int T = 64, BK = 16, F = 2;
+};
+
+template <bool AK, bool BKC>
+__global__ __launch_bounds__(256, 8) void sgemm_short_kernel(SgemmArgs P) {
+    constexpr int T = SgemmShort::T, BK = SgemmShort::BK, F = SgemmShort::F, LC = T + 4;
+    using OA = Staged<float, AK, T, BK>;
+    using OB = Staged<float, BKC, T, BK>;
+    constexpr int STAGE = OA::BYTES + OB::BYTES, TILE = T * LC * 4;
+    __shared__ __attribute__((aligned(16))) char lds[STAGE > TILE ? STAGE : TILE];
+    const int64_t bid = blockIdx.x + (int64_t)blockIdx.y * gridDim.x;
+    if (bid >= P.tiles_m * P.tiles_n) return;
+    const int tile = xcd_remap((int)bid, P.tiles_m * P.tiles_n);
+    const int per_group = sk::GROUP_M * P.tiles_n;
+    const int group = tile / per_group;
+    const int first_m = group * sk::GROUP_M;
+    const int gsize = min(P.tiles_m - first_m, sk::GROUP_M);
+    const int in_group = tile - group * per_group;
+    const int64_t m0 = (int64_t)(first_m + in_group % gsize) * T;
+    const int64_t n0 = (int64_t)(in_group / gsize) * T;
+    const int rows = (int)min(P.m - m0, (int64_t)T), cols = (int)min(P.n - n0, (int64_t)T);
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
+    const int lr = lane & 15, lg = lane >> 4;
+
+    OA oa;
+    OB ob;
+    oa.start(P.a, P.lda, m0, rows);
+    ob.start(P.b, P.ldb, n0, cols);
+    int64_t left = P.k;
+    const int last = (AK || rows == T) && (BKC || cols == T) ? 0 : 1;
+    fv4 va[OA::NL], vb[OB::NL];
+    auto read = [&]() {
+        if (!P.by_elements && left >= BK + last) {
+            oa.read(va);
+            ob.read(vb);
+        } else {
+            const int real = (int)min(left, (int64_t)BK);
+            oa.read_last(va, real, rows);
+            ob.read_last(vb, real, cols);
+        }
+        left -= BK;
+    };
+    read();
+    fv4 acc[F][F];
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = fv4{0.f, 0.f, 0.f, 0.f};
+    while (true) {
+        OA::store(lds, va);
+        OB::store(lds + OA::BYTES, vb);
+        __syncthreads();
+        const bool more = left > 0;
+        if (more) read();
+        float fa[F][4], fb[F][4];
+        staged_fragments<OA, AK>(fa, lds, wm, lr, lg, 0);
+        staged_fragments<OB, BKC>(fb, lds + OA::BYTES, wn, lr, lg, 0);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < F; ++i)
+#pragma unroll
+                for (int j = 0; j < F; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[i][q], fb[j][q], acc[i][j], 0, 0, 0);
+        __syncthreads();
+        if (!more) break;
+    }
+    // this thread's elements of C: row `lane` of every fourth column
+    typedef __attribute__((address_space(1))) float gf;
+    float* const c = P.c + m0 + n0 * P.ldc;
+    const uint32_t row = min(lane, rows - 1);
+    const float alpha = P.alpha, beta = P.beta;
+    float old[T / 4];
+    if (beta != 0.f) {
+#pragma unroll
+        for (int x = 0; x < T / 4; ++x) old[x] = ((gf*)(c + (int64_t)min(wave + 4 * x, cols - 1) * P.ldc))[row];
+    }
+    // acc[i][j][v] as in sgemm_kernel
+    float* const t = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int j = 0; j < F; ++j)
+#pragma unroll
+        for (int b = 0; b < F; ++b) {
+            const int r = wm + (AK ? 16 * b + 4 * lg : 4 * F * lg + 4 * b), n = wn + (BKC ? 16 * j + lr : F * lr + j);
+            fv4 val;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                if constexpr (AK) val[v] = acc[b][j][v];
+                else val[v] = acc[(4 * b + v) % F][j][(4 * b + v) / F];
+            }
+            *reinterpret_cast<fv4*>(t + n * LC + r) = val;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int x = 0; x < T / 4; ++x) {
+        const int n = wave + 4 * x;
+        float val = alpha * t[n * LC + lane];
+        if (beta != 0.f) val = fmaf(beta, old[x], val);
+        if (lane < rows && n < cols) ((gf*)(c + (int64_t)n * P.ldc))[row] = val;
+    }
+}
+
 __global__ void sgemm_scale_kernel(int64_t m, int64_t n, float beta, float* __restrict__ C, int64_t ldc) {
     const int64_t total = m * n;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
@@ -800,6 +914,14 @@ void launch_sgemm(SgemmArgs a, hipStream_t st) {
     hipLaunchKernelGGL((sgemm_kernel<C, AK, BKC>), tile_grid(a.tiles_m * a.tiles_n), dim3(256), 0, st, a);
 }
 
+template <bool AK, bool BKC>
+void launch_sgemm_short(SgemmArgs a, hipStream_t st) {
+    a.tiles_m = (int)((a.m + SgemmShort::T - 1) / SgemmShort::T);
+    a.tiles_n = (int)((a.n + SgemmShort::T - 1) / SgemmShort::T);
+    a.by_elements = by_elements<SgemmShort, AK, BKC>(a);
+    hipLaunchKernelGGL((sgemm_short_kernel<AK, BKC>), tile_grid(a.tiles_m * a.tiles_n), dim3(256), 0, st, a);
+}
+
 // Time (us) of one launch, to choose between the tiles: the fullest CU's c
 // tiles at the rate that as many reach (eff), plus 4 us of prologue and
 // epilogue per round of `conc` resident tiles.  Measured rates, share of 157.3
@@ -826,7 +948,7 @@ constexpr double kEff64[6] = {0.87, 0.89, 0.90, 0.91, 0.945, 0.915}, kEff32[6] =
 // tiles, into its interior block (register-operand kernel) and strips after
 // it (rows past the interior, then the columns past it beside the interior
 // rows), which the register-staged kernel runs; else whole on the edge kernel.
-// The register-staged kernel takes the others, and those whose estimated time
+// The register-staged kernels take the others, and those whose estimated time
 // on 64x64 or 32x32 tiles is less: 128x128 tiles leave CUs idle until there
 // are a few hundred of them.  Every kernel sums an element in the same order:
 // neither the cut nor the tile changes a result bit.  DG_GEMM_TILE forces a
@@ -846,6 +968,7 @@ void run_sgemm(const SgemmArgs& a, bool dma, hipStream_t st) {
     auto time64 = [&](int64_t m, int64_t n) { return sgemm_time(m, n, a.k, 64, 4, kEff64, el64); };
     auto time32 = [&](int64_t m, int64_t n) { return sgemm_time(m, n, a.k, 32, 4, kEff32, el32); };
     auto staged = [&](const SgemmArgs& p) {
+        if (forced == DG_GEMM_TILE_AUTO && sgemm_is_short(p.m, p.k)) return launch_sgemm_short<AK, BKC>(p, st);
         const bool small = forced == DG_GEMM_TILE_32x32 || (forced != DG_GEMM_TILE_64x64 && time32(p.m, p.n) < time64(p.m, p.n));
         if (small) launch_sgemm<Sgemm32, AK, BKC>(p, st); else launch_sgemm<Sgemm64, AK, BKC>(p, st);
     };

@@ -312,6 +312,19 @@ static void check_grids() {
     }
 }
 
+// Where FP32 products of short K take their own kernel: below one whole
+// 32-deep stage, and with few rows in tiles that are not whole below two.
+static void check_sgemm_short() {
+    for (int64_t m : {1, 37, 64, 103, 128, 4096, 100000})
+        for (int64_t k : {1, 4, 8, 16, 31}) CHECK(dg::sgemm_is_short(m, k));
+    for (int64_t k : {32, 33, 48, 63}) {
+        CHECK(dg::sgemm_is_short(37, k) && dg::sgemm_is_short(103, k));
+        CHECK(!dg::sgemm_is_short(64, k) && !dg::sgemm_is_short(128, k) && !dg::sgemm_is_short(130, k) && !dg::sgemm_is_short(2000, k));
+    }
+    for (int64_t m : {1, 37, 64, 4096})
+        for (int64_t k : {64, 65, 1024}) CHECK(!dg::sgemm_is_short(m, k));
+}
+
 // The lists of one FP64 problem under DG_GEMM_TILE: sizes of the five.
 static void print_lists(char** v) {
     const char oa = v[0][0], ob = v[1][0];
@@ -331,6 +344,7 @@ int main(int argc, char** argv) {
     else if (what == "parts") check_parts();
     else if (what == "long") check_long();
     else if (what == "short") check_short();
+    else if (what == "sgemm_short") check_sgemm_short();
     else if (what == "trials") check_trials();
     else if (what == "grids") check_grids();
     else if (what == "forced") std::printf("%d\n", dg::forced_tile());

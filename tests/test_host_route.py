@@ -62,6 +62,12 @@ def test_short_segments(check):
     check("short")
 
 
+def test_short_fp32_products(check):
+    """FP32 products of short K go to the kernel that is not slower than
+    what they had before the register-staged tiles."""
+    check("sgemm_short")
+
+
 def test_first_use_times_distinct_choices(check):
     """An autotuned plan's first use times each distinct tile choice, and
     what is clearly slower only once."""
