@@ -137,6 +137,13 @@ inline dim3 run_grid(int64_t chunks, unsigned cols) {
     return dim3((unsigned)((chunks + z - 1) / z), cols, (unsigned)z);
 }
 
+// `chunks` run chunks cut into eight ranges, one for each XCD (workgroups go
+// to the XCDs in turn, by their number): a launch of 8 * eighth(chunks)
+// workgroups in x, of which number x takes chunk eighth_chunk(x, eighth(chunks)),
+// if there is one.
+inline uint32_t eighth(uint32_t chunks) { return (chunks + 7) / 8; }
+__host__ __device__ __forceinline__ uint32_t eighth_chunk(uint32_t x, uint32_t per) { return (x & 7) * per + (x >> 3); }
+
 // Tile scheduling of the FP64 GEMM launch.
 enum {
     DG_GEMM_MODE_ROUND_ROBIN = 0,  // tile = workgroup id (tiles dealt round-robin over XCDs)

@@ -183,13 +183,19 @@ struct Cyclic {
 // columns top to bottom (blockIdx.x, blockIdx.z = row block * chunks + chunk,
 // blockIdx.y = column group).  Unpacking in this order, against each rank's
 // local matrix front to back: 5003 x 7001 on 3 x 2 in blocks of 128 x 96
-// 110 -> 106 us, 11003 x 12000 on 3 x 4 in 32 x 32 913 -> 806 us, 16384^2 on
-// 4 x 4 in 512 x 512 649 -> 651 us.
+// 110 -> 106 us, 16384^2 on 4 x 4 in 512 x 512 649 -> 651 us.
+// Unpacking row blocks of 16 to 32, of which most lines hold parts of two,
+// each XCD takes an eighth of the column (per_xcd, of eighth()), so that both
+// parts of a line meet in one L2: written from two XCDs a little apart they
+// cost more than far apart, as in the packed order.  12288 x 7168 on 2 x 2 in
+// 16 x 64, ldg 12291: 512 us (block by block over the XCDs 810, packed order
+// 590); over 1368 unpackings of such blocks 0.86 of the time on average, 0.66 of
+// the packed order's.  Blocks of 48 and more gain nothing, those of 8 lose 2 %.
 template <bool PACK, bool LINES>
 __global__ __launch_bounds__(kThreads) void cyclic_kernel(const double* __restrict__ src, double* __restrict__ dst,
-                                                          Cyclic g, int lanes_log2) {
+                                                          Cyclic g, int lanes_log2, uint32_t per_xcd) {
     const uint32_t chunk = 2u << lanes_log2;
-    const uint32_t x = blockIdx.z * gridDim.x + blockIdx.x;
+    const uint32_t x = !PACK && !LINES && per_xcd ? eighth_chunk(blockIdx.x, per_xcd) : blockIdx.z * gridDim.x + blockIdx.x;
     const uint32_t blk = fdiv(x, g.dchunks);
     const uint32_t q0 = (x - blk * g.dchunks.d) * chunk;  // first row of the chunk within its row block
     const int lane = threadIdx.x & ((1 << lanes_log2) - 1);
@@ -353,10 +359,12 @@ int cyclic(const char* who, const double* src, double* dst, int64_t ldg, int64_t
     g.dchunks = make_fastdiv((uint32_t)rs.chunks);
     const int64_t row_blocks = (rows + mb - 1) / mb;
     if (row_blocks > INT32_MAX / rs.chunks) return fail(DG_ERR_INVALID, "%s: too many row chunks", who);
-    const dim3 grid = run_grid(row_blocks * rs.chunks, col_groups(cols, rs.cols_per_wg));
+    dim3 grid = run_grid(row_blocks * rs.chunks, col_groups(cols, rs.cols_per_wg));
     const bool lines = whole_lines(src, dst, 8 * (ldg | rows | std::min(mb, rows)));
+    const uint32_t per_xcd = !PACK && !lines && mb >= 16 && mb <= 32 && grid.z == 1 ? eighth(grid.x) : 0;
+    if (per_xcd) grid.x = 8 * per_xcd;
     const auto kernel = lines ? cyclic_kernel<PACK, true> : cyclic_kernel<PACK, false>;
-    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, as_stream(stream), src, dst, g, rs.lanes_log2);
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, as_stream(stream), src, dst, g, rs.lanes_log2, per_xcd);
     DG_LAUNCH_CHECK();
     return DG_OK;
 }

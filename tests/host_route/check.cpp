@@ -310,6 +310,20 @@ static void check_grids() {
         CHECK((int64_t)g.x * 64 < (int64_t)1 << 32 && g.y == 7 && g.z < 65536);
         CHECK((int64_t)g.x * g.z >= chunks && (int64_t)g.x * (g.z - 1) < chunks);
     }
+    // eight ranges: every chunk once, neighbours on one XCD (workgroup number modulo 8) but at the seams
+    for (uint32_t chunks : {1u, 2u, 7u, 8u, 9u, 15u, 64u, 313u, 768u, 100001u}) {
+        const uint32_t per = dg::eighth(chunks);
+        CHECK(8 * per >= chunks && 8 * per < chunks + 8);
+        std::vector<int> xcd(8 * per, -1);
+        for (uint32_t x = 0; x < 8 * per; ++x) {
+            const uint32_t c = dg::eighth_chunk(x, per);
+            CHECK(c < 8 * per && xcd[c] < 0);
+            xcd[c] = x % 8;
+        }
+        int seams = 0;
+        for (uint32_t c = 1; c < 8 * per; ++c) seams += xcd[c] != xcd[c - 1];
+        CHECK(seams == 7);
+    }
 }
 
 // Where FP32 products of short K take their own kernel: below one whole
