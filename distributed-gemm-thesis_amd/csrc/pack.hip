@@ -92,9 +92,10 @@ unsigned col_groups(int64_t cols, int cols_per_wg) {
     return (unsigned)(g < 1 ? 1 : g);
 }
 
-// Whether two addresses and a length in bytes are whole lines.
-bool whole_lines(const void* a, const void* b, int64_t bytes) {
-    return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)bytes) & 127) == 0;
+// Whether two addresses and a length in bytes are whole lines (or parts of
+// `unit` bytes).
+bool whole_lines(const void* a, const void* b, int64_t bytes, int unit = 128) {
+    return (((uintptr_t)a | (uintptr_t)b | (uintptr_t)bytes) & (unit - 1)) == 0;
 }
 
 struct Bands {
@@ -360,7 +361,10 @@ int cyclic(const char* who, const double* src, double* dst, int64_t ldg, int64_t
     const int64_t row_blocks = (rows + mb - 1) / mb;
     if (row_blocks > INT32_MAX / rs.chunks) return fail(DG_ERR_INVALID, "%s: too many row chunks", who);
     dim3 grid = run_grid(row_blocks * rs.chunks, col_groups(cols, rs.cols_per_wg));
-    const bool lines = whole_lines(src, dst, 8 * (ldg | rows | std::min(mb, rows)));
+    bool lines = whole_lines(src, dst, 8 * (ldg | rows | std::min(mb, rows)));
+    // packed runs of half a line each want the hint too (12288 x 7168 in 8 x 64:
+    // 618 us without, 594 with it; runs of three halves lose 8 % with it)
+    if (PACK && mb == 8) lines = whole_lines(src, dst, 8 * (ldg | rows), 64);
     const uint32_t per_xcd = !PACK && !lines && mb >= 16 && mb <= 32 && grid.z == 1 ? eighth(grid.x) : 0;
     if (per_xcd) grid.x = 8 * per_xcd;
     const auto kernel = lines ? cyclic_kernel<PACK, true> : cyclic_kernel<PACK, false>;
