@@ -191,7 +191,8 @@ struct Cyclic {
 // cost more than far apart, as in the packed order.  12288 x 7168 on 2 x 2 in
 // 16 x 64, ldg 12291: 512 us (block by block over the XCDs 810, packed order
 // 590); over 1368 unpackings of such blocks 0.86 of the time on average, 0.66 of
-// the packed order's.  Blocks of 48 and more gain nothing, those of 8 lose 2 %.
+// the packed order's.  Blocks of 48 and more gain nothing, those of 8 lose 2 %,
+// and those that share no half line 3 to 5 %.
 template <bool PACK, bool LINES>
 __global__ __launch_bounds__(kThreads) void cyclic_kernel(const double* __restrict__ src, double* __restrict__ dst,
                                                           Cyclic g, int lanes_log2, uint32_t per_xcd) {
@@ -365,7 +366,8 @@ int cyclic(const char* who, const double* src, double* dst, int64_t ldg, int64_t
     // packed runs of half a line each want the hint too (12288 x 7168 in 8 x 64:
     // 618 us without, 594 with it; runs of three halves lose 8 % with it)
     if (PACK && mb == 8) lines = whole_lines(src, dst, 8 * (ldg | rows), 64);
-    const uint32_t per_xcd = !PACK && !lines && mb >= 16 && mb <= 32 && grid.z == 1 ? eighth(grid.x) : 0;
+    const bool halves = whole_lines(dst, dst, 8 * (ldg | mb), 64);
+    const uint32_t per_xcd = !PACK && !halves && mb >= 16 && mb <= 32 && grid.z == 1 ? eighth(grid.x) : 0;
     if (per_xcd) grid.x = 8 * per_xcd;
     const auto kernel = lines ? cyclic_kernel<PACK, true> : cyclic_kernel<PACK, false>;
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, as_stream(stream), src, dst, g, rs.lanes_log2, per_xcd);
