@@ -218,39 +218,33 @@ int prepare_gemm(char opA, char opB, const std::vector<Prob>& probs, std::vector
 bool same_lists(const GemmBatch& a, const GemmBatch& b);
 
 // Times the scheduling modes of each tile choice in `choices` and keeps the
-// fastest: trial(choice, mode, &ms) runs one and returns a status.  The
-// variants run in turn, in rounds, because the clock moves by a tenth during
-// the first 60 ms of load.  The first round's runs are cold, up to 1.34 times
-// the steady time (a process's very first one more, it loads the code: run
-// twice); only what is half as slow again as the least drops out.  After the
-// second round, what is a tenth slower.  Two rounds of two runs then decide:
-// the first run after another variant's finds the caches as that one left
-// them (0.61 to 0.65 against 0.58 ms for a batch of 2100 with 40 products), so
-// the second one counts.
+// fastest: trial(choice, mode, &ms) runs one and returns a status.  The best of
+// three runs in a row counts.  A variant's first run is cold (up to 1.34 times
+// its steady time: the 7 x 5 batch of 5000 with 256 products, 6.1 against 5.5 ms
+// for its best variant), so only one that is half as slow again as the best so
+// far, and 0.2 ms, ends there.  25 batches in four processes each: the choice is
+// 0.7 % behind the best one on average (0.8 % with three runs of all); taking turns
+// in rounds, with the second run of a pair or the settled run of up to eight
+// counting, came out 1.3 to 1.4 % behind.
 template <class F>
 int fastest_variant(const std::vector<int>& choices, const F& trial, int* choice, int* mode) {
-    struct Variant { int choice, mode; float sum, ms; };
-    std::vector<Variant> in;
+    float best = 1e30f;
     for (int c : choices)
-        for (int v : {(int)DG_GEMM_MODE_XCD, (int)DG_GEMM_MODE_ROUND_ROBIN, (int)DG_GEMM_MODE_PERSISTENT})
-            in.push_back({c, v, 0.f, 0.f});
-    const struct { int runs; float factor, gap; } rounds[4] = {{1, 1.5f, 0.2f}, {1, 1.1f, 0.03f}, {2, 1.05f, 0.02f}, {2, 1e30f, 0.f}};
-    for (int r = 0; r < 4; ++r) {
-        float least = 1e30f;
-        for (Variant& x : in) {
-            for (int n = r == 0 && &x == &in[0] ? 2 : rounds[r].runs; n > 0; --n) {
-                const int rc = trial(x.choice, x.mode, &x.ms);
+        for (int v : {(int)DG_GEMM_MODE_XCD, (int)DG_GEMM_MODE_ROUND_ROBIN, (int)DG_GEMM_MODE_PERSISTENT}) {
+            float least = 1e30f;
+            for (int run = 0; run < 3; ++run) {
+                float ms = 0.f;
+                const int rc = trial(c, v, &ms);
                 if (rc) return rc;
+                least = std::min(least, ms);
+                if (least > std::max(1.5f * best, best + 0.2f)) break;
             }
-            if (r >= 2) x.sum += x.ms;
-            least = std::min(least, x.ms);
+            if (least < best) {
+                best = least;
+                *choice = c;
+                *mode = v;
+            }
         }
-        const float most = std::max(rounds[r].factor * least, least + rounds[r].gap);
-        in.erase(std::remove_if(in.begin(), in.end(), [&](const Variant& x) { return x.ms > most; }), in.end());
-    }
-    const Variant best = *std::min_element(in.begin(), in.end(), [](const Variant& a, const Variant& b) { return a.sum < b.sum; });
-    *choice = best.choice;
-    *mode = best.mode;
     return DG_OK;
 }
 
