@@ -191,7 +191,10 @@ int launch_gemm_f64(char opA, char opB, const std::vector<Prob>& probs, std::vec
 // the work is padding (DG_GEMM_TILE forces a choice, DG_GEMM_NO_DMA routes
 // everything to the register-staged kernel).  Every kernel and tile sums an
 // element in the same order, so a problem gives the same bits alone, in any
-// batch and on any tile.
+// batch and on any tile, with one exception: a sum of -0 (negative products
+// that all underflow) comes out +0 where zeros follow it.  Each segment's k is
+// padded with them to whole stages, 8 deep in the direct-to-LDS kernels, 16 on
+// 128x128 and 64x64 tiles and 32 on 32x32 ones, and the tile depends on the batch.
 // Direct-to-LDS problems whose tiles are all interior (no row shift, m and n
 // multiples of 128, whole k-steps, an even step count) go to `dma`, which
 // the A-in-registers kernel runs; the others go to `dmae` (the edge-handling

@@ -37,7 +37,8 @@
 // leading dimensions not multiples of 4, K % 4 != 0 with a k-contiguous
 // operand), strips, products too small to fill the chip with 128x128 tiles,
 // and long-K products of any size (run_sgemm chooses; all kernels give the
-// same bits).  TFLOP/s before (FMA kernel without matrix cores, or 128x128
+// same bits, but for the sign of a sum of -0 where a kernel pads K with zeros,
+// to 16 with direct loads, 32 on 64x64 tiles and 64 on 32x32 ones).  TFLOP/s before (FMA kernel without matrix cores, or 128x128
 // tiles) and after: 4001^3 38.8 -> 136.5, 1537 x 2051 x 1023 28.5 -> 93.8, 512^3
 // 7.7 -> 36.7, 1024^3 31.5 -> 90, 3072^3 105.9 -> 142.8, 4096^3 142.2 -> 146.1.
 //
@@ -522,7 +523,7 @@ __global__ __launch_bounds__(256, 2) void sgemm_dma_xr_kernel(SgemmArgs P) {
 // MFMA: 1024 x 1024 x 8192, one tile per CU, 147 -> 129 us, 2048^3 127 -> 124).  The k order of an element
 // is sgemm_dma_kernel's: lane group lg supplies k = 4lg + s of a 16-deep step
 // to MFMA s, A the first operand, so the tile choice changes no bit (but the
-// sign of an exactly zero sum).
+// sign of a sum of -0).
 // A row-contiguous operand's block row r stands for row F*r + i of block i, so
 // that a lane's rows of all F blocks are one LDS read.
 template <int T_, int BK_, int OCC_>
@@ -1040,6 +1041,7 @@ extern "C" int dg_sgemm(char opA, char opB, int64_t m, int64_t n, int64_t k, flo
     if (!A || !B) return fail(DG_ERR_INVALID, "dg_sgemm: null matrix pointer");
     const bool ak = oa == 'T', bkc = ob == 'N';  // operands stored contiguous along k
     const int64_t tm = (m + sk::BM - 1) / sk::BM, tn = (n + sk::BN - 1) / sk::BN;
+    // part of the interface, not of the grids: every tile count fits those
     if (tm * tn > INT32_MAX || (m + 63) / 64 > INT32_MAX || (n + 63) / 64 > 65535)
         return fail(DG_ERR_INVALID, "dg_sgemm: %lld x %lld output is too large", (long long)m, (long long)n);
     SgemmArgs a{A, B, C, lda, ldb, ldc, m, n, k, alpha, beta, 0, 0, 0, 0};

@@ -1,8 +1,8 @@
 // FP64 GEMM on the CDNA4 matrix cores (v_mfma_f64_16x16x4_f64), grouped over
 // problems and segmented along K.
 //
-// One launch computes every 128x128 output tile of every problem in the
-// problem table.  A problem is C = alpha * sum_s opA(seg s) * opB(seg s)
+// One launch computes every output tile of every problem in its problem
+// table.  A problem is C = alpha * sum_s opA(seg s) * opB(seg s)
 // + beta*C, where segment s supplies its own A/B base pointers and leading
 // dimensions.  A plain DGEMM is one problem with one segment; a virtual-grid
 // Cannon rank is one problem whose segments are the tiles the rotations
@@ -13,15 +13,16 @@
 // whose 128x128 tiles are all interior run gemm_f64_dma_ar_kernel (A straight
 // into registers, B direct to LDS); the others that take direct loads run
 // gemm_f64_dma_kernel (both operands direct to LDS); both are described below.
-// gemm_f64_kernel takes everything else on 64x64 or 32x32 tiles: operands that
-// direct loads do not take (odd leading dimensions, odd K), strips cut off
-// uneven problems, and batches too small to fill the chip with 128x128 tiles
-// (prepare_gemm chooses).  It stages both operands through registers into a
-// double-buffered LDS; four waves a workgroup, each owning a quarter of the
-// tile.
+// gemm_f64_kernel takes everything else, on 128x128, 64x64 or 32x32 tiles:
+// operands that direct loads do not take (odd leading dimensions, odd K),
+// strips cut off uneven problems, and what it is estimated to run faster, such
+// as products with few 128x128 tiles per CU (prepare_gemm chooses; a single
+// problem goes to gemm_f64_one_kernel, the same code).  It stages both
+// operands through registers into a double-buffered LDS; four waves a
+// workgroup, each owning a quarter of the tile.
 // What bounds it: the FP64 MFMA (64 cycles each, on the vector ALU's pipes).
 // Measured (TFLOP/s, against the 128x128 tiles and guarded loads before):
-// 512^3 3.8 -> 28.9 (32x32 tiles; 70 -> 9.3 us), 1024^3 16.6 -> 50.4, 2000^3
+// 512^3 3.8 -> 32.1 (32x32 tiles; 70 -> 8.4 us), 1024^3 16.6 -> 50.4, 2000^3
 // 32.8 -> 65.9, 3072^3 55.3 -> 70.9, 4097^3 (odd leading dimensions) 48.6 ->
 // 64.4, TN 1500 x 1333 x 2001 22.7 -> 61.8.
 // Lane l of an MFMA supplies k = 2*(l/16) + q to sub-step q for both operands,
@@ -31,7 +32,6 @@
 // Result layout of v_mfma_f64_16x16x4_f64: lane l, register v holds
 // D(l/16 + 4v, l%16) (checked on the device by the exact-integer tests).
 #include <algorithm>
-#include <string>
 
 #include "dg_internal.hpp"
 #include "staged.hpp"
@@ -62,6 +62,9 @@ struct TileCfg {
     static constexpr int FM = WM / 16, FN = WN / 16;
     static_assert((BM / WM) * (BN / WN) * 64 == NTH, "one wave per WM x WN sub-tile");
 };
+// The 128x128 kernels fill their 256 VGPRs and spill 4 to 13 values of the
+// code around the steady turns (the last stages' addresses, the epilogue),
+// the 64x64 walks of NN two; no steady turn touches scratch.
 using Cfg128 = TileCfg<128, 128, 64, 64, 16, 1, 2>;
 using Cfg64 = TileCfg<64, 64, 32, 32, 16, 2, 4>;
 using Cfg32 = TileCfg<32, 32, 16, 16, 32, 2, 3>;
@@ -193,7 +196,7 @@ __device__ __forceinline__ void gemm_tile(const Prob& P, const Seg* __restrict__
     // summed in their order: lane group lg supplies k = 8h + 2lg + q to MFMA q,
     // so every element takes the same sequence of MFMAs in all FP64 kernels
     // and a problem cut between them, or run on other tiles, gives the same
-    // bits (but for the sign of an exactly zero sum when K leaves this kernel
+    // bits (but for the sign of a sum of -0 when K leaves this kernel
     // zero-padded parts).
     // A part's fragments are read while the part before it is multiplied, the
     // first part's of stage s + 1 during the last part of stage s: the stage's
@@ -364,7 +367,8 @@ __device__ __forceinline__ void walk_xcd(int total_tiles, const F& run) {
 }
 
 // MODE 0: one workgroup per tile, tile = blockIdx.x (round-robin over XCDs);
-// MODE 1: one workgroup per tile, XCD-contiguous tile ranges (xcd_remap);
+// MODE 1: XCD-contiguous tile ranges (walk_xcd), a workgroup per tile or
+//         fewer that walk several (xcd_grid);
 // MODE 2: persistent: every workgroup takes tiles from `counter` (zeroed
 //         before the launch) until the tile space is exhausted.
 template <class C, bool TA, bool TB, int MODE>
@@ -403,8 +407,8 @@ __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_kernel(const Prob* __
 // One problem of one segment, passed by value: nothing is uploaded on the
 // first call with new buffers, and a workgroup's first loads wait on no table
 // reads (512^3: 9.3 -> 8.4 us a call, 7.9 of them on the GPU).  One workgroup
-// per tile, XCD-contiguous ranges; the walk of several tiles per workgroup
-// would spill registers here and stays with the tables.
+// per tile, XCD-contiguous ranges; problems whose tiles are walked several per
+// workgroup (xcd_grid) stay with the tables.
 template <class C, bool TA, bool TB>
 __global__ __launch_bounds__(C::NTH, C::OCC) void gemm_f64_one_kernel(Prob P, Seg S) {
     __shared__ __attribute__((aligned(16))) char lds[2 * TileLds<C, TA, TB>::STAGE];
@@ -1129,10 +1133,10 @@ static_assert(dmak::DBM == 128 && dmak::DBN == 128 && Cfg128::BM == 128 && Cfg64
 // first, per round of `conc` resident tiles.
 // Measured: A in registers 0.91 with one tile per CU, 0.95 with more (both
 // operands in LDS 0.85, 0.93); register-staged 128x128 0.95 with one, 0.965 up
-// to 15 (4096^3: 1812 us against 1838 with A in registers), then less, 0.89
-// from 32 on: its matrix cores are 99 % busy, but its workgroups drift apart,
-// fetch their operands from beyond the L2 (16384^3: 374 GB against 101) and
-// the clock falls; 64x64 0.92, 0.88 from 25 tiles per CU on, 0.85 from 64 on;
+// to 15 (4096^3: 1816 us against 1836 with A in registers), then less, 0.89
+// from 32 on: its workgroups drift apart and fetch four times as much from
+// beyond the L2 (16384^3: 398 GB against 103), and with 98.5 % busy matrix cores
+// it is no faster than A in registers (116.5 ms both, SUMMA too); 64x64 0.92, 0.88 from 25 tiles per CU on, 0.85 from 64 on;
 // 32x32 0.67, 0.72, 0.76, 0.78 with one to four, 0.80 with more.  Loads by
 // elements: kElementRate of these (TN 500 x 4096 x 4096 with 2^22 + 2 rows to a
 // column, 64x64 tiles: 403 us, 257 with whole runs; NN 4096 x 4096 x 480, odd:

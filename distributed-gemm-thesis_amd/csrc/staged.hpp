@@ -33,8 +33,9 @@ inline dim3 tile_grid(int tiles) {
 // BK-deep stages of ROWS rows for a workgroup of 256 threads, loaded in runs
 // of E elements (16 bytes) at any alignment -- a run per load instead of
 // single elements is what lets odd leading dimensions run like even ones --
-// and stored to LDS in the direction memory has, so that both the stores and
-// the fragment reads are conflict-free.
+// and stored to LDS in the direction memory has, so that the stores and the
+// fragment reads spread over the banks (4096^3 on FP64 128x128 tiles: conflicts
+// in 3 % of a CU's cycles).
 //  * KC, element (row, k) at base[k + row*ld]: a thread takes the run at
 //    k = E*(t % CH) of rows t/CH + RPP*q; LDS [row][k], rows padded by a run.
 //  * else, element (row, k) at base[row + k*ld]: a thread takes the run at row
